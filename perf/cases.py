@@ -108,23 +108,31 @@ class _FeedForward(nn.Module):
         return self.w2(F.silu(self.w1(x)) * self.w3(x))
 
 
-def prepare(case, seed):
+def _made(case, seed):
+    """The model in high precision, its input and, to train, the gradients of its outputs."""
     torch.manual_seed(seed)
     m, k, n, dtype = case["m"], case["k"], case["n"], _DTYPES[case["dtype"]]
     normal = lambda *shape, dt=dtype, std=1.0: torch.empty(shape, device="cuda", dtype=dt).normal_(0.0, std)
     if case["what"] == "infer":
         model = _FeedForward(k, n, case["bias"], dtype) if case["block"] == "ffn" else nn.Linear(k, n, bias=case["bias"], device="cuda", dtype=dtype)
+        return model, normal(m, k), None
+    act = torch.bfloat16 if case["autocast"] else dtype  # what the layers before and after this one hand over
+    model = _Parallel(k, n, case["linears"], case["bias"], dtype)
+    return model, normal(m, k, dt=act), [normal(m, n, dt=act, std=1e-2) for _ in range(case["linears"])]
+
+
+def prepare(case, seed):
+    model, x, dys = _made(case, seed)
+    if case["what"] == "infer":
         if case["casting"] == "static":  # as calibrated on activations that reach about 7
             quant = QuantConfig(ActivationCasting.STATIC, static_quantization_scale=torch.tensor([64.0], device="cuda"))
         else:
             quant = QuantConfig(ActivationCasting.DYNAMIC if case["casting"] == "dynamic" else ActivationCasting.WEIGHT_ONLY)
-        return {"case": case, "model": quantize_to_float8(model, quant), "x": normal(m, k)}
+        return {"case": case, "model": quantize_to_float8(model, quant), "x": x}
     kind = f8.CastConfig(scaling_type=f8.ScalingType.DELAYED if case["scaling"] == "delayed" else f8.ScalingType.DYNAMIC)
     config = f8.Float8LinearConfig(cast_config_input=kind, cast_config_weight=kind, cast_config_grad_output=kind)
-    model = f8.convert_to_float8_training(_Parallel(k, n, case["linears"], case["bias"], dtype), config=config)
-    act = torch.bfloat16 if case["autocast"] else dtype  # what the layers before and after this one hand over
-    state = {"case": case, "model": model, "x": normal(m, k, dt=act).requires_grad_(),
-             "dys": [normal(m, n, dt=act, std=1e-2) for _ in range(case["linears"])]}
+    model = f8.convert_to_float8_training(model, config=config)
+    state = {"case": case, "model": model, "x": x.requires_grad_(), "dys": dys}
     if case["scaling"] == "delayed":
         _step(state)  # the first iteration, which initialises the amaxes, is behind a program that trains
     return state
@@ -190,3 +198,51 @@ def tolerance(case):
             # scaling, may move their scale by one ulp, which rounds a tenth of them the other way (1.5e-2)
             rel, most = (0.02, 0.15) if case["casting"] == "dynamic" and out == "bf16" else (7e-3, 0.06)
     return {"rel": rel, "max": most}
+
+
+def _dequantised(t, kind, scale=None, buffered=False):
+    """t cast to fp8 as the path defines it, and back, in 64 bits: an operand of the exact products.  With the scale in a
+    buffer (delayed, or given beforehand) its arithmetic and the product are in fp32, else in t's own type."""
+    top = torch.finfo(kind).max
+    buffered = buffered or scale is not None
+    if scale is None:
+        amax = t.abs().max()
+        scale = (amax.float() if buffered else amax).clamp(min=1e-12).reciprocal() * top
+        if t.dtype is torch.float16:
+            scale = scale.clamp(max=65504.0)
+        scale = scale.float()
+    product = (t.float() if buffered else t) * scale
+    return product.clamp(-top, top).to(kind).double() / scale.double()
+
+
+def exact(case, seed):
+    """The same outputs with every product of the fp8 operands in 64 bits; None for the buffers of delayed scaling."""
+    model, x, dys = _made(case, seed)
+    e4m3, e5m2 = torch.float8_e4m3fn, torch.float8_e5m2
+    with torch.no_grad():
+        if case["what"] == "infer":
+            def linear(layer, x):
+                if case["casting"] == "weight_only":  # the dequantised weight has the model's type, and no bias is added
+                    return x.double() @ _dequantised(layer.weight, e4m3).to(x.dtype).double().t()
+                static = torch.tensor([64.0], device="cuda") if case["casting"] == "static" else None
+                y = _dequantised(x, e4m3, static) @ _dequantised(layer.weight, e4m3).t()
+                return y if layer.bias is None else y + layer.bias.double()
+
+            if case["block"] != "ffn":
+                return linear(model, x)
+            return linear(model.w2, F.silu(linear(model.w1, x).to(x.dtype)) * linear(model.w3, x).to(x.dtype))
+        delayed = case["scaling"] == "delayed"
+        x8 = _dequantised(x, e4m3, buffered=delayed)
+        ys, dx, grads = [], 0.0, []
+        for layer, dy in zip(model.layers, dys):
+            w8, dy8 = _dequantised(layer.weight, e4m3, buffered=delayed), _dequantised(dy, e5m2, buffered=delayed)
+            y = x8 @ w8.t()
+            ys.append(y if layer.bias is None else y + layer.bias.to(x.dtype).double())
+            dx = dx + dy8 @ w8
+            grads.append(dy8.t() @ x8)
+            if layer.bias is not None:
+                grads.append(dy.double().sum(0))
+        out = {"y": ys, "dx": dx, "grads": grads}
+        if delayed:
+            out["buffers"] = [None] * (9 * case["linears"])
+        return out
