@@ -44,6 +44,8 @@ EXPORTS = (
     "f8mi_delayed_workspace_bytes",
     "f8mi_cast_dynamic",
     "f8mi_cast_dynamic_static",
+    "f8mi_gemm_weight_only",
+    "f8mi_dequant",
     "f8mi_gemm_nt",
     "f8mi_gemm_nt_kb",
     "f8mi_gemm_kb_ex",
@@ -123,6 +125,10 @@ def lib() -> C.CDLL:
         L.f8mi_gemm_plan.argtypes = [i64, i64, i64, i32, i64]
         L.f8mi_gemm_nt_kb_ws.restype = i32
         L.f8mi_gemm_nt_kb_ws.argtypes = [vp, i32, vp, i32, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp, i64, vp]
+        L.f8mi_gemm_weight_only.restype = i32
+        L.f8mi_gemm_weight_only.argtypes = [vp, i64, i32, vp, i32, i64, i64, i64, i64, fp, vp, i64, vp]
+        L.f8mi_dequant.restype = i32
+        L.f8mi_dequant.argtypes = [vp, i32, i64, fp, i32, vp, vp]
         L.f8mi_sync.restype = i32
         L.f8mi_sync.argtypes = [vp, i32, i32, i32, i32, vp]
         L.f8mi_sync_host.restype = i32
@@ -653,6 +659,35 @@ def scaled_mm(a: torch.Tensor, a_scale: torch.Tensor, b: torch.Tensor, b_scale: 
             _check(rc, "f8mi_gemm_ex")
     # the copies: gemm_nt makes an operand contiguous along k when it is not
     return gemm_nt(a, a_scale, b.t(), b_scale, out_dtype, bias=bias)
+
+
+def gemm_weight_only(x: torch.Tensor, w_data: torch.Tensor, w_scale: torch.Tensor) -> torch.Tensor:
+    """``x @ (w_data.to(x.dtype) / w_scale).t()`` for x [m, k] and an fp8 weight [n, k], without the dequantised tensor.
+    See f8mi_gemm_weight_only."""
+    _require_gpu(x, "x")
+    assert x.dim() == 2 and w_data.dim() == 2 and x.shape[1] == w_data.shape[1], f"shape mismatch {tuple(x.shape)} x {tuple(w_data.shape)}^T"
+    assert w_data.is_contiguous() and w_data.device == x.device
+    assert w_scale.dtype == torch.float32 and w_scale.numel() == 1 and w_scale.device == x.device
+    (m, k), n = x.shape, w_data.shape[0]
+    if x.stride(1) != 1 or (m > 1 and x.stride(0) < k):
+        x = x.contiguous()
+    _check_device(x.device)
+    out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    rc = lib().f8mi_gemm_weight_only(x.data_ptr(), x.stride(0) if m > 1 else k, _DT[x.dtype], w_data.data_ptr(), _F8[w_data.dtype], k, m, n, k,
+                                     w_scale.data_ptr(), out.data_ptr(), n, _stream(x))
+    _check(rc, "f8mi_gemm_weight_only")
+    return out
+
+
+def dequant(data: torch.Tensor, scale: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """``data.to(dtype) / scale`` (a 0-dim scale) of a contiguous fp8 tensor in one launch.  See f8mi_dequant."""
+    _require_gpu(data, "data")
+    assert data.is_contiguous() and scale.dtype == torch.float32 and scale.numel() == 1 and scale.device == data.device
+    _check_device(data.device)
+    out = torch.empty(data.shape, dtype=dtype, device=data.device)
+    rc = lib().f8mi_dequant(data.data_ptr(), _F8[data.dtype], data.numel(), scale.data_ptr(), _DT[dtype], out.data_ptr(), _stream(data))
+    _check(rc, "f8mi_dequant")
+    return out
 
 
 def sync_table(entries, device: torch.device) -> torch.Tensor:

@@ -232,6 +232,16 @@ int f8mi_cast_dynamic_static(const void* x, int64_t rows, int64_t cols, int64_t 
                              float* scale_dev, uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout,
                              void* stream);
 
+/* Weight-only inference for few rows: c[m][n] = sum_k x[m][k] * W[n][k] with x, c and W = w / *scale_dev in `dtype`,
+ * the fp8 weight w (rows of ldw bytes) dequantised in registers: the quotient is taken in fp32 and rounded to `dtype`,
+ * as torch divides (the scale rounded to `dtype` before); fp32 accumulation.  Any k >= 1, any alignment of rows to the
+ * element size.  Replaces to_original_precision + linear (reference inference.py:104-107). */
+int f8mi_gemm_weight_only(const void* x, int64_t ldx, int dtype, const uint8_t* w, int fp8_fmt, int64_t ldw, int64_t m,
+                          int64_t n, int64_t k, const float* scale_dev, void* c, int64_t ldc, void* stream);
+/* out[i] = in[i] / *scale_dev in `dtype`, the same quotient, for n consecutive elements (float8_tensor.py:198-212 of the
+ * reference). */
+int f8mi_dequant(const uint8_t* in, int fp8_fmt, int64_t n, const float* scale_dev, int dtype, void* out, void* stream);
+
 /* f8mi_gemm_nt on k-blocked operands: a = [k/64][m][64], bt = [k/64][n][64], both 16-byte
  * aligned.  Needs k % 64 == 0 and k >= 384 (F8MI_ERR_UNSUPPORTED otherwise: keep such operands
  * row-major and call f8mi_gemm_nt).  Same arithmetic, same result bits as f8mi_gemm_nt. */

@@ -232,3 +232,64 @@ def test_fp8_training_then_save_load_then_inference_is_bit_identical(f8, dtype):
     sd = torch.load(buf, weights_only=True)
     assert isinstance(sd["w1.weight"], f8.Float8Tensor)
     assert torch.equal(sd["w1.weight"]._data.view(torch.uint8), new.w1.weight._data.view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("fmt", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_dequant_gives_the_bits_of_the_division(f8, dtype, fmt):
+    """Every code and sizes around the 16-element pieces, over scales whose reciprocal product differs from the quotient
+    for some code, that push codes below the type's normal range, and that are no value of the type."""
+    from float8_experimental_amd import _native
+
+    gen = torch.Generator().manual_seed(3)
+    scales = [1.0, 3.0, 448.0 / 0.0156, 65504.0, 1e-3] + (torch.rand(24, generator=gen) * 1e4).tolist()
+    for i, scale in enumerate(scales):
+        n = (256, 257, 255, 271, 1, 16, 4096 * 3 + 5)[i % 7]
+        data = (torch.arange(n) % 256).to(torch.uint8).to(DEV).view(fmt)
+        s = torch.tensor(scale, device=DEV)
+        want, got = data.to(dtype) / s, _native.dequant(data, s, dtype)
+        assert got.dtype == want.dtype and torch.equal(want.isnan(), got.isnan())
+        assert torch.equal(want.nan_to_num(0.0), got.nan_to_num(0.0)), scale
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(1, 16, 64), (1, 8192, 512), (4, 33, 640), (16, 8208, 1024), (17, 40, 4097), (32, 31, 63), (33, 257, 1),
+                                   (64, 96, 8191), (48, 8193, 192), (64, 12352, 128), (65, 144, 640), (128, 100, 200)])
+def test_weight_only_dequantises_inside_the_product(f8, dtype, m, n, k):
+    """Edges of the row and column tiles (16, 32, 64; 16 and 32 columns), of the 64-deep steps and of their split over the
+    waves; x as a view with a row pitch.  Bound: 2 k roundings of the fp32 sum and one of the output."""
+    from float8_experimental_amd import inference
+
+    torch.manual_seed(m + n + k)
+    lin = torch.nn.Linear(k, n, bias=False, device=DEV, dtype=dtype)
+    lin = inference.quantize_to_float8(lin, inference.QuantConfig(inference.ActivationCasting.WEIGHT_ONLY))
+    x = torch.randn(m, k + 3, device=DEV).to(dtype)[:, :k]
+    with torch.no_grad():
+        assert inference._weight_only_kernels_take(x, lin.weight)
+        got = lin(x)
+    w = (lin.weight._data.to(dtype) / lin.weight._scale).double()
+    want, mag = x.double() @ w.t(), x.double().abs() @ w.abs().t()
+    out_ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
+    tiny = 2.0 ** -24 if dtype is torch.float16 else 0.0
+    assert got.shape == (m, n) and got.dtype == dtype
+    assert ((got.double() - want).abs() <= out_ulp * want.abs() + 2 * k * 2.0 ** -24 * mag + tiny).all()
+    assert not inference._weight_only_kernels_take(x.clone().requires_grad_(), lin.weight)
+
+
+def test_weight_only_leaves_other_calls_to_the_library_product(f8):
+    """Calls that record a gradient, run under autocast, a functional transform or forward-mode differentiation."""
+    from float8_experimental_amd import inference
+
+    lin = torch.nn.Linear(128, 64, bias=False, device=DEV, dtype=torch.bfloat16)
+    lin = inference.quantize_to_float8(lin, inference.QuantConfig(inference.ActivationCasting.WEIGHT_ONLY))
+    w = lin.weight._data.to(torch.bfloat16) / lin.weight._scale
+    x = torch.randn(3, 128, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    lin(x).sum().backward()
+    assert torch.allclose(x.grad, w.sum(0, dtype=torch.float32).to(torch.bfloat16).expand(3, -1), rtol=2.0 ** -6, atol=1e-2)
+    x = x.detach()
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert lin(x).dtype == torch.float16
+    tangent = torch.randn_like(x)
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        y = lin(torch.autograd.forward_ad.make_dual(x, tangent))
+        assert torch.equal(torch.autograd.forward_ad.unpack_dual(y).tangent, torch.nn.functional.linear(tangent, w))
