@@ -289,8 +289,8 @@ static RowSplit split_last_round(int64_t tiles_m, int64_t tiles_n, int64_t k) {
     if (rows_large < 1 || rows_large >= tiles_m) return {0, 0};
     const int mid = use_mid_tiles((tiles_m - rows_large) * BM, tiles_n * BN, k);
     if (!mid) return {0, 0};
-    // in rounds of the large-tile kernel: a round of 128 x 128 tiles takes about 0.5, one of 128 x 256 tiles 0.8 (measured)
-    const double cost = (double)((rows_large * tiles_n + per_round - 1) / per_round) + (mid == 1 ? 0.5 : 0.8);
+    // in rounds of the large-tile kernel (50 us at k = 4096): a round of 128 x 128 tiles takes about 0.4 (19 us), one of 128 x 256 tiles 0.65 (30 us)
+    const double cost = (double)((rows_large * tiles_n + per_round - 1) / per_round) + (mid == 1 ? 0.4 : 0.65);
     if (cost > (double)((tiles + per_round - 1) / per_round) - 0.1) return {0, 0};
     return {rows_large, mid};
 }

@@ -576,6 +576,15 @@ def test_gemm_mid_tile_kernel_shapes(nat, m, n, k, out_dt):
     _gemm_check(nat, m, n, k, fm[0], fm[1], out_dt, seed=m + n + k, bias=(n % 2 == 0))
 
 
+# One to eight 128-deep steps: shorter and longer than the three (128 x 256) and five (128 x 128) stages in flight.
+@pytest.mark.parametrize("steps", range(1, 9))
+@pytest.mark.parametrize("m,n,mid", [(257, 200, 1), (1300, 4008, 2)])
+def test_gemm_mid_tile_kernel_step_counts(nat, m, n, mid, steps):
+    assert nat.gemm_plan(m, n, 128 * steps) == ("tiles128", 0, mid)
+    for out_dt in (torch.bfloat16, torch.float32):
+        _gemm_check(nat, m, n, 128 * steps, "e4m3", "e5m2", out_dt, seed=m + steps, bias=True)
+
+
 # Few 128-row tiles and a long contraction: with the stream's scratch buffer k is split over workgroups and a second
 # kernel adds the parts in a fixed order.
 @pytest.mark.parametrize("m,n,k", [(256, 2048, 16384), (512, 1024, 8192), (100, 4096, 16384)])
