@@ -6,6 +6,8 @@ current HIP stream to the library.  There is no fallback: if the library is
 missing, cannot be loaded, or the tensors are not on a GPU, the call raises.
 """
 import ctypes as C
+import functools
+import importlib.util
 import os
 import threading
 from typing import Optional, Tuple
@@ -148,6 +150,28 @@ def lib() -> C.CDLL:
                 "F8MI_ALLOW_MEASUREMENT_BUILD=1 to load it anyway")
         _lib = L
     return _lib
+
+
+_EXT_PATH = os.path.join(_HERE, "_f8mi_torch.so")
+_ext = None
+
+
+def ext():
+    """The CPython module with the fused linear's host path (csrc/f8mi_torch.cpp), on the loaded library."""
+    global _ext
+    if _ext is None:
+        lib()
+        with _lock:
+            if _ext is None:
+                if not os.path.exists(_EXT_PATH):
+                    raise Float8NativeError(f"{_EXT_PATH} not found: build it with `python -c 'import __graft_entry__ as g; g.build()'` "
+                                            "(or `python float8_experimental_amd/_build.py`)")
+                spec = importlib.util.spec_from_file_location("float8_experimental_amd._f8mi_torch", _EXT_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                module.load(LIB_PATH, Float8NativeError)
+                _ext = module
+    return _ext
 
 
 def build_knobs() -> str:
@@ -422,6 +446,49 @@ def tn_ok(m: int, k: int, n: int) -> bool:
         return False
     tiles = lambda rows, cols: -(-rows // 128) * -(-cols // 128)  # of 128 x 128: at most one per CU -> that kernel
     return tiles(m, k) > 256 and tiles(n, k) > 256
+
+
+@functools.lru_cache(maxsize=4096)
+def linear_layouts(m: int, k: int, n: int):
+    """(one copy per tensor?, layouts of the operands of output, grad_input and grad_weight) of the fused Float8Linear."""
+    if tn_ok(m, k, n):
+        return True, KBLOCK, KBLOCK, KBLOCK
+    return False, kblock_layout(k), kblock_layout(n), kblock_layout(m)
+
+
+def linear_forward(x: torch.Tensor, weight: torch.Tensor, layouts, need_dx: bool, need_dw: bool, delayed_x, delayed_w, weight_scale):
+    """Casts and product of the fused Float8Linear's forward as one native call: (y, copy of x for backward, copy of the
+    weight for backward, scale of x, scale of the weight); None for arguments that the step-by-step functions have to
+    take (or refuse).  ``delayed_x`` / ``delayed_w``: (amax, scale) buffers of a tensor with delayed scaling."""
+    if not x.is_cuda:
+        return None
+    _check_device(x.device)
+    idx = torch._C._cuda_getDevice()
+    ws = delayed_workspace(x.device) if delayed_x is not None or delayed_w is not None else None
+    return ext().linear_forward(x, weight, *layouts, need_dx, need_dw, delayed_x, delayed_w, weight_scale,
+                                None if ws is None else ws.data_ptr(), idx, torch._C._cuda_getCurrentRawStream(idx))
+
+
+def linear_backward(dy: torch.Tensor, x_saved, w_saved, x_scale, w_scale, k: int, layouts, need_dx: bool, need_dw: bool, delayed_dy):
+    """Cast and products of the fused Float8Linear's backward as one native call: (grad_input, grad_weight), or None (see
+    ``linear_forward``)."""
+    if not dy.is_cuda:
+        return None
+    idx = torch._C._cuda_getDevice()
+    ws = delayed_workspace(dy.device) if delayed_dy is not None else None
+    one_copy, _, kb_dx, kb_dw = layouts
+    return ext().linear_backward(dy, x_saved, w_saved, x_scale, w_scale, k, one_copy, kb_dx, kb_dw, need_dx, need_dw, delayed_dy,
+                                 None if ws is None else ws.data_ptr(), idx, torch._C._cuda_getCurrentRawStream(idx))
+
+
+def inference_linear(x: torch.Tensor, weight: torch.Tensor, n: int, layout: int, weight_scale: torch.Tensor,
+                     static_scale: Optional[torch.Tensor], bias: Optional[torch.Tensor]):
+    """Activation cast and product of an inference linear as one native call; None as for ``linear_forward``."""
+    if not x.is_cuda:
+        return None
+    _check_device(x.device)
+    idx = torch._C._cuda_getDevice()
+    return ext().inference_linear(x, weight, n, layout, weight_scale, static_scale, bias, idx, torch._C._cuda_getCurrentRawStream(idx))
 
 
 def kblock_ok(k: int) -> bool:

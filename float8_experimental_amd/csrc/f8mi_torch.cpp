@@ -1,0 +1,309 @@
+// The host path of the fused linear (training forward, backward; inference) over libf8mi's C ABI, as a CPython module on
+// torch tensors: one call allocates what the kernels write and queues all launches of a direction.  Host code only.
+//
+// Why: a layer of 512 tokens, 1024 -> 1024, is 59 us of kernels; issued launch by launch from Python (allocation, checks,
+// pointer and stream look-ups and a ctypes call each) the same step was bound by the host at 172 - 218 us.
+//
+// Every function returns None, without having queued or allocated anything, for arguments that it does not take (subclasses,
+// other devices, layouts that need a copy, odd scales): the caller then goes through the checked Python functions of
+// _native.py, which raise what there is to raise.  Workspaces are temporaries of torch's caching allocator: it hands their
+// memory out again in stream order, so calls on any number of threads, streams and captures share nothing.
+#include <dlfcn.h>
+
+#include <ATen/ATen.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/f8mi.h"
+
+namespace {
+
+struct Lib {
+    decltype(&f8mi_cast_dynamic) cast_dynamic;
+    decltype(&f8mi_cast_layout) cast_layout;
+    decltype(&f8mi_cast_delayed) cast_delayed;
+    decltype(&f8mi_gemm_nt_ws) gemm_nt_ws;
+    decltype(&f8mi_gemm_nt_kb_ws) gemm_nt_kb_ws;
+    decltype(&f8mi_gemm_kb_ex) gemm_kb_ex;
+    decltype(&f8mi_gemm_plan) gemm_plan;
+    decltype(&f8mi_last_error) last_error;
+    size_t workspace_bytes;
+} L;
+PyObject* native_error = nullptr;  // float8_experimental_amd._native.Float8NativeError
+
+struct NativeFailure {
+    const char* what;
+    int rc;
+};
+void check(int rc, const char* what) {
+    if (rc != 0) throw NativeFailure{what, rc};
+}
+
+int dtype_code(at::ScalarType t) {
+    return t == at::kBFloat16 ? F8MI_BF16 : t == at::kHalf ? F8MI_FP16 : t == at::kFloat ? F8MI_FP32 : -1;
+}
+int fp8_code(at::ScalarType t) { return t == at::kFloat8_e4m3fn ? F8MI_E4M3FN : t == at::kFloat8_e5m2 ? F8MI_E5M2 : -1; }
+at::ScalarType fp8_type(int fmt) { return fmt == F8MI_E4M3FN ? at::kFloat8_e4m3fn : at::kFloat8_e5m2; }
+int64_t padded(int64_t k, int layout) { return layout == F8MI_LAYOUT_KBLOCK64_PAD128 ? (k + 127) / 128 * 128 : k; }
+
+// a plain tensor (or Parameter) on the current device: nothing of a subclass, no other layout
+const at::Tensor* plain(PyObject* o, int device) {
+    if (!THPVariable_CheckExact(o)) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.get_device() == device ? &t : nullptr;
+}
+// ... that the cast kernels read as it is: 2-D, not empty, unit column stride
+const at::Tensor* matrix(PyObject* o, int device) {
+    const at::Tensor* t = plain(o, device);
+    return t && t->dim() == 2 && dtype_code(t->scalar_type()) >= 0 && t->size(0) > 0 && t->size(1) > 0 && t->stride(1) == 1 && t->stride(0) >= t->size(1) ? t : nullptr;
+}
+// ... one fp32 element: a scale or an amax
+const at::Tensor* one_float(PyObject* o, int device) {
+    const at::Tensor* t = plain(o, device);
+    return t && t->scalar_type() == at::kFloat && t->numel() == 1 ? t : nullptr;
+}
+
+// How one tensor is scaled: dynamically, with a scale known beforehand, or delayed (with its amax buffer).
+struct Scaling {
+    const at::Tensor* scale = nullptr;
+    const at::Tensor* amax = nullptr;
+    // `known`: a scale or None; `delayed`: (amax, scale) or None.  False: not taken.
+    bool parse(PyObject* known, PyObject* delayed, int device) {
+        if (delayed != Py_None) {
+            if (!PyTuple_Check(delayed) || PyTuple_GET_SIZE(delayed) != 2) return false;
+            amax = one_float(PyTuple_GET_ITEM(delayed, 0), device);
+            scale = one_float(PyTuple_GET_ITEM(delayed, 1), device);
+            return amax && scale;
+        }
+        if (known == Py_None) return true;
+        scale = one_float(known, device);
+        return scale != nullptr;
+    }
+};
+
+struct Call {
+    void* stream;
+    int device;
+    void* delayed_ws;
+
+    at::Tensor make(at::IntArrayRef sizes, at::ScalarType t) const {
+        return at::empty(sizes, at::TensorOptions().dtype(t).device(at::Device(at::kCUDA, (c10::DeviceIndex)device)));
+    }
+    // fp8 copy of `rows` rows that contracts over kc, in the layout
+    at::Tensor copy(int64_t rows, int64_t kc, int layout, int fmt) const {
+        if (layout == F8MI_LAYOUT_ROWMAJOR) return make({rows, kc}, fp8_type(fmt));
+        return make({padded(kc, layout) / 64, rows, 64}, fp8_type(fmt));
+    }
+
+    // The fp8 copies of x: `row` contracts over the columns, `tr` (the transpose) over the rows.
+    void cast(const at::Tensor& x, const Scaling& s, int fmt, bool want_row, int row_layout, bool want_tr, int tr_layout, at::Tensor& row,
+              at::Tensor& tr, at::Tensor& scale, int scale_dtype = -1) const {
+        const int64_t m = x.size(0), k = x.size(1), ld = x.stride(0);
+        const int dt = dtype_code(x.scalar_type());
+        if (want_row) row = copy(m, k, row_layout, fmt);
+        if (want_tr) tr = copy(k, m, tr_layout, fmt);
+        uint8_t* pr = want_row ? (uint8_t*)row.data_ptr() : nullptr;
+        uint8_t* pt = want_tr ? (uint8_t*)tr.data_ptr() : nullptr;
+        if (!s.scale) {
+            scale = make({}, at::kFloat);
+            const at::Tensor ws = make({(int64_t)L.workspace_bytes / 4}, at::kInt);
+            check(L.cast_dynamic(x.data_ptr(), m, k, ld, dt, fmt, (float*)scale.data_ptr(), pr, row_layout, pt, tr_layout, ws.data_ptr(), stream),
+                  "f8mi_cast_dynamic");
+            return;
+        }
+        scale = *s.scale;
+        if (s.amax)
+            check(L.cast_delayed(x.data_ptr(), m, k, ld, dt, (const float*)scale.data_ptr(), fmt, pr, row_layout, pt, tr_layout,
+                                 (float*)s.amax->data_ptr(), delayed_ws, stream), "f8mi_cast_delayed");
+        else
+            check(L.cast_layout(x.data_ptr(), m, k, ld, dt, (const float*)scale.data_ptr(), scale_dtype < 0 ? dt : scale_dtype, fmt, pr, row_layout,
+                                pt, tr_layout, nullptr, stream), "f8mi_cast_layout");
+    }
+
+    // a [m][k] times bt [n][k] in the layout, both contracting over kc (before padding)
+    at::Tensor gemm(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& bt, const at::Tensor& sb, int layout, int64_t m, int64_t n,
+                    int64_t kc, at::ScalarType out, const at::Tensor* bias = nullptr) const {
+        at::Tensor c = make({m, n}, out), ws;
+        const int64_t k = padded(kc, layout);
+        int64_t ws_bytes = 0;
+        if (m >= 17 && k >= 2048 && (layout != F8MI_LAYOUT_ROWMAJOR || k % 16 == 0)) {  // below these no product is split over k
+            const int plan = L.gemm_plan(m, n, k, 1, F8MI_GEMM_WORKSPACE_BYTES);
+            if ((plan & 0xff) == F8MI_PLAN_TILES128_SPLIT_K) {
+                ws_bytes = (int64_t)((plan >> 8) & 0xff) * m * n * 4;
+                ws = make({ws_bytes / 4}, at::kFloat);
+            }
+        }
+        void* pws = ws_bytes ? ws.data_ptr() : nullptr;
+        const float *pa = (const float*)sa.data_ptr(), *pb = (const float*)sb.data_ptr();
+        const int fa = fp8_code(a.scalar_type()), fb = fp8_code(bt.scalar_type()), dt = dtype_code(out);
+        const void* pbias = bias ? bias->data_ptr() : nullptr;
+        if (layout == F8MI_LAYOUT_ROWMAJOR)
+            check(L.gemm_nt_ws(a.data_ptr(), fa, k, bt.data_ptr(), fb, k, m, n, k, pa, pb, c.data_ptr(), dt, n, pbias, pws, ws_bytes, stream), "f8mi_gemm_nt_ws");
+        else
+            check(L.gemm_nt_kb_ws(a.data_ptr(), fa, bt.data_ptr(), fb, m, n, k, pa, pb, c.data_ptr(), dt, n, pbias, pws, ws_bytes, stream), "f8mi_gemm_nt_kb_ws");
+        return c;
+    }
+    at::Tensor gemm_tr(const at::Tensor& a, bool a_tr, const at::Tensor& sa, const at::Tensor& bt, const at::Tensor& sb, int64_t m, int64_t n,
+                       int64_t k, at::ScalarType out) const {
+        at::Tensor c = make({m, n}, out);
+        check(L.gemm_kb_ex(a.data_ptr(), fp8_code(a.scalar_type()), a_tr, bt.data_ptr(), fp8_code(bt.scalar_type()), 1, m, n, k, (const float*)sa.data_ptr(),
+                           (const float*)sb.data_ptr(), c.data_ptr(), dtype_code(out), n, nullptr, stream), "f8mi_gemm_kb_ex");
+        return c;
+    }
+};
+
+PyObject* wrap(const at::Tensor& t) {
+    if (!t.defined()) Py_RETURN_NONE;
+    return THPVariable_Wrap(t);
+}
+template <typename... T>
+PyObject* wrap_all(const T&... t) {
+    PyObject* r = PyTuple_New(sizeof...(t));
+    if (!r) return nullptr;
+    Py_ssize_t i = 0;
+    for (PyObject* o : {wrap(t)...}) PyTuple_SET_ITEM(r, i++, o);
+    return r;
+}
+template <typename F>
+PyObject* guarded(F body) {
+    HANDLE_TH_ERRORS
+    try {
+        return body();
+    } catch (const NativeFailure& f) {
+        PyErr_Format(native_error, "%s failed with code %d: %s", f.what, f.rc, L.last_error());
+        return nullptr;
+    }
+    END_HANDLE_TH_ERRORS
+}
+bool expect(Py_ssize_t got, Py_ssize_t want, const char* name) {
+    if (!L.gemm_plan) PyErr_SetString(PyExc_RuntimeError, "f8mi_torch: load() has not been called");
+    else if (got != want) PyErr_Format(PyExc_TypeError, "%s takes %zd arguments, got %zd", name, want, got);
+    else return true;
+    return false;
+}
+int as_int(PyObject* o) { return (int)PyLong_AsLong(o); }
+void* as_ptr(PyObject* o) { return o == Py_None ? nullptr : PyLong_AsVoidPtr(o); }
+
+// linear_forward(x [m, k], weight [n, k], one_copy, kb_fwd, kb_dx, kb_dw, need_dx, need_dw, delayed_x, delayed_w, weight_scale,
+//                delayed_workspace, device, stream) -> (y, saved of x, saved of weight, scale of x, scale of weight) or None
+PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    if (!expect(n_args, 14, "linear_forward")) return nullptr;
+    return guarded([&]() -> PyObject* {
+        const Call c{as_ptr(a[13]), as_int(a[12]), as_ptr(a[11])};
+        const at::Tensor *x = matrix(a[0], c.device), *w = matrix(a[1], c.device);
+        Scaling in, we;
+        if (!x || !w || x->size(1) != w->size(1) || !in.parse(Py_None, a[8], c.device) || !we.parse(a[10], a[9], c.device)) Py_RETURN_NONE;
+        if ((in.amax || we.amax) && !c.delayed_ws) Py_RETURN_NONE;
+        const bool one_copy = as_int(a[2]), need_dx = as_int(a[6]), need_dw = as_int(a[7]);
+        const int kb_fwd = as_int(a[3]), kb_dx = as_int(a[4]), kb_dw = as_int(a[5]);
+        const int64_t m = x->size(0), k = x->size(1), n = w->size(0);
+        at::Tensor x8, x8t, sx, w8, w8t, sw;
+        c.cast(*x, in, F8MI_E4M3FN, true, kb_fwd, !one_copy && need_dw, kb_dw, x8, x8t, sx);
+        c.cast(*w, we, F8MI_E4M3FN, true, kb_fwd, !one_copy && need_dx, kb_dx, w8, w8t, sw);
+        const at::Tensor y = c.gemm(x8, sx, w8, sw, kb_fwd, m, n, k, x->scalar_type());
+        if (one_copy) return wrap_all(y, x8, w8, sx, sw);
+        return wrap_all(y, x8t, w8t, sx, sw);
+    });
+}
+
+// linear_backward(dy [m, n], saved of x, saved of weight, scale of x, scale of weight, k, one_copy, kb_dx, kb_dw, need_dx, need_dw,
+//                 delayed_dy, delayed_workspace, device, stream) -> (grad of x [m, k], grad of weight [n, k]) or None
+PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    if (!expect(n_args, 15, "linear_backward")) return nullptr;
+    return guarded([&]() -> PyObject* {
+        const Call c{as_ptr(a[14]), as_int(a[13]), as_ptr(a[12])};
+        const at::Tensor* dy = matrix(a[0], c.device);
+        const bool one_copy = as_int(a[6]), need_dx = as_int(a[9]), need_dw = as_int(a[10]);
+        const at::Tensor *xs = need_dw ? plain(a[1], c.device) : nullptr, *ws = need_dx ? plain(a[2], c.device) : nullptr;
+        const at::Tensor *sx = one_float(a[3], c.device), *sw = one_float(a[4], c.device);
+        Scaling go;
+        if (!dy || !sx || !sw || (need_dw && !xs) || (need_dx && !ws) || !(need_dx || need_dw) || !go.parse(Py_None, a[11], c.device)) Py_RETURN_NONE;
+        if (go.amax && !c.delayed_ws) Py_RETURN_NONE;
+        const int kb_dx = as_int(a[7]), kb_dw = as_int(a[8]);
+        const int64_t m = dy->size(0), n = dy->size(1), k = PyLong_AsLongLong(a[5]);
+        // what saved-tensor hooks hand back has to be what was saved: dense fp8 copies of the sizes the products assume
+        for (const at::Tensor* t : {xs, ws}) {
+            if (!t) continue;
+            const int64_t rows = one_copy ? (t == xs ? m : n) : k, kc = one_copy ? k : (t == xs ? m : n);
+            const int layout = one_copy ? F8MI_LAYOUT_KBLOCK64 : t == xs ? kb_dw : kb_dx;
+            if (fp8_code(t->scalar_type()) < 0 || !t->is_contiguous() || t->numel() != rows * padded(kc, layout)) Py_RETURN_NONE;
+        }
+        at::Tensor g8, g8t, sg, dx, dw;
+        if (one_copy) {
+            c.cast(*dy, go, F8MI_E5M2, true, F8MI_LAYOUT_KBLOCK64, false, 0, g8, g8t, sg);
+            if (need_dx) dx = c.gemm_tr(g8, false, sg, *ws, *sw, m, k, n, dy->scalar_type());
+            if (need_dw) dw = c.gemm_tr(g8, true, sg, *xs, *sx, n, k, m, dy->scalar_type());
+        } else {
+            c.cast(*dy, go, F8MI_E5M2, need_dx, kb_dx, need_dw, kb_dw, g8, g8t, sg);
+            if (need_dx) dx = c.gemm(g8, sg, *ws, *sw, kb_dx, m, k, n, dy->scalar_type());
+            if (need_dw) dw = c.gemm(g8t, sg, *xs, *sx, kb_dw, n, k, m, dy->scalar_type());
+        }
+        return wrap_all(dx, dw);
+    });
+}
+
+// inference_linear(x [m, k], weight (fp8, [n, k] or k-blocked), n, layout, weight_scale, static_scale, bias, device, stream) -> y or None
+PyObject* inference_linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    if (!expect(n_args, 9, "inference_linear")) return nullptr;
+    return guarded([&]() -> PyObject* {
+        const Call c{as_ptr(a[8]), as_int(a[7]), nullptr};
+        const at::Tensor *x = matrix(a[0], c.device), *w = plain(a[1], c.device), *sw = one_float(a[4], c.device);
+        const at::Tensor* bias = a[6] == Py_None ? nullptr : plain(a[6], c.device);
+        const int64_t n = PyLong_AsLongLong(a[2]);
+        const int layout = as_int(a[3]);
+        Scaling in;
+        if (!x || !w || !sw || (a[6] != Py_None && !bias) || !in.parse(a[5], Py_None, c.device)) Py_RETURN_NONE;
+        const int64_t m = x->size(0), k = x->size(1);
+        if (n <= 0 || fp8_code(w->scalar_type()) < 0 || !w->is_contiguous() || w->numel() != n * padded(k, layout)) Py_RETURN_NONE;
+        if (bias && (bias->scalar_type() != x->scalar_type() || bias->numel() != n || !bias->is_contiguous())) Py_RETURN_NONE;
+        at::Tensor x8, none, sx;
+        // a 0-dim scale leaves the product in x's dtype, a scale with a dimension promotes it to fp32
+        c.cast(*x, in, F8MI_E4M3FN, true, layout, false, 0, x8, none, sx, in.scale && in.scale->dim() > 0 ? F8MI_FP32 : -1);
+        return wrap(c.gemm(x8, sx, *w, *sw, layout, m, n, k, x->scalar_type(), bias));
+    });
+}
+
+// load(path of libf8mi.so, error class): resolves the entry points
+PyObject* load(PyObject*, PyObject* args) {
+    const char* path;
+    PyObject* error;
+    if (!PyArg_ParseTuple(args, "sO", &path, &error)) return nullptr;
+    void* h = dlopen(path, RTLD_NOW | RTLD_LOCAL);
+    if (!h) return PyErr_Format(PyExc_ImportError, "%s", dlerror());
+    const char* missing = nullptr;
+    auto get = [&](auto& f, const char* name) {
+        f = reinterpret_cast<std::decay_t<decltype(f)>>(dlsym(h, name));
+        if (!f) missing = name;
+    };
+    decltype(&f8mi_workspace_bytes) workspace_bytes;
+    get(workspace_bytes, "f8mi_workspace_bytes");
+    get(L.cast_dynamic, "f8mi_cast_dynamic");
+    get(L.cast_layout, "f8mi_cast_layout");
+    get(L.cast_delayed, "f8mi_cast_delayed");
+    get(L.gemm_nt_ws, "f8mi_gemm_nt_ws");
+    get(L.gemm_nt_kb_ws, "f8mi_gemm_nt_kb_ws");
+    get(L.gemm_kb_ex, "f8mi_gemm_kb_ex");
+    get(L.last_error, "f8mi_last_error");
+    get(L.gemm_plan, "f8mi_gemm_plan");
+    if (missing) {
+        L.gemm_plan = nullptr;
+        return PyErr_Format(PyExc_ImportError, "%s does not export %s", path, missing);
+    }
+    L.workspace_bytes = workspace_bytes();
+    Py_INCREF(error);
+    native_error = error;
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"load", load, METH_VARARGS, nullptr},
+    {"linear_forward", (PyCFunction)(void (*)(void))linear_forward, METH_FASTCALL, nullptr},
+    {"linear_backward", (PyCFunction)(void (*)(void))linear_backward, METH_FASTCALL, nullptr},
+    {"inference_linear", (PyCFunction)(void (*)(void))inference_linear, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_f8mi_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__f8mi_torch(void) { return PyModule_Create(&module); }

@@ -124,6 +124,20 @@ class _float8_linear_fn(torch.autograd.Function):
         emulate = mod.linear_mm_config.output.emulate
         emulate_bw = mod.linear_mm_config.grad_input.emulate or mod.linear_mm_config.grad_weight.emulate
         dl = mod._delayed_buffers
+        ctx.mod = mod
+        ctx.is_amax_initialized = is_amax_initialized
+        ctx.x_shape = x.shape
+        ctx.layouts = None
+        if not emulate and not emulate_bw and (is_amax_initialized or not mod.has_any_delayed_scaling):
+            layouts = _native.linear_layouts(m, k, n)
+            done = _native.linear_forward(x2, weight, layouts, need_dx, need_dw, mod._delayed_pair("input"), mod._delayed_pair("weight"),
+                                          mod._precomputed_weight_scale)
+            if done is not None:
+                y, xs, ws, sx, sw = done
+                ctx.layouts = layouts
+                ctx.kb = None if layouts[0] else layouts[2:]
+                ctx.save_for_backward(xs, ws, sx, sw)
+                return y if x.dim() == 2 else y.reshape(*x.shape[:-1], n)
         tn = not emulate and not emulate_bw and _native.tn_ok(m, k, n)
         if tn:
             x8, _, sx = _cast_for_gemm(x2, e4m3_dtype, dl("input"), is_amax_initialized, True, False, True, False)
@@ -145,9 +159,6 @@ class _float8_linear_fn(torch.autograd.Function):
                 y = _gemm(x8, sx, w8, sw, x.dtype, kb_fwd)
             ctx.kb = (kb_dx, kb_dw)
             ctx.save_for_backward(x8t, w8t, sx, sw)
-        ctx.mod = mod
-        ctx.is_amax_initialized = is_amax_initialized
-        ctx.x_shape = x.shape
         return y.reshape(*x.shape[:-1], n)
 
     @staticmethod
@@ -155,8 +166,14 @@ class _float8_linear_fn(torch.autograd.Function):
         mod = ctx.mod
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         dy2 = dy.reshape(-1, dy.shape[-1])
-        dlg = mod._delayed_buffers("grad_output")
         dx = dw = None
+        if ctx.layouts is not None and (need_dx or need_dw):
+            done = _native.linear_backward(dy2, *ctx.saved_tensors, ctx.x_shape[-1], ctx.layouts, need_dx, need_dw,
+                                           mod._delayed_pair("grad_output"))
+            if done is not None:
+                dx, dw = done
+                return dx if dx is None or len(ctx.x_shape) == 2 else dx.reshape(ctx.x_shape), dw, None, None
+        dlg = mod._delayed_buffers("grad_output")
         if ctx.kb is None:  # one copy per tensor: x8 [K/64, M, 64], w8 [K/64, N, 64], g8 [N/64, M, 64]
             x8, w8, sx, sw = ctx.saved_tensors
             g8, _, sg = _cast_for_gemm(dy2, e5m2_dtype, dlg, ctx.is_amax_initialized, True, False, True, False)
@@ -268,6 +285,12 @@ class Float8Linear(torch.nn.Linear):
             return None
         return _DelayedBuffers(getattr(self, f"fp8_amax_{kind}"), getattr(self, f"fp8_amax_history_{kind}"),
                                getattr(self, f"fp8_scale_{kind}"))
+
+    def _delayed_pair(self, kind: str):
+        """(amax, scale) buffers of a tensor with delayed scaling, None for dynamic scaling."""
+        if not self.has_any_delayed_scaling or getattr(self, f"scaling_type_{kind}") is not ScalingType.DELAYED:
+            return None
+        return self._buffers[f"fp8_amax_{kind}"], self._buffers[f"fp8_scale_{kind}"]
 
     # ---- the reference's building blocks (same numbers as the fused path) -----------------
 

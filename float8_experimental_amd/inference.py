@@ -101,6 +101,9 @@ def _fp8_linear(x2: torch.Tensor, w_data: torch.Tensor, w_scale: torch.Tensor, s
     given, else dynamic) and the scaled GEMM with the bias in its epilogue."""
     k = x2.shape[1]
     use_kb = _native.kblock_layout(k)  # row-major for a short contraction, else k-blocked (zero-padded when ragged)
+    y = _native.inference_linear(x2, _kblocked_weight(w_data) if use_kb else w_data, w_data.shape[0], use_kb, w_scale, static_scale, bias)
+    if y is not None:
+        return y
     if static_scale is not None:
         scale = static_scale
         x8, _ = _native.cast(x2, scale, e4m3_dtype, product_dtype=_product_dtype(x2, scale), out_kblock=use_kb)

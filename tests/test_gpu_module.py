@@ -767,3 +767,61 @@ def test_frozen_weight_and_no_grad(f8):
     y2 = mod(x)  # input without grad
     y2.sum().backward()
     assert lin.weight.grad is not None
+
+
+@pytest.mark.parametrize("m,k,n", [(512, 1024, 1024), (384, 384, 384), (100, 257, 130), (17, 64, 4096), (1, 512, 512), (2048, 4096, 4224)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("delayed", [False, True])
+def test_native_host_path_equals_the_step_by_step_functions(f8, monkeypatch, m, k, n, dtype, delayed):
+    """One native call per direction against the Python functions it stands for: the same bits for dense and row-strided
+    inputs and gradients, with the input's or the weight's gradient left out, dynamic and delayed."""
+    from float8_experimental_amd import _native
+
+    kind = f8.CastConfig(scaling_type=f8.ScalingType.DELAYED if delayed else f8.ScalingType.DYNAMIC)
+    config = f8.Float8LinearConfig(cast_config_input=kind, cast_config_weight=kind, cast_config_grad_output=kind)
+    g = torch.Generator().manual_seed(m + k + n)
+    base = torch.randn(m, k + 9, generator=g).to(dtype).to(DEV)
+    dbase = torch.randn(m, n + 3, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(n, k, generator=g) / 30).to(dtype).to(DEV)
+    taken = []
+
+    def steps(native):
+        lin = torch.nn.Linear(k, n, bias=False, device=DEV, dtype=dtype)
+        lin.weight.data.copy_(w)
+        mod = f8.convert_to_float8_training(torch.nn.Sequential(lin), config=config)
+        out = []
+        for it, (strided, dx, dw) in enumerate([(False, True, True), (True, True, True), (False, True, False), (True, False, True)]):
+            if delayed and it:
+                f8.sync_float8_amax_and_scale_history(mod)
+            with monkeypatch.context() as p:
+                for name in ("linear_forward", "linear_backward"):
+                    real = getattr(_native, name)
+                    spy = lambda *a, real=real: taken.append(real(*a)) or taken[-1]
+                    p.setattr(_native, name, spy if native else lambda *a: None)
+                x = base[:, :k] if strided else base[:, :k].contiguous()
+                x = x.detach().requires_grad_(dx)
+                mod[0].weight.requires_grad_(dw)
+                mod[0].weight.grad = None
+                y = mod(x)
+                y.backward(dbase[:, :n] if strided else dbase[:, :n].contiguous())
+            out += [y.detach(), x.grad, mod[0].weight.grad] + [b.clone() for b in mod.buffers()]
+        return out
+
+    for got, want in zip(steps(True), steps(False)):
+        assert (got is None) == (want is None)
+        assert got is None or torch.equal(got, want)
+    assert len(taken) == (6 if delayed else 8) and all(t is not None for t in taken)  # the first delayed step initialises its buffers
+
+
+def test_native_host_path_leaves_what_it_does_not_take_to_the_step_by_step_functions(f8):
+    from float8_experimental_amd import _native
+
+    x, w = torch.randn(64, 512, device=DEV), torch.randn(256, 512, device=DEV)
+    layouts = _native.linear_layouts(64, 512, 256)
+    call = lambda x, w, **kw: _native.linear_forward(x, w, layouts, True, True, kw.get("dx"), kw.get("dw"), kw.get("scale"))
+    one = torch.ones(1, device=DEV)
+    assert call(x, w) is not None
+    assert call(x.expand(2, 64, 512)[:, 0], w) is not None
+    for bad in (call(x.t().contiguous().t(), w), call(x[0].expand(64, 512), w), call(x[:0], w), call(x.double(), w), call(x, w[:, :-1]),
+                call(x, w, scale=one.double()), call(x, w, scale=torch.ones(2, device=DEV)), call(x, w, dx=(one, one.cpu()))):
+        assert bad is None
