@@ -821,7 +821,7 @@ def test_native_host_path_leaves_what_it_does_not_take_to_the_step_by_step_funct
     call = lambda x, w, **kw: _native.linear_forward(x, w, layouts, True, True, kw.get("dx"), kw.get("dw"), kw.get("scale"))
     one = torch.ones(1, device=DEV)
     assert call(x, w) is not None
-    assert call(x.expand(2, 64, 512)[:, 0], w) is not None
+    assert call(torch.randn(64, 600, device=DEV)[:, :512], w) is not None
     for bad in (call(x.t().contiguous().t(), w), call(x[0].expand(64, 512), w), call(x[:0], w), call(x.double(), w), call(x, w[:, :-1]),
                 call(x, w, scale=one.double()), call(x, w, scale=torch.ones(2, device=DEV)), call(x, w, dx=(one, one.cpu()))):
         assert bad is None
