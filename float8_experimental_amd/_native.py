@@ -46,6 +46,7 @@ EXPORTS = (
     "f8mi_delayed_workspace_bytes",
     "f8mi_cast_dynamic",
     "f8mi_cast_dynamic_static",
+    "f8mi_linear_few_rows",
     "f8mi_gemm_weight_only",
     "f8mi_dequant",
     "f8mi_gemm_nt",
@@ -127,6 +128,8 @@ def lib() -> C.CDLL:
         L.f8mi_gemm_plan.argtypes = [i64, i64, i64, i32, i64]
         L.f8mi_gemm_nt_kb_ws.restype = i32
         L.f8mi_gemm_nt_kb_ws.argtypes = [vp, i32, vp, i32, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp, i64, vp]
+        L.f8mi_linear_few_rows.restype = i32
+        L.f8mi_linear_few_rows.argtypes = [vp, i64, i32, fp, i32, vp, i32, i32, fp, i64, i64, i64, vp, i64, vp, vp]
         L.f8mi_gemm_weight_only.restype = i32
         L.f8mi_gemm_weight_only.argtypes = [vp, i64, i32, vp, i32, i64, i64, i64, i64, fp, vp, i64, vp]
         L.f8mi_dequant.restype = i32

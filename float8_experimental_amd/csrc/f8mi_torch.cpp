@@ -26,6 +26,7 @@ struct Lib {
     decltype(&f8mi_gemm_nt_kb_ws) gemm_nt_kb_ws;
     decltype(&f8mi_gemm_kb_ex) gemm_kb_ex;
     decltype(&f8mi_gemm_plan) gemm_plan;
+    decltype(&f8mi_linear_few_rows) linear_few_rows;
     decltype(&f8mi_last_error) last_error;
     size_t workspace_bytes;
 } L;
@@ -97,7 +98,7 @@ struct Call {
 
     // The fp8 copies of x: `row` contracts over the columns, `tr` (the transpose) over the rows.
     void cast(const at::Tensor& x, const Scaling& s, int fmt, bool want_row, int row_layout, bool want_tr, int tr_layout, at::Tensor& row,
-              at::Tensor& tr, at::Tensor& scale, int scale_dtype = -1) const {
+              at::Tensor& tr, at::Tensor& scale, int product_dtype = -1) const {
         const int64_t m = x.size(0), k = x.size(1), ld = x.stride(0);
         const int dt = dtype_code(x.scalar_type());
         if (want_row) row = copy(m, k, row_layout, fmt);
@@ -116,7 +117,7 @@ struct Call {
             check(L.cast_delayed(x.data_ptr(), m, k, ld, dt, (const float*)scale.data_ptr(), fmt, pr, row_layout, pt, tr_layout,
                                  (float*)s.amax->data_ptr(), delayed_ws, stream), "f8mi_cast_delayed");
         else
-            check(L.cast_layout(x.data_ptr(), m, k, ld, dt, (const float*)scale.data_ptr(), scale_dtype < 0 ? dt : scale_dtype, fmt, pr, row_layout,
+            check(L.cast_layout(x.data_ptr(), m, k, ld, dt, (const float*)scale.data_ptr(), product_dtype < 0 ? dt : product_dtype, fmt, pr, row_layout,
                                 pt, tr_layout, nullptr, stream), "f8mi_cast_layout");
     }
 
@@ -256,9 +257,20 @@ PyObject* inference_linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         const int64_t m = x->size(0), k = x->size(1);
         if (n <= 0 || fp8_code(w->scalar_type()) < 0 || !w->is_contiguous() || w->numel() != n * padded(k, layout)) Py_RETURN_NONE;
         if (bias && (bias->scalar_type() != x->scalar_type() || bias->numel() != n || !bias->is_contiguous())) Py_RETURN_NONE;
-        at::Tensor x8, none, sx;
         // a 0-dim scale leaves the product in x's dtype, a scale with a dimension promotes it to fp32
-        c.cast(*x, in, F8MI_E4M3FN, true, layout, false, 0, x8, none, sx, in.scale && in.scale->dim() > 0 ? F8MI_FP32 : -1);
+        const int dt = dtype_code(x->scalar_type()), product = in.scale && in.scale->dim() > 0 ? F8MI_FP32 : dt;
+        if (m <= 16 && m * k <= F8MI_FEW_ROWS_ELEMS && layout != F8MI_LAYOUT_KBLOCK64_PAD128) {  // cast and product in one kernel
+            const at::Tensor y = c.make({m, n}, x->scalar_type());
+            const int rc = L.linear_few_rows(x->data_ptr(), x->stride(0), dt, in.scale ? (const float*)in.scale->data_ptr() : nullptr, product, w->data_ptr(),
+                                             fp8_code(w->scalar_type()), layout, (const float*)sw->data_ptr(), m, n, k, y.data_ptr(), n,
+                                             bias ? bias->data_ptr() : nullptr, c.stream);
+            if (rc != F8MI_ERR_UNSUPPORTED) {
+                check(rc, "f8mi_linear_few_rows");
+                return wrap(y);
+            }
+        }
+        at::Tensor x8, none, sx;
+        c.cast(*x, in, F8MI_E4M3FN, true, layout, false, 0, x8, none, sx, product);
         return wrap(c.gemm(x8, sx, *w, *sw, layout, m, n, k, x->scalar_type(), bias));
     });
 }
@@ -283,6 +295,7 @@ PyObject* load(PyObject*, PyObject* args) {
     get(L.gemm_nt_ws, "f8mi_gemm_nt_ws");
     get(L.gemm_nt_kb_ws, "f8mi_gemm_nt_kb_ws");
     get(L.gemm_kb_ex, "f8mi_gemm_kb_ex");
+    get(L.linear_few_rows, "f8mi_linear_few_rows");
     get(L.last_error, "f8mi_last_error");
     get(L.gemm_plan, "f8mi_gemm_plan");
     if (missing) {

@@ -232,6 +232,17 @@ int f8mi_cast_dynamic_static(const void* x, int64_t rows, int64_t cols, int64_t 
                              float* scale_dev, uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout,
                              void* stream);
 
+/* A whole linear of at most 16 rows and F8MI_FEW_ROWS_ELEMS activations in one kernel: c[m][n] = sum_k x8[m][k] * w[n][k]
+ * / (scale_x * scale_w) (+ bias[n]) with x8 the saturated e4m3 cast of x, which every workgroup makes for itself.  The same
+ * bits as f8mi_cast_dynamic (scale_x_dev null) or f8mi_cast_layout (scale_x_dev given, product in product_dtype) followed by
+ * f8mi_gemm_nt / f8mi_gemm_nt_kb.  x: rows of ldx elements at element alignment; w: row-major (w_layout
+ * F8MI_LAYOUT_ROWMAJOR, rows of k bytes) or k-blocked (F8MI_LAYOUT_KBLOCK64), 16-byte aligned; c in x's dtype.
+ * F8MI_ERR_UNSUPPORTED, with nothing queued: more rows or activations, k % 128 != 0, an unaligned weight. */
+#define F8MI_FEW_ROWS_ELEMS 32768
+int f8mi_linear_few_rows(const void* x, int64_t ldx, int dtype, const float* scale_x_dev, int product_dtype, const void* w,
+                         int w_fmt, int w_layout, const float* scale_w_dev, int64_t m, int64_t n, int64_t k, void* c,
+                         int64_t ldc, const void* bias_dev, void* stream);
+
 /* Weight-only inference for few rows: c[m][n] = sum_k x[m][k] * W[n][k] with x, c and W = w / *scale_dev in `dtype`,
  * the fp8 weight w (rows of ldw bytes) dequantised in registers: the quotient is taken in fp32 and rounded to `dtype`,
  * as torch divides (the scale rounded to `dtype` before); fp32 accumulation.  Any k >= 1, any alignment of rows to the

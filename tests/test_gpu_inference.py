@@ -293,3 +293,35 @@ def test_weight_only_leaves_other_calls_to_the_library_product(f8):
     with torch.no_grad(), torch.autograd.forward_ad.dual_level():
         y = lin(torch.autograd.forward_ad.make_dual(x, tangent))
         assert torch.equal(torch.autograd.forward_ad.unpack_dual(y).tangent, torch.nn.functional.linear(tangent, w))
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 8192, 512), (1, 128, 16), (2, 256, 100), (16, 384, 8200), (16, 2048, 1000), (16, 2176, 24), (7, 4096, 8197),
+                                   (5, 1152, 33), (16, 14336, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_few_row_linear_equals_cast_and_gemm(m, k, n, dtype):
+    """At most 16 rows: the kernel that casts the activations in registers against the cast and GEMM it stands for, bit for
+    bit -- dynamic (one and two launches), static with a 0-dim and a 1-element scale, NaN and infinities, strided rows."""
+    from float8_experimental_amd import _native as nat
+    from float8_experimental_amd.inference import _to_kblock
+
+    g = torch.Generator().manual_seed(m + k + n)
+    w = (torch.randn(n, k, generator=g) * 30).to([torch.float8_e4m3fn, torch.float8_e5m2][(m + n) % 2]).to(DEV)
+    sw, bias = torch.tensor(3.5, device=DEV), torch.randn(n, generator=g).to(dtype).to(DEV)
+    kb = nat.kblock_layout(k)
+    wk = _to_kblock(w) if kb else w
+    plain = torch.randn(m, k + 5, generator=g).to(dtype).to(DEV)
+    odd = plain.clone()
+    odd[m // 2, 3], odd[0, k - 1] = float("inf"), 1e4
+    nan = plain.clone()
+    nan[m - 1, k // 2] = float("nan")
+    for base in (plain, odd, nan, torch.zeros_like(plain)):
+        for x in (base[:, :k], base[:, :k].contiguous()):
+            for static, b in ((None, None), (None, bias), (torch.tensor(64.0, device=DEV), bias), (torch.tensor([0.3], device=DEV), None)):
+                if static is None:
+                    x8, _, s = nat.cast_dynamic(x, torch.float8_e4m3fn, out_kblock=kb)
+                else:
+                    s = static
+                    x8, _ = nat.cast(x, s, torch.float8_e4m3fn, product_dtype=dtype if s.dim() == 0 else torch.float32, out_kblock=kb)
+                want = (nat.gemm_nt_kb if kb else nat.gemm_nt)(x8, s, wk, sw, dtype, bias=b)
+                got = nat.inference_linear(x, wk, n, kb, sw, static, b)
+                assert torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)) and torch.equal(got.isnan(), want.isnan())
