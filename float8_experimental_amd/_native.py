@@ -440,15 +440,21 @@ def _kb_alloc(rows: int, kc: int, layout: int, float8_dtype, device) -> torch.Te
     return torch.empty((kc // KB, rows, KB), dtype=float8_dtype, device=device)
 
 
+TN_MIN_TILES = 32
+
+
 def tn_ok(m: int, k: int, n: int) -> bool:
     """True if a linear layer with m tokens, k in_features and n out_features should keep one k-blocked fp8 copy per
     tensor and let the backward GEMMs read it transposed (f8mi_gemm_kb_ex): every dimension a multiple of 128 and at
-    least 384 -- and grad_input and grad_weight large enough for the 256 x 256-tile kernels, the only ones that read
-    transposed operands (smaller outputs are faster from transposed copies through the 128 x 128-tile kernel)."""
+    least 384, and neither backward product one that is faster split over k (the kernels that read transposed operands
+    are not split).  Reading an operand transposed costs the GEMM nothing (2048 x 4096 over 4096: 29.9 us as it is, 30.9
+    transposed), writing the transposed copy costs the cast a sixth (2048 x 4096: 14.2 us with one copy, 16.7 with two).
+    Layers with a backward product of fewer than TN_MIN_TILES tiles of 128 x 128 are bound by launches either way and keep
+    their transposed copies."""
     if not all(d % 128 == 0 and d >= KB_MIN_K for d in (m, k, n)):
         return False
-    tiles = lambda rows, cols: -(-rows // 128) * -(-cols // 128)  # of 128 x 128: at most one per CU -> that kernel
-    return tiles(m, k) > 256 and tiles(n, k) > 256
+    return all((rows // 128) * (cols // 128) >= TN_MIN_TILES and gemm_plan(rows, cols, kc)[0] != "tiles128_split_k"
+               for rows, cols, kc in ((m, k, n), (n, k, m)))
 
 
 @functools.lru_cache(maxsize=4096)

@@ -329,6 +329,28 @@ static GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, bool aligned, int64_t
     return p;
 }
 
+// The kernels that read Bt (a_transposed: and A) transposed, by the same rule: outputs of at most 256 tiles of 128 rows go to
+// those, which take as long as on operands as they are (2048 x 4096 over k = 4096, half a round of 256 x 256 tiles: 40.3 -> 30.9 us,
+// both operands transposed 41.9 -> 30.9; 1024 x 4096 over 8192: 69.1 -> 30.6 and 72.0 -> 31.6), and a sparse last round of large
+// tiles is split off (4352 x 4096 over 1024: 32.5 -> 25.7).
+static int launch_transposed(bool a_transposed, int a_fmt, int b_fmt, int c_dtype, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
+                             const uint8_t* Bt, int64_t ldb, int64_t b_unit, int64_t m, int64_t n, int64_t k, const float* sa, const float* sb,
+                             void* c, int64_t ldc, const void* bias, int c_vec_ok) {
+    const auto mid_kernel = a_transposed ? launch_gemm_mid_tt : launch_gemm_mid_nt;
+    const auto large_kernel = a_transposed ? launch_gemm_dma16_tt : launch_gemm_dma16_nt;
+    if (const int mid = use_mid_tiles(m, n, k))
+        return mid_kernel(a_fmt, b_fmt, c_dtype, mid == 2, stream, A, lda, a_unit, Bt, ldb, b_unit, (int)m, (int)n, (int)k, sa, sb, c, ldc, bias, c_vec_ok);
+    const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
+    const RowSplit split = split_last_round(tiles_m, tiles_n, k);
+    const int64_t rows = split.rows_large ? split.rows_large : tiles_m, m1 = split.rows_large ? rows * BM : m;
+    if (int rc = large_kernel(a_fmt, b_fmt, c_dtype, dim3((unsigned)(rows * tiles_n)), stream, A, lda, a_unit, Bt, ldb, b_unit, (int)m1, (int)n, (int)k, sa, sb,
+                              c, ldc, bias, (int)rows, (int)tiles_n, c_vec_ok))
+        return rc;
+    if (m1 == m) return F8MI_OK;
+    return mid_kernel(a_fmt, b_fmt, c_dtype, split.mid == 2, stream, A + (a_transposed ? m1 / 64 * a_unit : m1 * lda), lda, a_unit, Bt, ldb, b_unit, (int)(m - m1),
+                      (int)n, (int)k, sa, sb, (uint8_t*)c + m1 * ldc * (c_dtype == F8MI_FP32 ? 4 : 2), ldc, bias, c_vec_ok);
+}
+
 extern "C" int f8mi_gemm_plan(int64_t m, int64_t n, int64_t k, int aligned, int64_t workspace_bytes) {
     if (m <= 0 || n <= 0 || k < 0) return 0;
     const GemmPlan p = gemm_plan(m, n, k, aligned != 0, workspace_bytes);
@@ -466,16 +488,11 @@ extern "C" int f8mi_gemm_kb_ex(const void* a, int a_fmt, int a_transposed, const
     if (m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff - BK || k * 64 * 4 > 0x7fffffffLL) { set_error("f8mi_gemm_kb_ex: dimension too large"); return F8MI_ERR_UNSUPPORTED; }
     const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
     if (tiles_m * tiles_n > 0x7fffffff) { set_error("f8mi_gemm_kb_ex: too many tiles"); return F8MI_ERR_UNSUPPORTED; }
-    const int64_t csz = c_dtype == F8MI_FP32 ? 4 : 2;
-    const int c_vec_ok = (uintptr_t)c % csz == 0;  // 16-byte stores at element alignment: any row pitch will do
-    dim3 g((unsigned)(tiles_m * tiles_n));
+    const int c_vec_ok = (uintptr_t)c % (c_dtype == F8MI_FP32 ? 4 : 2) == 0;  // 16-byte stores at element alignment: any row pitch will do
     ProfScope prof(F8MI_K_GEMM, 2.0 * (double)m * (double)n * (double)k, stream);
     // a transposed operand: 64 bytes between contraction rows, k * 64 between blocks of 64 rows
-    if (a_transposed)
-        return launch_gemm_dma16_tt(a_fmt, b_fmt, c_dtype, g, stream, (const uint8_t*)a, 64, k * 64, (const uint8_t*)bt, 64, k * 64, (int)m, (int)n,
-                                    (int)k, scale_a_dev, scale_b_dev, c, ldc, bias_dev, (int)tiles_m, (int)tiles_n, c_vec_ok);
-    return launch_gemm_dma16_nt(a_fmt, b_fmt, c_dtype, g, stream, (const uint8_t*)a, 64, m * 64, (const uint8_t*)bt, 64, k * 64, (int)m, (int)n,
-                                (int)k, scale_a_dev, scale_b_dev, c, ldc, bias_dev, (int)tiles_m, (int)tiles_n, c_vec_ok);
+    return launch_transposed(a_transposed != 0, a_fmt, b_fmt, c_dtype, stream, (const uint8_t*)a, 64, a_transposed ? k * 64 : m * 64, (const uint8_t*)bt, 64, k * 64,
+                             m, n, k, scale_a_dev, scale_b_dev, c, ldc, bias_dev, c_vec_ok);
 }
 
 extern "C" int f8mi_gemm_ex(const void* a, int a_fmt, int a_transposed, int64_t lda, const void* bt, int b_fmt, int b_transposed, int64_t ldb,
@@ -498,14 +515,9 @@ extern "C" int f8mi_gemm_ex(const void* a, int a_fmt, int a_transposed, int64_t 
     if (m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff - BK || 128 * ldb + 256 > 0x7fffffffLL || (a_transposed ? 128 * lda + 256 : lda * (BM - 1) + k + BK) > 0x7fffffffLL) { set_error("f8mi_gemm_ex: dimension or row stride too large"); return F8MI_ERR_UNSUPPORTED; }
     const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
     if (tiles_m * tiles_n > 0x7fffffff) { set_error("f8mi_gemm_ex: too many tiles"); return F8MI_ERR_UNSUPPORTED; }
-    const int64_t csz = c_dtype == F8MI_FP32 ? 4 : 2;
-    const int c_vec_ok = (uintptr_t)c % csz == 0;
-    dim3 g((unsigned)(tiles_m * tiles_n));
+    const int c_vec_ok = (uintptr_t)c % (c_dtype == F8MI_FP32 ? 4 : 2) == 0;
     ProfScope prof(F8MI_K_GEMM, 2.0 * (double)m * (double)n * (double)k, stream);
     // a row-major matrix read transposed: row stride between contraction rows, 64 bytes between blocks of 64 rows
-    if (a_transposed)
-        return launch_gemm_dma16_tt(a_fmt, b_fmt, c_dtype, g, stream, (const uint8_t*)a, lda, 64, (const uint8_t*)bt, ldb, 64, (int)m, (int)n, (int)k,
-                                    scale_a_dev, scale_b_dev, c, ldc, bias_dev, (int)tiles_m, (int)tiles_n, c_vec_ok);
-    return launch_gemm_dma16_nt(a_fmt, b_fmt, c_dtype, g, stream, (const uint8_t*)a, lda, 64, (const uint8_t*)bt, ldb, 64, (int)m, (int)n, (int)k,
-                                scale_a_dev, scale_b_dev, c, ldc, bias_dev, (int)tiles_m, (int)tiles_n, c_vec_ok);
+    return launch_transposed(a_transposed != 0, a_fmt, b_fmt, c_dtype, stream, (const uint8_t*)a, lda, 64, (const uint8_t*)bt, ldb, 64, m, n, k, scale_a_dev,
+                             scale_b_dev, c, ldc, bias_dev, c_vec_ok);
 }

@@ -166,25 +166,6 @@ __device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[8][8], int m0, in
     }
 }
 
-typedef int v2i __attribute__((ext_vector_type(2)));
-
-// Four transpose reads = the 32 contraction bytes of one lane's MFMA operand (rows k0 + 8t .. + 7, t = 0..3, of
-// the lane's column): in every group of 16 lanes, lane i receives byte i%8 of the 8 bytes addressed by lanes
-// 2b + i/8 (b = 0..7); callers point lane j at (row k0 + j/2, column n0 + 8*(j%2)), so lane i gets column n0 + i.
-__device__ __forceinline__ v8i read_frag_tr(const uint8_t* p) {
-    typedef __attribute__((address_space(3))) v2i* lds_v2i;
-    const v2i r0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i)(p));
-    const v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i)(p + 2048));
-    const v2i r2 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i)(p + 4096));
-    const v2i r3 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i)(p + 6144));
-    return (v8i){r0.x, r0.y, r1.x, r1.y, r2.x, r2.y, r3.x, r3.y};
-}
-
-// f(k) of the transposed-slab swizzle: the 16-byte slot c of contraction row k sits at slot c ^ f(k).  One
-// transpose read touches rows 8t..8t+7 of two 32-row quarters per 32 lanes; f makes those 16 rows hit 16
-// different slots.
-__device__ __forceinline__ int tr_swizzle(int k) { return (k & 7) | (((k >> 5) & 1) << 3); }
-
 // ODD (from the host): the number of steps K/128 is odd.
 // A_TR / B_TR: the operand is given "transposed": its memory holds the matrix [contraction][rows] (the layout
 // in which another GEMM contracts over `rows`), a slab is 128 contraction rows x 256 row-bytes, and fragments

@@ -35,6 +35,26 @@ __device__ __forceinline__ v8i read_frag(const uint8_t* p0, const uint8_t* p1) {
     return (v8i){(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
 }
 
+typedef int v2i __attribute__((ext_vector_type(2)));
+
+// Four transpose reads = the 32 contraction bytes of one lane's MFMA operand (rows k0 + 8t .. + 7, t = 0..3, of
+// the lane's column): in every group of 16 lanes, lane i receives byte i%8 of the 8 bytes addressed by lanes
+// 2b + i/8 (b = 0..7); callers point lane j at (row k0 + j/2, column n0 + 8*(j%2)), so lane i gets column n0 + i.
+template <int ROW_BYTES = 256>
+__device__ __forceinline__ v8i read_frag_tr(const uint8_t* p) {
+    typedef __attribute__((address_space(3))) v2i* lds_v2i;
+    const v2i r0 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i)(p));
+    const v2i r1 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i)(p + 8 * ROW_BYTES));
+    const v2i r2 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i)(p + 16 * ROW_BYTES));
+    const v2i r3 = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i)(p + 24 * ROW_BYTES));
+    return (v8i){r0.x, r0.y, r1.x, r1.y, r2.x, r2.y, r3.x, r3.y};
+}
+
+// f(k) of the transposed-slab swizzle: the 16-byte slot c of contraction row k sits at slot c ^ f(k).  One
+// transpose read touches rows 8t..8t+7 of two 32-row quarters per 32 lanes; f makes those 16 rows hit 16
+// different slots.
+__device__ __forceinline__ int tr_swizzle(int k) { return (k & 7) | (((k >> 5) & 1) << 3); }
+
 template <int C_DT>
 __device__ __forceinline__ float load_bias(const void* bias, int col) {
     if constexpr (C_DT == F8MI_BF16) return bf16_bits_to_float(((const uint16_t*)bias)[col]);
@@ -238,6 +258,13 @@ int launch_gemm_mid_splitk(int a_fmt, int b_fmt, int c_dtype, bool wide, int k_s
 int launch_gemm_skinny(int a_fmt, int b_fmt, int c_dtype, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
                        const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C,
                        int64_t ldc, const void* bias);
+// The 128-row-tile kernel on the same transposed operands (f8mi_gemm_mid_nt.hip, f8mi_gemm_mid_tt.hip).
+int launch_gemm_mid_nt(int a_fmt, int b_fmt, int c_dtype, bool wide, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
+                       const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C,
+                       int64_t ldc, const void* bias, int c_vec_ok);
+int launch_gemm_mid_tt(int a_fmt, int b_fmt, int c_dtype, bool wide, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
+                       const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C,
+                       int64_t ldc, const void* bias, int c_vec_ok);
 int launch_gemm_dma16_nt(int a_fmt, int b_fmt, int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
                          const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb,
                          void* C, int64_t ldc, const void* bias, int tiles_m, int tiles_n, int c_vec_ok);

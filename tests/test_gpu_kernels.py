@@ -585,6 +585,27 @@ def test_gemm_mid_tile_kernel_step_counts(nat, m, n, mid, steps):
         _gemm_check(nat, m, n, 128 * steps, "e4m3", "e5m2", out_dt, seed=m + steps, bias=True)
 
 
+# Both tile widths of the 128-row kernel (1: 128 x 128, 2: 128 x 256) and large tiles with a sparse last round (0), edges at half
+# a tile, three to nine steps (the stages in flight are five and three).
+@pytest.mark.parametrize("m,n,k,mid", [(192, 320, 384, 1), (64, 64, 640, 1), (1024, 1088, 512, 1), (128, 4096, 1152, 1), (448, 8128, 768, 1),
+                                       (1344, 4032, 384, 2), (2048, 2304, 512, 2), (1984, 4096, 640, 2), (1088, 6464, 1152, 2),
+                                       (4352, 4096, 512, 0), (4416, 4032, 384, 0)])
+@pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float32])
+def test_gemm_mid_tile_kernel_reads_transposed_operands(nat, m, n, k, mid, out_dt):
+    """The same bits as on operands that are not transposed, for one and for both of them transposed."""
+    plan = nat.gemm_plan(m, n, k, split_k=False)
+    assert plan[0] == ("tiles256_and_128" if mid == 0 else "tiles128") and (mid == 0 or plan[2] == mid) or m <= 256
+    a = _rand_fp8((m, k), torch.float8_e5m2, m + k, 4.0).to(DEV)
+    bt = _rand_fp8((n, k), torch.float8_e4m3fn, n + k, 4.0).to(DEV)
+    sa, sb = torch.tensor(2.0, device=DEV), torch.tensor(0.25, device=DEV)
+    turned = lambda t: _to_kb(t.view(torch.uint8).t().contiguous().view(t.dtype))
+    bias = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 3).to(out_dt).to(DEV)
+    tall = torch.cat([a.view(torch.uint8), torch.zeros(272 - m if m <= 256 else 0, k, dtype=torch.uint8, device=DEV)]).view(a.dtype)  # past the few-row kernel
+    want = nat.gemm_nt_kb(_to_kb(tall), sa, _to_kb(bt), sb, out_dt, bias=bias, split_k=False)[:m]
+    assert torch.equal(nat.gemm_kb_ex(_to_kb(a), False, sa, turned(bt), True, sb, out_dt, bias=bias), want)
+    assert torch.equal(nat.gemm_kb_ex(turned(a), True, sa, turned(bt), True, sb, out_dt, bias=bias), want)
+
+
 # Few 128-row tiles and a long contraction: with the stream's scratch buffer k is split over workgroups and a second
 # kernel adds the parts in a fixed order.
 @pytest.mark.parametrize("m,n,k", [(256, 2048, 16384), (512, 1024, 8192), (100, 4096, 16384)])
