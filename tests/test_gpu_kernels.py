@@ -482,6 +482,29 @@ def test_cast_dynamic_equals_amax_scale_then_cast(nat, dt, shape):
     assert s.item() == s_want.item()
 
 
+# One copy of more than 32 K elements and at most 512 KB: one launch, whose workgroups take 8192 elements each.  The first such
+# size, a whole number of workgroups, one item more and less, the largest of 16-bit and of 32-bit types, the first beyond.
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("shape", [(1, 32776), (4097, 8), (5, 8192), (1, 40968), (3, 13656), (16, 4096), (16, 14336), (1, 131072), (1, 131080),
+                                   (64, 4096), (1, 262144), (1, 262152)])
+def test_cast_dynamic_one_copy_equals_amax_scale_then_cast(nat, dt, shape):
+    tdt = TORCH_DT[dt]
+    x = heavy(shape, tdt, 22).to(DEV)
+    shifted = torch.zeros(x.numel() + 1, device=DEV, dtype=tdt)[1:].view(shape)  # rows start at odd multiples of the element size
+    shifted.copy_(x)
+    wide = torch.cat([x, x], dim=1)[:, :shape[1]]  # more than one row: strided, the two kernels
+    first, last = x.clone(), x.clone()
+    first.view(-1)[0], last.view(-1)[-1] = float("inf"), float("nan")
+    for v in (x, shifted, wide, first, last, torch.zeros_like(x)):
+        for fmt, (code, f8dt) in F8.items():
+            _, s_want = nat.amax_scale(v, f8dt, want_amax=False)
+            for kb in {False, shape[1] % 64 == 0}:
+                o_want, _ = nat.cast(v, s_want, f8dt, out_kblock=kb)
+                o, _, s = nat.cast_dynamic(v, f8dt, out_kblock=kb)
+                assert s.view(torch.int32).item() == s_want.view(torch.int32).item() or (torch.isnan(s) and torch.isnan(s_want))
+                assert same_bytes_mod_nan_sign(fp8_bytes(o), fp8_bytes(o_want)), (dt, shape, fmt, kb)
+
+
 def _rand_fp8(shape, tdt, seed, scale=1.0):
     g = torch.Generator().manual_seed(seed)
     v = torch.randn(shape, generator=g) * scale
