@@ -443,6 +443,23 @@ def _kb_alloc(rows: int, kc: int, layout: int, float8_dtype, device) -> torch.Te
 TN_MIN_TILES = 32
 
 
+def _faster_split_over_k(rows, cols, kc) -> bool:
+    """``gemm_plan(rows, cols, kc)[0] == "tiles128_split_k"`` for dimensions that are multiples of 128 and at least 384, where the
+    few-row kernel plays no part: pick_k_splits of f8mi_gemm_util.h (an output of more than 128 tiles is not split; ``s`` parts
+    are taken if 4.4 ns per unit of k / s, the two launches and the traffic of the parts stay below 0.9 of 4.4 ns per unit of k) in
+    whole numbers, units of 0.1 ps.  Written out here because torch.compile works the rule out on symbolic sizes, which a call
+    into the library would pin to the values of the first call."""
+    tiles = (rows // 128) * (cols // 128)
+    if tiles > 128:
+        return False
+    for s in (2, 4, 8):
+        if tiles * s > 256 or kc < 1024 * s or kc % (128 * s) != 0 or 4 * s * rows * cols > GEMM_WORKSPACE_BYTES:
+            return False
+        if 44000 * kc + 70000000 * s + 16 * s * s * rows * cols < 39600 * kc * s:
+            return True
+    return False
+
+
 def tn_ok(m: int, k: int, n: int) -> bool:
     """True if a linear layer with m tokens, k in_features and n out_features should keep one k-blocked fp8 copy per
     tensor and let the backward GEMMs read it transposed (f8mi_gemm_kb_ex): every dimension a multiple of 128 and at
@@ -453,7 +470,7 @@ def tn_ok(m: int, k: int, n: int) -> bool:
     their transposed copies."""
     if not all(d % 128 == 0 and d >= KB_MIN_K for d in (m, k, n)):
         return False
-    return all((rows // 128) * (cols // 128) >= TN_MIN_TILES and gemm_plan(rows, cols, kc)[0] != "tiles128_split_k"
+    return all((rows // 128) * (cols // 128) >= TN_MIN_TILES and not _faster_split_over_k(rows, cols, kc)
                for rows, cols, kc in ((m, k, n), (n, k, m)))
 
 

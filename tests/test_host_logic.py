@@ -331,3 +331,30 @@ def test_sync_table_cache_does_not_trust_a_recycled_object_id(monkeypatch):
     layer.fp8_amax_input = torch.zeros(())
     assert flu._sync_table([layer]) is not fresh and len(built) == 3
     assert built[-1][0][0] is layer.fp8_amax_input
+
+
+def test_layout_rule_agrees_with_the_library_on_what_is_split_over_k():
+    """``tn_ok`` works out for itself which backward products the library would split over k."""
+    sizes = (384, 512, 640, 768, 1024, 1280, 1536, 2048, 2560, 3072, 4096, 5120)
+    lengths = (384, 1024, 2048, 2176, 2560, 3072, 3584, 4096, 4224, 4608, 5120, 6144, 7168, 8192, 10240, 11008, 14336, 16384, 28672, 57344)
+    split = [(r, c, k) for r in sizes for c in sizes for k in lengths if _native.gemm_plan(r, c, k)[0] == "tiles128_split_k"]
+    assert split and split == [(r, c, k) for r in sizes for c in sizes for k in lengths if _native._faster_split_over_k(r, c, k)]
+
+
+@pytest.mark.parametrize("m,k,n", [(512, 1024, 1024), (640, 4096, 8192), (1024, 4096, 4096), (4096, 1024, 1024), (16384, 1024, 8192)])
+def test_compiled_linear_keeps_a_symbolic_number_of_tokens(m, k, n):
+    """torch.compile with dynamic shapes: the layout rule must not pin the number of tokens to the first call's (a graph for
+    every size, and an error where the program has marked the dimension dynamic)."""
+    from torch._dynamo.source import ConstantSource
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.symbolic_shapes import ShapeEnv
+
+    env = ShapeEnv()
+    tokens = env.create_symintnode(env.create_symbol(m, ConstantSource("tokens")), hint=m)
+    with FakeTensorMode(shape_env=env):
+        x = torch.empty(tokens, k, device="cuda", dtype=torch.bfloat16)
+        w = torch.empty(n, k, device="cuda", dtype=torch.bfloat16)
+        y, xs, ws, sx, sw, _, _ = torch.ops.f8mi.linear_fwd(x, w, True, True, None, None)
+        dx, dw, _ = torch.ops.f8mi.linear_bwd(torch.empty_like(y), xs, ws, sx, sw, k, True, True, None)
+    assert not env.replacements, env.guards  # no symbol was replaced by a number
+    assert tuple(int(d) for d in y.shape) == (m, n) and tuple(int(d) for d in dx.shape) == (m, k)
