@@ -167,22 +167,23 @@ class _float8_linear_fn(torch.autograd.Function):
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         dy2 = dy.reshape(-1, dy.shape[-1])
         dx = dw = None
+        saved = ctx.saved_tensors  # once: non-reentrant checkpointing refuses to unpack a tensor a second time
         if ctx.layouts is not None and (need_dx or need_dw):
-            done = _native.linear_backward(dy2, *ctx.saved_tensors, ctx.x_shape[-1], ctx.layouts, need_dx, need_dw,
+            done = _native.linear_backward(dy2, *saved, ctx.x_shape[-1], ctx.layouts, need_dx, need_dw,
                                            mod._delayed_pair("grad_output"))
             if done is not None:
                 dx, dw = done
                 return dx if dx is None or len(ctx.x_shape) == 2 else dx.reshape(ctx.x_shape), dw, None, None
         dlg = mod._delayed_buffers("grad_output")
         if ctx.kb is None:  # one copy per tensor: x8 [K/64, M, 64], w8 [K/64, N, 64], g8 [N/64, M, 64]
-            x8, w8, sx, sw = ctx.saved_tensors
+            x8, w8, sx, sw = saved
             g8, _, sg = _cast_for_gemm(dy2, e5m2_dtype, dlg, ctx.is_amax_initialized, True, False, True, False)
             if need_dx:  # grad_input = dY @ W: dY as it is, W read transposed
                 dx = _native.gemm_kb_ex(g8, False, sg, w8, True, sw, dy.dtype).reshape(ctx.x_shape)
             if need_dw:  # grad_weight = dY^T @ x: both read transposed
                 dw = _native.gemm_kb_ex(g8, True, sg, x8, True, sx, dy.dtype)
             return dx, dw, None, None
-        x8t, w8t, sx, sw = ctx.saved_tensors
+        x8t, w8t, sx, sw = saved
         kb_dx, kb_dw = ctx.kb
         g8, g8t, sg = _cast_for_gemm(dy2, e5m2_dtype, dlg, ctx.is_amax_initialized, need_dx, need_dw, kb_dx, kb_dw)
         emulate = mod.linear_mm_config.grad_input.emulate

@@ -5,6 +5,7 @@ import logging
 import pytest
 import torch
 import torch.nn as nn
+import torch.utils.checkpoint
 
 import float8_experimental_amd as f8
 from float8_experimental_amd import _native
@@ -358,3 +359,24 @@ def test_compiled_linear_keeps_a_symbolic_number_of_tokens(m, k, n):
         dx, dw, _ = torch.ops.f8mi.linear_bwd(torch.empty_like(y), xs, ws, sx, sw, k, True, True, None)
     assert not env.replacements, env.guards  # no symbol was replaced by a number
     assert tuple(int(d) for d in y.shape) == (m, n) and tuple(int(d) for d in dx.shape) == (m, k)
+
+
+@pytest.mark.parametrize("one_copy", [True, False])
+def test_backward_unpacks_its_saved_tensors_once(monkeypatch, one_copy):
+    """Under non-reentrant checkpointing a saved tensor may be unpacked once.  A gradient that the native host path leaves to
+    the step-by-step functions (an expanded one, as ``y.sum().backward()`` hands it over) must not unpack it again.  The
+    kernels are stood in for by plain products: only who is called, and with what, is looked at."""
+    m, k, n = 4, 6, 8
+    layouts = (one_copy, 1, 1, 1)
+    scale = torch.ones(())
+    monkeypatch.setattr(_native, "linear_layouts", lambda *a: layouts)
+    monkeypatch.setattr(_native, "linear_forward", lambda x, w, *a: (x @ w.t(), x if one_copy else x.t(), w if one_copy else w.t(), scale, scale))
+    monkeypatch.setattr(_native, "linear_backward", lambda *a: None)
+    monkeypatch.setattr(_native, "cast_dynamic", lambda t, *a, **kw: (t, t.t(), scale))
+    monkeypatch.setattr(_native, "gemm_kb_ex", lambda a, at, sa, b, bt, sb, dtype: (a.t() if at else a) @ b)
+    monkeypatch.setattr(_native, "gemm_nt_kb", lambda a, sa, b, sb, dtype: a @ b.t())
+    mod = Float8Linear.from_float(nn.Linear(k, n, bias=False), config=cfg())
+    x = torch.randn(m, k, requires_grad=True)
+    torch.utils.checkpoint.checkpoint(mod, x, use_reentrant=False).sum().backward()
+    assert torch.allclose(x.grad, mod.weight.detach().sum(0).expand(m, -1))
+    assert torch.allclose(mod.weight.grad, x.detach().sum(0).expand(n, -1))
