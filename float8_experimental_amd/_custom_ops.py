@@ -126,8 +126,8 @@ def linear_fwd(x2: torch.Tensor, weight: torch.Tensor, need_dx: bool, need_dw: b
     """y = x2 W^T in fp8; also the fp8 copies and the dynamic scales backward needs, and the amaxes delayed scaling records.
 
     Returns (y, xs, ws, sx, sw, amax_x, amax_w).  When the sizes allow it (``_native.tn_ok``) xs / ws are the
-    forward's own k-blocked operands (backward reads them transposed); otherwise they are the transposed copies,
-    and one that backward will not need is an empty tensor.  sx / sw are the scales of dynamically scaled
+    forward's own k-blocked operands (backward reads them transposed); otherwise they are the transposed copies.
+    One that backward will not need is an empty tensor.  sx / sw are the scales of dynamically scaled
     tensors; for a tensor with delayed scaling (``scale_*`` given: the module's scale buffer) the slot holds an empty
     tensor and ``amax_*`` this step's amax, [1] fp32 (empty for dynamic scaling)."""
     with _native.transient_workspaces():
@@ -142,11 +142,12 @@ def _linear_fwd_impl(x2, weight, need_dx, need_dw, scale_x, scale_w):
     if _native.tn_ok(m, k, n):
         x8, _, sx, ax = _cast(x2, e4m3_dtype, scale_x, True, False, True, False)
         w8, _, sw, aw = _cast(weight, e4m3_dtype, scale_w, True, False, True, False)
-        return _native.gemm_nt_kb(x8, sx, w8, sw, x2.dtype), x8, w8, out_s(sx, scale_x), out_s(sw, scale_w), ax, aw
-    kb_fwd, kb_dx, kb_dw = _native.kblock_layout(k), _native.kblock_layout(n), _native.kblock_layout(m)
-    x8, x8t, sx, ax = _cast(x2, e4m3_dtype, scale_x, True, need_dw, kb_fwd, kb_dw)
-    w8, w8t, sw, aw = _cast(weight, e4m3_dtype, scale_w, True, need_dx, kb_fwd, kb_dx)
-    y = _gemm(x8, sx, w8, sw, x2.dtype, kb_fwd)
+        y, x8t, w8t = _native.gemm_nt_kb(x8, sx, w8, sw, x2.dtype), x8, w8
+    else:
+        kb_fwd, kb_dx, kb_dw = _native.kblock_layout(k), _native.kblock_layout(n), _native.kblock_layout(m)
+        x8, x8t, sx, ax = _cast(x2, e4m3_dtype, scale_x, True, need_dw, kb_fwd, kb_dw)
+        w8, w8t, sw, aw = _cast(weight, e4m3_dtype, scale_w, True, need_dx, kb_fwd, kb_dx)
+        y = _gemm(x8, sx, w8, sw, x2.dtype, kb_fwd)
     return (y, (x8t if need_dw else none(e4m3_dtype)), (w8t if need_dx else none(e4m3_dtype)),
             out_s(sx, scale_x), out_s(sw, scale_w), ax, aw)
 
@@ -160,10 +161,10 @@ def _(x2, weight, need_dx, need_dw, scale_x, scale_w):
     a = lambda buf: torch.empty((0,) if buf is None else (1,), dtype=torch.float32, device=x2.device)
     y = torch.empty((m, n), dtype=x2.dtype, device=x2.device)
     if _native.tn_ok(m, k, n):
-        return y, f8((k // _KB, m, _KB)), f8((k // _KB, n, _KB)), s(scale_x), s(scale_w), a(scale_x), a(scale_w)
-    kb_dx, kb_dw = _native.kblock_layout(n), _native.kblock_layout(m)
-    return (y, f8(_layout(k, m, kb_dw)) if need_dw else f8((0,)), f8(_layout(k, n, kb_dx)) if need_dx else f8((0,)),
-            s(scale_x), s(scale_w), a(scale_x), a(scale_w))
+        xs, ws = (k // _KB, m, _KB), (k // _KB, n, _KB)
+    else:
+        xs, ws = _layout(k, m, _native.kblock_layout(m)), _layout(k, n, _native.kblock_layout(n))
+    return (y, f8(xs if need_dw else (0,)), f8(ws if need_dx else (0,)), s(scale_x), s(scale_w), a(scale_x), a(scale_w))
 
 
 @torch.library.custom_op("f8mi::linear_bwd", mutates_args=())

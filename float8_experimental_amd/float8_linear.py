@@ -136,7 +136,7 @@ class _float8_linear_fn(torch.autograd.Function):
                 y, xs, ws, sx, sw = done
                 ctx.layouts = layouts
                 ctx.kb = None if layouts[0] else layouts[2:]
-                ctx.save_for_backward(xs, ws, sx, sw)
+                ctx.save_for_backward(xs if need_dw else None, ws if need_dx else None, sx, sw)
                 return y if x.dim() == 2 else y.reshape(*x.shape[:-1], n)
         tn = not emulate and not emulate_bw and _native.tn_ok(m, k, n)
         if tn:
@@ -145,7 +145,7 @@ class _float8_linear_fn(torch.autograd.Function):
                                         known_scale=mod._precomputed_weight_scale)
             y = _native.gemm_nt_kb(x8, sx, w8, sw, x.dtype)
             ctx.kb = None
-            ctx.save_for_backward(x8, w8, sx, sw)
+            ctx.save_for_backward(x8 if need_dw else None, w8 if need_dx else None, sx, sw)
         else:
             kb_fwd = 0 if emulate else _native.kblock_layout(k)      # y = x W^T contracts in_features
             kb_dx = 0 if emulate_bw else _native.kblock_layout(n)    # dx = dy W contracts out_features

@@ -380,3 +380,26 @@ def test_backward_unpacks_its_saved_tensors_once(monkeypatch, one_copy):
     torch.utils.checkpoint.checkpoint(mod, x, use_reentrant=False).sum().backward()
     assert torch.allclose(x.grad, mod.weight.detach().sum(0).expand(m, -1))
     assert torch.allclose(mod.weight.grad, x.detach().sum(0).expand(n, -1))
+
+
+@pytest.mark.parametrize("need_dx,need_dw", [(True, False), (False, True), (True, True)])
+def test_layers_with_one_fp8_copy_save_only_what_backward_reads(monkeypatch, need_dx, need_dw):
+    """A frozen weight needs no fp8 copy of the activations in backward, a first layer none of the weight."""
+    m, k, n = 512, 1024, 1152
+    assert _native.tn_ok(m, k, n)
+    f8t = lambda *shape: torch.zeros(shape, dtype=torch.float8_e4m3fn)
+    one = torch.ones(())
+    monkeypatch.setattr(_native, "linear_forward", lambda x, w, *a: (x @ w.t(), f8t(k // 64, m, 64), f8t(k // 64, n, 64), one, one))
+    mod = Float8Linear.from_float(nn.Linear(k, n, bias=False), config=cfg())
+    mod.weight.requires_grad_(need_dw)
+    saved = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(tuple(t.shape)) or t, lambda t: t):
+        mod(torch.randn(m, k, requires_grad=need_dx))
+    assert (k // 64, m, 64) in saved if need_dw else (k // 64, m, 64) not in saved
+    assert (k // 64, n, 64) in saved if need_dx else (k // 64, n, 64) not in saved
+
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():  # the same through torch.compile's node
+        x, w = (torch.empty(r, k, device="cuda", dtype=torch.bfloat16) for r in (m, n))
+        _, xs, ws, *_ = torch.ops.f8mi.linear_fwd(x, w, need_dx, need_dw, None, None)
+    assert xs.numel() == (m * k if need_dw else 0) and ws.numel() == (n * k if need_dx else 0)
