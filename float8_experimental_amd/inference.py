@@ -15,6 +15,8 @@ from typing import Callable, Optional
 
 import torch
 import torch.nn as nn
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _custom_ops  # noqa: F401  (registers torch.ops.f8mi.*)
 from . import _native
@@ -140,11 +142,19 @@ def _inference_linear_traced(x2: torch.Tensor, weight: "Float8Tensor", static_sc
 WEIGHT_ONLY_MAX_ROWS = 128
 
 
+def _function_mode_active() -> bool:
+    """True under a ``TorchFunctionMode`` that may want to see ``F.linear``; ``torch.set_default_device`` is one that does not."""
+    return torch._C._len_torch_function_stack() > 0 and any(not isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack())
+
+
 def _weight_only_kernels_take(input: torch.Tensor, weight: "Float8Tensor") -> bool:
     """True if the weight-only kernels compute what ``F.linear(input, weight.to_original_precision())`` would: plain
-    tensors of the weight's own type on the current device, nothing to record for autograd and nobody (a compiler, a
-    functional transform, a dispatch mode) who has to see the operators."""
+    tensors of the weight's own type on the current device whose memory holds their values (not sparse, nested or a lazy
+    negation), nothing to record for autograd and nobody (a compiler, a functional transform, a dispatch or function mode)
+    who has to see the operators."""
     if torch.compiler.is_compiling() or type(weight) is not Float8Tensor or type(input) not in (torch.Tensor, nn.Parameter):
+        return False
+    if input.layout is not torch.strided or input.is_nested or input.is_neg() or input._is_zerotensor() or _function_mode_active():
         return False
     data, scale = weight._data, weight._scale
     return (input.is_cuda and input.dtype == weight._orig_dtype and input.dtype in _native._DT and data.dtype in _native._F8

@@ -295,6 +295,36 @@ def test_weight_only_leaves_other_calls_to_the_library_product(f8):
         assert torch.equal(torch.autograd.forward_ad.unpack_dual(y).tangent, torch.nn.functional.linear(tangent, w))
 
 
+def test_weight_only_leaves_function_modes_and_lazy_or_nested_inputs_to_the_library_product(f8):
+    """A TorchFunctionMode sees (and may replace) F.linear as on any nn.Linear; a nested tensor has no sizes for the kernel, a
+    lazily negated one not its own values in memory.  torch.set_default_device is a function mode that asks for nothing."""
+    from float8_experimental_amd import inference
+
+    lin = torch.nn.Linear(128, 64, bias=False, device=DEV, dtype=torch.bfloat16)
+    lin = inference.quantize_to_float8(lin, inference.QuantConfig(inference.ActivationCasting.WEIGHT_ONLY))
+    w = lin.weight._data.to(torch.bfloat16) / lin.weight._scale
+    x = torch.randn(3, 128, device=DEV, dtype=torch.bfloat16)
+
+    class Doubles(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            out = func(*args, **(kwargs or {}))
+            return out * 2 if func is torch.nn.functional.linear else out
+
+    with torch.no_grad():
+        want = torch.nn.functional.linear(x, w)
+        with Doubles():
+            got = lin(x)
+        assert torch.equal(got, want * 2)
+        with torch.device("cuda"):
+            assert inference._weight_only_kernels_take(x, lin.weight)
+        neg = torch._neg_view(x)
+        assert neg.is_neg() and torch.equal(lin(neg), torch.nn.functional.linear(-x, w))
+        nested = torch.nested.nested_tensor([x[:1], x[:2]], device=DEV)
+        for got, rows in zip(lin(nested).unbind(), (x[:1], x[:2])):
+            assert torch.allclose(got.float(), torch.nn.functional.linear(rows, w).float(), rtol=2.0 ** -7, atol=1e-2)
+        assert not inference._weight_only_kernels_take(x.to_sparse_csr(), lin.weight)
+
+
 @pytest.mark.parametrize("m,k,n", [(1, 8192, 512), (1, 128, 16), (2, 256, 100), (16, 384, 8200), (16, 2048, 1000), (16, 2176, 24), (7, 4096, 8197),
                                    (5, 1152, 33), (16, 14336, 64)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
