@@ -13,6 +13,7 @@
 // the tile is read back as 16-byte row pieces: 8 lanes = one 128-byte segment of
 // a row of the transposed output.
 #include <atomic>
+#include <mutex>
 
 #include "f8mi_cast_util.h"
 
@@ -601,11 +602,22 @@ extern "C" int f8mi_cast(const void* x, int64_t rows, int64_t cols, int64_t ld, 
 
 extern "C" size_t f8mi_delayed_workspace_bytes(void) { return SPREAD_WORDS * sizeof(uint32_t); }
 
+namespace f8mi {
+// Host threads that share a workspace (and with it a stream) queue the cast and its finalize launch one pair at a time: with the
+// finalize of one between the cast and the finalize of another, the first would take, and clear, both maxima.  The workspaces of
+// different streams mostly find different locks; none is held for longer than two launches take to queue.
+static std::mutex& delayed_lock(const void* workspace) {
+    static std::mutex locks[64];
+    return locks[((uintptr_t)workspace >> 12) % 64];
+}
+}  // namespace f8mi
+
 extern "C" int f8mi_cast_delayed(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, const float* scale_dev, int fp8_fmt,
                                  uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout, float* amax_dev, void* workspace,
                                  void* stream) {
     if (!amax_dev) { set_error("f8mi_cast_delayed: null amax"); return F8MI_ERR_INVALID_ARG; }
     if (!workspace || (uintptr_t)workspace % 4 != 0) { set_error("f8mi_cast_delayed: null or misaligned workspace"); return F8MI_ERR_INVALID_ARG; }
+    const std::lock_guard<std::mutex> guard(f8mi::delayed_lock(workspace));
     return cast_layout_impl(x, rows, cols, ld, in_dtype, scale_dev, F8MI_FP32, fp8_fmt, out, out_layout, out_t, out_t_layout, amax_dev,
                             (hipStream_t)stream, AmaxSource{nullptr, 0, nullptr, (uint32_t*)workspace});
 }

@@ -825,3 +825,30 @@ def test_native_host_path_leaves_what_it_does_not_take_to_the_step_by_step_funct
     for bad in (call(x.t().contiguous().t(), w), call(x[0].expand(64, 512), w), call(x[:0], w), call(x.double(), w), call(x, w[:, :-1]),
                 call(x, w, scale=one.double()), call(x, w, scale=torch.ones(2, device=DEV)), call(x, w, dx=(one, one.cpu()))):
         assert bad is None
+
+
+def test_delayed_casts_of_two_threads_on_one_stream_keep_their_maxima_apart(f8):
+    """Cast and finalize of one call are two launches over words that calls on one stream share: another thread's cast must not
+    come between them."""
+    import threading
+
+    from float8_experimental_amd import _native
+
+    calls, scale = 2000, torch.ones(1, device=DEV)
+    amaxes = {v: torch.zeros(calls, device=DEV) for v in (1.0, 300.0)}
+    start = threading.Barrier(2)
+
+    def work(v):
+        x = torch.full((64, 128), v, device=DEV, dtype=torch.bfloat16)
+        out = amaxes[v]
+        start.wait()
+        for i in range(calls):
+            _native.cast(x, scale, torch.float8_e4m3fn, product_dtype=torch.float32, amax_out=out[i:i + 1])
+
+    _native.delayed_workspace(scale.device)
+    threads = [threading.Thread(target=work, args=(v,)) for v in amaxes]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all((got == v).all() for v, got in amaxes.items())
