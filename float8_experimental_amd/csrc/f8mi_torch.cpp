@@ -7,7 +7,11 @@
 // Every function returns None, without having queued or allocated anything, for arguments that it does not take (subclasses,
 // other devices, layouts that need a copy, odd scales): the caller then goes through the checked Python functions of
 // _native.py, which raise what there is to raise.  Workspaces are temporaries of torch's caching allocator: it hands their
-// memory out again in stream order, so calls on any number of threads, streams and captures share nothing.
+// memory out again in stream order, so calls on any number of threads, streams and captures share nothing but the delayed
+// cast's words, which the library guards.
+//
+// The Python arguments are read first, tensors by value; allocations and launches then run without the GIL, as under ctypes and
+// torch's own bindings: a launch may block on a full queue, an allocation on hipMalloc, and other Python threads go on.
 #include <dlfcn.h>
 
 #include <ATen/ATen.h>
@@ -47,38 +51,37 @@ int fp8_code(at::ScalarType t) { return t == at::kFloat8_e4m3fn ? F8MI_E4M3FN : 
 at::ScalarType fp8_type(int fmt) { return fmt == F8MI_E4M3FN ? at::kFloat8_e4m3fn : at::kFloat8_e5m2; }
 int64_t padded(int64_t k, int layout) { return layout == F8MI_LAYOUT_KBLOCK64_PAD128 ? (k + 127) / 128 * 128 : k; }
 
-// a plain tensor (or Parameter) on the current device: nothing of a subclass, no other layout
-const at::Tensor* plain(PyObject* o, int device) {
-    if (!THPVariable_CheckExact(o)) return nullptr;
+// Undefined: not taken.  A plain tensor (or Parameter) on the current device: nothing of a subclass, no other layout ...
+at::Tensor plain(PyObject* o, int device) {
+    if (!THPVariable_CheckExact(o)) return {};
     const at::Tensor& t = THPVariable_Unpack(o);
-    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.get_device() == device ? &t : nullptr;
+    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.get_device() == device ? t : at::Tensor();
 }
 // ... that the cast kernels read as it is: 2-D, not empty, unit column stride
-const at::Tensor* matrix(PyObject* o, int device) {
-    const at::Tensor* t = plain(o, device);
-    return t && t->dim() == 2 && dtype_code(t->scalar_type()) >= 0 && t->size(0) > 0 && t->size(1) > 0 && t->stride(1) == 1 && t->stride(0) >= t->size(1) ? t : nullptr;
+at::Tensor matrix(PyObject* o, int device) {
+    const at::Tensor t = plain(o, device);
+    return t.defined() && t.dim() == 2 && dtype_code(t.scalar_type()) >= 0 && t.size(0) > 0 && t.size(1) > 0 && t.stride(1) == 1 && t.stride(0) >= t.size(1) ? t : at::Tensor();
 }
 // ... one fp32 element: a scale or an amax
-const at::Tensor* one_float(PyObject* o, int device) {
-    const at::Tensor* t = plain(o, device);
-    return t && t->scalar_type() == at::kFloat && t->numel() == 1 ? t : nullptr;
+at::Tensor one_float(PyObject* o, int device) {
+    const at::Tensor t = plain(o, device);
+    return t.defined() && t.scalar_type() == at::kFloat && t.numel() == 1 ? t : at::Tensor();
 }
 
 // How one tensor is scaled: dynamically, with a scale known beforehand, or delayed (with its amax buffer).
 struct Scaling {
-    const at::Tensor* scale = nullptr;
-    const at::Tensor* amax = nullptr;
+    at::Tensor scale, amax;
     // `known`: a scale or None; `delayed`: (amax, scale) or None.  False: not taken.
     bool parse(PyObject* known, PyObject* delayed, int device) {
         if (delayed != Py_None) {
             if (!PyTuple_Check(delayed) || PyTuple_GET_SIZE(delayed) != 2) return false;
             amax = one_float(PyTuple_GET_ITEM(delayed, 0), device);
             scale = one_float(PyTuple_GET_ITEM(delayed, 1), device);
-            return amax && scale;
+            return amax.defined() && scale.defined();
         }
         if (known == Py_None) return true;
         scale = one_float(known, device);
-        return scale != nullptr;
+        return scale.defined();
     }
 };
 
@@ -105,17 +108,17 @@ struct Call {
         if (want_tr) tr = copy(k, m, tr_layout, fmt);
         uint8_t* pr = want_row ? (uint8_t*)row.data_ptr() : nullptr;
         uint8_t* pt = want_tr ? (uint8_t*)tr.data_ptr() : nullptr;
-        if (!s.scale) {
+        if (!s.scale.defined()) {
             scale = make({}, at::kFloat);
             const at::Tensor ws = make({(int64_t)L.workspace_bytes / 4}, at::kInt);
             check(L.cast_dynamic(x.data_ptr(), m, k, ld, dt, fmt, (float*)scale.data_ptr(), pr, row_layout, pt, tr_layout, ws.data_ptr(), stream),
                   "f8mi_cast_dynamic");
             return;
         }
-        scale = *s.scale;
-        if (s.amax)
+        scale = s.scale;
+        if (s.amax.defined())
             check(L.cast_delayed(x.data_ptr(), m, k, ld, dt, (const float*)scale.data_ptr(), fmt, pr, row_layout, pt, tr_layout,
-                                 (float*)s.amax->data_ptr(), delayed_ws, stream), "f8mi_cast_delayed");
+                                 (float*)s.amax.data_ptr(), delayed_ws, stream), "f8mi_cast_delayed");
         else
             check(L.cast_layout(x.data_ptr(), m, k, ld, dt, (const float*)scale.data_ptr(), product_dtype < 0 ? dt : product_dtype, fmt, pr, row_layout,
                                 pt, tr_layout, nullptr, stream), "f8mi_cast_layout");
@@ -123,7 +126,7 @@ struct Call {
 
     // a [m][k] times bt [n][k] in the layout, both contracting over kc (before padding)
     at::Tensor gemm(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& bt, const at::Tensor& sb, int layout, int64_t m, int64_t n,
-                    int64_t kc, at::ScalarType out, const at::Tensor* bias = nullptr) const {
+                    int64_t kc, at::ScalarType out, const at::Tensor& bias = {}) const {
         at::Tensor c = make({m, n}, out), ws;
         const int64_t k = padded(kc, layout);
         int64_t ws_bytes = 0;
@@ -137,7 +140,7 @@ struct Call {
         void* pws = ws_bytes ? ws.data_ptr() : nullptr;
         const float *pa = (const float*)sa.data_ptr(), *pb = (const float*)sb.data_ptr();
         const int fa = fp8_code(a.scalar_type()), fb = fp8_code(bt.scalar_type()), dt = dtype_code(out);
-        const void* pbias = bias ? bias->data_ptr() : nullptr;
+        const void* pbias = bias.defined() ? bias.data_ptr() : nullptr;
         if (layout == F8MI_LAYOUT_ROWMAJOR)
             check(L.gemm_nt_ws(a.data_ptr(), fa, k, bt.data_ptr(), fb, k, m, n, k, pa, pb, c.data_ptr(), dt, n, pbias, pws, ws_bytes, stream), "f8mi_gemm_nt_ws");
         else
@@ -165,6 +168,10 @@ PyObject* wrap_all(const T&... t) {
     for (PyObject* o : {wrap(t)...}) PyTuple_SET_ITEM(r, i++, o);
     return r;
 }
+struct WithoutGil {
+    PyThreadState* state = PyEval_SaveThread();
+    ~WithoutGil() { PyEval_RestoreThread(state); }
+};
 template <typename F>
 PyObject* guarded(F body) {
     HANDLE_TH_ERRORS
@@ -191,17 +198,19 @@ PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (!expect(n_args, 14, "linear_forward")) return nullptr;
     return guarded([&]() -> PyObject* {
         const Call c{as_ptr(a[13]), as_int(a[12]), as_ptr(a[11])};
-        const at::Tensor *x = matrix(a[0], c.device), *w = matrix(a[1], c.device);
+        const at::Tensor x = matrix(a[0], c.device), w = matrix(a[1], c.device);
         Scaling in, we;
-        if (!x || !w || x->size(1) != w->size(1) || !in.parse(Py_None, a[8], c.device) || !we.parse(a[10], a[9], c.device)) Py_RETURN_NONE;
-        if ((in.amax || we.amax) && !c.delayed_ws) Py_RETURN_NONE;
+        if (!x.defined() || !w.defined() || x.size(1) != w.size(1) || !in.parse(Py_None, a[8], c.device) || !we.parse(a[10], a[9], c.device)) Py_RETURN_NONE;
+        if ((in.amax.defined() || we.amax.defined()) && !c.delayed_ws) Py_RETURN_NONE;
         const bool one_copy = as_int(a[2]), need_dx = as_int(a[6]), need_dw = as_int(a[7]);
         const int kb_fwd = as_int(a[3]), kb_dx = as_int(a[4]), kb_dw = as_int(a[5]);
-        const int64_t m = x->size(0), k = x->size(1), n = w->size(0);
-        at::Tensor x8, x8t, sx, w8, w8t, sw;
-        c.cast(*x, in, F8MI_E4M3FN, true, kb_fwd, !one_copy && need_dw, kb_dw, x8, x8t, sx);
-        c.cast(*w, we, F8MI_E4M3FN, true, kb_fwd, !one_copy && need_dx, kb_dx, w8, w8t, sw);
-        const at::Tensor y = c.gemm(x8, sx, w8, sw, kb_fwd, m, n, k, x->scalar_type());
+        at::Tensor y, x8, x8t, sx, w8, w8t, sw;
+        {
+            const WithoutGil no_gil;
+            c.cast(x, in, F8MI_E4M3FN, true, kb_fwd, !one_copy && need_dw, kb_dw, x8, x8t, sx);
+            c.cast(w, we, F8MI_E4M3FN, true, kb_fwd, !one_copy && need_dx, kb_dx, w8, w8t, sw);
+            y = c.gemm(x8, sx, w8, sw, kb_fwd, x.size(0), w.size(0), x.size(1), x.scalar_type());
+        }
         if (one_copy) return wrap_all(y, x8, w8, sx, sw);
         return wrap_all(y, x8t, w8t, sx, sw);
     });
@@ -213,31 +222,36 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (!expect(n_args, 15, "linear_backward")) return nullptr;
     return guarded([&]() -> PyObject* {
         const Call c{as_ptr(a[14]), as_int(a[13]), as_ptr(a[12])};
-        const at::Tensor* dy = matrix(a[0], c.device);
+        const at::Tensor dy = matrix(a[0], c.device);
         const bool one_copy = as_int(a[6]), need_dx = as_int(a[9]), need_dw = as_int(a[10]);
-        const at::Tensor *xs = need_dw ? plain(a[1], c.device) : nullptr, *ws = need_dx ? plain(a[2], c.device) : nullptr;
-        const at::Tensor *sx = one_float(a[3], c.device), *sw = one_float(a[4], c.device);
+        const at::Tensor xs = need_dw ? plain(a[1], c.device) : at::Tensor(), ws = need_dx ? plain(a[2], c.device) : at::Tensor();
+        const at::Tensor sx = one_float(a[3], c.device), sw = one_float(a[4], c.device);
         Scaling go;
-        if (!dy || !sx || !sw || (need_dw && !xs) || (need_dx && !ws) || !(need_dx || need_dw) || !go.parse(Py_None, a[11], c.device)) Py_RETURN_NONE;
-        if (go.amax && !c.delayed_ws) Py_RETURN_NONE;
+        if (!dy.defined() || !sx.defined() || !sw.defined() || xs.defined() != need_dw || ws.defined() != need_dx || !(need_dx || need_dw) ||
+            !go.parse(Py_None, a[11], c.device))
+            Py_RETURN_NONE;
+        if (go.amax.defined() && !c.delayed_ws) Py_RETURN_NONE;
         const int kb_dx = as_int(a[7]), kb_dw = as_int(a[8]);
-        const int64_t m = dy->size(0), n = dy->size(1), k = PyLong_AsLongLong(a[5]);
+        const int64_t m = dy.size(0), n = dy.size(1), k = PyLong_AsLongLong(a[5]);
         // what saved-tensor hooks hand back has to be what was saved: dense fp8 copies of the sizes the products assume
-        for (const at::Tensor* t : {xs, ws}) {
-            if (!t) continue;
-            const int64_t rows = one_copy ? (t == xs ? m : n) : k, kc = one_copy ? k : (t == xs ? m : n);
-            const int layout = one_copy ? F8MI_LAYOUT_KBLOCK64 : t == xs ? kb_dw : kb_dx;
+        for (const at::Tensor* t : {&xs, &ws}) {
+            if (!t->defined()) continue;
+            const int64_t rows = one_copy ? (t == &xs ? m : n) : k, kc = one_copy ? k : (t == &xs ? m : n);
+            const int layout = one_copy ? F8MI_LAYOUT_KBLOCK64 : t == &xs ? kb_dw : kb_dx;
             if (fp8_code(t->scalar_type()) < 0 || !t->is_contiguous() || t->numel() != rows * padded(kc, layout)) Py_RETURN_NONE;
         }
         at::Tensor g8, g8t, sg, dx, dw;
-        if (one_copy) {
-            c.cast(*dy, go, F8MI_E5M2, true, F8MI_LAYOUT_KBLOCK64, false, 0, g8, g8t, sg);
-            if (need_dx) dx = c.gemm_tr(g8, false, sg, *ws, *sw, m, k, n, dy->scalar_type());
-            if (need_dw) dw = c.gemm_tr(g8, true, sg, *xs, *sx, n, k, m, dy->scalar_type());
-        } else {
-            c.cast(*dy, go, F8MI_E5M2, need_dx, kb_dx, need_dw, kb_dw, g8, g8t, sg);
-            if (need_dx) dx = c.gemm(g8, sg, *ws, *sw, kb_dx, m, k, n, dy->scalar_type());
-            if (need_dw) dw = c.gemm(g8t, sg, *xs, *sx, kb_dw, n, k, m, dy->scalar_type());
+        {
+            const WithoutGil no_gil;
+            if (one_copy) {
+                c.cast(dy, go, F8MI_E5M2, true, F8MI_LAYOUT_KBLOCK64, false, 0, g8, g8t, sg);
+                if (need_dx) dx = c.gemm_tr(g8, false, sg, ws, sw, m, k, n, dy.scalar_type());
+                if (need_dw) dw = c.gemm_tr(g8, true, sg, xs, sx, n, k, m, dy.scalar_type());
+            } else {
+                c.cast(dy, go, F8MI_E5M2, need_dx, kb_dx, need_dw, kb_dw, g8, g8t, sg);
+                if (need_dx) dx = c.gemm(g8, sg, ws, sw, kb_dx, m, k, n, dy.scalar_type());
+                if (need_dw) dw = c.gemm(g8t, sg, xs, sx, kb_dw, n, k, m, dy.scalar_type());
+            }
         }
         return wrap_all(dx, dw);
     });
@@ -248,30 +262,38 @@ PyObject* inference_linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (!expect(n_args, 9, "inference_linear")) return nullptr;
     return guarded([&]() -> PyObject* {
         const Call c{as_ptr(a[8]), as_int(a[7]), nullptr};
-        const at::Tensor *x = matrix(a[0], c.device), *w = plain(a[1], c.device), *sw = one_float(a[4], c.device);
-        const at::Tensor* bias = a[6] == Py_None ? nullptr : plain(a[6], c.device);
+        const at::Tensor x = matrix(a[0], c.device), w = plain(a[1], c.device), sw = one_float(a[4], c.device);
+        const at::Tensor bias = a[6] == Py_None ? at::Tensor() : plain(a[6], c.device);
         const int64_t n = PyLong_AsLongLong(a[2]);
         const int layout = as_int(a[3]);
         Scaling in;
-        if (!x || !w || !sw || (a[6] != Py_None && !bias) || !in.parse(a[5], Py_None, c.device)) Py_RETURN_NONE;
-        const int64_t m = x->size(0), k = x->size(1);
-        if (n <= 0 || fp8_code(w->scalar_type()) < 0 || !w->is_contiguous() || w->numel() != n * padded(k, layout)) Py_RETURN_NONE;
-        if (bias && (bias->scalar_type() != x->scalar_type() || bias->numel() != n || !bias->is_contiguous())) Py_RETURN_NONE;
+        if (!x.defined() || !w.defined() || !sw.defined() || (a[6] != Py_None && !bias.defined()) || !in.parse(a[5], Py_None, c.device)) Py_RETURN_NONE;
+        const int64_t m = x.size(0), k = x.size(1);
+        if (n <= 0 || fp8_code(w.scalar_type()) < 0 || !w.is_contiguous() || w.numel() != n * padded(k, layout)) Py_RETURN_NONE;
+        if (bias.defined() && (bias.scalar_type() != x.scalar_type() || bias.numel() != n || !bias.is_contiguous())) Py_RETURN_NONE;
         // a 0-dim scale leaves the product in x's dtype, a scale with a dimension promotes it to fp32
-        const int dt = dtype_code(x->scalar_type()), product = in.scale && in.scale->dim() > 0 ? F8MI_FP32 : dt;
-        if (m <= 16 && m * k <= F8MI_FEW_ROWS_ELEMS && layout != F8MI_LAYOUT_KBLOCK64_PAD128) {  // cast and product in one kernel
-            const at::Tensor y = c.make({m, n}, x->scalar_type());
-            const int rc = L.linear_few_rows(x->data_ptr(), x->stride(0), dt, in.scale ? (const float*)in.scale->data_ptr() : nullptr, product, w->data_ptr(),
-                                             fp8_code(w->scalar_type()), layout, (const float*)sw->data_ptr(), m, n, k, y.data_ptr(), n,
-                                             bias ? bias->data_ptr() : nullptr, c.stream);
-            if (rc != F8MI_ERR_UNSUPPORTED) {
-                check(rc, "f8mi_linear_few_rows");
-                return wrap(y);
+        const int dt = dtype_code(x.scalar_type()), product = in.scale.defined() && in.scale.dim() > 0 ? F8MI_FP32 : dt;
+        const auto compute = [&]() -> at::Tensor {
+            if (m <= 16 && m * k <= F8MI_FEW_ROWS_ELEMS && layout != F8MI_LAYOUT_KBLOCK64_PAD128) {  // cast and product in one kernel
+                const at::Tensor y = c.make({m, n}, x.scalar_type());
+                const int rc = L.linear_few_rows(x.data_ptr(), x.stride(0), dt, in.scale.defined() ? (const float*)in.scale.data_ptr() : nullptr, product,
+                                                 w.data_ptr(), fp8_code(w.scalar_type()), layout, (const float*)sw.data_ptr(), m, n, k, y.data_ptr(), n,
+                                                 bias.defined() ? bias.data_ptr() : nullptr, c.stream);
+                if (rc != F8MI_ERR_UNSUPPORTED) {
+                    check(rc, "f8mi_linear_few_rows");
+                    return y;
+                }
             }
+            at::Tensor x8, none, sx;
+            c.cast(x, in, F8MI_E4M3FN, true, layout, false, 0, x8, none, sx, product);
+            return c.gemm(x8, sx, w, sw, layout, m, n, k, x.scalar_type(), bias);
+        };
+        at::Tensor y;
+        {
+            const WithoutGil no_gil;
+            y = compute();
         }
-        at::Tensor x8, none, sx;
-        c.cast(*x, in, F8MI_E4M3FN, true, layout, false, 0, x8, none, sx, product);
-        return wrap(c.gemm(x8, sx, *w, *sw, layout, m, n, k, x->scalar_type(), bias));
+        return wrap(y);
     });
 }
 

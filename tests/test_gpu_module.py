@@ -852,3 +852,66 @@ def test_delayed_casts_of_two_threads_on_one_stream_keep_their_maxima_apart(f8):
     for t in threads:
         t.join()
     assert all((got == v).all() for v, got in amaxes.items())
+
+
+_SLOW_LIBRARY = """
+#include <stddef.h>
+#include <stdint.h>
+#include <unistd.h>
+static int slow(void) { usleep(150000); return 0; }
+size_t f8mi_workspace_bytes(void) { return 4096; }
+const char* f8mi_last_error(void) { return ""; }
+int f8mi_gemm_plan(int64_t m, int64_t n, int64_t k, int a, int64_t w) { return 0; }
+int f8mi_cast_dynamic(void) { return slow(); }
+int f8mi_cast_layout(void) { return slow(); }
+int f8mi_cast_delayed(void) { return slow(); }
+int f8mi_gemm_nt_ws(void) { return slow(); }
+int f8mi_gemm_nt_kb_ws(void) { return slow(); }
+int f8mi_gemm_kb_ex(void) { return slow(); }
+int f8mi_linear_few_rows(void) { return slow(); }
+"""
+
+
+def test_native_host_path_lets_other_python_threads_run(f8, tmp_path):
+    """A launch may block on a full queue: the calls release the GIL, as ctypes does around the step-by-step functions.  A
+    second copy of the module over a stand-in library whose entry points sleep (and launch nothing)."""
+    import importlib.util
+    import shutil
+    import subprocess
+    import threading
+    import time
+
+    from float8_experimental_amd import _native
+
+    (tmp_path / "slow.c").write_text(_SLOW_LIBRARY)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / "slow.so"), str(tmp_path / "slow.c")], check=True)
+    copy = shutil.copy(_native._EXT_PATH, tmp_path / "_f8mi_torch.so")
+    spec = importlib.util.spec_from_file_location("_f8mi_torch", copy)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    module.load(str(tmp_path / "slow.so"), RuntimeError)
+
+    x, w, dy = (torch.zeros(s, device=DEV) for s in ((512, 1024), (1024, 1024), (512, 1024)))
+    saved, one = torch.zeros(16, 512, 64, dtype=torch.float8_e4m3fn, device=DEV), torch.ones((), device=DEV)
+    w8 = torch.zeros(16, 1024, 64, dtype=torch.float8_e4m3fn, device=DEV)
+    ticks, done = [], threading.Event()
+
+    def tick():
+        while not done.is_set():
+            ticks.append(time.perf_counter())
+            time.sleep(0.002)
+
+    thread = threading.Thread(target=tick)
+    thread.start()
+    try:
+        for call in (lambda: module.linear_forward(x, w, 1, 1, 1, 1, 1, 1, None, None, None, None, 0, 0),
+                     lambda: module.linear_backward(dy, saved, w8, one, one, 1024, 1, 1, 1, 1, 1, None, None, 0, 0),
+                     lambda: module.inference_linear(x, w8, 1024, 1, one, None, None, 0, 0)):
+            begin = time.perf_counter()
+            assert call() is not None
+            end = time.perf_counter()
+            assert end - begin > 0.25
+            assert sum(begin + 0.05 < t < end - 0.05 for t in ticks) > 10
+    finally:
+        done.set()
+        thread.join()
