@@ -51,6 +51,12 @@ int fp8_code(at::ScalarType t) { return t == at::kFloat8_e4m3fn ? F8MI_E4M3FN : 
 at::ScalarType fp8_type(int fmt) { return fmt == F8MI_E4M3FN ? at::kFloat8_e4m3fn : at::kFloat8_e5m2; }
 int64_t padded(int64_t k, int layout) { return layout == F8MI_LAYOUT_KBLOCK64_PAD128 ? (k + 127) / 128 * 128 : k; }
 
+// sizes of the fp8 copy of `rows` rows that contracts over kc, in the layout
+std::vector<int64_t> copy_sizes(int64_t rows, int64_t kc, int layout) {
+    if (layout == F8MI_LAYOUT_ROWMAJOR) return {rows, kc};
+    return {padded(kc, layout) / 64, rows, 64};
+}
+
 // Undefined: not taken.  A plain tensor (or Parameter) on the current device: nothing of a subclass, no other layout ...
 at::Tensor plain(PyObject* o, int device) {
     if (!THPVariable_CheckExact(o)) return {};
@@ -93,10 +99,8 @@ struct Call {
     at::Tensor make(at::IntArrayRef sizes, at::ScalarType t) const {
         return at::empty(sizes, at::TensorOptions().dtype(t).device(at::Device(at::kCUDA, (c10::DeviceIndex)device)));
     }
-    // fp8 copy of `rows` rows that contracts over kc, in the layout
     at::Tensor copy(int64_t rows, int64_t kc, int layout, int fmt) const {
-        if (layout == F8MI_LAYOUT_ROWMAJOR) return make({rows, kc}, fp8_type(fmt));
-        return make({padded(kc, layout) / 64, rows, 64}, fp8_type(fmt));
+        return make(copy_sizes(rows, kc, layout), fp8_type(fmt));
     }
 
     // The fp8 copies of x: `row` contracts over the columns, `tr` (the transpose) over the rows.
@@ -238,7 +242,7 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             if (!t->defined()) continue;
             const int64_t rows = one_copy ? (t == &xs ? m : n) : k, kc = one_copy ? k : (t == &xs ? m : n);
             const int layout = one_copy ? F8MI_LAYOUT_KBLOCK64 : t == &xs ? kb_dw : kb_dx;
-            if (fp8_code(t->scalar_type()) < 0 || !t->is_contiguous() || t->numel() != rows * padded(kc, layout)) Py_RETURN_NONE;
+            if (fp8_code(t->scalar_type()) < 0 || !t->is_contiguous() || t->sizes() != copy_sizes(rows, kc, layout)) Py_RETURN_NONE;
         }
         at::Tensor g8, g8t, sg, dx, dw;
         {

@@ -915,3 +915,15 @@ def test_native_host_path_lets_other_python_threads_run(f8, tmp_path):
     finally:
         done.set()
         thread.join()
+
+
+@pytest.mark.parametrize("m,k,n", [(512, 1024, 1024), (100, 512, 512)])
+def test_native_host_path_refuses_saved_copies_of_another_shape(f8, m, k, n):
+    """A saved-tensor hook that hands back something else than it was given is refused, as the step-by-step functions do."""
+    x = torch.randn(m, k, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    mod = f8.convert_to_float8_training(torch.nn.Sequential(torch.nn.Linear(k, n, bias=False, device=DEV, dtype=torch.bfloat16)))
+    turn = lambda t: t.view(torch.uint8).reshape(t.shape[1], -1).view(t.dtype) if t.dim() == 3 else t
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, turn):
+        y = mod(x)
+    with pytest.raises(Exception):
+        y.backward(torch.randn_like(y))
