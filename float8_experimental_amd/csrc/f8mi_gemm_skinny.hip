@@ -2,14 +2,18 @@
 // work there is (a decode step of an inference linear: A is a handful of tokens, Bt the weight).
 //
 // The 256 x 256 tile kernels would put n / 256 workgroups on 256 CUs and walk the whole k on each, which is
-// 70 us for k = n = 8192 whatever m is.  Here a workgroup of eight waves owns 32 columns of C (two 16-row tiles
+// 70 us for k = n = 8192 whatever m is.  Here a workgroup of eight waves owns 16 or 32 columns of C (one or two 16-row tiles
 // of Bt) and all rows of A (of its block of A, past 64 rows); the waves split k among themselves, eight ways, and
 // each streams its part of Bt straight from memory into MFMA operands: a lane's operand of
-// v_mfma_f32_16x16x128_f8f6f4 is 32 consecutive k bytes of one row, two 16-byte loads, no LDS on the way.  With up
-// to 32 rows of A four steps of 128 k are loaded back to back before the first is multiplied (16 loads of 16
-// bytes per lane in flight for Bt alone), with more rows two or one.  The A fragments come the same
-// way (A is small and stays in the L2).  At the end the eight partial sums meet in LDS, are added in a
+// v_mfma_f32_16x16x128_f8f6f4 is 32 consecutive k bytes of one row, two 16-byte loads, no LDS on the way.  The A fragments
+// come the same way (A is small and stays in the L2).  SK_DEPTH steps of 128 k are in flight per wave -- four with up to 32 rows
+// of A (16 loads of 16 bytes per lane for Bt alone), two with up to 64, one with more -- and a slot is filled again as soon as
+// it has been multiplied.  At the end the eight partial sums meet in LDS, are added in a
 // fixed order, scaled, biased, converted and stored.
+//
+// No more slots than a wave has steps: with k <= 1024 it has one, and four slots asked for that step four times and held the registers
+// of four, which left fewer workgroups on a CU.  us, always the most slots / as many as steps: 1 row, 1024 x 1024: 3.6 / 2.9;
+// 17 rows: 5.6 / 3.7; 64 rows: 6.1 / 5.2; 8 rows, 28672 x 1024: 13.6 / 8.4; 16 rows, 131072 x 1024: 62 / 38, 131072 x 2048: 74 / 59.
 //
 // Operands are addressed as (row stride, stride of a 64-deep k block): row-major (ld, 64) or k-blocked
 // (64, rows * 64).  Needs k % 128 == 0 and 16-byte aligned operands and strides; any n.  Up to 64 rows of A go
@@ -24,7 +28,7 @@ typedef float v4f_s __attribute__((ext_vector_type(4)));
 
 constexpr int SK_WAVES = 8;
 constexpr int SK_THREADS = SK_WAVES * 64;
-// 128-deep steps loaded before the first is multiplied: four where the A fragments leave registers for it
+// 128-deep steps in flight: at most what the A fragments leave registers for
 constexpr int sk_depth(int mt) { return mt <= 2 ? 4 : mt <= 4 ? 2 : 1; }
 
 __device__ __forceinline__ v8i load_frag_global(const uint8_t* p) {
@@ -33,12 +37,11 @@ __device__ __forceinline__ v8i load_frag_global(const uint8_t* p) {
     return (v8i){(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
 }
 
-template <int AF, int BF, int C_DT, int MT, int SK_NT>
+template <int AF, int BF, int C_DT, int MT, int SK_NT, int SK_DEPTH>
 __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(
     const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
     int M_all, int N, int K, const float* __restrict__ sa_dev, const float* __restrict__ sb_dev, void* __restrict__ C_all,
     int64_t ldc, const void* __restrict__ bias) {
-    constexpr int SK_DEPTH = sk_depth(MT);
     // blockIdx.y: which block of 16 * MT rows of A (and C) this workgroup multiplies
     // 1 / (sa * sb) for the epilogue: fetched first, so that the round trip to memory is over long before it is needed
     const float inv = __fdiv_rn(1.0f, *sa_dev) * __fdiv_rn(1.0f, *sb_dev);
@@ -143,12 +146,24 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(
     }
 }
 
+template <int AF, int BF, int C_DT, int MT, int SK_NT, int SK_DEPTH>
+static int launch_skinny5(hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt, int64_t ldb, int64_t b_unit,
+                          int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc, const void* bias) {
+    const dim3 g((unsigned)((N + 16 * SK_NT - 1) / (16 * SK_NT)), (unsigned)((M + 16 * MT - 1) / (16 * MT)));
+    hipLaunchKernelGGL((gemm_skinny_kernel<AF, BF, C_DT, MT, SK_NT, SK_DEPTH>), g, dim3(SK_THREADS), 0, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias);
+    return check_hip(hipGetLastError(), "skinny gemm kernel launch");
+}
+
 template <int AF, int BF, int C_DT, int MT, int SK_NT>
 static int launch_skinny4(hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt, int64_t ldb, int64_t b_unit,
                           int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc, const void* bias) {
-    const dim3 g((unsigned)((N + 16 * SK_NT - 1) / (16 * SK_NT)), (unsigned)((M + 16 * MT - 1) / (16 * MT)));
-    hipLaunchKernelGGL((gemm_skinny_kernel<AF, BF, C_DT, MT, SK_NT>), g, dim3(SK_THREADS), 0, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias);
-    return check_hip(hipGetLastError(), "skinny gemm kernel launch");
+    constexpr int DEPTH = sk_depth(MT);
+    const int steps = (K / 128 + SK_WAVES - 1) / SK_WAVES;  // of the wave that has most
+    if constexpr (DEPTH > 1)
+        if (steps <= 1) return launch_skinny5<AF, BF, C_DT, MT, SK_NT, 1>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias);
+    if constexpr (DEPTH > 2)
+        if (steps <= 2) return launch_skinny5<AF, BF, C_DT, MT, SK_NT, 2>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias);
+    return launch_skinny5<AF, BF, C_DT, MT, SK_NT, DEPTH>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias);
 }
 
 template <int AF, int BF, int C_DT>

@@ -629,6 +629,15 @@ def test_gemm_mid_tile_kernel_reads_transposed_operands(nat, m, n, k, mid, out_d
     assert torch.equal(nat.gemm_kb_ex(turned(a), True, sa, turned(bt), True, sb, out_dt, bias=bias), want)
 
 
+# Few rows: one to three 128-deep steps per wave and one more or less of them, on each block of rows and both widths.
+@pytest.mark.parametrize("m,n,k", [(m, n, k) for m, n in ((1, 1000), (16, 4104), (17, 40), (32, 1000), (33, 40), (64, 1000))
+                                   for k in (128, 896, 1024, 1152, 2048, 2176, 3200) if m <= 16 or k > 128])
+def test_gemm_few_rows_step_counts(nat, m, n, k):
+    assert nat.gemm_plan(m, n, k)[0] == "few_rows"
+    for out_dt in (torch.bfloat16, torch.float32):
+        _gemm_check(nat, m, n, k, "e5m2", "e4m3", out_dt, seed=m + k, bias=(k % 256 == 0))
+
+
 # Few 128-row tiles and a long contraction: with the stream's scratch buffer k is split over workgroups and a second
 # kernel adds the parts in a fixed order.
 @pytest.mark.parametrize("m,n,k", [(256, 2048, 16384), (512, 1024, 8192), (100, 4096, 16384)])

@@ -87,3 +87,17 @@ def test_no_spills_and_accumulators_stay_in_place(listings, unit):
     assert "v_accvgpr_mov" not in text
     sizes = [int(x) for x in re.findall(r"; ScratchSize: (\d+)", text)]
     assert sizes and not any(sizes)
+
+
+def test_few_row_kernels_of_one_step_per_wave_leave_room_for_two_workgroups(tmp_path):
+    """With one 128-deep step per wave the few-row kernels are bound by latency and by how many workgroups a CU holds: up to 32
+    rows they keep to the 128 registers that two workgroups of eight waves can have each."""
+    text = "\n".join(_asm("f8mi_gemm_skinny.hip", str(tmp_path)))
+    vgprs = {}
+    for name, n in re.findall(r"\.globl\s+\S*gemm_skinny_kernelI(\S+?)EEv.*?; TotalNumVgprs: (\d+)", text, re.S):
+        af, bf, dt, mt, nt, depth = (int(v) for v in re.findall(r"Li(\d+)E?", name))
+        vgprs[af, bf, dt, mt, nt, depth] = int(n)
+    one_step = [v for (af, bf, dt, mt, nt, depth), v in vgprs.items() if depth == 1 and mt <= 2]
+    assert len(one_step) == 4 * 3 * 3 and max(one_step) <= 128
+    sizes = [int(x) for x in re.findall(r"; ScratchSize: (\d+)", text)]
+    assert len(sizes) >= len(vgprs) and not any(sizes)
