@@ -25,7 +25,8 @@ typedef float v4f_l __attribute__((ext_vector_type(4)));
 constexpr int FR_WAVES = 8;
 constexpr int FR_THREADS = FR_WAVES * 64;
 constexpr int FR_MAX_M = 16;
-constexpr int fr_depth(int nt, int dt) { return nt == 2 && dt == F8MI_FP32 ? 2 : 4; }  // steps in flight per wave: what the registers next to x allow
+// Steps in flight per wave: at most what the registers next to x allow (128 a lane, with two workgroups a CU; fp32 x takes 64 of them)
+constexpr int fr_depth(int nt, int dt) { return nt == 2 && dt == F8MI_FP32 ? 2 : 4; }
 constexpr int FR_LDS_PAD = 16;  // bytes between rows of x8 in LDS
 
 __device__ __forceinline__ v8i fr_load_weight(const uint8_t* p) {
@@ -67,11 +68,11 @@ __device__ __forceinline__ uint32_t absmax16bytes(uint4 v, uint32_t m) {  // 16-
     return m;
 }
 
-template <int DT, int PROD, int BF, int NT>
+template <int DT, int PROD, int BF, int NT, int DEPTH>
 __global__ __launch_bounds__(FR_THREADS, 4) void linear_few_rows_kernel(
     const uint8_t* __restrict__ x, int64_t ldx, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit, int M, int N, int K,
     const float* __restrict__ sx_dev, const float* __restrict__ sb_dev, void* __restrict__ C, int64_t ldc, const void* __restrict__ bias) {
-    constexpr int ESZ = DT == F8MI_FP32 ? 4 : 2, EPV = 16 / ESZ, DEPTH = fr_depth(NT, DT);
+    constexpr int ESZ = DT == F8MI_FP32 ? 4 : 2, EPV = 16 / ESZ;
     constexpr int PIECES = F8MI_FEW_ROWS_ELEMS / EPV / FR_THREADS;
     extern __shared__ __align__(16) uint8_t x8[];  // [M][K + FR_LDS_PAD]
     __shared__ float4 part[FR_WAVES / 2][NT][64];
@@ -96,15 +97,18 @@ __global__ __launch_bounds__(FR_THREADS, 4) void linear_few_rows_kernel(
             v[u] = make_uint4(t.x, t.y, t.z, t.w);
         }
     }
-    // a lane's 32 bytes of step s: row * ld + (2s + lq / 2) * unit + 32 * (lq % 2); rows past the end re-read the last one
-    const uint8_t* pb[NT];
+    // a lane's 32 bytes of step s: row * ld + (2s + lq / 2) * unit + 32 * (lq % 2); rows past the end re-read the last one.  The wave's
+    // part of the address is scalar, the lane's 32 bits (the host has checked): with a 64-bit pointer per lane fp32 x with 32 columns
+    // spilled, and one step in flight instead of two cost more on long k (1 row, 14336 x 32768: 88.7 us with one, 84.4 with two)
+    const uint8_t* const base = Bt + (int64_t)n0 * ldb;
+    uint32_t off[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) pb[nt] = Bt + (int64_t)min(n0 + nt * 16 + lm, N - 1) * ldb + (lq >> 1) * b_unit + (lq & 1) * 32;
+    for (int nt = 0; nt < NT; nt++) off[nt] = (uint32_t)(min(nt * 16 + lm, N - 1 - n0) * ldb + (lq >> 1) * b_unit + (lq & 1) * 32);
     v8i fb[DEPTH][NT];
     auto load = [&](int d, int s) __attribute__((always_inline)) {  // past the wave's range: a valid address, the product is skipped
         const int sd = min(s, s1 - 1);
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) fb[d][nt] = fr_load_weight(pb[nt] + 2 * (int64_t)sd * b_unit);
+        for (int nt = 0; nt < NT; nt++) fb[d][nt] = fr_load_weight(base + 2 * (int64_t)sd * b_unit + off[nt]);
     };
     if (s0 < s1) {
 #pragma unroll
@@ -202,11 +206,22 @@ struct FewRowsArgs {
     const uint8_t* x; int64_t ldx; const uint8_t* w; int64_t ldb, b_unit; int M, N, K;
     const float* sx; const float* sb; void* C; int64_t ldc; const void* bias;
 };
-template <int DT, int PROD, int BF, int NT>
-static int launch_fr3(hipStream_t stream, const FewRowsArgs& a) {
-    hipLaunchKernelGGL((linear_few_rows_kernel<DT, PROD, BF, NT>), dim3((unsigned)((a.N + 16 * NT - 1) / (16 * NT))), dim3(FR_THREADS), (size_t)a.M * (a.K + FR_LDS_PAD), stream,
+template <int DT, int PROD, int BF, int NT, int DEPTH>
+static int launch_fr4(hipStream_t stream, const FewRowsArgs& a) {
+    hipLaunchKernelGGL((linear_few_rows_kernel<DT, PROD, BF, NT, DEPTH>), dim3((unsigned)((a.N + 16 * NT - 1) / (16 * NT))), dim3(FR_THREADS), (size_t)a.M * (a.K + FR_LDS_PAD), stream,
                        a.x, a.ldx, a.w, a.ldb, a.b_unit, a.M, a.N, a.K, a.sx, a.sb, a.C, a.ldc, a.bias);
     return check_hip(hipGetLastError(), "few-row linear kernel launch");
+}
+template <int DT, int PROD, int BF, int NT>
+static int launch_fr3(hipStream_t stream, const FewRowsArgs& a) {
+    // no more slots than a wave has steps, as in f8mi_gemm_skinny.hip (1 row, 131072 x 512: 36.9 / 24.0 us; 8 rows, 8192 x 1024: 7.1 / 6.5)
+    constexpr int DEPTH = fr_depth(NT, DT);
+    const int steps = (a.K / 128 + FR_WAVES - 1) / FR_WAVES;
+    if constexpr (DEPTH > 1)
+        if (steps <= 1) return launch_fr4<DT, PROD, BF, NT, 1>(stream, a);
+    if constexpr (DEPTH > 2)
+        if (steps <= 2) return launch_fr4<DT, PROD, BF, NT, 2>(stream, a);
+    return launch_fr4<DT, PROD, BF, NT, DEPTH>(stream, a);
 }
 template <int DT, int PROD, int BF>
 static int launch_fr2(hipStream_t stream, const FewRowsArgs& a) {
@@ -232,7 +247,7 @@ extern "C" int f8mi_linear_few_rows(const void* x, int64_t ldx, int dtype, const
     if (scale_x_dev && product_dtype != dtype && product_dtype != F8MI_FP32) { set_error("f8mi_linear_few_rows: product_dtype must be the input dtype or fp32"); return F8MI_ERR_INVALID_ARG; }
     if (m < 0 || n < 0 || k < 0 || ldx < k || ldc < n) { set_error("f8mi_linear_few_rows: bad shape m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k); return F8MI_ERR_INVALID_ARG; }
     if (m == 0 || n == 0) return F8MI_OK;
-    if (m > FR_MAX_M || k < 128 || k % 128 != 0 || m * k > F8MI_FEW_ROWS_ELEMS || n > 0x7fffff00LL || (w_layout != F8MI_LAYOUT_ROWMAJOR && w_layout != F8MI_LAYOUT_KBLOCK64) || (uintptr_t)w % 16 != 0) { set_error("f8mi_linear_few_rows: at most 16 rows and 32768 activations, k a multiple of 128, a 16-byte aligned row-major or k-blocked weight (m=%lld k=%lld layout=%d)", (long long)m, (long long)k, w_layout); return F8MI_ERR_UNSUPPORTED; }
+    if (m > FR_MAX_M || k < 128 || k % 128 != 0 || m * k > F8MI_FEW_ROWS_ELEMS || n > (w_layout ? 0x3ffff00LL : 0x7fffff00LL) || (w_layout != F8MI_LAYOUT_ROWMAJOR && w_layout != F8MI_LAYOUT_KBLOCK64) || (uintptr_t)w % 16 != 0) { set_error("f8mi_linear_few_rows: at most 16 rows and 32768 activations, k a multiple of 128, a 16-byte aligned row-major or k-blocked weight (m=%lld k=%lld layout=%d)", (long long)m, (long long)k, w_layout); return F8MI_ERR_UNSUPPORTED; }
     if (!x || !w || !scale_w_dev || !c) { set_error("f8mi_linear_few_rows: null pointer"); return F8MI_ERR_INVALID_ARG; }
     FewRowsArgs a{(const uint8_t*)x, ldx, (const uint8_t*)w, w_layout ? 64 : k, w_layout ? n * 64 : 64, (int)m, (int)n, (int)k, scale_x_dev,
                   scale_w_dev, c, ldc, bias_dev};

@@ -101,3 +101,12 @@ def test_few_row_kernels_of_one_step_per_wave_leave_room_for_two_workgroups(tmp_
     assert len(one_step) == 4 * 3 * 3 and max(one_step) <= 128
     sizes = [int(x) for x in re.findall(r"; ScratchSize: (\d+)", text)]
     assert len(sizes) >= len(vgprs) and not any(sizes)
+
+
+def test_few_row_linear_keeps_to_its_registers(tmp_path):
+    """Two workgroups a CU leave a lane 128 registers; the activations take up to 64 of them and the weights in flight the
+    rest: no instantiation may spill."""
+    text = "\n".join(_asm("f8mi_linear_few_rows.hip", str(tmp_path)))
+    assert len(re.findall(r"\.globl\s+\S*linear_few_rows_kernel", text)) >= 5 * 2 * 2
+    assert "scratch_store" not in text and "scratch_load" not in text
+    assert not any(int(x) for x in re.findall(r"; ScratchSize: (\d+)", text))
