@@ -99,7 +99,7 @@ __global__ __launch_bounds__(FR_THREADS, 4) void linear_few_rows_kernel(
     }
     // a lane's 32 bytes of step s: row * ld + (2s + lq / 2) * unit + 32 * (lq % 2); rows past the end re-read the last one.  The wave's
     // part of the address is scalar, the lane's 32 bits (the host has checked): with a 64-bit pointer per lane fp32 x with 32 columns
-    // spilled, and one step in flight instead of two cost more on long k (1 row, 14336 x 32768: 88.7 us with one, 84.4 with two)
+    // spilled, and one step in flight instead of two cost more on long k (1 row, 14336 x 32768: 88.9 us with one, 83.2 with two)
     const uint8_t* const base = Bt + (int64_t)n0 * ldb;
     uint32_t off[NT];
 #pragma unroll

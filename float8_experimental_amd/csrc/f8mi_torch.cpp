@@ -261,6 +261,16 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     });
 }
 
+// Cast and product of a few rows in one kernel: every workgroup of 16 or 32 columns converts all of the activations for itself, which
+// costs more than the launch it saves once there are many of them and many rows.  us, two launches / one kernel, bf16: 1 row, 65536 x
+// 4096: 67.4 / 64.3; 8 rows, 24576 x 4096: 26.2 / 25.4, 98304 x 4096: 81.2 / 86.9; 16 rows, 14336 x 2048: 15.0 / 12.9, 24576 x 2048: 18.3 /
+// 19.2, 131072 x 2048: 67.3 / 84.0.  fp32 holds twice the registers and reaches the line earlier: 4 rows, 14336 x 8192: 29.9 / 24.9, 24576
+// x 8192: 44.5 / 46.1; 8 rows, 24576 x 4096: 28.8 / 29.3, 98304 x 4096: 88.9 / 107.8.
+bool one_kernel_pays(int64_t m, int64_t n, int64_t k, int dt) {
+    if (m > 16 || m * k > F8MI_FEW_ROWS_ELEMS) return false;
+    return dt == F8MI_FP32 ? n <= 16384 || m * n <= 65536 : m * n <= 262144;
+}
+
 // inference_linear(x [m, k], weight (fp8, [n, k] or k-blocked), n, layout, weight_scale, static_scale, bias, device, stream) -> y or None
 PyObject* inference_linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (!expect(n_args, 9, "inference_linear")) return nullptr;
@@ -278,7 +288,7 @@ PyObject* inference_linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         // a 0-dim scale leaves the product in x's dtype, a scale with a dimension promotes it to fp32
         const int dt = dtype_code(x.scalar_type()), product = in.scale.defined() && in.scale.dim() > 0 ? F8MI_FP32 : dt;
         const auto compute = [&]() -> at::Tensor {
-            if (m <= 16 && m * k <= F8MI_FEW_ROWS_ELEMS && layout != F8MI_LAYOUT_KBLOCK64_PAD128) {  // cast and product in one kernel
+            if (one_kernel_pays(m, n, k, dt) && layout != F8MI_LAYOUT_KBLOCK64_PAD128) {  // cast and product in one kernel
                 const at::Tensor y = c.make({m, n}, x.scalar_type());
                 const int rc = L.linear_few_rows(x.data_ptr(), x.stride(0), dt, in.scale.defined() ? (const float*)in.scale.data_ptr() : nullptr, product,
                                                  w.data_ptr(), fp8_code(w.scalar_type()), layout, (const float*)sw.data_ptr(), m, n, k, y.data_ptr(), n,

@@ -355,3 +355,24 @@ def test_few_row_linear_equals_cast_and_gemm(m, k, n, dtype):
                 want = (nat.gemm_nt_kb if kb else nat.gemm_nt)(x8, s, wk, sw, dtype, bias=b)
                 got = nat.inference_linear(x, wk, n, kb, sw, static, b)
                 assert torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)) and torch.equal(got.isnan(), want.isnan())
+
+
+@pytest.mark.parametrize("m,n,dtype,one_kernel", [(16, 16384, torch.bfloat16, True), (16, 16400, torch.bfloat16, False), (1, 65536, torch.float16, True),
+                                                  (8, 49152, torch.bfloat16, False), (16, 16384, torch.float32, True), (4, 16400, torch.float32, False),
+                                                  (1, 65536, torch.float32, True), (17, 512, torch.bfloat16, False)])
+def test_few_row_linear_is_taken_where_its_workgroups_are_few(m, n, dtype, one_kernel):
+    """Every workgroup converts all of the activations: with many columns and rows the two launches are faster."""
+    from float8_experimental_amd import _native as nat
+
+    k = 512
+    x, one = torch.randn(m, k, device=DEV).to(dtype), torch.ones((), device=DEV)
+    w = torch.zeros(k // 64, n, 64, dtype=torch.float8_e4m3fn, device=DEV)
+    nat.prof_reset()
+    nat.prof_enable(True)
+    try:
+        nat.inference_linear(x, w, n, nat.KBLOCK, one, None, None)
+    finally:
+        nat.prof_enable(False)
+    launches = [nat.prof_read(kernel)[0] for kernel in (nat.K_CAST, nat.K_GEMM)]
+    nat.prof_reset()
+    assert launches == [0 if one_kernel else 1, 1]
