@@ -353,8 +353,17 @@ def test_few_row_linear_equals_cast_and_gemm(m, k, n, dtype):
                     s = static
                     x8, _ = nat.cast(x, s, torch.float8_e4m3fn, product_dtype=dtype if s.dim() == 0 else torch.float32, out_kblock=kb)
                 want = (nat.gemm_nt_kb if kb else nat.gemm_nt)(x8, s, wk, sw, dtype, bias=b)
-                got = nat.inference_linear(x, wk, n, kb, sw, static, b)
-                assert torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)) and torch.equal(got.isnan(), want.isnan())
+                same = lambda got: torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)) and torch.equal(got.isnan(), want.isnan())
+                assert same(nat.inference_linear(x, wk, n, kb, sw, static, b))  # whichever of the two it takes
+                got = torch.full((m, n), 3.0, dtype=dtype, device=DEV)
+                rc = nat.lib().f8mi_linear_few_rows(x.data_ptr(), x.stride(0), nat._DT[dtype], None if static is None else static.data_ptr(),
+                                                    nat._DT[dtype if static is None or static.dim() == 0 else torch.float32], wk.data_ptr(),
+                                                    nat._F8[w.dtype], kb, sw.data_ptr(), m, n, k, got.data_ptr(), n,
+                                                    None if b is None else b.data_ptr(), torch.cuda.current_stream().cuda_stream)
+                if m * k <= 32768:
+                    assert rc == 0 and same(got)
+                else:  # nothing queued
+                    assert rc == nat.ERR_UNSUPPORTED and (got == 3.0).all()
 
 
 @pytest.mark.parametrize("m,n,dtype,one_kernel", [(16, 16384, torch.bfloat16, True), (16, 16400, torch.bfloat16, False), (1, 65536, torch.float16, True),

@@ -616,14 +616,15 @@ def test_gemm_mid_tile_kernel_step_counts(nat, m, n, mid, steps):
 @pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float32])
 def test_gemm_mid_tile_kernel_reads_transposed_operands(nat, m, n, k, mid, out_dt):
     """The same bits as on operands that are not transposed, for one and for both of them transposed."""
-    plan = nat.gemm_plan(m, n, k, split_k=False)
-    assert plan[0] == ("tiles256_and_128" if mid == 0 else "tiles128") and (mid == 0 or plan[2] == mid) or m <= 256
+    rows = m if m > 256 else 272  # past the few-row kernel, for the operands that are not transposed
+    plan = nat.gemm_plan(rows, n, k, split_k=False)
+    assert plan[0] == ("tiles256_and_128" if mid == 0 else "tiles128") and (mid == 0 or plan[2] == mid)
     a = _rand_fp8((m, k), torch.float8_e5m2, m + k, 4.0).to(DEV)
     bt = _rand_fp8((n, k), torch.float8_e4m3fn, n + k, 4.0).to(DEV)
     sa, sb = torch.tensor(2.0, device=DEV), torch.tensor(0.25, device=DEV)
     turned = lambda t: _to_kb(t.view(torch.uint8).t().contiguous().view(t.dtype))
     bias = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 3).to(out_dt).to(DEV)
-    tall = torch.cat([a.view(torch.uint8), torch.zeros(272 - m if m <= 256 else 0, k, dtype=torch.uint8, device=DEV)]).view(a.dtype)  # past the few-row kernel
+    tall = torch.cat([a.view(torch.uint8), torch.zeros(rows - m, k, dtype=torch.uint8, device=DEV)]).view(a.dtype)
     want = nat.gemm_nt_kb(_to_kb(tall), sa, _to_kb(bt), sb, out_dt, bias=bias, split_k=False)[:m]
     assert torch.equal(nat.gemm_kb_ex(_to_kb(a), False, sa, turned(bt), True, sb, out_dt, bias=bias), want)
     assert torch.equal(nat.gemm_kb_ex(turned(a), True, sa, turned(bt), True, sb, out_dt, bias=bias), want)

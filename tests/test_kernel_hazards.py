@@ -2,7 +2,8 @@
 ones: it neither knows that their results arrive passes later nor inserts the wait states an accumulator read
 needs.  The kernel keeps that distance by construction (hand-placed v_accvgpr_read_b32 between later MFMAs, wait
 states before the last reads).  This test compiles the kernel's translation units to assembly (no GPU needed) and
-checks the distance on what the compiler actually emitted, for every instantiation.
+checks the distance on what the compiler actually emitted, for every instantiation.  The LDS-DMA sequences of the
+128-row-tile kernels and the register budgets of the few-row ones are checked the same way.
 """
 import os
 import re
@@ -14,6 +15,7 @@ import pytest
 from float8_experimental_amd import _build
 
 UNITS = ["f8mi_gemm_dma16.hip", "f8mi_gemm_dma16_nt.hip", "f8mi_gemm_dma16_tt.hip"]
+MID_UNITS = ["f8mi_gemm_mid.hip", "f8mi_gemm_mid_nt.hip", "f8mi_gemm_mid_tt.hip"]
 MIN_MFMAS = 8        # MFMAs issued after the producing one (each occupies the matrix core for 8 passes of 4 cycles) ...
 MIN_WAIT_STATES = 18  # ... or this many wait states of s_nop between the two
 
@@ -29,8 +31,8 @@ def _asm(unit, out_dir):
 @pytest.fixture(scope="module")
 def listings(tmp_path_factory):
     d = str(tmp_path_factory.mktemp("asm"))
-    with ThreadPoolExecutor(max_workers=3) as ex:
-        return dict(zip(UNITS, ex.map(lambda u: _asm(u, d), UNITS)))
+    with ThreadPoolExecutor(max_workers=6) as ex:
+        return dict(zip(UNITS + MID_UNITS, ex.map(lambda u: _asm(u, d), UNITS + MID_UNITS)))
 
 
 @pytest.mark.parametrize("unit", UNITS)
@@ -62,7 +64,7 @@ def test_accumulator_reads_keep_their_distance_from_the_mfma_that_writes_them(li
         start = end + 1
 
 
-@pytest.mark.parametrize("unit", UNITS)
+@pytest.mark.parametrize("unit", UNITS + MID_UNITS)
 def test_every_lds_dma_sets_m0_itself_with_the_wait_state_it_needs(listings, unit):
     """A global load into the LDS takes its LDS address from M0.  The scalar write of M0 needs one wait state before
     the vector memory instruction that reads it, and nothing may change M0 in between: every such load must come
@@ -75,7 +77,10 @@ def test_every_lds_dma_sets_m0_itself_with_the_wait_state_it_needs(listings, uni
             n += 1
             assert code[i - 1].startswith("s_nop"), f"{unit}: `{l}` follows `{code[i - 1]}`"
             assert code[i - 2].startswith("s_mov_b32 m0,"), f"{unit}: `{l}`: M0 written by `{code[i - 2]}`"
-    assert n >= 12 * 16 * 3  # every instantiation has the prologue's 32 and at least two steps with 16
+    if unit in UNITS:
+        assert n >= 12 * 16 * 3  # every instantiation has the prologue's 32 and at least two steps with 16
+    else:  # 12 instantiations of each width: 8 a step with five stages, 12 with three; the prologue and at least two steps
+        assert n >= 12 * (8 * (5 + 2) + 12 * (3 + 2))
 
 
 @pytest.mark.parametrize("unit", UNITS)
@@ -110,3 +115,13 @@ def test_few_row_linear_keeps_to_its_registers(tmp_path):
     assert len(re.findall(r"\.globl\s+\S*linear_few_rows_kernel", text)) >= 5 * 2 * 2
     assert "scratch_store" not in text and "scratch_load" not in text
     assert not any(int(x) for x in re.findall(r"; ScratchSize: (\d+)", text))
+
+
+@pytest.mark.parametrize("unit", MID_UNITS)
+def test_128_row_tile_kernels_keep_both_fragment_sets_in_registers(listings, unit):
+    """Two sets of fragments beside up to 128 accumulator registers at one wave per SIMD: nothing may go to scratch."""
+    text = "\n".join(listings[unit])
+    assert len(re.findall(r"\.globl\s+\S*gemm_mid_kernel", text)) == 4 * 3 * 2
+    assert "scratch_store" not in text and "scratch_load" not in text
+    sizes = [int(x) for x in re.findall(r"; ScratchSize: (\d+)", text)]
+    assert sizes and not any(sizes)
