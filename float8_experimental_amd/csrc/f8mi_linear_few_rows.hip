@@ -97,18 +97,27 @@ __global__ __launch_bounds__(FR_THREADS, 4) void linear_few_rows_kernel(
             v[u] = make_uint4(t.x, t.y, t.z, t.w);
         }
     }
-    // a lane's 32 bytes of step s: row * ld + (2s + lq / 2) * unit + 32 * (lq % 2); rows past the end re-read the last one.  The wave's
-    // part of the address is scalar, the lane's 32 bits (the host has checked): with a 64-bit pointer per lane fp32 x with 32 columns
-    // spilled, and one step in flight instead of two cost more on long k (1 row, 14336 x 32768: 88.9 us with one, 83.2 with two)
+    // a lane's 32 bytes of step s: row * ld + (2s + lq / 2) * unit + 32 * (lq % 2); rows past the end re-read the last one.  Next to fp32 x
+    // the wave's part of the address is scalar and the lane's 32 bits (the host has checked that they do): with a 64-bit pointer per
+    // lane 32 columns spilled, and one step in flight instead of two cost more on long k (1 row, 14336 x 32768: 88.9 us with one, 83.2
+    // with two).  16-bit x leaves the registers for pointers, which are faster (1 row, 8192 x 8192, weights in cache: 13.2 / 12.7 us).
+    constexpr bool SCALAR_BASE = DT == F8MI_FP32;
     const uint8_t* const base = Bt + (int64_t)n0 * ldb;
+    const uint8_t* pb[NT];
     uint32_t off[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) off[nt] = (uint32_t)(min(nt * 16 + lm, N - 1 - n0) * ldb + (lq >> 1) * b_unit + (lq & 1) * 32);
+    for (int nt = 0; nt < NT; nt++) {
+        if constexpr (SCALAR_BASE) off[nt] = (uint32_t)(min(nt * 16 + lm, N - 1 - n0) * ldb + (lq >> 1) * b_unit + (lq & 1) * 32);
+        else pb[nt] = Bt + (int64_t)min(n0 + nt * 16 + lm, N - 1) * ldb + (lq >> 1) * b_unit + (lq & 1) * 32;
+    }
     v8i fb[DEPTH][NT];
     auto load = [&](int d, int s) __attribute__((always_inline)) {  // past the wave's range: a valid address, the product is skipped
         const int sd = min(s, s1 - 1);
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) fb[d][nt] = fr_load_weight(base + 2 * (int64_t)sd * b_unit + off[nt]);
+        for (int nt = 0; nt < NT; nt++) {
+            if constexpr (SCALAR_BASE) fb[d][nt] = fr_load_weight(base + 2 * (int64_t)sd * b_unit + off[nt]);
+            else fb[d][nt] = fr_load_weight(pb[nt] + 2 * (int64_t)sd * b_unit);
+        }
     };
     if (s0 < s1) {
 #pragma unroll
@@ -247,7 +256,7 @@ extern "C" int f8mi_linear_few_rows(const void* x, int64_t ldx, int dtype, const
     if (scale_x_dev && product_dtype != dtype && product_dtype != F8MI_FP32) { set_error("f8mi_linear_few_rows: product_dtype must be the input dtype or fp32"); return F8MI_ERR_INVALID_ARG; }
     if (m < 0 || n < 0 || k < 0 || ldx < k || ldc < n) { set_error("f8mi_linear_few_rows: bad shape m=%lld n=%lld k=%lld", (long long)m, (long long)n, (long long)k); return F8MI_ERR_INVALID_ARG; }
     if (m == 0 || n == 0) return F8MI_OK;
-    if (m > FR_MAX_M || k < 128 || k % 128 != 0 || m * k > F8MI_FEW_ROWS_ELEMS || n > (w_layout ? 0x3ffff00LL : 0x7fffff00LL) || (w_layout != F8MI_LAYOUT_ROWMAJOR && w_layout != F8MI_LAYOUT_KBLOCK64) || (uintptr_t)w % 16 != 0) { set_error("f8mi_linear_few_rows: at most 16 rows and 32768 activations, k a multiple of 128, a 16-byte aligned row-major or k-blocked weight (m=%lld k=%lld layout=%d)", (long long)m, (long long)k, w_layout); return F8MI_ERR_UNSUPPORTED; }
+    if (m > FR_MAX_M || k < 128 || k % 128 != 0 || m * k > F8MI_FEW_ROWS_ELEMS || n > (w_layout && dtype == F8MI_FP32 ? 0x3ffff00LL : 0x7fffff00LL) || (w_layout != F8MI_LAYOUT_ROWMAJOR && w_layout != F8MI_LAYOUT_KBLOCK64) || (uintptr_t)w % 16 != 0) { set_error("f8mi_linear_few_rows: at most 16 rows and 32768 activations, k a multiple of 128, a 16-byte aligned row-major or k-blocked weight (m=%lld k=%lld layout=%d)", (long long)m, (long long)k, w_layout); return F8MI_ERR_UNSUPPORTED; }
     if (!x || !w || !scale_w_dev || !c) { set_error("f8mi_linear_few_rows: null pointer"); return F8MI_ERR_INVALID_ARG; }
     FewRowsArgs a{(const uint8_t*)x, ldx, (const uint8_t*)w, w_layout ? 64 : k, w_layout ? n * 64 : 64, (int)m, (int)n, (int)k, scale_x_dev,
                   scale_w_dev, c, ldc, bias_dev};

@@ -238,8 +238,8 @@ int f8mi_cast_dynamic_static(const void* x, int64_t rows, int64_t cols, int64_t 
  * bits as f8mi_cast_dynamic (scale_x_dev null) or f8mi_cast_layout (scale_x_dev given, product in product_dtype) followed by
  * f8mi_gemm_nt / f8mi_gemm_nt_kb.  x: rows of ldx elements at element alignment; w: row-major (w_layout
  * F8MI_LAYOUT_ROWMAJOR, rows of k bytes) or k-blocked (F8MI_LAYOUT_KBLOCK64), 16-byte aligned; c in x's dtype.
- * F8MI_ERR_UNSUPPORTED, with nothing queued: more rows or activations, k % 128 != 0, an unaligned weight, a k-blocked
- * weight of more than 2^26 - 256 rows. */
+ * F8MI_ERR_UNSUPPORTED, with nothing queued: more rows or activations, k % 128 != 0, an unaligned weight; fp32
+ * with a k-blocked weight of more than 2^26 - 256 rows. */
 #define F8MI_FEW_ROWS_ELEMS 32768
 int f8mi_linear_few_rows(const void* x, int64_t ldx, int dtype, const float* scale_x_dev, int product_dtype, const void* w,
                          int w_fmt, int w_layout, const float* scale_w_dev, int64_t m, int64_t n, int64_t k, void* c,
