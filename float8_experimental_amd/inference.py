@@ -144,7 +144,7 @@ WEIGHT_ONLY_MAX_ROWS = 128
 
 def _function_mode_active() -> bool:
     """True under a ``TorchFunctionMode`` that may want to see ``F.linear``; ``torch.set_default_device`` is one that does not."""
-    return torch._C._len_torch_function_stack() > 0 and any(not isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack())
+    return any(not isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack())
 
 
 def _weight_only_kernels_take(input: torch.Tensor, weight: "Float8Tensor") -> bool:
@@ -154,17 +154,17 @@ def _weight_only_kernels_take(input: torch.Tensor, weight: "Float8Tensor") -> bo
     who has to see the operators."""
     if torch.compiler.is_compiling() or type(weight) is not Float8Tensor or type(input) not in (torch.Tensor, nn.Parameter):
         return False
-    if input.layout is not torch.strided or input.is_nested or input.is_neg() or input._is_zerotensor() or _function_mode_active():
+    if input.layout is not torch.strided or input.is_nested or input.is_neg() or input._is_zerotensor():
         return False
     data, scale = weight._data, weight._scale
     return (input.is_cuda and input.dtype == weight._orig_dtype and input.dtype in _native._DT and data.dtype in _native._F8
-            and input.device == data.device == scale.device and input.device.index == torch.cuda.current_device()
+            and input.get_device() == data.get_device() == scale.get_device() == torch._C._cuda_getDevice()
             and input.dim() >= 1 and data.dim() == 2 and input.shape[-1] == data.shape[1] and input.numel() > 0 and data.shape[0] > 0
             and data.is_contiguous() and scale.dim() == 0 and scale.dtype == torch.float32
             and not (torch.is_grad_enabled() and (input.requires_grad or weight.requires_grad or data.requires_grad))
             and not torch.is_autocast_enabled() and torch.autograd.forward_ad._current_level < 0
             and torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0
-            and not torch.jit.is_tracing())
+            and not (torch._C._len_torch_function_stack() and _function_mode_active()) and not torch.jit.is_tracing())
 
 
 def _weight_only_linear(input: torch.Tensor, weight: "Float8Tensor") -> torch.Tensor:
