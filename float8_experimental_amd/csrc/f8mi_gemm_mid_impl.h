@@ -205,7 +205,12 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
     asm volatile("" : "+s"(sa_dev), "+s"(sb_dev)::"memory");
     const float inv = k_splits > 1 ? 1.0f : __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(
         int, __fdiv_rn(1.0f, load_scalar(sa_dev)) * __fdiv_rn(1.0f, load_scalar(sb_dev)))));
+    // step 0's data is there; what was asked for behind it, min(steps, NSTAGE) - 1 steps, may still be in flight (with fewer steps than
+    // stages too: waiting for all of it cost 512-deep products of many columns a tenth, 17 rows, 28672 x 512: 7.8 / 7.25 us)
     if (steps >= NSTAGE) mid_wait_barrier<(NSTAGE - 1) * NDMA>();
+    else if (NSTAGE == 5 && steps == 4) mid_wait_barrier<3 * NDMA>();
+    else if (NSTAGE == 5 && steps == 3) mid_wait_barrier<2 * NDMA>();
+    else if (steps == 2) mid_wait_barrier<NDMA>();
     else mid_wait_barrier<0>();
     if (steps & 1) fetch_all(c0);
     else fetch_all(c1);
