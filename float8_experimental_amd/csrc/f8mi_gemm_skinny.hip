@@ -161,8 +161,10 @@ static int launch_skinny4(hipStream_t stream, const uint8_t* A, int64_t lda, int
     const int steps = (K / 128 + SK_WAVES - 1) / SK_WAVES;  // of the wave that has most
     if constexpr (DEPTH > 1)
         if (steps <= 1) return launch_skinny5<AF, BF, C_DT, MT, SK_NT, 1>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias);
+    // with 17 - 32 rows two slots leave room for two workgroups on a CU, four only for one: taken where there are more workgroups than
+    // CUs and no slot would be filled again (32 rows, 16384 x 4096: 18.5 us with four, 16.9 with two)
     if constexpr (DEPTH > 2)
-        if (steps <= 2) return launch_skinny5<AF, BF, C_DT, MT, SK_NT, 2>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias);
+        if (steps <= 2 || (MT == 2 && steps <= 4 && N > 32 * cu_count())) return launch_skinny5<AF, BF, C_DT, MT, SK_NT, 2>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias);
     return launch_skinny5<AF, BF, C_DT, MT, SK_NT, DEPTH>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias);
 }
 
