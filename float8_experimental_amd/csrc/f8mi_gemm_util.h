@@ -230,10 +230,10 @@ inline double tiles_time_us(int64_t m, int64_t n, int64_t k) {
 inline bool use_skinny(int64_t m, int64_t n, int64_t k) {
     if (m > SKINNY_MAX_M || k <= 0 || k % 128 != 0) return false;
     if (m <= 16) return true;
-    // With 33 - 64 rows the few-row kernel has one workgroup on a CU: more than 256 of them run in turn, and tiles are faster (us, few-row /
-    // tiles: 33 rows, 8320 x 1024: 8.4 / 7.8, 9216 x 4096: 17.6 / 16.3; 48 rows, 10240 x 3072: 17.9 / 14.4; 64 rows, 14336 x 4096: 22.1 / 19.0;
-    // with 256: 48 rows, 8192 x 3072: 10.4 / 13.9, 8192 x 8192: 20.4 / 29.6).
-    if (m > 32 && m <= 64 && n > 8192 && use_mid_tiles(m, n, k)) return false;
+    // With 33 - 128 rows the few-row kernel has one workgroup on a CU: more than 256 of them run in turn, and tiles are faster (us, few-row /
+    // tiles: 33 rows, 8320 x 1024: 8.4 / 7.8, 9216 x 4096: 17.6 / 16.3; 48 rows, 10240 x 3072: 17.9 / 14.4; 64 rows, 14336 x 4096: 22.1 / 19.0; 96
+    // rows, 14336 x 2048: 20.5 / 12.9; with 256: 48 rows, 8192 x 3072: 10.4 / 13.9, 8192 x 8192: 20.4 / 29.6).
+    if (m > 32 && m <= 128 && n > 8192 && use_mid_tiles(m, n, k)) return false;
     return skinny_time_us(m, n, k) <= tiles_time_us(m, n, k);
 }
 // An output of at most 128 of the 128-row tiles and a long k: with `ws_bytes` of scratch for the partial sums, k is

@@ -117,8 +117,8 @@ def test_gemm_plan_names_the_kernel_each_shape_class_takes():
         assert plan(m, n, k)[0] == "few_rows", (m, n, k)
     # a wide weight at 17 - 256 rows, and outputs of at most 256 small tiles: 128-row tiles
     assert plan(64, 28672, 512) == ("tiles128", 0, 1) and plan(20, 16384, 256) == ("tiles128", 0, 1)
-    # 33 - 64 rows: as soon as the few-row kernel would have more workgroups (of 32 columns) than CUs
-    for m in (33, 48, 64):
+    # 33 - 128 rows: as soon as the few-row kernel would have more workgroups (of 32 columns) than CUs
+    for m in (33, 48, 64, 65, 128):
         assert plan(m, 8192, 3072)[0] == "few_rows" and plan(m, 8200, 3072) == ("tiles128", 0, 1) == plan(m, 14336, 4096)
     assert plan(32, 14336, 4096)[0] == "few_rows"
     assert plan(200, 8192, 512) == ("tiles128", 0, 1) and plan(300, 520, 1024) == ("tiles128", 0, 1)
