@@ -422,7 +422,9 @@ static int launch_cast_small(int fmt, hipStream_t stream, const void* x, int64_t
 // kernels' time does not.  Same arithmetic, element for element, as those: the same bits.
 //
 // us a call, back to back, two kernels / this one: bf16, 16 x 4096: 6.8 / 3.5, 32 x 4096: 7.3 / 4.4, 64 x 4096 (512 KB): 7.3 / 6.3,
-// 64 x 8192: 7.4 / 9.9; fp32, 16 x 4096: 6.8 / 4.3, 32 x 4096 (512 KB): 6.9 / 6.1, 16 x 14336 (896 KB): 6.9 / 8.7.  Hence the line.
+// 64 x 8192: 7.4 / 9.9; fp32, 16 x 4096: 6.8 / 4.3, 32 x 4096 (512 KB): 6.9 / 6.1, 16 x 14336 (896 KB): 6.9 / 8.7.  In place, between
+// products with a cold weight of 4096 rows, cast and product together: bf16, 16 x 4096: 15.0 / 10.6, 64 x 4096 (512 KB): 20.7 / 19.1, 32 x
+// 8192 (512 KB): 22.8 / 21.6, 16 x 14336 (448 KB): 23.5 / 22.1; fp32, 16 x 4096: 15.3 / 12.1, 16 x 8192 (512 KB): 18.8 / 18.3.  Hence the line.
 constexpr int FLAT_THREADS = 1024;
 constexpr int FLAT_UNROLL = 8;  // 16-byte loads in flight per lane of the scan
 constexpr int64_t FLAT_MAX_BYTES = 512 << 10;

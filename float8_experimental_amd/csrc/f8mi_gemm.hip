@@ -510,7 +510,7 @@ extern "C" int f8mi_gemm_ex(const void* a, int a_fmt, int a_transposed, int64_t 
     if (k % 128 != 0 || k < 384) { set_error("f8mi_gemm_ex: transposed operands need k %% 128 == 0 and k >= 384 (k=%lld)", (long long)k); return F8MI_ERR_UNSUPPORTED; }
     if (n % 64 != 0 || (a_transposed && m % 64 != 0)) { set_error("f8mi_gemm_ex: a transposed operand needs its row count to be a multiple of 64 (m=%lld n=%lld)", (long long)m, (long long)n); return F8MI_ERR_UNSUPPORTED; }
     if ((uintptr_t)a % 16 != 0 || (uintptr_t)bt % 16 != 0 || lda % 16 != 0 || ldb % 16 != 0) { set_error("f8mi_gemm_ex: transposed operands need 16-byte aligned addresses and row strides"); return F8MI_ERR_UNSUPPORTED; }
-    if (((m + 127) / 128) * ((n + 127) / 128) <= 256) { set_error("f8mi_gemm_ex: an output of at most 256 tiles of 128 x 128 is faster from transposed copies (128-row tiles read no operand transposed)"); return F8MI_ERR_UNSUPPORTED; }
+    if (((m + 127) / 128) * ((n + 127) / 128) <= 256) { set_error("f8mi_gemm_ex: an output of at most 256 tiles of 128 x 128 is left to copies (f8mi_gemm_nt may take the few-row kernel or split k for them)"); return F8MI_ERR_UNSUPPORTED; }
     // 32-bit offsets inside a step: 128 contraction rows of a transposed operand, 256 rows of a normal one
     if (m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff - BK || 128 * ldb + 256 > 0x7fffffffLL || (a_transposed ? 128 * lda + 256 : lda * (BM - 1) + k + BK) > 0x7fffffffLL) { set_error("f8mi_gemm_ex: dimension or row stride too large"); return F8MI_ERR_UNSUPPORTED; }
     const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;

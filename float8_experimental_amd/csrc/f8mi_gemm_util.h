@@ -186,7 +186,7 @@ static int allow_big_lds(K kern, int bytes, std::atomic<uint64_t>& done_mask) {
 
 // The 16x16x128 kernel with Bt (nt) or both operands (tt) given transposed: memory holds [contraction][rows];
 // lda / ldb = bytes between contraction rows, a_unit / b_unit = bytes between blocks of 64 rows.
-// 128-row-tile kernels (f8mi_gemm_mid.hip) for outputs of few 256 x 256 tiles: K % 128 == 0, aligned operands.
+// 128-row-tile kernels (f8mi_gemm_mid_impl.h) for outputs of few 256 x 256 tiles: K % 128 == 0, aligned operands.
 // wide = false: 128 x 128 tiles, true: 128 x 256.
 int launch_gemm_mid(int a_fmt, int b_fmt, int c_dtype, bool wide, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
                     const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C,
@@ -204,9 +204,13 @@ inline int use_mid_tiles(int64_t m, int64_t n, int64_t k) {
 // few-row kernel (f8mi_gemm_skinny.hip): m <= SKINNY_MAX_M, K % 128 == 0, aligned operands.
 constexpr int SKINNY_MAX_M = 256;
 // Time estimates in us behind the choice between the few-row kernel, a round of 128-row tiles, and the same tiles
-// with k split over workgroups -- fitted to measurements (rows, n x k: few-row / tiles): 128, 8192 x 8192: 27 / 37;
-// 128, 28672 x 8192: 83 / 37; 64, 28672 x 8192: 53 / 37; 64, 4096 x 14336: 27 / 63; 144 - 256, 4096 x 4096: 14 / 20;
-// 4096 x 14336: 36 / 60; 8192 x 8192: 41 - 48 / 37; 14336 x 4096: 39 - 47 / 22; 28672 x 8192: 119 - 143 / 59.
+// with k split over workgroups.  They were fitted to earlier forms of these kernels and rank them, no more.  As the kernels are now,
+// weights cold (rows, n x k: few-row / tiles / k split 8, 4 or 2 ways): 128, 8192 x 8192: 30 / 38 / 24; 128, 28672 x 8192: 110 / 46;
+// 64, 28672 x 8192: 72 / 39; 64, 4096 x 14336: 30 / 45 / 20; 192, 4096 x 4096: 15.4 / 17.6 / 17.8; 4096 x 14336: 40 / 49 / 24; 8192 x
+// 8192: 50 / 32 / 26; 14336 x 4096: 54 / 20; 28672 x 8192: 162 / 56.  Of 820 sizes with 17 - 1024 rows, n and k from 512 to 57344 and 28672,
+// the choice is within 5 % of the best of the three in 671.  Where it is not, the few-row kernel is kept for narrow weights with a
+// long k that a split would take in half the time (128, 512 x 28672: 67 / 71 / 20; 64, 2048 x 14336: 29 / 49 / 16), and tiles for 17 - 64 rows
+// with k = 512 that the few-row kernel takes in two thirds of it (17, 4096 x 512: 3.5 / 6.0).
 // They depend on the shape only, so the row-major and the k-blocked entry point decide alike.
 //
 // Few-row kernel: Bt at 6.5 TB/s from memory plus A (n / 32 workgroups x 16 row_tiles x k bytes) at 20 TB/s from L2,
@@ -218,8 +222,8 @@ inline double skinny_time_us(int64_t m, int64_t n, int64_t k) {
     const double idle = wgs < 256.0 ? __builtin_sqrt(256.0 / wgs) : 1.0;
     return passes * (2.0 + (double)n * (double)k * (0.154 + 0.025 * row_tiles) * 1e-6 * idle);
 }
-// Tiles: a round of 128 x 128 tiles takes 4.4 ns per unit of k, of 128 x 256 tiles 7.8 ns, of 256 x 256 tiles 10.6 ns,
-// for 1 row or 128.
+// Tiles: a round of 128 x 128 tiles was taken to cost 4.4 ns per unit of k, of 128 x 256 tiles 7.8 ns, of 256 x 256 tiles 10.6 ns, for
+// 1 row or 128 (128 x 128 now: 5 us and 2.3 ns with few tiles, 4.2 with 128 and more; 128 x 256: 6 us and 6 - 7.3 ns).
 inline double tiles_time_us(int64_t m, int64_t n, int64_t k) {
     const int64_t rt = (m + 127) / 128;
     if (rt * ((n + 127) / 128) <= 256) return 4.4e-3 * (double)k;

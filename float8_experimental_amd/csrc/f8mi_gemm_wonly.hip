@@ -2,7 +2,7 @@
 // fp32, fp32 accumulation.  HBM-bound for few rows: the fp8 weight, one byte per element, is all that has to be read.
 //
 // Dequantising into a tensor first reads n k, writes 2 n k, reads 2 n k and divides element by element: 14336 x 4096 took
-// 143 us (conversion) + 149 us (division) + 20 us (library GEMM) for four tokens, now 18 us in all (reading the weight at
+// 143 us (conversion) + 149 us (division) + 20 us (library GEMM) for four tokens, now 16.5 us in all (reading the weight at
 // 7 TB/s: 8.4; what is left is launch and ramp, and the conversions, which the few waves per SIMD do not all hide).  Here the weight goes from memory to
 // registers, is dequantised there and multiplied, as in the few-row fp8 kernel: a workgroup of eight waves owns 16 NT columns
 // of C and 16 MT rows, the waves split k eight ways, a lane's load is 16 consecutive k bytes of one weight row and the
