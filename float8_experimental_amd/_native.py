@@ -46,6 +46,7 @@ EXPORTS = (
     "f8mi_delayed_workspace_bytes",
     "f8mi_cast_dynamic",
     "f8mi_cast_dynamic_static",
+    "f8mi_cast_dynamic_resident",
     "f8mi_linear_few_rows",
     "f8mi_gemm_weight_only",
     "f8mi_dequant",
@@ -114,6 +115,8 @@ def lib() -> C.CDLL:
         L.f8mi_cast_dynamic.argtypes = [vp, i64, i64, i64, i32, i32, fp, vp, i32, vp, i32, vp, vp]
         L.f8mi_cast_dynamic_static.restype = i32
         L.f8mi_cast_dynamic_static.argtypes = [vp, i64, i64, i64, i32, i32, fp, vp, i32, vp, i32, vp]
+        L.f8mi_cast_dynamic_resident.restype = i32
+        L.f8mi_cast_dynamic_resident.argtypes = [vp, i64, i64, i64, i32, i32, fp, vp, i32, vp, i32, C.c_uint32, vp]
         L.f8mi_gemm_nt_kb.restype = i32
         L.f8mi_gemm_nt_kb.argtypes = [vp, i32, vp, i32, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp]
         L.f8mi_gemm_kb_ex.restype = i32

@@ -12,6 +12,7 @@
 // (so the 64 lanes of a store hit 32 banks twice: the floor for 256 bytes), and
 // the tile is read back as 16-byte row pieces: 8 lanes = one 128-byte segment of
 // a row of the transposed output.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -133,110 +134,69 @@ __device__ __forceinline__ void load_row8(Row8<DT>& r, const void* x, int64_t ro
     }
 }
 
-// out_kb / out_t_kb: F8MI_LAYOUT_* code of the respective output.
-template <int DT, int PROD, int FMT>
-__global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restrict__ x, int64_t rows, int64_t cols,
-                                                            int64_t ld, const float* __restrict__ scale_dev,
-                                                            uint8_t* __restrict__ out, uint8_t* __restrict__ out_t,
-                                                            float* amax_out, uint32_t tiles_x, uint32_t tiles_y,
-                                                            int out_kb, int out_t_kb, const uint32_t* __restrict__ amax_ws,
-                                                            int amax_nblocks, float* scale_out, uint32_t* amax_spread) {
-    __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];  // [column][row/4] dwords, swizzled
-    __shared__ uint32_t red[CAST_THREADS / 64];
-
-    const int t = threadIdx.x;
-    const int a = t & 15;   // column group: columns 8a .. 8a+7 of the tile
-    const int b = t >> 4;   // row group: rows 4b .. 4b+3 of each 64-row half
-    // Tiles are walked in bands of CAST_GROUP tile rows and, inside a band, in groups of CAST_GROUP tile
-    // columns: the blocks in flight then read 2 KB runs of each input row and write 1 KB runs of each
-    // transposed row, instead of one of the two walking through memory with a huge stride.
-    int ty, tx;
-    {
-        // Consecutive workgroup ids go to the 8 XCDs round-robin; re-deal them so that one XCD (one L2) gets whole
-        // groups of 64 neighbouring tiles (an 8 x 8 supertile where the tile grid divides evenly) and can merge
-        // their adjacent output segments, while consecutive groups go to consecutive XCDs: the workgroups in flight
-        // on the whole chip then cover ONE contiguous stretch of the tensor that advances through memory.  (Giving
-        // each XCD its own eighth of the tensor instead, eight fronts far apart, measured 5 % slower in the
-        // benchmark step: 5.36 -> 5.63 TB/s; up to 20 % on tensors below 300 MB.)
-        // (32-bit arithmetic: the host has checked that the tiles number at most 2^31 - 1; the 64-bit divisions of before cost every
-        // workgroup 0.4 us: 8192 x 4096 with both copies 30.6 -> 28.2 us, 16 x 4096 4.7 -> 4.3)
-        uint32_t bid = blockIdx.x;
-        const uint32_t nb = gridDim.x, nb_full = nb - nb % 512;  // ids past the last whole round of 8 groups stay
-        if (bid < nb_full) {
-            const uint32_t xcd = bid % 8, j = bid / 8;
-            bid = ((j / 64) * 8 + xcd) * 64 + (j % 64);
-        }
+// Which tile (ty, tx) of a tiles_y x tiles_x grid workgroup `bid` of `nb` takes.  Tiles are walked in bands of CAST_GROUP tile
+// rows and, inside a band, in groups of CAST_GROUP tile columns: the blocks in flight then read 2 KB runs of each input row
+// and write 1 KB runs of each transposed row, instead of one of the two walking through memory with a huge stride.
+__device__ __forceinline__ void cast_tile_of(uint32_t bid, uint32_t nb, uint32_t tiles_x, uint32_t tiles_y, int& ty, int& tx) {
+    // Consecutive workgroup ids go to the 8 XCDs round-robin; re-deal them so that one XCD (one L2) gets whole
+    // groups of 64 neighbouring tiles (an 8 x 8 supertile where the tile grid divides evenly) and can merge
+    // their adjacent output segments, while consecutive groups go to consecutive XCDs: the workgroups in flight
+    // on the whole chip then cover ONE contiguous stretch of the tensor that advances through memory.  (Giving
+    // each XCD its own eighth of the tensor instead, eight fronts far apart, measured 5 % slower in the
+    // benchmark step: 5.36 -> 5.63 TB/s; up to 20 % on tensors below 300 MB.)
+    // (32-bit arithmetic: the host has checked that the tiles number at most 2^31 - 1; the 64-bit divisions of before cost every
+    // workgroup 0.4 us: 8192 x 4096 with both copies 30.6 -> 28.2 us, 16 x 4096 4.7 -> 4.3)
+    const uint32_t nb_full = nb - nb % 512;  // ids past the last whole round of 8 groups stay
+    if (bid < nb_full) {
+        const uint32_t xcd = bid % 8, j = bid / 8;
+        bid = ((j / 64) * 8 + xcd) * 64 + (j % 64);
+    }
 #if F8MI_CAST_REVERSE_WALK  // measurement builds only: last tiles first, the reverse of the order the amax pass read in
-        bid = nb - 1 - bid;
+    bid = nb - 1 - bid;
 #endif
-        const uint32_t band = tiles_y <= CAST_GROUP ? 0 : bid / (CAST_GROUP * tiles_x);  // (one band: the product may not fit)
-        const uint32_t rem = bid - band * CAST_GROUP * tiles_x;
-        const uint32_t rows_in_band = min((uint32_t)CAST_GROUP, tiles_y - band * CAST_GROUP);
-        const uint32_t gcol = rem / (rows_in_band * CAST_GROUP);
-        const uint32_t r2 = rem - gcol * rows_in_band * CAST_GROUP;
-        const uint32_t cols_in_g = min((uint32_t)CAST_GROUP, tiles_x - gcol * CAST_GROUP);
-        ty = (int)(band * CAST_GROUP + r2 / cols_in_g);
-        tx = (int)(gcol * CAST_GROUP + r2 % cols_in_g);
-    }
-    const int64_t r0 = (int64_t)ty * CAST_TILE;
-    const int64_t c0 = (int64_t)tx * CAST_TILE;
-    const int64_t col = c0 + 8 * a;
+    const uint32_t band = tiles_y <= CAST_GROUP ? 0 : bid / (CAST_GROUP * tiles_x);  // (one band: the product may not fit)
+    const uint32_t rem = bid - band * CAST_GROUP * tiles_x;
+    const uint32_t rows_in_band = min((uint32_t)CAST_GROUP, tiles_y - band * CAST_GROUP);
+    const uint32_t gcol = rem / (rows_in_band * CAST_GROUP);
+    const uint32_t r2 = rem - gcol * rows_in_band * CAST_GROUP;
+    const uint32_t cols_in_g = min((uint32_t)CAST_GROUP, tiles_x - gcol * CAST_GROUP);
+    ty = (int)(band * CAST_GROUP + r2 / cols_in_g);
+    tx = (int)(gcol * CAST_GROUP + r2 % cols_in_g);
+}
 
-    // dynamic scaling: the amax kernel's per-workgroup maxima (at most WS_WORDS = 4 x 64 lanes x 4 words), requested
-    // ahead of the tile so that they arrive first.  Every wave fetches all of them: no LDS, no barrier.
-    static_assert(WS_WORDS <= 4 * 64 * 4, "four 16-byte loads per lane cover the workspace");
-    uint4 ws_words[4];
-    if (amax_ws) {
+// A tile of 64 H rows x 128 columns at (r0, c0), one per workgroup of 256 lanes: lane t holds columns 8 (t % 16) .. + 7 of rows
+// 64 h + 4 (t / 16) .. + 3 for h < H.
+template <int DT, int H>
+__device__ __forceinline__ void load_tile(Row8<DT> (&in)[H][4], const void* x, int64_t r0, int64_t c0, int64_t rows, int64_t cols, int64_t ld) {
+    const int a = threadIdx.x & 15, b = threadIdx.x >> 4;
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-            ws_words[q] = q * 256 < amax_nblocks ? ((const uint4*)amax_ws)[q * 64 + (t & 63)] : make_uint4(0u, 0u, 0u, 0u);
-    }
-
-    Row8<DT> in[2][4];
+    for (int h = 0; h < H; h++)
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) load_row8<DT>(in[h][j], x, r0 + 64 * h + 4 * b + j, col, rows, cols, ld);
-
-    // The scale: given -- or, for dynamic scaling, derived here from the per-workgroup maxima the amax kernel left in
-    // amax_ws (every wave of every workgroup reduces the <= 1024 words itself; saves the one-block launch that would do
-    // it once).  The words were requested before the tile and nothing here waits for anybody else, so the reduction
-    // runs while the tile's loads are still in flight.  (A first version shared the work among the four waves through
-    // LDS: its two barriers, in the middle of the block, cost more than the redundant loads do.)  Words past
-    // amax_nblocks are leftovers of an earlier, larger call and are masked.  Same arithmetic as amax_finalize_kernel,
-    // in the tensor's dtype.
-    float scale;
-    if (amax_ws) {
-        uint32_t wm = 0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int first = q * 256 + (t & 63) * 4;
-            const uint32_t w[4] = {ws_words[q].x, ws_words[q].y, ws_words[q].z, ws_words[q].w};
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const uint32_t v = first + c < amax_nblocks ? w[c] : 0u;
-                wm = wm > v ? wm : v;
-            }
-        }
-        wm = wave_max_u32(wm);
-        scale = amax_to_scale_dev(abs_bits_to_float(wm, DT), DT, FMT, DT == F8MI_FP16);
-        if (blockIdx.x == 0 && t == 0) *scale_out = scale;
-    } else {
-        scale = *scale_dev;
-    }
-    constexpr float fmax = FMT == F8MI_E4M3FN ? 448.0f : 57344.0f;
-
+        for (int j = 0; j < 4; j++) load_row8<DT>(in[h][j], x, r0 + 64 * h + 4 * b + j, c0 + 8 * a, rows, cols, ld);
+}
+template <int DT, int H>
+__device__ __forceinline__ uint32_t absmax_tile(const Row8<DT> (&in)[H][4]) {
     uint32_t m = 0;
-    if (amax_out) {
 #pragma unroll
-        for (int h = 0; h < 2; h++)
+    for (int h = 0; h < H; h++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) m = absmax_row<DT>(in[h][j], m);
-        m = absmax_done<DT>(m);
-    }
+        for (int j = 0; j < 4; j++) m = absmax_row<DT>(in[h][j], m);
+    return absmax_done<DT>(m);
+}
 
+// Scales, converts and stores such a tile: `out` row by row from registers, `out_t` through tileT.  out_kb / out_t_kb:
+// F8MI_LAYOUT_* code of the respective output.
+template <int DT, int PROD, int FMT, int H>
+__device__ __forceinline__ void emit_tile(const Row8<DT> (&in)[H][4], uint32_t* tileT, float scale, int64_t r0, int64_t c0, int64_t rows, int64_t cols,
+                                          uint8_t* __restrict__ out, uint8_t* __restrict__ out_t, int out_kb, int out_t_kb) {
+    constexpr int DWORDS = 16 * H;                  // of a tile column: four rows each
+    constexpr int SWIZZLE = 4 * H - 1;              // 16-byte pieces of a tile column, less one
+    const int t = threadIdx.x;
+    const int a = t & 15, b = t >> 4;
+    const int64_t col = c0 + 8 * a;
+    constexpr float fmax = FMT == F8MI_E4M3FN ? 448.0f : 57344.0f;
     // Zero-padded k-blocked outputs (F8MI_LAYOUT_KBLOCK64_PAD128): the tile grid ends exactly where the padding does, so
-    // a tile writes all of its 128 columns (`out`) or rows (`out_t`); what lies past the tensor's edge is forced to
+    // a tile writes all of its columns (`out`) or rows (`out_t`); what lies past the tensor's edge is forced to
     // zero bytes (elements read as +0 would become NaN codes under a NaN scale).
     const bool pad = out_kb == F8MI_LAYOUT_KBLOCK64_PAD128 || out_t_kb == F8MI_LAYOUT_KBLOCK64_PAD128;
     uint32_t keep_lo = 0xffffffffu, keep_hi = 0xffffffffu;  // bytes of the lane's eight columns that lie inside the row
@@ -246,7 +206,7 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restri
         keep_hi = valid > 4 ? (1u << (8 * (valid - 4))) - 1u : 0u;
     }
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
+    for (int h = 0; h < H; h++) {
         uint32_t lo[4], hi[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -277,21 +237,21 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restri
             uint32_t tc[8];
             transpose4x4_bytes(lo[0], lo[1], lo[2], lo[3], tc[0], tc[1], tc[2], tc[3]);
             transpose4x4_bytes(hi[0], hi[1], hi[2], hi[3], tc[4], tc[5], tc[6], tc[7]);
-            const int d = 16 * h + b;              // dword index (rows 4d .. 4d+3) within a tile column
-            const int dsw = d ^ ((a & 7) << 2);    // swizzle by column group
+            const int d = 16 * h + b;                    // dword index (rows 4d .. 4d+3) within a tile column
+            const int dsw = d ^ ((a & SWIZZLE) << 2);    // swizzle by column group
 #pragma unroll
-            for (int cc = 0; cc < 8; cc++) tileT[(8 * a + cc) * (CAST_TILE / 4) + dsw] = tc[cc];
+            for (int cc = 0; cc < 8; cc++) tileT[(8 * a + cc) * DWORDS + dsw] = tc[cc];
         }
     }
 
     if (out_t) {
         __syncthreads();
 #pragma unroll
-        for (int p = 0; p < 4; p++) {
+        for (int p = 0; p < 2 * H; p++) {
             const int id = p * CAST_THREADS + t;
-            const int c = id >> 3, q = id & 7;  // tile column c (a row of out_t), 16-byte piece q
-            const int qsw = q ^ ((c >> 3) & 7);
-            const uint4 v = *(const uint4*)&tileT[c * (CAST_TILE / 4) + 4 * qsw];
+            const int c = id / (4 * H), q = id % (4 * H);  // tile column c (a row of out_t), 16-byte piece q
+            const int qsw = q ^ ((c >> 3) & SWIZZLE);
+            const uint4 v = *(const uint4*)&tileT[c * DWORDS + 4 * qsw];
             const int64_t gc = c0 + c;
             const int64_t gr = r0 + 16 * q;
             if (gc < cols && (gr < rows || out_t_kb == F8MI_LAYOUT_KBLOCK64_PAD128)) {
@@ -308,6 +268,67 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restri
             }
         }
     }
+}
+
+template <int DT, int PROD, int FMT>
+__global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restrict__ x, int64_t rows, int64_t cols,
+                                                            int64_t ld, const float* __restrict__ scale_dev,
+                                                            uint8_t* __restrict__ out, uint8_t* __restrict__ out_t,
+                                                            float* amax_out, uint32_t tiles_x, uint32_t tiles_y,
+                                                            int out_kb, int out_t_kb, const uint32_t* __restrict__ amax_ws,
+                                                            int amax_nblocks, float* scale_out, uint32_t* amax_spread) {
+    __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];  // [column][row/4] dwords, swizzled
+    __shared__ uint32_t red[CAST_THREADS / 64];
+
+    const int t = threadIdx.x;
+    int ty, tx;
+    cast_tile_of(blockIdx.x, gridDim.x, tiles_x, tiles_y, ty, tx);
+    const int64_t r0 = (int64_t)ty * CAST_TILE;
+    const int64_t c0 = (int64_t)tx * CAST_TILE;
+
+    // dynamic scaling: the amax kernel's per-workgroup maxima (at most WS_WORDS = 4 x 64 lanes x 4 words), requested
+    // ahead of the tile so that they arrive first.  Every wave fetches all of them: no LDS, no barrier.
+    static_assert(WS_WORDS <= 4 * 64 * 4, "four 16-byte loads per lane cover the workspace");
+    uint4 ws_words[4];
+    if (amax_ws) {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            ws_words[q] = q * 256 < amax_nblocks ? ((const uint4*)amax_ws)[q * 64 + (t & 63)] : make_uint4(0u, 0u, 0u, 0u);
+    }
+
+    Row8<DT> in[2][4];
+    load_tile<DT, 2>(in, x, r0, c0, rows, cols, ld);
+
+    // The scale: given -- or, for dynamic scaling, derived here from the per-workgroup maxima the amax kernel left in
+    // amax_ws (every wave of every workgroup reduces the <= 1024 words itself; saves the one-block launch that would do
+    // it once).  The words were requested before the tile and nothing here waits for anybody else, so the reduction
+    // runs while the tile's loads are still in flight.  (A first version shared the work among the four waves through
+    // LDS: its two barriers, in the middle of the block, cost more than the redundant loads do.)  Words past
+    // amax_nblocks are leftovers of an earlier, larger call and are masked.  Same arithmetic as amax_finalize_kernel,
+    // in the tensor's dtype.
+    float scale;
+    if (amax_ws) {
+        uint32_t wm = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int first = q * 256 + (t & 63) * 4;
+            const uint32_t w[4] = {ws_words[q].x, ws_words[q].y, ws_words[q].z, ws_words[q].w};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const uint32_t v = first + c < amax_nblocks ? w[c] : 0u;
+                wm = wm > v ? wm : v;
+            }
+        }
+        wm = wave_max_u32(wm);
+        scale = amax_to_scale_dev(abs_bits_to_float(wm, DT), DT, FMT, DT == F8MI_FP16);
+        if (blockIdx.x == 0 && t == 0) *scale_out = scale;
+    } else {
+        scale = *scale_dev;
+    }
+
+    uint32_t m = 0;
+    if (amax_out) m = absmax_tile<DT, 2>(in);
+    emit_tile<DT, PROD, FMT, 2>(in, tileT, scale, r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
 
     if (amax_out && amax_spread) {
         // Every wave folds its maximum (the bit pattern in the input's dtype) into one of SPREAD_WORDS words with an
@@ -488,6 +509,79 @@ static int launch_cast_flat(int fmt, hipStream_t stream, const void* x, int64_t 
     return check_hip(hipGetLastError(), "cast (dynamic, few rows) kernel launch");
 }
 
+// Dynamic scaling of a tensor that the chip can hold, any layout and both copies, in ONE launch that reads it once: every
+// workgroup loads its tile (64 H rows x 128 columns) into registers, publishes the tile's maximum, collects everybody's and casts
+// what it holds.  The two kernels it replaces read the tensor twice and pay a launch and a ramp more.
+//
+// A workgroup publishes one 64-bit word, {launch tag, maximum}, with an agent-scope store and reads the others' with agent-scope
+// loads: the words carry all there is to exchange, so no fence is needed.  The tag is the host's count of such launches, never
+// used twice, so a word of any other launch just reads as "not there yet" and nothing has to be cleared; the host keeps launches
+// that may run at the same time (other streams) on other words.  All workgroups fit on the chip at once (see
+// resident_tile_rows), but nothing depends on it: a workgroup that has waited for wait_ticks of the 100 MHz clock -- because
+// other work holds the CUs that the missing ones need -- finds the maximum itself by reading the whole tensor, and goes on.  So every wave
+// ends whatever else runs, and the result is the same bits either way.
+//
+// us a call, back to back, inputs cold, amax and cast / this one: one copy, bf16, 512 x 1024: 8.8 / 6.6, 2048 x 2048: 10.6 / 9.0, 2726 x 934
+// (padded): 16.1 / 10.7, 2048 x 4096: 14.3 / 12.2, 4096 x 4096: 20.5 / 18.9; both copies, 512 x 1024: 8.8 / 6.6, 4096 x 4096: 21.8 / 20.4; fp32,
+// 512 x 1024: 9.9 / 6.9, 4096 x 4096: 30.7 / 28.9.  Inside a launch of 4096 x 4096 bf16 (1024 workgroups): the last tile has arrived after 9.5
+// us, everybody has everybody's maximum after 11.3 (2 us is what a word takes to memory and back, 512 x 1024 waits as long), the
+// last byte is stored after 15.  Loads in smaller batches, other tile shapes and linear tile orders all took the same or longer.
+constexpr int RESIDENT_WORDS = 1024;  // workgroups at most
+constexpr uint32_t RESIDENT_WAIT_TICKS = 200000;  // 2 ms: several rounds of the longest tiles of the GEMMs that may hold the CUs
+
+template <int DT, int FMT, int H>
+__global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_kernel(const void* __restrict__ x, int64_t rows, int64_t cols, int64_t ld,
+                                                                             float* __restrict__ scale_out, uint8_t* __restrict__ out,
+                                                                             uint8_t* __restrict__ out_t, uint32_t tiles_x, uint32_t tiles_y,
+                                                                             int out_kb, int out_t_kb, uint64_t* __restrict__ words, uint32_t tag,
+                                                                             uint32_t wait_ticks) {
+    __shared__ uint32_t tileT[32 * 64 * H];
+    __shared__ uint32_t red[CAST_THREADS / 64], late;
+    const int t = threadIdx.x;
+    int ty, tx;
+    cast_tile_of(blockIdx.x, gridDim.x, tiles_x, tiles_y, ty, tx);
+    const int64_t r0 = (int64_t)ty * (64 * H), c0 = (int64_t)tx * CAST_TILE;
+    Row8<DT> in[H][4];
+    load_tile<DT, H>(in, x, r0, c0, rows, cols, ld);
+    uint32_t m = wave_max_u32(absmax_tile<DT, H>(in));
+    if ((t & 63) == 0) red[t >> 6] = m;
+    if (t == 0) late = 0u;
+    __syncthreads();
+    static_assert(CAST_THREADS == 256, "four waves");
+    m = max(max(red[0], red[1]), max(red[2], red[3]));
+    if (t == 0) __hip_atomic_store(&words[blockIdx.x], (uint64_t)tag << 32 | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t start = wall_clock64();
+    bool here = true;
+    for (uint32_t i = t; i < gridDim.x; i += CAST_THREADS) {
+        uint64_t w;
+        while ((uint32_t)((w = __hip_atomic_load(&words[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) != tag) {
+            if (wall_clock64() - start >= wait_ticks) { here = false; break; }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        if (here) m = max(m, (uint32_t)w);
+        else break;
+    }
+    if (!here) late = 1u;
+    m = wave_max_u32(m);
+    __syncthreads();  // everybody has read `red` and written `late`
+    if (late) {  // the same for the whole workgroup
+        uint32_t own = 0;
+        for (int64_t r = 0; r < (ld ? rows : 1); r++)
+            for (int64_t c = 8 * t; c < cols; c += 8 * CAST_THREADS) {
+                Row8<DT> v;
+                load_row8<DT>(v, x, r, c, rows, cols, ld);
+                own = absmax_row<DT>(v, own);
+            }
+        m = wave_max_u32(absmax_done<DT>(own));
+    }
+    if ((t & 63) == 0) red[t >> 6] = m;
+    __syncthreads();
+    m = max(max(red[0], red[1]), max(red[2], red[3]));
+    const float scale = amax_to_scale_dev(abs_bits_to_float(m, DT), DT, FMT, DT == F8MI_FP16);
+    if (blockIdx.x == 0 && t == 0) *scale_out = scale;
+    emit_tile<DT, DT, FMT, H>(in, tileT, scale, r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
+}
+
 // where a dynamic-scaling cast takes its scale from (see cast_layout_impl)
 struct AmaxSource {
     const uint32_t* ws;
@@ -531,15 +625,20 @@ static int launch_cast1(int fmt, dim3 g, hipStream_t stream, const void* x, int6
     return launch_cast2<DT, PROD, F8MI_E5M2>(g, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src);
 }
 
+static int check_cast_layouts(int64_t rows, int64_t cols, const void* out, int out_layout, const void* out_t, int out_t_layout) {
+    if (out_layout < F8MI_LAYOUT_ROWMAJOR || out_layout > F8MI_LAYOUT_KBLOCK64_PAD128 || out_t_layout < F8MI_LAYOUT_ROWMAJOR || out_t_layout > F8MI_LAYOUT_KBLOCK64_PAD128) { set_error("f8mi_cast: unknown layout code"); return F8MI_ERR_INVALID_ARG; }
+    if (out && out_layout == F8MI_LAYOUT_KBLOCK64 && cols % 64 != 0) { set_error("f8mi_cast: k-blocked `out` needs cols %% 64 == 0 (cols=%lld); F8MI_LAYOUT_KBLOCK64_PAD128 takes any", (long long)cols); return F8MI_ERR_UNSUPPORTED; }
+    if (out_t && out_t_layout == F8MI_LAYOUT_KBLOCK64 && rows % 64 != 0) { set_error("f8mi_cast: k-blocked `out_t` needs rows %% 64 == 0 (rows=%lld); F8MI_LAYOUT_KBLOCK64_PAD128 takes any", (long long)rows); return F8MI_ERR_UNSUPPORTED; }
+    return F8MI_OK;
+}
+
 // Validates and launches the cast.  `src.ws` null: the scale is read from scale_dev (f8mi_cast_layout).  Not null
 // (dynamic scaling, product in the input's dtype): the kernel derives the scale from the src.nblocks per-workgroup
 // maxima in src.ws and workgroup 0 stores it to src.scale_out.
 static int cast_layout_impl(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, const float* scale_dev,
                             int product_dtype, int fp8_fmt, uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout,
                             float* amax_dev, hipStream_t stream, const AmaxSource& src) {
-    if (out_layout < F8MI_LAYOUT_ROWMAJOR || out_layout > F8MI_LAYOUT_KBLOCK64_PAD128 || out_t_layout < F8MI_LAYOUT_ROWMAJOR || out_t_layout > F8MI_LAYOUT_KBLOCK64_PAD128) { set_error("f8mi_cast: unknown layout code"); return F8MI_ERR_INVALID_ARG; }
-    if (out && out_layout == F8MI_LAYOUT_KBLOCK64 && cols % 64 != 0) { set_error("f8mi_cast: k-blocked `out` needs cols %% 64 == 0 (cols=%lld); F8MI_LAYOUT_KBLOCK64_PAD128 takes any", (long long)cols); return F8MI_ERR_UNSUPPORTED; }
-    if (out_t && out_t_layout == F8MI_LAYOUT_KBLOCK64 && rows % 64 != 0) { set_error("f8mi_cast: k-blocked `out_t` needs rows %% 64 == 0 (rows=%lld); F8MI_LAYOUT_KBLOCK64_PAD128 takes any", (long long)rows); return F8MI_ERR_UNSUPPORTED; }
+    if (const int rc = check_cast_layouts(rows, cols, out, out_layout, out_t, out_t_layout)) return rc;
     // the kernel takes the layout codes as they are (0: row-major, otherwise k-blocked; PAD128: whole tiles are written)
     const int out_kb = out ? out_layout : F8MI_LAYOUT_ROWMAJOR, out_t_kb = out_t ? out_t_layout : F8MI_LAYOUT_ROWMAJOR;
     // ld == 0: every row reads the same `cols` elements (the kernels address row * ld + col)
@@ -624,6 +723,104 @@ extern "C" int f8mi_cast_delayed(const void* x, int64_t rows, int64_t cols, int6
                             (hipStream_t)stream, AmaxSource{nullptr, 0, nullptr, (uint32_t*)workspace});
 }
 
+namespace f8mi {
+
+constexpr int STATIC_MAX_DEVICES = 64;
+
+// Device address of a device array of this library on the current device, looked up once per device and kept (nullptr + error
+// message on failure).  Two threads racing here store the same value.
+template <typename T>
+static T* device_array(const void* symbol, std::atomic<T*> (&known)[STATIC_MAX_DEVICES], const char* what) {
+    int dev = -1;
+    if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
+    if (dev < 0 || dev >= STATIC_MAX_DEVICES) { set_error("%s: device index %d, at most %d devices", what, dev, STATIC_MAX_DEVICES); return nullptr; }
+    if (T* p = known[dev].load(std::memory_order_acquire)) return p;
+    void* addr = nullptr;
+    if (check_hip(hipGetSymbolAddress(&addr, symbol), what)) return nullptr;
+    if (!addr) { set_error("%s: no address on device %d", what, dev); return nullptr; }
+    known[dev].store((T*)addr, std::memory_order_release);
+    return (T*)addr;
+}
+
+// The words of the one-launch cast: a set for each of the first RESIDENT_STREAMS streams that use it, so that launches which may
+// run at the same time do not share any (sharing would be slow, not wrong: see the kernel).  Later streams take the two
+// launches.  A stream handle that comes back for a new stream finds the old one's set: its work is done.
+constexpr int RESIDENT_STREAMS = 64;
+static __device__ __align__(256) uint64_t resident_words[RESIDENT_STREAMS][RESIDENT_WORDS];
+static std::atomic<uint64_t*> g_resident_words[STATIC_MAX_DEVICES];
+static std::atomic<uintptr_t> g_resident_streams[STATIC_MAX_DEVICES][RESIDENT_STREAMS];
+static std::atomic<uint32_t> g_resident_tag{0};
+
+static uint64_t* resident_words_of(hipStream_t stream) {
+    uint64_t* base = device_array(HIP_SYMBOL(resident_words), g_resident_words, "resident_words");
+    if (!base) return nullptr;
+    int dev = 0;
+    if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
+    const uintptr_t key = (uintptr_t)stream + 1;  // the default stream is a null handle
+    for (int i = 0; i < RESIDENT_STREAMS; i++) {
+        uintptr_t have = g_resident_streams[dev][i].load(std::memory_order_relaxed);
+        if (!have && g_resident_streams[dev][i].compare_exchange_strong(have, key, std::memory_order_relaxed)) have = key;
+        if (have == key) return base + (size_t)i * RESIDENT_WORDS;
+    }
+    return nullptr;
+}
+
+// Rows of the tiles that the one-launch cast gives a tensor, 0: it does not take it.  At most four workgroups a CU (RESIDENT_WORDS on
+// 256): it holds eight of them (five of 128 rows of fp32), so that all are there at once also beside other streams' kernels.
+static int resident_tile_rows(int64_t rows, int64_t cols) {
+    const int64_t tx = (cols + CAST_TILE - 1) / CAST_TILE, ty = (rows + CAST_TILE - 1) / CAST_TILE, most = std::min(RESIDENT_WORDS, 4 * cu_count());
+    if (ty > most || tx > most) return 0;
+    // tiles of 64 rows while they number at most two a CU: more workgroups share a small tensor (512 x 1024: 7.6 -> 6.6 us); beyond that
+    // they only add words to collect (2048 x 4096 as 512 or 1024 tiles: 12.2 / 12.5)
+    return 2 * tx * ty <= most / 2 ? 64 : tx * ty <= most ? 128 : 0;
+}
+
+template <int DT, int FMT>
+static int launch_cast_resident1(int tile_rows, dim3 g, hipStream_t stream, const void* x, int64_t rows, int64_t cols, int64_t ld, float* scale_dev,
+                                 uint8_t* out, uint8_t* out_t, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb, uint64_t* words, uint32_t tag,
+                                 uint32_t wait_ticks) {
+    if (tile_rows == 64) hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 1>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+    else hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 2>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+    return check_hip(hipGetLastError(), "cast (dynamic, resident) kernel launch");
+}
+template <int DT>
+static int launch_cast_resident(int fmt, int tile_rows, dim3 g, hipStream_t stream, const void* x, int64_t rows, int64_t cols, int64_t ld, float* scale_dev,
+                                uint8_t* out, uint8_t* out_t, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb, uint64_t* words, uint32_t tag,
+                                uint32_t wait_ticks) {
+    if (fmt == F8MI_E4M3FN) return launch_cast_resident1<DT, F8MI_E4M3FN>(tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+    return launch_cast_resident1<DT, F8MI_E5M2>(tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+}
+
+}  // namespace f8mi
+
+extern "C" int f8mi_cast_dynamic_resident(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, int fp8_fmt, float* scale_dev,
+                                          uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout, uint32_t wait_ticks, void* stream_) {
+    hipStream_t stream = (hipStream_t)stream_;
+    if (rows <= 0 || cols <= 0 || (ld < cols && ld != 0) || in_dtype < 0 || in_dtype > 2 || fp8_fmt < 0 || fp8_fmt > 1) { set_error("f8mi_cast_dynamic_resident: bad shape or dtype/format code"); return F8MI_ERR_INVALID_ARG; }
+    if (!x || !scale_dev || (!out && !out_t)) { set_error("f8mi_cast_dynamic_resident: null tensor or scale, or no output"); return F8MI_ERR_INVALID_ARG; }
+    if (const int rc = check_cast_layouts(rows, cols, out, out_layout, out_t, out_t_layout)) return rc;
+    const int tile_rows = resident_tile_rows(rows, cols);
+    if (!tile_rows) { set_error("f8mi_cast_dynamic_resident: %lld x %lld is more than the chip holds", (long long)rows, (long long)cols); return F8MI_ERR_UNSUPPORTED; }
+    // a captured launch would use its tag again on every replay
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (check_hip(hipStreamIsCapturing(stream, &capture), "hipStreamIsCapturing")) return F8MI_ERR_HIP;
+    if (capture != hipStreamCaptureStatusNone) { set_error("f8mi_cast_dynamic_resident: the stream is being captured"); return F8MI_ERR_UNSUPPORTED; }
+    uint64_t* words = resident_words_of(stream);
+    if (!words) { set_error("f8mi_cast_dynamic_resident: %d other streams use it", RESIDENT_STREAMS); return F8MI_ERR_UNSUPPORTED; }
+    uint32_t tag = g_resident_tag.fetch_add(1, std::memory_order_relaxed) + 1;
+    if (!tag) tag = g_resident_tag.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 is what the words start with
+    const int out_kb = out ? out_layout : F8MI_LAYOUT_ROWMAJOR, out_t_kb = out_t ? out_t_layout : F8MI_LAYOUT_ROWMAJOR;
+    // whole 128 x 128 tiles, as the padded layouts are
+    const uint32_t tiles_x = (uint32_t)((cols + CAST_TILE - 1) / CAST_TILE), tiles_y = (uint32_t)((rows + CAST_TILE - 1) / CAST_TILE) * (CAST_TILE / tile_rows);
+    const dim3 g(tiles_x * tiles_y);
+    const size_t esz = in_dtype == F8MI_FP32 ? 4 : 2;
+    const double n = (double)rows * (double)cols;
+    ProfScope prof(F8MI_K_CAST, (ld == 0 ? (double)cols : n) * esz + n * ((out ? 1 : 0) + (out_t ? 1 : 0)), stream);
+    if (in_dtype == F8MI_BF16) return launch_cast_resident<F8MI_BF16>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+    if (in_dtype == F8MI_FP16) return launch_cast_resident<F8MI_FP16>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+    return launch_cast_resident<F8MI_FP32>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+}
+
 extern "C" int f8mi_cast_dynamic(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, int fp8_fmt, float* scale_dev,
                                  uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout, void* workspace, void* stream_) {
     hipStream_t stream = (hipStream_t)stream_;
@@ -659,6 +856,10 @@ extern "C" int f8mi_cast_dynamic(const void* x, int64_t rows, int64_t cols, int6
         if (in_dtype == F8MI_FP16) return launch_cast_flat<F8MI_FP16>(fp8_fmt, stream, x, rows, cols, scale_dev, out, out_kb);
         return launch_cast_flat<F8MI_FP32>(fp8_fmt, stream, x, rows, cols, scale_dev, out, out_kb);
     }
+    if (resident_tile_rows(rows, cols)) {
+        const int rc = f8mi_cast_dynamic_resident(x, rows, cols, ld, in_dtype, fp8_fmt, scale_dev, out, out_layout, out_t, out_t_layout, RESIDENT_WAIT_TICKS, stream_);
+        if (rc != F8MI_ERR_UNSUPPORTED) return rc;
+    }
     // amax pass: per-workgroup maxima into the workspace; the cast's workgroups reduce them and derive the scale
     // themselves (no one-block finalize launch in between), workgroup 0 stores it to *scale_dev
     int nblocks = 0;
@@ -681,22 +882,7 @@ namespace f8mi {
 static __device__ __align__(256) uint32_t scratch[WS_WORDS];
 static_assert(sizeof(scratch) == F8MI_STATIC_SCRATCH_BYTES, "f8mi.h states the size of the static scratch");
 
-constexpr int STATIC_MAX_DEVICES = 64;
 static std::atomic<uint32_t*> g_scratch_ptr[STATIC_MAX_DEVICES];
-
-// Device address of `scratch` on the current device (nullptr + error message on failure).
-static uint32_t* static_scratch_ptr() {
-    int dev = -1;
-    if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
-    if (dev < 0 || dev >= STATIC_MAX_DEVICES) { set_error("f8mi_cast_dynamic_static: device index %d, at most %d devices", dev, STATIC_MAX_DEVICES); return nullptr; }
-    uint32_t* p = g_scratch_ptr[dev].load(std::memory_order_acquire);
-    if (p) return p;
-    void* addr = nullptr;
-    if (check_hip(hipGetSymbolAddress(&addr, HIP_SYMBOL(scratch)), "hipGetSymbolAddress(scratch)")) return nullptr;
-    if (!addr) { set_error("f8mi_cast_dynamic_static: the static scratch has no address on device %d", dev); return nullptr; }
-    g_scratch_ptr[dev].store((uint32_t*)addr, std::memory_order_release);  // two threads racing here store the same value
-    return (uint32_t*)addr;
-}
 
 }  // namespace f8mi
 
@@ -708,7 +894,7 @@ extern "C" int f8mi_cast_dynamic_static(const void* x, int64_t rows, int64_t col
                   (long long)rows, (long long)cols, (long long)F8MI_STATIC_MAX_ELEMS);
         return F8MI_ERR_INVALID_ARG;
     }
-    uint32_t* ws = f8mi::static_scratch_ptr();
+    uint32_t* ws = device_array(HIP_SYMBOL(scratch), g_scratch_ptr, "f8mi_cast_dynamic_static");
     if (!ws) return F8MI_ERR_HIP;
     return f8mi_cast_dynamic(x, rows, cols, ld, in_dtype, fp8_fmt, scale_dev, out, out_layout, out_t, out_t_layout, ws, stream);
 }

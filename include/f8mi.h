@@ -233,6 +233,16 @@ int f8mi_cast_dynamic_static(const void* x, int64_t rows, int64_t cols, int64_t 
                              float* scale_dev, uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout,
                              void* stream);
 
+/* f8mi_cast_dynamic in one launch that reads x once, for tensors that the chip holds: at most 1024 tiles of 128 x 128 (fewer
+ * on a device of fewer than 256 CUs).  f8mi_cast_dynamic takes it by itself; the same bits.  The workgroups exchange their
+ * maxima inside the launch; one that has waited wait_ticks of the 100 MHz clock for the others reads the whole tensor
+ * itself, so the launch ends and is right whatever else runs (wait_ticks 0: nobody waits).  Refused with
+ * F8MI_ERR_UNSUPPORTED, nothing queued: larger tensors, a stream that is being captured, more than 64 streams of one
+ * device. */
+int f8mi_cast_dynamic_resident(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, int fp8_fmt,
+                               float* scale_dev, uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout,
+                               uint32_t wait_ticks, void* stream);
+
 /* A whole linear of at most 16 rows and F8MI_FEW_ROWS_ELEMS activations in one kernel: c[m][n] = sum_k x8[m][k] * w[n][k]
  * / (scale_x * scale_w) (+ bias[n]) with x8 the saturated e4m3 cast of x, which every workgroup makes for itself.  The same
  * bits as f8mi_cast_dynamic (scale_x_dev null) or f8mi_cast_layout (scale_x_dev given, product in product_dtype) followed by

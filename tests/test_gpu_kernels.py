@@ -505,6 +505,65 @@ def test_cast_dynamic_one_copy_equals_amax_scale_then_cast(nat, dt, shape):
                 assert same_bytes_mod_nan_sign(fp8_bytes(o), fp8_bytes(o_want)), (dt, shape, fmt, kb)
 
 
+# The one-launch cast of a tensor that the chip holds: a single tile, tiles of 64 rows and of 128, one row or column into the next tile,
+# the last size of either kind and the largest of all; nobody waits (every workgroup finds the maximum itself) or as shipped.
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("shape", [(1, 1), (64, 128), (65, 129), (200, 1000), (513, 1031), (2048, 2048), (2049, 2048), (1000, 3001), (4096, 4096)])
+def test_cast_dynamic_resident_equals_amax_scale_then_cast(nat, dt, shape):
+    tdt = TORCH_DT[dt]
+    x = heavy(shape, tdt, 23).to(DEV)
+    rows, cols = shape
+    big = rows * cols > 1 << 22
+    first, last = x.clone(), x.clone()
+    first.view(-1)[0], last.view(-1)[-1] = float("-inf"), float("nan")
+    odd = torch.zeros(rows, cols + 5, device=DEV, dtype=tdt)[:, 3:cols + 3]  # rows at any multiple of the element size
+    odd.copy_(x)
+    variants = [x, last] if big else [x, first, last, odd, x[:1].expand(rows, cols), torch.zeros_like(x)]
+    for v in variants:
+        for fmt, (code, f8dt) in F8.items():
+            _, s_want = nat.amax_scale(v, f8dt, want_amax=False)
+            for layout in {0, nat.KBLOCK_PAD}:
+                want = nat.cast(v.contiguous(), s_want, f8dt, want_out_t=True, out_kblock=layout, out_t_kblock=layout)
+                for ticks in (0, 200000) if not big or layout == 0 and v is x and dt == "bf16" and shape[0] < 4096 else (200000,):
+                    got = [torch.zeros_like(w.view(torch.uint8)) for w in want]
+                    s = torch.zeros((), device=DEV)
+                    rc = nat.lib().f8mi_cast_dynamic_resident(v.data_ptr(), rows, cols, v.stride(0), nat._DT[tdt], code, s.data_ptr(), got[0].data_ptr(),
+                                                              layout, got[1].data_ptr(), layout, ticks, nat._stream(x))
+                    assert rc == 0, nat.lib().f8mi_last_error()
+                    assert s.view(torch.int32).item() == s_want.view(torch.int32).item() or (torch.isnan(s) and torch.isnan(s_want))
+                    for g, w in zip(got, want):
+                        assert same_bytes_mod_nan_sign(fp8_bytes(g), fp8_bytes(w)), (dt, shape, fmt, layout, ticks)
+
+
+def test_cast_dynamic_resident_on_several_streams_and_what_it_refuses(nat):
+    streams = [torch.cuda.Stream() for _ in range(4)]
+    xs = [heavy((1024, 1024), torch.bfloat16, 30 + i).to(DEV) for i in range(4)]
+    want = [nat.cast(x, nat.amax_scale(x, torch.float8_e4m3fn, want_amax=False)[1], torch.float8_e4m3fn)[0] for x in xs]
+    torch.cuda.synchronize()
+    got = []
+    for _ in range(20):
+        for st, x in zip(streams, xs):
+            with torch.cuda.stream(st):
+                got.append(nat.cast_dynamic(x, torch.float8_e4m3fn)[0])
+    torch.cuda.synchronize()
+    for i, g in enumerate(got):
+        assert torch.equal(g.view(torch.uint8), want[i % 4].view(torch.uint8))
+    big = torch.zeros(4097, 4096, device=DEV, dtype=torch.bfloat16)
+    o, s = torch.empty(4097, 4096, device=DEV, dtype=torch.uint8), torch.empty((), device=DEV)
+    call = lambda stream, rows=4096: nat.lib().f8mi_cast_dynamic_resident(big.data_ptr(), rows, 4096, 4096, 0, 0, s.data_ptr(), o.data_ptr(), 0, None, 0, 100,
+                                                                          stream.cuda_stream)
+    assert call(torch.cuda.current_stream(), 4097) == -2
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):  # its word would be the same on every replay: the two launches instead
+        assert call(torch.cuda.current_stream()) == -2
+        q, _, sq = nat.cast_dynamic(xs[0], torch.float8_e4m3fn)
+    for _ in range(3):
+        xs[0].mul_(0.5)
+        graph.replay()
+        assert torch.equal(sq, nat.amax_scale(xs[0], torch.float8_e4m3fn, want_amax=False)[1])
+        assert torch.equal(q.view(torch.uint8), nat.cast(xs[0], sq, torch.float8_e4m3fn)[0].view(torch.uint8))
+
+
 def _rand_fp8(shape, tdt, seed, scale=1.0):
     g = torch.Generator().manual_seed(seed)
     v = torch.randn(shape, generator=g) * scale
