@@ -270,13 +270,79 @@ __device__ __forceinline__ void emit_tile(const Row8<DT> (&in)[H][4], uint32_t* 
     }
 }
 
-template <int DT, int PROD, int FMT>
+// An exchange of maxima inside a launch.  Whoever has one publishes a 64-bit word, {launch tag, maximum}, with an agent-scope store;
+// whoever needs them all reads the words with agent-scope loads until each carries the tag: the words are all there is to
+// exchange, so no fence is needed.  The tag is the host's count of such launches, never used twice, so a word of any other launch
+// just reads as "not there yet" and nothing has to be cleared; the host keeps launches that may run at the same time (other
+// streams) on other words.  Nothing depends on the others being on the chip: a workgroup that has waited for wait_ticks of the 100
+// MHz clock finds the maximum itself by reading the whole tensor.  So every wave ends whatever else runs, and the result is the same
+// bits either way.
+struct TaggedWords {
+    uint64_t* words;  // null: no exchange
+    uint32_t tag, wait_ticks;
+};
+constexpr uint32_t EXCHANGE_WAIT_TICKS = 200000;  // 2 ms: several rounds of the longest tiles of the GEMMs that may hold the CUs
+
+__device__ __forceinline__ void publish_word(const TaggedWords& e, uint32_t i, uint32_t m) {
+    __hip_atomic_store(&e.words[i], (uint64_t)e.tag << 32 | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The maximum of the first n words and of every lane's m, the same in all lanes of the workgroup.  Every lane asks for BATCH words at
+// a time, from the last ones (which come last) down: one round trip to memory (0.7 us) for each batch.  With every workgroup
+// collecting, BATCH is 1: more words polled at a time hold up the loads that are waited for (4096 x 4096 bf16: 18.9 us, with four 24.7).
+template <int DT, int BATCH>
+__device__ __forceinline__ uint32_t collect_words(const TaggedWords& e, uint32_t n, uint32_t m, uint32_t (&red)[CAST_THREADS / 64], const void* x,
+                                                  int64_t rows, int64_t cols, int64_t ld) {
+    const int t = threadIdx.x;
+    const uint64_t start = wall_clock64();
+    constexpr uint32_t STEP = BATCH * CAST_THREADS, LATE = 0x80000000u;  // no maximum has the top bit
+    for (uint32_t left = (n + STEP - 1) / STEP; left > 0 && !(m & LATE); left--) {
+        const uint32_t i = (left - 1) * STEP + t;
+        uint64_t w[BATCH];
+        for (;;) {
+            bool all = true;
+#pragma unroll
+            for (int u = 0; u < BATCH; u++)  // past the end: the last word again
+                w[u] = __hip_atomic_load(&e.words[min(i + u * CAST_THREADS, n - 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int u = 0; u < BATCH; u++) all &= (uint32_t)(w[u] >> 32) == e.tag;
+            if (all) break;
+            if (wall_clock64() - start >= e.wait_ticks) { m |= LATE; break; }
+            __builtin_amdgcn_s_sleep(1);
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) m = max(m, (uint32_t)w[u]);
+    }
+    static_assert(CAST_THREADS == 256, "four waves");
+    m = wave_max_u32(m);
+    if ((t & 63) == 0) red[t >> 6] = m;
+    __syncthreads();
+    m = max(max(red[0], red[1]), max(red[2], red[3]));
+    if (m & LATE) {
+        m = 0;
+        for (int64_t r = 0; r < (ld ? rows : 1); r++)
+            for (int64_t c = 8 * t; c < cols; c += 8 * CAST_THREADS) {
+                Row8<DT> v;
+                load_row8<DT>(v, x, r, c, rows, cols, ld);
+                m = absmax_row<DT>(v, m);
+            }
+        m = wave_max_u32(absmax_done<DT>(m));
+        __syncthreads();  // everybody has read `red`
+        if ((t & 63) == 0) red[t >> 6] = m;
+        __syncthreads();
+        m = max(max(red[0], red[1]), max(red[2], red[3]));
+    }
+    return m;
+}
+
+template <int DT, int PROD, int FMT, bool TAGGED>
 __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restrict__ x, int64_t rows, int64_t cols,
                                                             int64_t ld, const float* __restrict__ scale_dev,
                                                             uint8_t* __restrict__ out, uint8_t* __restrict__ out_t,
                                                             float* amax_out, uint32_t tiles_x, uint32_t tiles_y,
                                                             int out_kb, int out_t_kb, const uint32_t* __restrict__ amax_ws,
-                                                            int amax_nblocks, float* scale_out, uint32_t* amax_spread) {
+                                                            int amax_nblocks, float* scale_out, uint32_t* amax_spread,
+                                                            TaggedWords tagged) {
     __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];  // [column][row/4] dwords, swizzled
     __shared__ uint32_t red[CAST_THREADS / 64];
 
@@ -327,10 +393,18 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restri
     }
 
     uint32_t m = 0;
-    if (amax_out) m = absmax_tile<DT, 2>(in);
+    if (TAGGED || amax_out) m = absmax_tile<DT, 2>(in);
     emit_tile<DT, PROD, FMT, 2>(in, tileT, scale, r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
 
-    if (amax_out && amax_spread) {
+    if constexpr (TAGGED) {
+        // Every wave leaves its maximum in a word of its own; the workgroup that was started last collects them.
+        m = wave_max_u32(m);
+        if ((t & 63) == 0) publish_word(tagged, blockIdx.x * (CAST_THREADS / 64) + (t >> 6), m);
+        if (blockIdx.x == gridDim.x - 1) {
+            m = collect_words<DT, 8>(tagged, gridDim.x * (CAST_THREADS / 64), m, red, x, rows, cols, ld);
+            if (t == 0) *amax_out = abs_bits_to_float(m, DT);
+        }
+    } else if (amax_out && amax_spread) {
         // Every wave folds its maximum (the bit pattern in the input's dtype) into one of SPREAD_WORDS words with an
         // atomic that returns nothing: no LDS, no barrier, no round trip to wait for, and a word sees about one atomic
         // per (tiles * 4 / SPREAD_WORDS) waves, spread over the whole run of the kernel.  cast_spread_finalize_kernel
@@ -513,30 +587,22 @@ static int launch_cast_flat(int fmt, hipStream_t stream, const void* x, int64_t 
 // workgroup loads its tile (64 H rows x 128 columns) into registers, publishes the tile's maximum, collects everybody's and casts
 // what it holds.  The two kernels it replaces read the tensor twice and pay a launch and a ramp more.
 //
-// A workgroup publishes one 64-bit word, {launch tag, maximum}, with an agent-scope store and reads the others' with agent-scope
-// loads: the words carry all there is to exchange, so no fence is needed.  The tag is the host's count of such launches, never
-// used twice, so a word of any other launch just reads as "not there yet" and nothing has to be cleared; the host keeps launches
-// that may run at the same time (other streams) on other words.  All workgroups fit on the chip at once (see
-// resident_tile_rows), but nothing depends on it: a workgroup that has waited for wait_ticks of the 100 MHz clock -- because
-// other work holds the CUs that the missing ones need -- finds the maximum itself by reading the whole tensor, and goes on.  So every wave
-// ends whatever else runs, and the result is the same bits either way.
+// All workgroups fit on the chip at once (see resident_tile_rows), but nothing depends on it.
 //
 // us a call, back to back, inputs cold, amax and cast / this one: one copy, bf16, 512 x 1024: 8.8 / 6.6, 2048 x 2048: 10.6 / 9.0, 2726 x 934
 // (padded): 16.1 / 10.7, 2048 x 4096: 14.3 / 12.2, 4096 x 4096: 20.5 / 18.9; both copies, 512 x 1024: 8.8 / 6.6, 4096 x 4096: 21.8 / 20.4; fp32,
 // 512 x 1024: 9.9 / 6.9, 4096 x 4096: 30.7 / 28.9.  Inside a launch of 4096 x 4096 bf16 (1024 workgroups): the last tile has arrived after 9.5
 // us, everybody has everybody's maximum after 11.3 (2 us is what a word takes to memory and back, 512 x 1024 waits as long), the
 // last byte is stored after 15.  Loads in smaller batches, other tile shapes and linear tile orders all took the same or longer.
-constexpr int RESIDENT_WORDS = 1024;  // workgroups at most
-constexpr uint32_t RESIDENT_WAIT_TICKS = 200000;  // 2 ms: several rounds of the longest tiles of the GEMMs that may hold the CUs
+constexpr int RESIDENT_TILES = 1024;  // workgroups at most
 
 template <int DT, int FMT, int H>
 __global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_kernel(const void* __restrict__ x, int64_t rows, int64_t cols, int64_t ld,
                                                                              float* __restrict__ scale_out, uint8_t* __restrict__ out,
                                                                              uint8_t* __restrict__ out_t, uint32_t tiles_x, uint32_t tiles_y,
-                                                                             int out_kb, int out_t_kb, uint64_t* __restrict__ words, uint32_t tag,
-                                                                             uint32_t wait_ticks) {
+                                                                             int out_kb, int out_t_kb, TaggedWords tagged) {
     __shared__ uint32_t tileT[32 * 64 * H];
-    __shared__ uint32_t red[CAST_THREADS / 64], late;
+    __shared__ uint32_t red[2][CAST_THREADS / 64];
     const int t = threadIdx.x;
     int ty, tx;
     cast_tile_of(blockIdx.x, gridDim.x, tiles_x, tiles_y, ty, tx);
@@ -544,42 +610,64 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_kernel(con
     Row8<DT> in[H][4];
     load_tile<DT, H>(in, x, r0, c0, rows, cols, ld);
     uint32_t m = wave_max_u32(absmax_tile<DT, H>(in));
-    if ((t & 63) == 0) red[t >> 6] = m;
-    if (t == 0) late = 0u;
+    if ((t & 63) == 0) red[0][t >> 6] = m;
     __syncthreads();
-    static_assert(CAST_THREADS == 256, "four waves");
-    m = max(max(red[0], red[1]), max(red[2], red[3]));
-    if (t == 0) __hip_atomic_store(&words[blockIdx.x], (uint64_t)tag << 32 | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint64_t start = wall_clock64();
-    bool here = true;
-    for (uint32_t i = t; i < gridDim.x; i += CAST_THREADS) {
-        uint64_t w;
-        while ((uint32_t)((w = __hip_atomic_load(&words[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) != tag) {
-            if (wall_clock64() - start >= wait_ticks) { here = false; break; }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        if (here) m = max(m, (uint32_t)w);
-        else break;
-    }
-    if (!here) late = 1u;
-    m = wave_max_u32(m);
-    __syncthreads();  // everybody has read `red` and written `late`
-    if (late) {  // the same for the whole workgroup
-        uint32_t own = 0;
-        for (int64_t r = 0; r < (ld ? rows : 1); r++)
-            for (int64_t c = 8 * t; c < cols; c += 8 * CAST_THREADS) {
-                Row8<DT> v;
-                load_row8<DT>(v, x, r, c, rows, cols, ld);
-                own = absmax_row<DT>(v, own);
-            }
-        m = wave_max_u32(absmax_done<DT>(own));
-    }
-    if ((t & 63) == 0) red[t >> 6] = m;
-    __syncthreads();
-    m = max(max(red[0], red[1]), max(red[2], red[3]));
+    if (t == 0) publish_word(tagged, blockIdx.x, max(max(red[0][0], red[0][1]), max(red[0][2], red[0][3])));
+    m = collect_words<DT, 1>(tagged, gridDim.x, m, red[1], x, rows, cols, ld);
     const float scale = amax_to_scale_dev(abs_bits_to_float(m, DT), DT, FMT, DT == F8MI_FP16);
     if (blockIdx.x == 0 && t == 0) *scale_out = scale;
     emit_tile<DT, DT, FMT, H>(in, tileT, scale, r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
+}
+
+constexpr int STATIC_MAX_DEVICES = 64;
+
+// Device address of a device array of this library on the current device, looked up once per device and kept (nullptr + error
+// message on failure).  Two threads racing here store the same value.
+template <typename T>
+static T* device_array(const void* symbol, std::atomic<T*> (&known)[STATIC_MAX_DEVICES], const char* what) {
+    int dev = -1;
+    if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
+    if (dev < 0 || dev >= STATIC_MAX_DEVICES) { set_error("%s: device index %d, at most %d devices", what, dev, STATIC_MAX_DEVICES); return nullptr; }
+    if (T* p = known[dev].load(std::memory_order_acquire)) return p;
+    void* addr = nullptr;
+    if (check_hip(hipGetSymbolAddress(&addr, symbol), what)) return nullptr;
+    if (!addr) { set_error("%s: no address on device %d", what, dev); return nullptr; }
+    known[dev].store((T*)addr, std::memory_order_release);
+    return (T*)addr;
+}
+
+// The words of the exchanges: a set for each of the first EXCHANGE_STREAMS streams that use one, so that launches which may run at
+// the same time do not share any (sharing would be slow, not wrong).  Later streams take the kernels that need no exchange, and so do
+// streams that are being captured: a captured launch would use its tag again on every replay.  A stream handle that comes back for a
+// new stream finds the old one's set: its work is done.
+constexpr int EXCHANGE_STREAMS = 64;
+constexpr int EXCHANGE_WORDS = 8192;
+static __device__ __align__(256) uint64_t exchange_words[EXCHANGE_STREAMS][EXCHANGE_WORDS];
+static std::atomic<uint64_t*> g_exchange_words[STATIC_MAX_DEVICES];
+static std::atomic<uintptr_t> g_exchange_streams[STATIC_MAX_DEVICES][EXCHANGE_STREAMS];
+static std::atomic<uint32_t> g_exchange_tag{0};
+
+// Words and a tag for one launch on `stream`; words null: none to be had.  An error code if the runtime reports one.
+static int begin_exchange(hipStream_t stream, uint32_t wait_ticks, TaggedWords& e) {
+    e = TaggedWords{nullptr, 0, wait_ticks};
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (check_hip(hipStreamIsCapturing(stream, &capture), "hipStreamIsCapturing")) return F8MI_ERR_HIP;
+    if (capture != hipStreamCaptureStatusNone) return F8MI_OK;
+    int dev = 0;
+    if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return F8MI_ERR_HIP;
+    uint64_t* base = device_array(HIP_SYMBOL(exchange_words), g_exchange_words, "exchange_words");
+    if (!base) return F8MI_ERR_HIP;
+    const uintptr_t key = (uintptr_t)stream + 1;  // the default stream is a null handle
+    for (int i = 0; i < EXCHANGE_STREAMS; i++) {
+        uintptr_t have = g_exchange_streams[dev][i].load(std::memory_order_relaxed);
+        if (!have && g_exchange_streams[dev][i].compare_exchange_strong(have, key, std::memory_order_relaxed)) have = key;
+        if (have != key) continue;
+        e.words = base + (size_t)i * EXCHANGE_WORDS;
+        e.tag = g_exchange_tag.fetch_add(1, std::memory_order_relaxed) + 1;
+        if (!e.tag) e.tag = g_exchange_tag.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 is what the words start with
+        break;
+    }
+    return F8MI_OK;
 }
 
 // where a dynamic-scaling cast takes its scale from (see cast_layout_impl)
@@ -588,6 +676,7 @@ struct AmaxSource {
     int nblocks;
     float* scale_out;
     uint32_t* spread;  // delayed scaling: the zeroed words the fused amax is folded into (null: straight into *amax_dev)
+    TaggedWords tagged;  // delayed scaling in one launch: instead of those
 };
 
 __global__ void cast_zero_amax_kernel(float* amax_out) {
@@ -613,7 +702,13 @@ template <int DT, int PROD, int FMT>
 static int launch_cast2(dim3 g, hipStream_t stream, const void* x, int64_t rows, int64_t cols, int64_t ld,
                         const float* scale_dev, uint8_t* out, uint8_t* out_t, float* amax_dev, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb,
                         const AmaxSource& src) {
-    hipLaunchKernelGGL((cast_kernel<DT, PROD, FMT>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src.ws, src.nblocks, src.scale_out, src.spread);
+    if constexpr (PROD == F8MI_FP32) {  // what delayed scaling computes in
+        if (src.tagged.words) {
+            hipLaunchKernelGGL((cast_kernel<DT, PROD, FMT, true>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src.ws, src.nblocks, src.scale_out, src.spread, src.tagged);
+            return check_hip(hipGetLastError(), "cast kernel launch");
+        }
+    }
+    hipLaunchKernelGGL((cast_kernel<DT, PROD, FMT, false>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src.ws, src.nblocks, src.scale_out, src.spread, src.tagged);
     return check_hip(hipGetLastError(), "cast kernel launch");
 }
 
@@ -663,7 +758,7 @@ static int cast_layout_impl(const void* x, int64_t rows, int64_t cols, int64_t l
     const double n = (double)rows * (double)cols;
     // every launch of this call: the cast and what a fused amax adds before or after it
     ProfScope prof(F8MI_K_CAST, (ld == 0 ? (double)cols : n) * esz + n * ((out ? 1 : 0) + (out_t ? 1 : 0)), stream);
-    if (amax_dev && !src.spread) {
+    if (amax_dev && !src.spread && !src.tagged.words) {
         hipLaunchKernelGGL(cast_zero_amax_kernel, dim3(1), dim3(64), 0, stream, amax_dev);
         if (int rc = check_hip(hipGetLastError(), "cast_zero_amax_kernel")) return rc;
     }
@@ -690,7 +785,7 @@ extern "C" int f8mi_cast_layout(const void* x, int64_t rows, int64_t cols, int64
                                 const float* scale_dev, int product_dtype, int fp8_fmt, uint8_t* out, int out_layout,
                                 uint8_t* out_t, int out_t_layout, float* amax_dev, void* stream) {
     return cast_layout_impl(x, rows, cols, ld, in_dtype, scale_dev, product_dtype, fp8_fmt, out, out_layout, out_t, out_t_layout, amax_dev,
-                            (hipStream_t)stream, AmaxSource{nullptr, 0, nullptr, nullptr});
+                            (hipStream_t)stream, AmaxSource{});
 }
 
 extern "C" int f8mi_cast(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, const float* scale_dev,
@@ -711,6 +806,12 @@ static std::mutex& delayed_lock(const void* workspace) {
     static std::mutex locks[64];
     return locks[((uintptr_t)workspace >> 12) % 64];
 }
+
+// The delayed cast in one launch: a word for every wave.
+static bool one_launch_delayed(int64_t rows, int64_t cols) {
+    const int64_t tx = (cols + CAST_TILE - 1) / CAST_TILE, ty = (rows + CAST_TILE - 1) / CAST_TILE, most = EXCHANGE_WORDS / (CAST_THREADS / 64);
+    return tx <= most && ty <= most && tx * ty <= most;
+}
 }  // namespace f8mi
 
 extern "C" int f8mi_cast_delayed(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, const float* scale_dev, int fp8_fmt,
@@ -718,57 +819,24 @@ extern "C" int f8mi_cast_delayed(const void* x, int64_t rows, int64_t cols, int6
                                  void* stream) {
     if (!amax_dev) { set_error("f8mi_cast_delayed: null amax"); return F8MI_ERR_INVALID_ARG; }
     if (!workspace || (uintptr_t)workspace % 4 != 0) { set_error("f8mi_cast_delayed: null or misaligned workspace"); return F8MI_ERR_INVALID_ARG; }
+    AmaxSource src{};
+    if (rows > 0 && cols > 0 && one_launch_delayed(rows, cols))
+        if (const int rc = begin_exchange((hipStream_t)stream, EXCHANGE_WAIT_TICKS, src.tagged)) return rc;
+    if (src.tagged.words)
+        return cast_layout_impl(x, rows, cols, ld, in_dtype, scale_dev, F8MI_FP32, fp8_fmt, out, out_layout, out_t, out_t_layout, amax_dev,
+                                (hipStream_t)stream, src);
+    src.spread = (uint32_t*)workspace;
     const std::lock_guard<std::mutex> guard(f8mi::delayed_lock(workspace));
     return cast_layout_impl(x, rows, cols, ld, in_dtype, scale_dev, F8MI_FP32, fp8_fmt, out, out_layout, out_t, out_t_layout, amax_dev,
-                            (hipStream_t)stream, AmaxSource{nullptr, 0, nullptr, (uint32_t*)workspace});
+                            (hipStream_t)stream, src);
 }
 
 namespace f8mi {
 
-constexpr int STATIC_MAX_DEVICES = 64;
-
-// Device address of a device array of this library on the current device, looked up once per device and kept (nullptr + error
-// message on failure).  Two threads racing here store the same value.
-template <typename T>
-static T* device_array(const void* symbol, std::atomic<T*> (&known)[STATIC_MAX_DEVICES], const char* what) {
-    int dev = -1;
-    if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
-    if (dev < 0 || dev >= STATIC_MAX_DEVICES) { set_error("%s: device index %d, at most %d devices", what, dev, STATIC_MAX_DEVICES); return nullptr; }
-    if (T* p = known[dev].load(std::memory_order_acquire)) return p;
-    void* addr = nullptr;
-    if (check_hip(hipGetSymbolAddress(&addr, symbol), what)) return nullptr;
-    if (!addr) { set_error("%s: no address on device %d", what, dev); return nullptr; }
-    known[dev].store((T*)addr, std::memory_order_release);
-    return (T*)addr;
-}
-
-// The words of the one-launch cast: a set for each of the first RESIDENT_STREAMS streams that use it, so that launches which may
-// run at the same time do not share any (sharing would be slow, not wrong: see the kernel).  Later streams take the two
-// launches.  A stream handle that comes back for a new stream finds the old one's set: its work is done.
-constexpr int RESIDENT_STREAMS = 64;
-static __device__ __align__(256) uint64_t resident_words[RESIDENT_STREAMS][RESIDENT_WORDS];
-static std::atomic<uint64_t*> g_resident_words[STATIC_MAX_DEVICES];
-static std::atomic<uintptr_t> g_resident_streams[STATIC_MAX_DEVICES][RESIDENT_STREAMS];
-static std::atomic<uint32_t> g_resident_tag{0};
-
-static uint64_t* resident_words_of(hipStream_t stream) {
-    uint64_t* base = device_array(HIP_SYMBOL(resident_words), g_resident_words, "resident_words");
-    if (!base) return nullptr;
-    int dev = 0;
-    if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
-    const uintptr_t key = (uintptr_t)stream + 1;  // the default stream is a null handle
-    for (int i = 0; i < RESIDENT_STREAMS; i++) {
-        uintptr_t have = g_resident_streams[dev][i].load(std::memory_order_relaxed);
-        if (!have && g_resident_streams[dev][i].compare_exchange_strong(have, key, std::memory_order_relaxed)) have = key;
-        if (have == key) return base + (size_t)i * RESIDENT_WORDS;
-    }
-    return nullptr;
-}
-
-// Rows of the tiles that the one-launch cast gives a tensor, 0: it does not take it.  At most four workgroups a CU (RESIDENT_WORDS on
+// Rows of the tiles that the one-launch cast gives a tensor, 0: it does not take it.  At most four workgroups a CU (RESIDENT_TILES on
 // 256): it holds eight of them (five of 128 rows of fp32), so that all are there at once also beside other streams' kernels.
 static int resident_tile_rows(int64_t rows, int64_t cols) {
-    const int64_t tx = (cols + CAST_TILE - 1) / CAST_TILE, ty = (rows + CAST_TILE - 1) / CAST_TILE, most = std::min(RESIDENT_WORDS, 4 * cu_count());
+    const int64_t tx = (cols + CAST_TILE - 1) / CAST_TILE, ty = (rows + CAST_TILE - 1) / CAST_TILE, most = std::min(RESIDENT_TILES, 4 * cu_count());
     if (ty > most || tx > most) return 0;
     // tiles of 64 rows while they number at most two a CU: more workgroups share a small tensor (512 x 1024: 7.6 -> 6.6 us); beyond that
     // they only add words to collect (2048 x 4096 as 512 or 1024 tiles: 12.2 / 12.5)
@@ -777,18 +845,16 @@ static int resident_tile_rows(int64_t rows, int64_t cols) {
 
 template <int DT, int FMT>
 static int launch_cast_resident1(int tile_rows, dim3 g, hipStream_t stream, const void* x, int64_t rows, int64_t cols, int64_t ld, float* scale_dev,
-                                 uint8_t* out, uint8_t* out_t, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb, uint64_t* words, uint32_t tag,
-                                 uint32_t wait_ticks) {
-    if (tile_rows == 64) hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 1>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
-    else hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 2>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+                                 uint8_t* out, uint8_t* out_t, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb, const TaggedWords& tagged) {
+    if (tile_rows == 64) hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 1>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
+    else hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 2>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
     return check_hip(hipGetLastError(), "cast (dynamic, resident) kernel launch");
 }
 template <int DT>
 static int launch_cast_resident(int fmt, int tile_rows, dim3 g, hipStream_t stream, const void* x, int64_t rows, int64_t cols, int64_t ld, float* scale_dev,
-                                uint8_t* out, uint8_t* out_t, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb, uint64_t* words, uint32_t tag,
-                                uint32_t wait_ticks) {
-    if (fmt == F8MI_E4M3FN) return launch_cast_resident1<DT, F8MI_E4M3FN>(tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
-    return launch_cast_resident1<DT, F8MI_E5M2>(tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+                                uint8_t* out, uint8_t* out_t, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb, const TaggedWords& tagged) {
+    if (fmt == F8MI_E4M3FN) return launch_cast_resident1<DT, F8MI_E4M3FN>(tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
+    return launch_cast_resident1<DT, F8MI_E5M2>(tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
 }
 
 }  // namespace f8mi
@@ -801,14 +867,9 @@ extern "C" int f8mi_cast_dynamic_resident(const void* x, int64_t rows, int64_t c
     if (const int rc = check_cast_layouts(rows, cols, out, out_layout, out_t, out_t_layout)) return rc;
     const int tile_rows = resident_tile_rows(rows, cols);
     if (!tile_rows) { set_error("f8mi_cast_dynamic_resident: %lld x %lld is more than the chip holds", (long long)rows, (long long)cols); return F8MI_ERR_UNSUPPORTED; }
-    // a captured launch would use its tag again on every replay
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (check_hip(hipStreamIsCapturing(stream, &capture), "hipStreamIsCapturing")) return F8MI_ERR_HIP;
-    if (capture != hipStreamCaptureStatusNone) { set_error("f8mi_cast_dynamic_resident: the stream is being captured"); return F8MI_ERR_UNSUPPORTED; }
-    uint64_t* words = resident_words_of(stream);
-    if (!words) { set_error("f8mi_cast_dynamic_resident: %d other streams use it", RESIDENT_STREAMS); return F8MI_ERR_UNSUPPORTED; }
-    uint32_t tag = g_resident_tag.fetch_add(1, std::memory_order_relaxed) + 1;
-    if (!tag) tag = g_resident_tag.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 is what the words start with
+    TaggedWords tagged;
+    if (const int rc = begin_exchange(stream, wait_ticks, tagged)) return rc;
+    if (!tagged.words) { set_error("f8mi_cast_dynamic_resident: the stream is being captured, or %d others use it", EXCHANGE_STREAMS); return F8MI_ERR_UNSUPPORTED; }
     const int out_kb = out ? out_layout : F8MI_LAYOUT_ROWMAJOR, out_t_kb = out_t ? out_t_layout : F8MI_LAYOUT_ROWMAJOR;
     // whole 128 x 128 tiles, as the padded layouts are
     const uint32_t tiles_x = (uint32_t)((cols + CAST_TILE - 1) / CAST_TILE), tiles_y = (uint32_t)((rows + CAST_TILE - 1) / CAST_TILE) * (CAST_TILE / tile_rows);
@@ -816,9 +877,9 @@ extern "C" int f8mi_cast_dynamic_resident(const void* x, int64_t rows, int64_t c
     const size_t esz = in_dtype == F8MI_FP32 ? 4 : 2;
     const double n = (double)rows * (double)cols;
     ProfScope prof(F8MI_K_CAST, (ld == 0 ? (double)cols : n) * esz + n * ((out ? 1 : 0) + (out_t ? 1 : 0)), stream);
-    if (in_dtype == F8MI_BF16) return launch_cast_resident<F8MI_BF16>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
-    if (in_dtype == F8MI_FP16) return launch_cast_resident<F8MI_FP16>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
-    return launch_cast_resident<F8MI_FP32>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, words, tag, wait_ticks);
+    if (in_dtype == F8MI_BF16) return launch_cast_resident<F8MI_BF16>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
+    if (in_dtype == F8MI_FP16) return launch_cast_resident<F8MI_FP16>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
+    return launch_cast_resident<F8MI_FP32>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
 }
 
 extern "C" int f8mi_cast_dynamic(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, int fp8_fmt, float* scale_dev,
@@ -857,7 +918,7 @@ extern "C" int f8mi_cast_dynamic(const void* x, int64_t rows, int64_t cols, int6
         return launch_cast_flat<F8MI_FP32>(fp8_fmt, stream, x, rows, cols, scale_dev, out, out_kb);
     }
     if (resident_tile_rows(rows, cols)) {
-        const int rc = f8mi_cast_dynamic_resident(x, rows, cols, ld, in_dtype, fp8_fmt, scale_dev, out, out_layout, out_t, out_t_layout, RESIDENT_WAIT_TICKS, stream_);
+        const int rc = f8mi_cast_dynamic_resident(x, rows, cols, ld, in_dtype, fp8_fmt, scale_dev, out, out_layout, out_t, out_t_layout, EXCHANGE_WAIT_TICKS, stream_);
         if (rc != F8MI_ERR_UNSUPPORTED) return rc;
     }
     // amax pass: per-workgroup maxima into the workspace; the cast's workgroups reduce them and derive the scale
@@ -868,7 +929,7 @@ extern "C" int f8mi_cast_dynamic(const void* x, int64_t rows, int64_t cols, int6
         if (int rc = launch_amax_partials(x, rows, cols, ld, in_dtype, (uint32_t*)workspace, stream, &nblocks)) return rc;
     }
     return cast_layout_impl(x, rows, cols, ld, in_dtype, nullptr, in_dtype, fp8_fmt, out, out_layout, out_t, out_t_layout, nullptr, stream,
-                            AmaxSource{(const uint32_t*)workspace, nblocks, scale_dev, nullptr});
+                            AmaxSource{(const uint32_t*)workspace, nblocks, scale_dev, nullptr, {}});
 }
 
 namespace f8mi {

@@ -309,6 +309,34 @@ def test_delayed_cast_with_workspace_equals_the_cast_without(nat, dt):
         assert not ws.any().item(), "the workspace must be all zero after a call"
 
 
+# One launch while every wave has a word (2048 tiles), which the workgroup started last collects: one tile, one more row or column,
+# the last size and the first beyond; captured, the two launches.
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("shape", [(1, 1), (128, 128), (129, 257), (1000, 3001), (8192, 4096), (8193, 4096)])
+def test_delayed_cast_collects_the_maximum_in_its_launch(nat, dt, shape):
+    tdt = TORCH_DT[dt]
+    x = heavy(shape, tdt, 24).to(DEV)
+    scale = torch.tensor([3.0], device=DEV)
+    for at, value in ((0, 1e4), (-1, -2e4), (x.numel() // 2, float("nan")), (0, float("-inf"))):
+        v = x.clone()
+        v.view(-1)[at] = value
+        amax = torch.full((1,), -1.0, device=DEV)
+        o, _ = nat.cast(v, scale, torch.float8_e4m3fn, product_dtype=torch.float32, amax_out=amax)
+        want, _ = nat.amax_scale(v, torch.float8_e4m3fn, want_scale=False)
+        assert torch.equal(amax.view(()).isnan(), want.isnan()) and (torch.isnan(want) or amax.item() == want.item()), (at, value)
+        plain, _ = nat.cast(v, scale, torch.float8_e4m3fn, product_dtype=torch.float32)
+        assert torch.equal(o.view(torch.uint8), plain.view(torch.uint8))
+    if shape != (129, 257):
+        return
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        nat.cast(x, scale, torch.float8_e4m3fn, product_dtype=torch.float32, amax_out=amax)
+    for _ in range(3):
+        x.mul_(0.5)
+        graph.replay()
+        assert amax.item() == x.abs().max().item()
+
+
 def _unblock(t_kb):
     """[kc/64, rows, 64] k-blocked bytes -> [rows, kc] row-major (numpy)."""
     b = fp8_bytes(t_kb)
