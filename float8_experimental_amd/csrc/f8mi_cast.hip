@@ -104,6 +104,13 @@ __device__ __forceinline__ uint32_t absmax_done(uint32_t m) {
     else return fold16(m);
 }
 
+// Eight elements -> eight fp8 bytes.
+template <int DT, int PROD, int FMT, bool WITHIN>
+__device__ __forceinline__ void cast_row8(const Row8<DT>& r, float scale, uint32_t& lo, uint32_t& hi) {
+    lo = cast4<PROD, FMT, WITHIN>(elem<DT>(r, 0), elem<DT>(r, 1), elem<DT>(r, 2), elem<DT>(r, 3), scale);
+    hi = cast4<PROD, FMT, WITHIN>(elem<DT>(r, 4), elem<DT>(r, 5), elem<DT>(r, 6), elem<DT>(r, 7), scale);
+}
+
 // Loads 8 elements of row `row` starting at column `col`; out-of-range elements read as +0.  Eight elements inside the
 // row are one 16-byte load (two for fp32) whatever the row pitch: a row only has to start at a multiple of the
 // element size.
@@ -185,16 +192,15 @@ __device__ __forceinline__ uint32_t absmax_tile(const Row8<DT> (&in)[H][4]) {
 }
 
 // Scales, converts and stores such a tile: `out` row by row from registers, `out_t` through tileT.  out_kb / out_t_kb:
-// F8MI_LAYOUT_* code of the respective output.
+// F8MI_LAYOUT_* code of the respective output.  within (the same for the whole wave): within_range holds for all of it.
 template <int DT, int PROD, int FMT, int H>
-__device__ __forceinline__ void emit_tile(const Row8<DT> (&in)[H][4], uint32_t* tileT, float scale, int64_t r0, int64_t c0, int64_t rows, int64_t cols,
+__device__ __forceinline__ void emit_tile(const Row8<DT> (&in)[H][4], uint32_t* tileT, float scale, bool within, int64_t r0, int64_t c0, int64_t rows, int64_t cols,
                                           uint8_t* __restrict__ out, uint8_t* __restrict__ out_t, int out_kb, int out_t_kb) {
     constexpr int DWORDS = 16 * H;                  // of a tile column: four rows each
     constexpr int SWIZZLE = 4 * H - 1;              // 16-byte pieces of a tile column, less one
     const int t = threadIdx.x;
     const int a = t & 15, b = t >> 4;
     const int64_t col = c0 + 8 * a;
-    constexpr float fmax = FMT == F8MI_E4M3FN ? 448.0f : 57344.0f;
     // Zero-padded k-blocked outputs (F8MI_LAYOUT_KBLOCK64_PAD128): the tile grid ends exactly where the padding does, so
     // a tile writes all of its columns (`out`) or rows (`out_t`); what lies past the tensor's edge is forced to
     // zero bytes (elements read as +0 would become NaN codes under a NaN scale).
@@ -208,14 +214,15 @@ __device__ __forceinline__ void emit_tile(const Row8<DT> (&in)[H][4], uint32_t* 
 #pragma unroll
     for (int h = 0; h < H; h++) {
         uint32_t lo[4], hi[4];
+        if (within) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) cast_row8<DT, PROD, FMT, true>(in[h][j], scale, lo[j], hi[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) cast_row8<DT, PROD, FMT, false>(in[h][j], scale, lo[j], hi[j]);
+        }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            float f[8];
-#pragma unroll
-            for (int i = 0; i < 8; i += 2)
-                scale_clamp2<PROD>(elem<DT>(in[h][j], i), elem<DT>(in[h][j], i + 1), scale, fmax, f[i], f[i + 1]);
-            lo[j] = cvt4_fp8<FMT>(f[0], f[1], f[2], f[3]);
-            hi[j] = cvt4_fp8<FMT>(f[4], f[5], f[6], f[7]);
             const int64_t row = r0 + 64 * h + 4 * b + j;
             if (pad) {
                 lo[j] = row < rows ? lo[j] & keep_lo : 0u;
@@ -373,6 +380,8 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restri
     // amax_nblocks are leftovers of an earlier, larger call and are masked.  Same arithmetic as amax_finalize_kernel,
     // in the tensor's dtype.
     float scale;
+    bool within;
+    uint32_t m = 0;
     if (amax_ws) {
         uint32_t wm = 0;
 #pragma unroll
@@ -388,13 +397,14 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restri
         wm = wave_max_u32(wm);
         scale = amax_to_scale_dev(abs_bits_to_float(wm, DT), DT, FMT, DT == F8MI_FP16);
         if (blockIdx.x == 0 && t == 0) *scale_out = scale;
+        within = within_range<FMT>(abs_bits_to_float(wm, DT), scale);
     } else {
         scale = *scale_dev;
+        m = absmax_tile<DT, 2>(in);
+        within = __all(within_range<FMT>(abs_bits_to_float(m, DT), scale));
     }
 
-    uint32_t m = 0;
-    if (TAGGED || amax_out) m = absmax_tile<DT, 2>(in);
-    emit_tile<DT, PROD, FMT, 2>(in, tileT, scale, r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
+    emit_tile<DT, PROD, FMT, 2>(in, tileT, scale, within, r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
 
     if constexpr (TAGGED) {
         // Every wave leaves its maximum in a word of its own; the workgroup that was started last collects them.
@@ -466,18 +476,17 @@ __global__ __launch_bounds__(SMALL_THREADS) void cast_dynamic_small_kernel(const
     }
     __syncthreads();
     // the scale in the tensor's own dtype, as tensor_to_scale computes it (fp16 tensors: clamped to 65504)
-    const float scale = amax_to_scale_dev(abs_bits_to_float(amax_bits, DT), DT, FMT, DT == F8MI_FP16);
+    const float amax = abs_bits_to_float(amax_bits, DT), scale = amax_to_scale_dev(amax, DT, FMT, DT == F8MI_FP16);
     if (t == 0) *scale_out = scale;
-    constexpr float fmax = FMT == F8MI_E4M3FN ? 448.0f : 57344.0f;
+    const bool within = within_range<FMT>(amax, scale);
 #pragma unroll
     for (int u = 0; u < SMALL_ITEMS_PER_THREAD; u++) {
         const int64_t it = t + (int64_t)u * SMALL_THREADS;
         if (it >= items) continue;
         const int64_t row = it / groups, col = (it % groups) * 8;
-        float f[8];
-#pragma unroll
-        for (int i = 0; i < 8; i += 2) scale_clamp2<DT>(elem<DT>(r[u], i), elem<DT>(r[u], i + 1), scale, fmax, f[i], f[i + 1]);
-        const uint32_t lo = cvt4_fp8<FMT>(f[0], f[1], f[2], f[3]), hi = cvt4_fp8<FMT>(f[4], f[5], f[6], f[7]);
+        uint32_t lo, hi;
+        if (within) cast_row8<DT, DT, FMT, true>(r[u], scale, lo, hi);
+        else cast_row8<DT, DT, FMT, false>(r[u], scale, lo, hi);
         if (out) {
             uint8_t* p = out_kb ? out + ((col >> 6) * rows + row) * 64 + (col & 63) : out + row * cols + col;
             if (col + 8 <= cols) {
@@ -559,19 +568,18 @@ __global__ __launch_bounds__(FLAT_THREADS) void cast_dynamic_flat_kernel(const u
     m = red[0];
 #pragma unroll
     for (int i = 1; i < FLAT_THREADS / 64; i++) m = max(m, red[i]);
-    const float scale = amax_to_scale_dev(abs_bits_to_float(m, DT), DT, FMT, DT == F8MI_FP16);
+    const float amax = abs_bits_to_float(m, DT), scale = amax_to_scale_dev(amax, DT, FMT, DT == F8MI_FP16);
     if (own == 0) *scale_out = scale;
     if (own >= items) return;
-    constexpr float fmax = FMT == F8MI_E4M3FN ? 448.0f : 57344.0f;
-    float f[8];
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) scale_clamp2<DT>(elem<DT>(r, i), elem<DT>(r, i + 1), scale, fmax, f[i], f[i + 1]);
+    uint32_t lo, hi;
+    if (within_range<FMT>(amax, scale)) cast_row8<DT, DT, FMT, true>(r, scale, lo, hi);
+    else cast_row8<DT, DT, FMT, false>(r, scale, lo, hi);
     size_t at = (size_t)own * 8;
     if (out_kb) {
         const uint32_t row = own / (cols / 8), col = (own - row * (cols / 8)) * 8;
         at = ((size_t)(col >> 6) * rows + row) * 64 + (col & 63);
     }
-    store8_any(out + at, cvt4_fp8<FMT>(f[0], f[1], f[2], f[3]), cvt4_fp8<FMT>(f[4], f[5], f[6], f[7]));
+    store8_any(out + at, lo, hi);
 }
 
 template <int DT>
@@ -589,9 +597,10 @@ static int launch_cast_flat(int fmt, hipStream_t stream, const void* x, int64_t 
 //
 // All workgroups fit on the chip at once (see resident_tile_rows), but nothing depends on it.
 //
-// us a call, back to back, inputs cold, amax and cast / this one: one copy, bf16, 512 x 1024: 8.8 / 6.6, 2048 x 2048: 10.6 / 9.0, 2726 x 934
-// (padded): 16.1 / 10.7, 2048 x 4096: 14.3 / 12.2, 4096 x 4096: 20.5 / 18.9; both copies, 512 x 1024: 8.8 / 6.6, 4096 x 4096: 21.8 / 20.4; fp32,
-// 512 x 1024: 9.9 / 6.9, 4096 x 4096: 30.7 / 28.9.  Inside a launch of 4096 x 4096 bf16 (1024 workgroups): the last tile has arrived after 9.5
+// us a call, back to back, inputs cold, amax and cast / this one: one copy, bf16, 512 x 1024: 8.8 / 6.4, 2048 x 2048: 10.6 / 9.0, 2726 x 934
+// (padded): 16.1 / 10.7, 2048 x 4096: 14.3 / 11.5, 4096 x 4096: 20.5 / 17.6; both copies, 4096 x 4096: 21.8 / 19.3; fp32,
+// 512 x 1024: 9.9 / 6.4, 4096 x 4096: 30.7 / 24.3.  (Twice as many tiles, all that eight workgroups a CU hold: 8192 x 4096 34.7 / 31.3 -- but then
+// one workgroup that finds no room, beside another stream's kernel, keeps all the others waiting: not taken.)  Inside a launch of 4096 x 4096 bf16 (1024 workgroups): the last tile has arrived after 9.5
 // us, everybody has everybody's maximum after 11.3 (2 us is what a word takes to memory and back, 512 x 1024 waits as long), the
 // last byte is stored after 15.  Loads in smaller batches, other tile shapes and linear tile orders all took the same or longer.
 constexpr int RESIDENT_TILES = 1024;  // workgroups at most
@@ -614,9 +623,9 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_kernel(con
     __syncthreads();
     if (t == 0) publish_word(tagged, blockIdx.x, max(max(red[0][0], red[0][1]), max(red[0][2], red[0][3])));
     m = collect_words<DT, 1>(tagged, gridDim.x, m, red[1], x, rows, cols, ld);
-    const float scale = amax_to_scale_dev(abs_bits_to_float(m, DT), DT, FMT, DT == F8MI_FP16);
+    const float amax = abs_bits_to_float(m, DT), scale = amax_to_scale_dev(amax, DT, FMT, DT == F8MI_FP16);
     if (blockIdx.x == 0 && t == 0) *scale_out = scale;
-    emit_tile<DT, DT, FMT, H>(in, tileT, scale, r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
+    emit_tile<DT, DT, FMT, H>(in, tileT, scale, within_range<FMT>(amax, scale), r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
 }
 
 constexpr int STATIC_MAX_DEVICES = 64;

@@ -197,6 +197,30 @@ def test_cast_fp32_bit_patterns(nat, fmt):
 
 
 @pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+def test_cast_of_tiles_around_the_largest_code(nat, dt, fmt):
+    """A wave leaves the clamp out where its products stay below the middle past the largest code: one magnitude a tile, below, at
+    and above that line, of either sign, under scales of either sign, and tiles of it with one larger, infinite or NaN element."""
+    code, tdt = F8[fmt]
+    top = 448.0 if fmt == "e4m3" else 57344.0
+    edge = [0.98, 1.0, 1.01, 460 / 448, 462 / 448, 464 / 448, 466 / 448, 480 / 448, 60000 / 57344, 61440 / 57344, 61696 / 57344, 1.15]
+    x = torch.empty(len(edge), 128, 4, 128)
+    for i, e in enumerate(edge):
+        x[i] = top * e / 8
+        x[i, ::2, :, 1::2] *= -1
+        x[i, 17, 1, 5], x[i, 99, 2, 127], x[i, 64, 3, 0] = top / 2, float("-inf"), float("nan")
+    x = x.reshape(len(edge) * 128, 512).to(TORCH_DT[dt])
+    for s in (8.0, -8.0, 8.5):
+        sc = torch.tensor(s, dtype=torch.float32)
+        for delayed in (False, True):
+            want = _ref_cast(x, sc, tdt, delayed)
+            amax = torch.zeros((), dtype=torch.float32, device=DEV) if delayed else None
+            out, out_t = nat.cast(x.to(DEV), sc.to(DEV), tdt, product_dtype=torch.float32 if delayed else TORCH_DT[dt], want_out_t=True, amax_out=amax)
+            assert same_bytes_mod_nan_sign(fp8_bytes(out), want), (s, delayed)
+            assert np.array_equal(fp8_bytes(out_t), fp8_bytes(out).T)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("shape", [(1, 1), (1, 129), (129, 1), (16, 16), (33, 47), (128, 128), (257, 131), (130, 1000),
                                    (1000, 136), (4099, 1000), (2, 3, 40)])
 def test_cast_shapes_dynamic_and_delayed(nat, dt, shape):
