@@ -47,6 +47,8 @@ EXPORTS = (
     "f8mi_cast_dynamic",
     "f8mi_cast_dynamic_static",
     "f8mi_cast_dynamic_resident",
+    "f8mi_cast_dynamic_pair",
+    "f8mi_cast_delayed_pair",
     "f8mi_linear_few_rows",
     "f8mi_gemm_weight_only",
     "f8mi_dequant",
@@ -117,6 +119,9 @@ def lib() -> C.CDLL:
         L.f8mi_cast_dynamic_static.argtypes = [vp, i64, i64, i64, i32, i32, fp, vp, i32, vp, i32, vp]
         L.f8mi_cast_dynamic_resident.restype = i32
         L.f8mi_cast_dynamic_resident.argtypes = [vp, i64, i64, i64, i32, i32, fp, vp, i32, vp, i32, C.c_uint32, vp]
+        for pair in (L.f8mi_cast_dynamic_pair, L.f8mi_cast_delayed_pair):
+            pair.restype = i32
+            pair.argtypes = [vp, vp, vp, vp]
         L.f8mi_gemm_nt_kb.restype = i32
         L.f8mi_gemm_nt_kb.argtypes = [vp, i32, vp, i32, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp]
         L.f8mi_gemm_kb_ex.restype = i32

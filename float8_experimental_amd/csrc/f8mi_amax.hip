@@ -8,6 +8,8 @@
 // writes amax + scale.  (One word plus a "last block" ticket, both updated with
 // atomics, cost about 80 ns per block, serialised at the end of the kernel: 40 us of
 // a 90 us kernel with 512 blocks.)
+#include <algorithm>
+
 #include "f8mi_common.h"
 
 namespace f8mi {
@@ -83,16 +85,15 @@ __global__ __launch_bounds__(AMAX_THREADS) void amax_finalize_kernel(const uint3
 // vectors, so every wave-level load is 1 KB of one DRAM page.  (Striding each lane's loads by the whole
 // grid instead costs more than half of the bandwidth.)
 template <int DT, bool NT>
-__global__ __launch_bounds__(AMAX_THREADS) void amax_dense_kernel(const void* __restrict__ x, int64_t n,
-                                                                   uint32_t* __restrict__ ws) {
-    __shared__ uint32_t red[AMAX_THREADS / 64];
+__device__ __forceinline__ void amax_dense_body(const void* __restrict__ x, int64_t n, uint32_t* __restrict__ ws, uint32_t bid, uint32_t nb,
+                                                uint32_t* red) {
     constexpr int EPV = DT == F8MI_FP32 ? 4 : 8;
     constexpr int64_t TILE = (int64_t)AMAX_THREADS * AMAX_UNROLL;
     const int64_t nvec = n / EPV;
     const uint4* xv = (const uint4*)x;
     uint32_t m = 0;
     const int64_t ntiles = (nvec + TILE - 1) / TILE;
-    for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    for (int64_t t = bid; t < ntiles; t += nb) {
         const int64_t base = t * TILE + threadIdx.x;
         uint4 v[AMAX_UNROLL];
         if (base - threadIdx.x + TILE <= nvec) {
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(AMAX_THREADS) void amax_dense_kernel(const void* __
         for (int u = 0; u < AMAX_UNROLL; u++) m = absmax_vec<DT>(v[u], m);
     }
     m = absmax_done<DT>(m);
-    if (blockIdx.x == 0) {  // scalar tail (< EPV elements)
+    if (bid == 0) {  // scalar tail (< EPV elements)
         int64_t t = nvec * EPV + threadIdx.x;
         if (t < n) {
             uint32_t a = absmax_elem<DT>(x, t);
@@ -117,7 +118,22 @@ __global__ __launch_bounds__(AMAX_THREADS) void amax_dense_kernel(const void* __
         }
     }
     m = block_max_u32(m, red);
-    if (threadIdx.x == 0) ws[blockIdx.x] = m;
+    if (threadIdx.x == 0) ws[bid] = m;
+}
+
+template <int DT, bool NT>
+__global__ __launch_bounds__(AMAX_THREADS) void amax_dense_kernel(const void* __restrict__ x, int64_t n, uint32_t* __restrict__ ws) {
+    __shared__ uint32_t red[AMAX_THREADS / 64];
+    amax_dense_body<DT, NT>(x, n, ws, blockIdx.x, gridDim.x, red);
+}
+
+// Two tensors in one launch, the first nb_a blocks for the first.
+template <int DTA, int DTB>
+__global__ __launch_bounds__(AMAX_THREADS) void amax_dense_pair_kernel(const void* __restrict__ xa, int64_t na, uint32_t* __restrict__ ws_a, uint32_t nb_a,
+                                                                       const void* __restrict__ xb, int64_t nb, uint32_t* __restrict__ ws_b) {
+    __shared__ uint32_t red[AMAX_THREADS / 64];
+    if (blockIdx.x < nb_a) amax_dense_body<DTA, true>(xa, na, ws_a, blockIdx.x, nb_a, red);
+    else amax_dense_body<DTB, true>(xb, nb, ws_b, blockIdx.x - nb_a, gridDim.x - nb_a, red);
 }
 
 // Any row stride / alignment: one element per thread step.
@@ -241,6 +257,13 @@ using namespace f8mi;
 
 namespace f8mi {
 
+static bool amax_dense(const void* x, int64_t rows, int64_t cols, int64_t ld) { return (ld == cols || rows == 1) && (uintptr_t)x % 16 == 0; }
+static int64_t amax_dense_blocks(int64_t n, int in_dtype) {
+    const int64_t per_block = (int64_t)AMAX_THREADS * AMAX_UNROLL, nvec = n / (in_dtype == F8MI_FP32 ? 4 : 8);
+    // few, long-lived blocks, two per CU; two tensors' words fit the workspace
+    return std::max<int64_t>(1, std::min<int64_t>((nvec + per_block - 1) / per_block, std::min(cu_count() * 2, WS_WORDS / 2)));
+}
+
 // First half of f8mi_amax_scale: per-workgroup maxima of the |x| bit patterns into ws[0 .. *nblocks).  rows * cols > 0,
 // arguments already validated.  The second half is amax_finalize_kernel -- or the consumer reduces the words itself
 // (the dynamic-scaling cast does: one launch less).
@@ -249,16 +272,9 @@ int launch_amax_partials(const void* x, int64_t rows, int64_t cols, int64_t ld, 
     if (ld == 0 && rows > 1) rows = 1;  // every row is the same `cols` elements: the maximum of one of them
     const int64_t n = rows * cols;
     const size_t esz = in_dtype == F8MI_FP32 ? 4 : 2;
-    const bool dense = (ld == cols || rows == 1) && ((uintptr_t)x % 16 == 0);
     int64_t blocks;
-    if (dense) {
-        const int64_t epv = 16 / esz;
-        const int64_t nvec = n / epv;
-        blocks = (nvec + (int64_t)AMAX_THREADS * AMAX_UNROLL - 1) / ((int64_t)AMAX_THREADS * AMAX_UNROLL);
-        int64_t cap = (int64_t)cu_count() * 2;  // few, long-lived blocks, two per CU
-        if (cap > WS_WORDS) cap = WS_WORDS;
-        if (blocks > cap) blocks = cap;
-        if (blocks < 1) blocks = 1;
+    if (amax_dense(x, rows, cols, ld)) {
+        blocks = amax_dense_blocks(n, in_dtype);
         dim3 g((unsigned)blocks), b(AMAX_THREADS);
         const bool nt = (int64_t)(n * esz) > (int64_t)F8MI_AMAX_PLAIN_LOADS_MAX_BYTES;
         if (in_dtype == F8MI_BF16) {
@@ -283,6 +299,29 @@ int launch_amax_partials(const void* x, int64_t rows, int64_t cols, int64_t ld, 
     }
     *nblocks = (int)blocks;
     return check_hip(hipGetLastError(), "amax kernel launch");
+}
+
+bool amax_pair_ok(const void* xa, int64_t rows_a, int64_t cols_a, int64_t ld_a, const void* xb, int64_t rows_b, int64_t cols_b, int64_t ld_b) {
+    return amax_dense(xa, rows_a, cols_a, ld_a) && amax_dense(xb, rows_b, cols_b, ld_b);
+}
+
+template <int DTA, int DTB>
+static int launch_amax_pair1(hipStream_t stream, const void* xa, int64_t na, uint32_t* ws_a, int blocks_a, const void* xb, int64_t nb, uint32_t* ws_b, int blocks_b) {
+    hipLaunchKernelGGL((amax_dense_pair_kernel<DTA, DTB>), dim3((unsigned)(blocks_a + blocks_b)), dim3(AMAX_THREADS), 0, stream, xa, na, ws_a, (uint32_t)blocks_a, xb, nb, ws_b);
+    return check_hip(hipGetLastError(), "amax (two tensors) kernel launch");
+}
+
+int launch_amax_pair(int dt_a, int dt_b, const void* xa, int64_t na, const void* xb, int64_t nb, uint32_t* ws, hipStream_t stream, const uint32_t** words_b,
+                     int* blocks_a, int* blocks_b) {
+    uint32_t* const ws_b = ws + WS_WORDS / 2;
+    *words_b = ws_b;
+    *blocks_a = (int)amax_dense_blocks(na, dt_a);
+    *blocks_b = (int)amax_dense_blocks(nb, dt_b);
+    if (dt_a == F8MI_BF16 && dt_b == F8MI_BF16) return launch_amax_pair1<F8MI_BF16, F8MI_BF16>(stream, xa, na, ws, *blocks_a, xb, nb, ws_b, *blocks_b);
+    if (dt_a == F8MI_FP16 && dt_b == F8MI_FP16) return launch_amax_pair1<F8MI_FP16, F8MI_FP16>(stream, xa, na, ws, *blocks_a, xb, nb, ws_b, *blocks_b);
+    if (dt_a == F8MI_BF16 && dt_b == F8MI_FP32) return launch_amax_pair1<F8MI_BF16, F8MI_FP32>(stream, xa, na, ws, *blocks_a, xb, nb, ws_b, *blocks_b);
+    if (dt_a == F8MI_FP16 && dt_b == F8MI_FP32) return launch_amax_pair1<F8MI_FP16, F8MI_FP32>(stream, xa, na, ws, *blocks_a, xb, nb, ws_b, *blocks_b);
+    return launch_amax_pair1<F8MI_FP32, F8MI_FP32>(stream, xa, na, ws, *blocks_a, xb, nb, ws_b, *blocks_b);
 }
 
 }  // namespace f8mi

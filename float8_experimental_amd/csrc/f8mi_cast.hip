@@ -342,20 +342,33 @@ __device__ __forceinline__ uint32_t collect_words(const TaggedWords& e, uint32_t
     return m;
 }
 
-template <int DT, int PROD, int FMT, bool TAGGED>
-__global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restrict__ x, int64_t rows, int64_t cols,
-                                                            int64_t ld, const float* __restrict__ scale_dev,
-                                                            uint8_t* __restrict__ out, uint8_t* __restrict__ out_t,
-                                                            float* amax_out, uint32_t tiles_x, uint32_t tiles_y,
-                                                            int out_kb, int out_t_kb, const uint32_t* __restrict__ amax_ws,
-                                                            int amax_nblocks, float* scale_out, uint32_t* amax_spread,
-                                                            TaggedWords tagged) {
-    __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];  // [column][row/4] dwords, swizzled
-    __shared__ uint32_t red[CAST_THREADS / 64];
+// One tensor of a launch, as the kernels take it.
+struct CastJob {
+    const void* x;
+    int64_t rows, cols, ld;
+    uint8_t *out, *out_t;
+    uint32_t tiles_x, tiles_y;
+    int out_kb, out_t_kb;      // F8MI_LAYOUT_* code of the respective output
+    const float* scale_dev;    // the scale, given beforehand; else
+    float* scale_out;          // where the one found here goes,
+    const uint32_t* amax_ws;   // found from the amax_nblocks maxima in amax_ws (the resident kernel: from the tensor itself)
+    int amax_nblocks;
+    float* amax_out;           // fused amax: its value, through
+    uint32_t* amax_spread;     // these words, or
+    TaggedWords tagged;        // an exchange
+};
 
+// Workgroup `bid` of the `nb` that cast the tensor.
+template <int DT, int PROD, int FMT, bool TAGGED>
+__device__ __forceinline__ void cast_body(const CastJob& j, uint32_t bid, uint32_t nb, uint32_t* tileT, uint32_t (&red)[CAST_THREADS / 64]) {
+    const void* const x = j.x;
+    const int64_t rows = j.rows, cols = j.cols, ld = j.ld;
+    float* const amax_out = j.amax_out;
+    const uint32_t* const amax_ws = j.amax_ws;
+    const int amax_nblocks = j.amax_nblocks;
     const int t = threadIdx.x;
     int ty, tx;
-    cast_tile_of(blockIdx.x, gridDim.x, tiles_x, tiles_y, ty, tx);
+    cast_tile_of(bid, nb, j.tiles_x, j.tiles_y, ty, tx);
     const int64_t r0 = (int64_t)ty * CAST_TILE;
     const int64_t c0 = (int64_t)tx * CAST_TILE;
 
@@ -396,25 +409,25 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restri
         }
         wm = wave_max_u32(wm);
         scale = amax_to_scale_dev(abs_bits_to_float(wm, DT), DT, FMT, DT == F8MI_FP16);
-        if (blockIdx.x == 0 && t == 0) *scale_out = scale;
+        if (bid == 0 && t == 0) *j.scale_out = scale;
         within = within_range<FMT>(abs_bits_to_float(wm, DT), scale);
     } else {
-        scale = *scale_dev;
+        scale = *j.scale_dev;
         m = absmax_tile<DT, 2>(in);
         within = __all(within_range<FMT>(abs_bits_to_float(m, DT), scale));
     }
 
-    emit_tile<DT, PROD, FMT, 2>(in, tileT, scale, within, r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
+    emit_tile<DT, PROD, FMT, 2>(in, tileT, scale, within, r0, c0, rows, cols, j.out, j.out_t, j.out_kb, j.out_t_kb);
 
     if constexpr (TAGGED) {
         // Every wave leaves its maximum in a word of its own; the workgroup that was started last collects them.
         m = wave_max_u32(m);
-        if ((t & 63) == 0) publish_word(tagged, blockIdx.x * (CAST_THREADS / 64) + (t >> 6), m);
-        if (blockIdx.x == gridDim.x - 1) {
-            m = collect_words<DT, 8>(tagged, gridDim.x * (CAST_THREADS / 64), m, red, x, rows, cols, ld);
+        if ((t & 63) == 0) publish_word(j.tagged, bid * (CAST_THREADS / 64) + (t >> 6), m);
+        if (bid == nb - 1) {
+            m = collect_words<DT, 8>(j.tagged, nb * (CAST_THREADS / 64), m, red, x, rows, cols, ld);
             if (t == 0) *amax_out = abs_bits_to_float(m, DT);
         }
-    } else if (amax_out && amax_spread) {
+    } else if (amax_out && j.amax_spread) {
         // Every wave folds its maximum (the bit pattern in the input's dtype) into one of SPREAD_WORDS words with an
         // atomic that returns nothing: no LDS, no barrier, no round trip to wait for, and a word sees about one atomic
         // per (tiles * 4 / SPREAD_WORDS) waves, spread over the whole run of the kernel.  cast_spread_finalize_kernel
@@ -424,7 +437,7 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restri
         // plus 4 us for the finalize launch.)
         m = wave_max_u32(m);
         if ((t & 63) == 0 && m)
-            (void)__hip_atomic_fetch_max(&amax_spread[(blockIdx.x * (CAST_THREADS / 64) + (t >> 6)) & (SPREAD_WORDS - 1)], m,
+            (void)__hip_atomic_fetch_max(&j.amax_spread[(bid * (CAST_THREADS / 64) + (t >> 6)) & (SPREAD_WORDS - 1)], m,
                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else if (amax_out) {
         m = wave_max_u32(m);
@@ -437,6 +450,22 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(const void* __restri
         }
         publish_amax_cast(m, amax_out, DT);
     }
+}
+
+template <int DT, int PROD, int FMT, bool TAGGED>
+__global__ __launch_bounds__(CAST_THREADS) void cast_kernel(CastJob j) {
+    __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];  // [column][row/4] dwords, swizzled
+    __shared__ uint32_t red[CAST_THREADS / 64];
+    cast_body<DT, PROD, FMT, TAGGED>(j, blockIdx.x, gridDim.x, tileT, red);
+}
+
+// Two tensors in one launch, the first nb_a workgroups for the first.  TAGGED: delayed scaling, the product in fp32.
+template <int DTA, int DTB, int FMT, bool TAGGED>
+__global__ __launch_bounds__(CAST_THREADS) void cast_pair_kernel(CastJob a, CastJob b, uint32_t nb_a) {
+    __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];
+    __shared__ uint32_t red[CAST_THREADS / 64];
+    if (blockIdx.x < nb_a) cast_body<DTA, TAGGED ? F8MI_FP32 : DTA, FMT, TAGGED>(a, blockIdx.x, nb_a, tileT, red);
+    else cast_body<DTB, TAGGED ? F8MI_FP32 : DTB, FMT, TAGGED>(b, blockIdx.x - nb_a, gridDim.x - nb_a, tileT, red);
 }
 
 // Dynamic scaling of a small tensor in ONE launch: amax, scale and cast by a single workgroup that holds the whole
@@ -606,26 +635,37 @@ static int launch_cast_flat(int fmt, hipStream_t stream, const void* x, int64_t 
 constexpr int RESIDENT_TILES = 1024;  // workgroups at most
 
 template <int DT, int FMT, int H>
-__global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_kernel(const void* __restrict__ x, int64_t rows, int64_t cols, int64_t ld,
-                                                                             float* __restrict__ scale_out, uint8_t* __restrict__ out,
-                                                                             uint8_t* __restrict__ out_t, uint32_t tiles_x, uint32_t tiles_y,
-                                                                             int out_kb, int out_t_kb, TaggedWords tagged) {
-    __shared__ uint32_t tileT[32 * 64 * H];
-    __shared__ uint32_t red[2][CAST_THREADS / 64];
+__device__ __forceinline__ void resident_body(const CastJob& j, uint32_t bid, uint32_t nb, uint32_t* tileT, uint32_t (&red)[2][CAST_THREADS / 64]) {
     const int t = threadIdx.x;
     int ty, tx;
-    cast_tile_of(blockIdx.x, gridDim.x, tiles_x, tiles_y, ty, tx);
+    cast_tile_of(bid, nb, j.tiles_x, j.tiles_y, ty, tx);
     const int64_t r0 = (int64_t)ty * (64 * H), c0 = (int64_t)tx * CAST_TILE;
     Row8<DT> in[H][4];
-    load_tile<DT, H>(in, x, r0, c0, rows, cols, ld);
+    load_tile<DT, H>(in, j.x, r0, c0, j.rows, j.cols, j.ld);
     uint32_t m = wave_max_u32(absmax_tile<DT, H>(in));
     if ((t & 63) == 0) red[0][t >> 6] = m;
     __syncthreads();
-    if (t == 0) publish_word(tagged, blockIdx.x, max(max(red[0][0], red[0][1]), max(red[0][2], red[0][3])));
-    m = collect_words<DT, 1>(tagged, gridDim.x, m, red[1], x, rows, cols, ld);
+    if (t == 0) publish_word(j.tagged, bid, max(max(red[0][0], red[0][1]), max(red[0][2], red[0][3])));
+    m = collect_words<DT, 1>(j.tagged, nb, m, red[1], j.x, j.rows, j.cols, j.ld);
     const float amax = abs_bits_to_float(m, DT), scale = amax_to_scale_dev(amax, DT, FMT, DT == F8MI_FP16);
-    if (blockIdx.x == 0 && t == 0) *scale_out = scale;
-    emit_tile<DT, DT, FMT, H>(in, tileT, scale, within_range<FMT>(amax, scale), r0, c0, rows, cols, out, out_t, out_kb, out_t_kb);
+    if (bid == 0 && t == 0) *j.scale_out = scale;
+    emit_tile<DT, DT, FMT, H>(in, tileT, scale, within_range<FMT>(amax, scale), r0, c0, j.rows, j.cols, j.out, j.out_t, j.out_kb, j.out_t_kb);
+}
+
+template <int DT, int FMT, int H>
+__global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_kernel(CastJob j) {
+    __shared__ uint32_t tileT[32 * 64 * H];
+    __shared__ uint32_t red[2][CAST_THREADS / 64];
+    resident_body<DT, FMT, H>(j, blockIdx.x, gridDim.x, tileT, red);
+}
+
+// Two tensors that fit together; each finds its own maximum.
+template <int DTA, int DTB, int FMT, int H>
+__global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_pair_kernel(CastJob a, CastJob b, uint32_t nb_a) {
+    __shared__ uint32_t tileT[32 * 64 * H];
+    __shared__ uint32_t red[2][CAST_THREADS / 64];
+    if (blockIdx.x < nb_a) resident_body<DTA, FMT, H>(a, blockIdx.x, nb_a, tileT, red);
+    else resident_body<DTB, FMT, H>(b, blockIdx.x - nb_a, gridDim.x - nb_a, tileT, red);
 }
 
 constexpr int STATIC_MAX_DEVICES = 64;
@@ -708,25 +748,21 @@ __global__ __launch_bounds__(SPREAD_WORDS) void cast_spread_finalize_kernel(uint
 }
 
 template <int DT, int PROD, int FMT>
-static int launch_cast2(dim3 g, hipStream_t stream, const void* x, int64_t rows, int64_t cols, int64_t ld,
-                        const float* scale_dev, uint8_t* out, uint8_t* out_t, float* amax_dev, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb,
-                        const AmaxSource& src) {
+static int launch_cast2(dim3 g, hipStream_t stream, const CastJob& j) {
     if constexpr (PROD == F8MI_FP32) {  // what delayed scaling computes in
-        if (src.tagged.words) {
-            hipLaunchKernelGGL((cast_kernel<DT, PROD, FMT, true>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src.ws, src.nblocks, src.scale_out, src.spread, src.tagged);
+        if (j.tagged.words) {
+            hipLaunchKernelGGL((cast_kernel<DT, PROD, FMT, true>), g, dim3(CAST_THREADS), 0, stream, j);
             return check_hip(hipGetLastError(), "cast kernel launch");
         }
     }
-    hipLaunchKernelGGL((cast_kernel<DT, PROD, FMT, false>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src.ws, src.nblocks, src.scale_out, src.spread, src.tagged);
+    hipLaunchKernelGGL((cast_kernel<DT, PROD, FMT, false>), g, dim3(CAST_THREADS), 0, stream, j);
     return check_hip(hipGetLastError(), "cast kernel launch");
 }
 
 template <int DT, int PROD>
-static int launch_cast1(int fmt, dim3 g, hipStream_t stream, const void* x, int64_t rows, int64_t cols,
-                        int64_t ld, const float* scale_dev, uint8_t* out, uint8_t* out_t, float* amax_dev,
-                        uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb, const AmaxSource& src) {
-    if (fmt == F8MI_E4M3FN) return launch_cast2<DT, PROD, F8MI_E4M3FN>(g, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src);
-    return launch_cast2<DT, PROD, F8MI_E5M2>(g, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src);
+static int launch_cast1(int fmt, dim3 g, hipStream_t stream, const CastJob& j) {
+    if (fmt == F8MI_E4M3FN) return launch_cast2<DT, PROD, F8MI_E4M3FN>(g, stream, j);
+    return launch_cast2<DT, PROD, F8MI_E5M2>(g, stream, j);
 }
 
 static int check_cast_layouts(int64_t rows, int64_t cols, const void* out, int out_layout, const void* out_t, int out_t_layout) {
@@ -763,6 +799,7 @@ static int cast_layout_impl(const void* x, int64_t rows, int64_t cols, int64_t l
     if (tx * ty > 0x7fffffffLL) { set_error("f8mi_cast: more than 2^31 tiles"); return F8MI_ERR_UNSUPPORTED; }
     dim3 g((unsigned)(tx * ty));
     const uint32_t tiles_x = (uint32_t)tx, tiles_y = (uint32_t)ty;
+    const CastJob j{x, rows, cols, ld, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, scale_dev, src.scale_out, src.ws, src.nblocks, amax_dev, src.spread, src.tagged};
     const size_t esz = in_dtype == F8MI_FP32 ? 4 : 2;
     const double n = (double)rows * (double)cols;
     // every launch of this call: the cast and what a fused amax adds before or after it
@@ -773,13 +810,13 @@ static int cast_layout_impl(const void* x, int64_t rows, int64_t cols, int64_t l
     }
     int rc;
     if (in_dtype == F8MI_BF16) {
-        if (product_dtype == F8MI_BF16) rc = launch_cast1<F8MI_BF16, F8MI_BF16>(fp8_fmt, g, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src);
-        else rc = launch_cast1<F8MI_BF16, F8MI_FP32>(fp8_fmt, g, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src);
+        if (product_dtype == F8MI_BF16) rc = launch_cast1<F8MI_BF16, F8MI_BF16>(fp8_fmt, g, stream, j);
+        else rc = launch_cast1<F8MI_BF16, F8MI_FP32>(fp8_fmt, g, stream, j);
     } else if (in_dtype == F8MI_FP16) {
-        if (product_dtype == F8MI_FP16) rc = launch_cast1<F8MI_FP16, F8MI_FP16>(fp8_fmt, g, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src);
-        else rc = launch_cast1<F8MI_FP16, F8MI_FP32>(fp8_fmt, g, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src);
+        if (product_dtype == F8MI_FP16) rc = launch_cast1<F8MI_FP16, F8MI_FP16>(fp8_fmt, g, stream, j);
+        else rc = launch_cast1<F8MI_FP16, F8MI_FP32>(fp8_fmt, g, stream, j);
     } else {
-        rc = launch_cast1<F8MI_FP32, F8MI_FP32>(fp8_fmt, g, stream, x, rows, cols, ld, scale_dev, out, out_t, amax_dev, tiles_x, tiles_y, out_kb, out_t_kb, src);
+        rc = launch_cast1<F8MI_FP32, F8MI_FP32>(fp8_fmt, g, stream, j);
     }
     if (rc || !(amax_dev && src.spread)) return rc;
     hipLaunchKernelGGL(cast_spread_finalize_kernel, dim3(1), dim3(SPREAD_WORDS), 0, stream, src.spread, amax_dev, in_dtype);
@@ -853,17 +890,15 @@ static int resident_tile_rows(int64_t rows, int64_t cols) {
 }
 
 template <int DT, int FMT>
-static int launch_cast_resident1(int tile_rows, dim3 g, hipStream_t stream, const void* x, int64_t rows, int64_t cols, int64_t ld, float* scale_dev,
-                                 uint8_t* out, uint8_t* out_t, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb, const TaggedWords& tagged) {
-    if (tile_rows == 64) hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 1>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
-    else hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 2>), g, dim3(CAST_THREADS), 0, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
+static int launch_cast_resident1(int tile_rows, dim3 g, hipStream_t stream, const CastJob& j) {
+    if (tile_rows == 64) hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 1>), g, dim3(CAST_THREADS), 0, stream, j);
+    else hipLaunchKernelGGL((cast_dynamic_resident_kernel<DT, FMT, 2>), g, dim3(CAST_THREADS), 0, stream, j);
     return check_hip(hipGetLastError(), "cast (dynamic, resident) kernel launch");
 }
 template <int DT>
-static int launch_cast_resident(int fmt, int tile_rows, dim3 g, hipStream_t stream, const void* x, int64_t rows, int64_t cols, int64_t ld, float* scale_dev,
-                                uint8_t* out, uint8_t* out_t, uint32_t tiles_x, uint32_t tiles_y, int out_kb, int out_t_kb, const TaggedWords& tagged) {
-    if (fmt == F8MI_E4M3FN) return launch_cast_resident1<DT, F8MI_E4M3FN>(tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
-    return launch_cast_resident1<DT, F8MI_E5M2>(tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
+static int launch_cast_resident(int fmt, int tile_rows, dim3 g, hipStream_t stream, const CastJob& j) {
+    if (fmt == F8MI_E4M3FN) return launch_cast_resident1<DT, F8MI_E4M3FN>(tile_rows, g, stream, j);
+    return launch_cast_resident1<DT, F8MI_E5M2>(tile_rows, g, stream, j);
 }
 
 }  // namespace f8mi
@@ -883,12 +918,13 @@ extern "C" int f8mi_cast_dynamic_resident(const void* x, int64_t rows, int64_t c
     // whole 128 x 128 tiles, as the padded layouts are
     const uint32_t tiles_x = (uint32_t)((cols + CAST_TILE - 1) / CAST_TILE), tiles_y = (uint32_t)((rows + CAST_TILE - 1) / CAST_TILE) * (CAST_TILE / tile_rows);
     const dim3 g(tiles_x * tiles_y);
+    const CastJob j{x, rows, cols, ld, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, nullptr, scale_dev, nullptr, 0, nullptr, nullptr, tagged};
     const size_t esz = in_dtype == F8MI_FP32 ? 4 : 2;
     const double n = (double)rows * (double)cols;
     ProfScope prof(F8MI_K_CAST, (ld == 0 ? (double)cols : n) * esz + n * ((out ? 1 : 0) + (out_t ? 1 : 0)), stream);
-    if (in_dtype == F8MI_BF16) return launch_cast_resident<F8MI_BF16>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
-    if (in_dtype == F8MI_FP16) return launch_cast_resident<F8MI_FP16>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
-    return launch_cast_resident<F8MI_FP32>(fp8_fmt, tile_rows, g, stream, x, rows, cols, ld, scale_dev, out, out_t, tiles_x, tiles_y, out_kb, out_t_kb, tagged);
+    if (in_dtype == F8MI_BF16) return launch_cast_resident<F8MI_BF16>(fp8_fmt, tile_rows, g, stream, j);
+    if (in_dtype == F8MI_FP16) return launch_cast_resident<F8MI_FP16>(fp8_fmt, tile_rows, g, stream, j);
+    return launch_cast_resident<F8MI_FP32>(fp8_fmt, tile_rows, g, stream, j);
 }
 
 extern "C" int f8mi_cast_dynamic(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, int fp8_fmt, float* scale_dev,
@@ -939,6 +975,141 @@ extern "C" int f8mi_cast_dynamic(const void* x, int64_t rows, int64_t cols, int6
     }
     return cast_layout_impl(x, rows, cols, ld, in_dtype, nullptr, in_dtype, fp8_fmt, out, out_layout, out_t, out_t_layout, nullptr, stream,
                             AmaxSource{(const uint32_t*)workspace, nblocks, scale_dev, nullptr, {}});
+}
+
+namespace f8mi {
+
+// Two tensors, the operands of one product, in one launch: what it saves is the second one's launch, ramp and, between them, the
+// tail of the first.  us, back to back, inputs cold, two calls / this, bf16, dynamic: 512 x 1024 and 1024 x 1024: 12.8 / 7.0; 2048 x 4096
+// twice (1024 tiles, one launch): 23.3 / 18.8; 8192 x 4096 and 1024 x 4096 (two launches): 42.9 / 37.5, and 14336 x 4096: 88.2 / 83.6;
+// delayed: 11.5 / 6.1, 18.2 / 13.5, 2048 x 4096 and 4096 x 4096 22.6 / 18.9; bf16 and fp32, dynamic, 512 x 1024 and 1024 x 1024: 13.2 / 7.5.
+static int64_t tiles_of(const f8mi_cast_job& j) {
+    const int64_t ty = (j.rows + CAST_TILE - 1) / CAST_TILE, tx = (j.cols + CAST_TILE - 1) / CAST_TILE;
+    return ty > 0x7fffffff || tx > 0x7fffffff || tx * ty > 0x3fffffff ? 0x40000000 : tx * ty;
+}
+// Whether both are what the pair kernels take; anything else, wrong arguments among it, is left to the two calls.
+static bool pair_ok(const f8mi_cast_job& a, const f8mi_cast_job& b) {
+    for (const f8mi_cast_job* j : {&a, &b})
+        if (j->rows <= 0 || j->cols <= 0 || (j->ld < j->cols && j->ld != 0) || !j->x || !j->scale_dev || (!j->out && !j->out_t) || j->in_dtype < 0 || j->in_dtype > 2 ||
+            check_cast_layouts(j->rows, j->cols, j->out, j->out_layout, j->out_t, j->out_t_layout) || tiles_of(*j) >= 0x40000000)
+            return false;
+    return a.in_dtype == b.in_dtype || b.in_dtype == F8MI_FP32;
+}
+static int64_t job_read(const f8mi_cast_job& j) { return j.rows * j.cols * (j.in_dtype == F8MI_FP32 ? 4 : 2); }
+// The maxima of both in one launch and their casts in another: where both take two launches by themselves, and where the one that
+// takes only one is small: it is read twice that way (8192 x 4096 with 1024 x 4096: 42.9 / 37.5 us, with 4096 x 4096 fp32: 59.5 / 61.7).
+static bool two_launches_pay(const f8mi_cast_job& a, const f8mi_cast_job& b) {
+    const bool one_a = resident_tile_rows(a.rows, a.cols) != 0, one_b = resident_tile_rows(b.rows, b.cols) != 0;
+    if (one_a && one_b) return false;
+    return (!one_a || job_read(a) <= 16 << 20) && (!one_b || job_read(b) <= 16 << 20);
+}
+// tile_rows: 64 or 128, whole 128 x 128 tiles either way
+static CastJob kernel_job(const f8mi_cast_job& j, int tile_rows) {
+    CastJob k{};
+    k.x = j.x; k.rows = j.rows; k.cols = j.cols; k.ld = j.ld; k.out = j.out; k.out_t = j.out_t;
+    k.tiles_x = (uint32_t)((j.cols + CAST_TILE - 1) / CAST_TILE);
+    k.tiles_y = (uint32_t)((j.rows + CAST_TILE - 1) / CAST_TILE) * (CAST_TILE / tile_rows);
+    k.out_kb = j.out ? j.out_layout : F8MI_LAYOUT_ROWMAJOR;
+    k.out_t_kb = j.out_t ? j.out_t_layout : F8MI_LAYOUT_ROWMAJOR;
+    return k;
+}
+static double job_bytes(const f8mi_cast_job& j) {
+    const double n = (double)j.rows * (double)j.cols;
+    return (j.ld == 0 ? (double)j.cols : n) * (j.in_dtype == F8MI_FP32 ? 4 : 2) + n * ((j.out ? 1 : 0) + (j.out_t ? 1 : 0));
+}
+
+// tile_rows != 0: the resident kernel with such tiles; else the cast behind an amax launch, or, TAGGED, the delayed one
+template <int DTA, int DTB, bool TAGGED>
+static int launch_cast_pair1(int tile_rows, hipStream_t stream, const CastJob& a, const CastJob& b) {
+    const uint32_t nb_a = a.tiles_x * a.tiles_y;
+    const dim3 g(nb_a + b.tiles_x * b.tiles_y), t(CAST_THREADS);
+    if constexpr (!TAGGED) {
+        if (tile_rows == 64) hipLaunchKernelGGL((cast_dynamic_resident_pair_kernel<DTA, DTB, F8MI_E4M3FN, 1>), g, t, 0, stream, a, b, nb_a);
+        else if (tile_rows == 128) hipLaunchKernelGGL((cast_dynamic_resident_pair_kernel<DTA, DTB, F8MI_E4M3FN, 2>), g, t, 0, stream, a, b, nb_a);
+        else hipLaunchKernelGGL((cast_pair_kernel<DTA, DTB, F8MI_E4M3FN, false>), g, t, 0, stream, a, b, nb_a);
+    } else {
+        hipLaunchKernelGGL((cast_pair_kernel<DTA, DTB, F8MI_E4M3FN, true>), g, t, 0, stream, a, b, nb_a);
+    }
+    return check_hip(hipGetLastError(), "cast (two tensors) kernel launch");
+}
+template <bool TAGGED>
+static int launch_cast_pair(int dt_a, int dt_b, int tile_rows, hipStream_t stream, const CastJob& a, const CastJob& b) {
+    if (dt_a == F8MI_BF16 && dt_b == F8MI_BF16) return launch_cast_pair1<F8MI_BF16, F8MI_BF16, TAGGED>(tile_rows, stream, a, b);
+    if (dt_a == F8MI_FP16 && dt_b == F8MI_FP16) return launch_cast_pair1<F8MI_FP16, F8MI_FP16, TAGGED>(tile_rows, stream, a, b);
+    if (dt_a == F8MI_BF16 && dt_b == F8MI_FP32) return launch_cast_pair1<F8MI_BF16, F8MI_FP32, TAGGED>(tile_rows, stream, a, b);
+    if (dt_a == F8MI_FP16 && dt_b == F8MI_FP32) return launch_cast_pair1<F8MI_FP16, F8MI_FP32, TAGGED>(tile_rows, stream, a, b);
+    return launch_cast_pair1<F8MI_FP32, F8MI_FP32, TAGGED>(tile_rows, stream, a, b);
+}
+
+}  // namespace f8mi
+
+extern "C" int f8mi_cast_dynamic_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream_) {
+    hipStream_t stream = (hipStream_t)stream_;
+    if (!a || !b) { set_error("f8mi_cast_dynamic_pair: null job"); return F8MI_ERR_INVALID_ARG; }
+    if (workspace && (uintptr_t)workspace % 16 == 0 && pair_ok(*a, *b)) {
+        const int64_t tiles_a = tiles_of(*a), tiles_b = tiles_of(*b);
+        CastJob ja, jb;
+        if (const int tile_rows = resident_tile_rows((tiles_a + tiles_b) * CAST_TILE, CAST_TILE)) {
+            TaggedWords tagged;
+            if (const int rc = begin_exchange(stream, EXCHANGE_WAIT_TICKS, tagged)) return rc;
+            if (tagged.words) {
+                ja = kernel_job(*a, tile_rows);
+                jb = kernel_job(*b, tile_rows);
+                ja.scale_out = a->scale_dev;
+                jb.scale_out = b->scale_dev;
+                ja.tagged = jb.tagged = tagged;
+                jb.tagged.words += ja.tiles_x * ja.tiles_y;
+                ProfScope prof(F8MI_K_CAST, job_bytes(*a) + job_bytes(*b), stream);
+                return launch_cast_pair<false>(a->in_dtype, b->in_dtype, tile_rows, stream, ja, jb);
+            }
+        }
+        // one of them too large for a launch of its own: both through the two launches it takes
+        if (two_launches_pay(*a, *b) && a->ld && b->ld &&
+            amax_pair_ok(a->x, a->rows, a->cols, a->ld, b->x, b->rows, b->cols, b->ld)) {
+            ja = kernel_job(*a, CAST_TILE);
+            jb = kernel_job(*b, CAST_TILE);
+            ja.scale_out = a->scale_dev;
+            jb.scale_out = b->scale_dev;
+            ja.amax_ws = (const uint32_t*)workspace;
+            {
+                ProfScope prof(F8MI_K_AMAX, (double)job_read(*a) + (double)job_read(*b), stream);
+                if (const int rc = launch_amax_pair(a->in_dtype, b->in_dtype, a->x, a->rows * a->cols, b->x, b->rows * b->cols, (uint32_t*)workspace, stream, &jb.amax_ws,
+                                                    &ja.amax_nblocks, &jb.amax_nblocks))
+                    return rc;
+            }
+            ProfScope prof(F8MI_K_CAST, job_bytes(*a) + job_bytes(*b), stream);
+            return launch_cast_pair<false>(a->in_dtype, b->in_dtype, 0, stream, ja, jb);
+        }
+    }
+    for (const f8mi_cast_job* j : {a, b})
+        if (const int rc = f8mi_cast_dynamic(j->x, j->rows, j->cols, j->ld, j->in_dtype, F8MI_E4M3FN, j->scale_dev, j->out, j->out_layout, j->out_t, j->out_t_layout, workspace, stream_))
+            return rc;
+    return F8MI_OK;
+}
+
+extern "C" int f8mi_cast_delayed_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream_) {
+    hipStream_t stream = (hipStream_t)stream_;
+    if (!a || !b) { set_error("f8mi_cast_delayed_pair: null job"); return F8MI_ERR_INVALID_ARG; }
+    if (pair_ok(*a, *b) && a->amax_dev && b->amax_dev && one_launch_delayed((tiles_of(*a) + tiles_of(*b)) * CAST_TILE, CAST_TILE)) {
+        TaggedWords tagged;
+        if (const int rc = begin_exchange(stream, EXCHANGE_WAIT_TICKS, tagged)) return rc;
+        if (tagged.words) {
+            CastJob ja = kernel_job(*a, CAST_TILE), jb = kernel_job(*b, CAST_TILE);
+            ja.scale_dev = a->scale_dev;
+            jb.scale_dev = b->scale_dev;
+            ja.amax_out = a->amax_dev;
+            jb.amax_out = b->amax_dev;
+            ja.tagged = jb.tagged = tagged;
+            jb.tagged.words += ja.tiles_x * ja.tiles_y * (CAST_THREADS / 64);
+            ProfScope prof(F8MI_K_CAST, job_bytes(*a) + job_bytes(*b), stream);
+            return launch_cast_pair<true>(a->in_dtype, b->in_dtype, 0, stream, ja, jb);
+        }
+    }
+    for (const f8mi_cast_job* j : {a, b})
+        if (const int rc = f8mi_cast_delayed(j->x, j->rows, j->cols, j->ld, j->in_dtype, j->scale_dev, F8MI_E4M3FN, j->out, j->out_layout, j->out_t, j->out_t_layout, j->amax_dev,
+                                             workspace, stream_))
+            return rc;
+    return F8MI_OK;
 }
 
 namespace f8mi {

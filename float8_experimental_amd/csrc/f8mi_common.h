@@ -33,6 +33,11 @@ constexpr int WS_WORDS = 1024;
 // f8mi_amax_scale.  rows * cols > 0, arguments already validated; no profiling bracket of its own.
 int launch_amax_partials(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, uint32_t* ws, hipStream_t stream,
                          int* nblocks);
+// The same for two dense tensors (amax_pair_ok) in one launch: ws[0 .. *blocks_a) and (*words_b)[0 .. *blocks_b), in the halves of the
+// workspace.  Types: equal, or 16-bit and fp32.
+bool amax_pair_ok(const void* xa, int64_t rows_a, int64_t cols_a, int64_t ld_a, const void* xb, int64_t rows_b, int64_t cols_b, int64_t ld_b);
+int launch_amax_pair(int dt_a, int dt_b, const void* xa, int64_t na, const void* xb, int64_t nb, uint32_t* ws, hipStream_t stream, const uint32_t** words_b,
+                     int* blocks_a, int* blocks_b);
 
 // ---------------------------------------------------------------- device side
 

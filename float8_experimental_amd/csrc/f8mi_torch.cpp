@@ -26,6 +26,8 @@ struct Lib {
     decltype(&f8mi_cast_dynamic) cast_dynamic;
     decltype(&f8mi_cast_layout) cast_layout;
     decltype(&f8mi_cast_delayed) cast_delayed;
+    decltype(&f8mi_cast_dynamic_pair) cast_dynamic_pair;
+    decltype(&f8mi_cast_delayed_pair) cast_delayed_pair;
     decltype(&f8mi_gemm_nt_ws) gemm_nt_ws;
     decltype(&f8mi_gemm_nt_kb_ws) gemm_nt_kb_ws;
     decltype(&f8mi_gemm_kb_ex) gemm_kb_ex;
@@ -128,6 +130,38 @@ struct Call {
                                 pt, tr_layout, nullptr, stream), "f8mi_cast_layout");
     }
 
+    // The e4m3 copies of two tensors, both scaled dynamically or both delayed, as one library call.
+    struct Cast {
+        const at::Tensor& x;
+        const Scaling& s;
+        bool want_tr;
+        int row_layout, tr_layout;
+        at::Tensor &row, &tr, &scale;
+    };
+    void cast_two(const Cast& a, const Cast& b) const {
+        const bool delayed = a.s.amax.defined() && b.s.amax.defined(), dynamic = !a.s.scale.defined() && !b.s.scale.defined();
+        if (!(delayed && L.cast_delayed_pair) && !(dynamic && L.cast_dynamic_pair)) {
+            for (const Cast* c : {&a, &b}) cast(c->x, c->s, F8MI_E4M3FN, true, c->row_layout, c->want_tr, c->tr_layout, c->row, c->tr, c->scale);
+            return;
+        }
+        f8mi_cast_job jobs[2];
+        int i = 0;
+        for (const Cast* c : {&a, &b}) {
+            const int64_t m = c->x.size(0), k = c->x.size(1);
+            c->row = copy(m, k, c->row_layout, F8MI_E4M3FN);
+            if (c->want_tr) c->tr = copy(k, m, c->tr_layout, F8MI_E4M3FN);
+            c->scale = delayed ? c->s.scale : make({}, at::kFloat);
+            jobs[i++] = {c->x.data_ptr(), m, k, c->x.stride(0), (float*)c->scale.data_ptr(), (uint8_t*)c->row.data_ptr(), c->want_tr ? (uint8_t*)c->tr.data_ptr() : nullptr,
+                         delayed ? (float*)c->s.amax.data_ptr() : nullptr, dtype_code(c->x.scalar_type()), c->row_layout, c->tr_layout};
+        }
+        if (delayed) {
+            check(L.cast_delayed_pair(&jobs[0], &jobs[1], delayed_ws, stream), "f8mi_cast_delayed_pair");
+        } else {
+            const at::Tensor ws = make({(int64_t)L.workspace_bytes / 4}, at::kInt);
+            check(L.cast_dynamic_pair(&jobs[0], &jobs[1], ws.data_ptr(), stream), "f8mi_cast_dynamic_pair");
+        }
+    }
+
     // a [m][k] times bt [n][k] in the layout, both contracting over kc (before padding)
     at::Tensor gemm(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& bt, const at::Tensor& sb, int layout, int64_t m, int64_t n,
                     int64_t kc, at::ScalarType out, const at::Tensor& bias = {}) const {
@@ -211,8 +245,7 @@ PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         at::Tensor y, x8, x8t, sx, w8, w8t, sw;
         {
             const WithoutGil no_gil;
-            c.cast(x, in, F8MI_E4M3FN, true, kb_fwd, !one_copy && need_dw, kb_dw, x8, x8t, sx);
-            c.cast(w, we, F8MI_E4M3FN, true, kb_fwd, !one_copy && need_dx, kb_dx, w8, w8t, sw);
+            c.cast_two({x, in, !one_copy && need_dw, kb_fwd, kb_dw, x8, x8t, sx}, {w, we, !one_copy && need_dx, kb_fwd, kb_dx, w8, w8t, sw});
             y = c.gemm(x8, sx, w8, sw, kb_fwd, x.size(0), w.size(0), x.size(1), x.scalar_type());
         }
         if (one_copy) return wrap_all(y, x8, w8, sx, sw);
@@ -334,6 +367,9 @@ PyObject* load(PyObject*, PyObject* args) {
     get(L.linear_few_rows, "f8mi_linear_few_rows");
     get(L.last_error, "f8mi_last_error");
     get(L.gemm_plan, "f8mi_gemm_plan");
+    // (a library may be without these: the calls they stand for are made one by one then)
+    L.cast_dynamic_pair = reinterpret_cast<decltype(L.cast_dynamic_pair)>(dlsym(h, "f8mi_cast_dynamic_pair"));
+    L.cast_delayed_pair = reinterpret_cast<decltype(L.cast_delayed_pair)>(dlsym(h, "f8mi_cast_delayed_pair"));
     if (missing) {
         L.gemm_plan = nullptr;
         return PyErr_Format(PyExc_ImportError, "%s does not export %s", path, missing);

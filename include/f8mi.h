@@ -243,6 +243,24 @@ int f8mi_cast_dynamic_resident(const void* x, int64_t rows, int64_t cols, int64_
                                float* scale_dev, uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout,
                                uint32_t wait_ticks, void* stream);
 
+/* One tensor of a call that casts two: the arguments of f8mi_cast_dynamic (scale_dev: written; amax_dev unused) or of
+ * f8mi_cast_delayed (scale_dev: read). */
+typedef struct f8mi_cast_job {
+    const void* x;
+    int64_t rows, cols, ld;
+    float* scale_dev;
+    uint8_t* out;
+    uint8_t* out_t;
+    float* amax_dev;
+    int in_dtype, out_layout, out_t_layout;
+} f8mi_cast_job;
+
+/* f8mi_cast_dynamic of `a`, then of `b`, both to e4m3: the same bits, in one launch where the chip holds both (at most 1024 tiles
+ * together), in two instead of three or four where one is larger than that.  Everything else is the two calls. */
+int f8mi_cast_dynamic_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream);
+/* f8mi_cast_delayed of `a`, then of `b`, both to e4m3, in one launch up to 2048 tiles together. */
+int f8mi_cast_delayed_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream);
+
 /* A whole linear of at most 16 rows and F8MI_FEW_ROWS_ELEMS activations in one kernel: c[m][n] = sum_k x8[m][k] * w[n][k]
  * / (scale_x * scale_w) (+ bias[n]) with x8 the saturated e4m3 cast of x, which every workgroup makes for itself.  The same
  * bits as f8mi_cast_dynamic (scale_x_dev null) or f8mi_cast_layout (scale_x_dev given, product in product_dtype) followed by

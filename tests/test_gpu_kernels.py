@@ -616,6 +616,54 @@ def test_cast_dynamic_resident_on_several_streams_and_what_it_refuses(nat):
         assert torch.equal(q.view(torch.uint8), nat.cast(xs[0], sq, torch.float8_e4m3fn)[0].view(torch.uint8))
 
 
+# Two tensors in one call: tiny, tiles of 64 and of 128 rows, the most that one launch takes together (1024 tiles, delayed 2048) and one row
+# more, one or both too large for it, ragged and row-strided.
+@pytest.mark.parametrize("dts", ["bf16 bf16", "fp16 fp16", "fp32 fp32", "bf16 fp32", "fp16 fp32", "fp32 bf16"])
+@pytest.mark.parametrize("shapes", [((1, 1), (1, 1)), ((64, 128), (65, 129)), ((512, 1024), (1024, 1024)), ((2048, 2048), (6144, 2048)), ((2049, 2048), (6144, 2048)),
+                                    ((8192, 2048), (8193, 1024)), ((8192, 4096), (300, 4096)), ((4099, 4097), (1001, 4097)), ((4099, 4096), (4480, 4096))])
+def test_cast_of_two_tensors_equals_two_casts(nat, dts, shapes):
+    import ctypes as C
+
+    class Job(C.Structure):
+        _fields_ = ([("x", C.c_void_p)] + [(f, C.c_int64) for f in ("rows", "cols", "ld")] + [(f, C.c_void_p) for f in ("scale", "out", "out_t", "amax")] +
+                    [(f, C.c_int) for f in ("dtype", "layout", "layout_t")])
+
+    f8dt, tdts = torch.float8_e4m3fn, [TORCH_DT[d] for d in dts.split()]
+    base = [heavy(s, t, 40 + i).to(DEV) for i, (s, t) in enumerate(zip(shapes, tdts))]
+    nan = [x.clone() for x in base]
+    nan[1].view(-1)[-1] = float("nan")
+    odd = [torch.zeros(r, c + 5, device=DEV, dtype=t)[:, 3:c + 3].copy_(x) for (r, c), t, x in zip(shapes, tdts, base)]
+    for xs in (base, nan, odd):
+        for layout, both in ((0, False), (nat.KBLOCK_PAD, True)):
+            for delayed in (False, True):
+                scales = [torch.tensor([s], device=DEV) if delayed else torch.zeros((), device=DEV) for s in (3.0, 700.0)]
+                amaxes, outs, want = [torch.full((1,), -1.0, device=DEV) for _ in xs], [], []
+                jobs = (Job * 2)()
+                for x, s, a, job in zip(xs, scales, amaxes, jobs):
+                    wa = torch.zeros((1,), device=DEV)
+                    if delayed:
+                        w = nat.cast(x, s, f8dt, product_dtype=torch.float32, want_out_t=both, amax_out=wa, out_kblock=layout, out_t_kblock=layout)
+                        want.append((*w, s, wa))
+                    else:
+                        ws = nat.amax_scale(x, f8dt, want_amax=False)[1]
+                        want.append((*nat.cast(x, ws, f8dt, want_out_t=both, out_kblock=layout, out_t_kblock=layout), ws, a))
+                    o = [torch.zeros_like(t.view(torch.uint8)) if t is not None else None for t in want[-1][:2]]
+                    outs.append(o)
+                    job.x, job.rows, job.cols, job.ld, job.dtype = x.data_ptr(), *x.shape, x.stride(0), nat._DT[x.dtype]
+                    job.scale, job.amax, job.layout, job.layout_t = s.data_ptr(), a.data_ptr(), layout, layout
+                    job.out, job.out_t = o[0].data_ptr(), o[1].data_ptr() if both else None
+                if delayed:
+                    rc = nat.lib().f8mi_cast_delayed_pair(C.byref(jobs[0]), C.byref(jobs[1]), nat.delayed_workspace(xs[0].device).data_ptr(), nat._stream(xs[0]))
+                else:
+                    rc = nat.lib().f8mi_cast_dynamic_pair(C.byref(jobs[0]), C.byref(jobs[1]), nat.workspace(xs[0].device).data_ptr(), nat._stream(xs[0]))
+                assert rc == 0, nat.lib().f8mi_last_error()
+                for (w, wt, ws, wa), o, s, a in zip(want, outs, scales, amaxes):
+                    assert same_bytes_mod_nan_sign(fp8_bytes(o[0]), fp8_bytes(w)), (dts, shapes, layout, delayed)
+                    assert not both or same_bytes_mod_nan_sign(fp8_bytes(o[1]), fp8_bytes(wt))
+                    assert torch.equal(s, ws) or (torch.isnan(s).all() and torch.isnan(ws).all())
+                    assert torch.equal(a, wa) or (torch.isnan(a).all() and torch.isnan(wa).all())
+
+
 def _rand_fp8(shape, tdt, seed, scale=1.0):
     g = torch.Generator().manual_seed(seed)
     v = torch.randn(shape, generator=g) * scale
