@@ -160,6 +160,7 @@ __device__ __forceinline__ uint4 load_nt16(const void* p) {
 typedef u32x4 u32x4_any __attribute__((aligned(1)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef u32x2 u32x2_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
 __device__ __forceinline__ uint4 load_nt16_any(const void* p) {
     u32x4 v = __builtin_nontemporal_load((const u32x4_any*)p);
     return make_uint4(v.x, v.y, v.z, v.w);

@@ -55,26 +55,30 @@ __device__ __forceinline__ float acc_read(float a) {
 // every lane holds 8 neighbouring columns (lq even: columns 4 lq .. 4 lq + 7 of tile 2p; lq odd: columns
 // 4 (lq - 1) .. + 7 of tile 2p + 1) and one 16-byte store per lane writes 64 contiguous bytes of 16 rows.
 // (Staging the tile through LDS for 256-byte row segments takes the same time and needs the slabs to be free.)
-template <int C_DT>
+// ODD_ROWS: rows of C start at odd multiples of two bytes too (see ShiftedRows); a piece is then stored behind the next one.
+template <int C_DT, bool ODD_ROWS>
 struct Epilogue16 {
     int M, N, c_vec_ok, lq, row0, col0, wcol0;
-    bool interior;   // the whole 256 x 256 tile lies inside C and rows of C take 16-byte stores (the same for every lane)
+    bool whole, interior;  // the 256 x 256 tile lies inside C; and its rows take 16-byte stores as they are (the same for every lane)
     uint16_t* base;  // of the lane's first piece: a piece's address is this plus an offset that is the same for every lane
     float inv;
     int64_t ldc;
     void* C;
     const void* bias;
+    ShiftedRows rows_shifted;
     float bv[8][4];
 
     __device__ __forceinline__ Epilogue16(int m0, int n0, int M_, int N_, float inv_, void* C_, int64_t ldc_, const void* bias_,
                                           int c_vec_ok_)
-        : M(M_), N(N_), c_vec_ok(c_vec_ok_), inv(inv_), ldc(ldc_), C(C_), bias(bias_) {
+        : M(M_), N(N_), c_vec_ok(c_vec_ok_), inv(inv_), ldc(ldc_), C(C_), bias(bias_),
+          rows_shifted(C_, ldc_, m0 + (int)(threadIdx.x >> 7) * 128 + (int)(threadIdx.x & 15)) {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         lq = lane >> 4;
         wcol0 = n0 + (wave & 1) * 128;
         row0 = m0 + (wave >> 1) * 128 + (lane & 15);
         col0 = wcol0 + (lq & 1) * 16 + (lq >> 1) * 8;  // of the lane's 8 columns in the first pair of tiles
-        interior = c_vec_ok && m0 + 256 <= M && n0 + 256 <= N;
+        whole = m0 + 256 <= M && n0 + 256 <= N;
+        interior = c_vec_ok && whole;
         base = (uint16_t*)C + (int64_t)row0 * ldc + col0;
     }
 
@@ -89,7 +93,17 @@ struct Epilogue16 {
         }
     }
 
-    // rows ti*16 .. +15, columns tp*32 .. +31 of the wave's quarter (C_DT: bf16 or fp16); every lane must call it
+    __device__ __forceinline__ void store_held(int ti, int tp) {
+        uint16_t* dst = base + ((int64_t)(ti * 16) * ldc + tp * 32);
+        if (whole) rows_shifted.store(dst, true, tp == 0, tp == 3, 0, 0, M, N);
+        else rows_shifted.store(dst, false, tp == 0, tp == 3, row0 + ti * 16, col0 + tp * 32, M, N);
+    }
+    __device__ __forceinline__ void finish() {  // behind the last piece
+        if constexpr (ODD_ROWS) store_held(7, 3);
+    }
+
+    // rows ti*16 .. +15, columns tp*32 .. +31 of the wave's quarter (C_DT: bf16 or fp16); every lane must call it; pieces of a row of
+    // tiles from left to right, rows from the top
     __device__ __forceinline__ void piece(v4f (&acc)[8][8], int ti, int tp) {
         const int te = 2 * tp, to = 2 * tp + 1;
         float e[4], o[4];
@@ -103,6 +117,12 @@ struct Epilogue16 {
         const uint32_t y1 = pack2<C_DT>(o[2] * inv + bv[to][2], o[3] * inv + bv[to][3]);
         const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
         const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
+        if constexpr (ODD_ROWS) {
+            if (tp > 0) store_held(ti, tp - 1);
+            else if (ti > 0) store_held(ti - 1, 3);
+            rows_shifted.hold(make_uint4(s0[0], s1[0], s0[1], s1[1]));
+            return;
+        }
         const int row = row0 + ti * 16, col = col0 + tp * 32;
         // A tile inside C checks nothing: one scalar branch instead of the per-lane comparisons, the address one vector
         // instruction (the lane's base plus an offset that is the same for all lanes), and the element-wise tail -- 60 of
@@ -172,7 +192,7 @@ __device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[8][8], int m0, in
 // are built with ds_read_b64_tr_b8.  For such an operand lda / ldb is the byte distance between contraction
 // rows (64 when k-blocked over `rows`, the row stride when row-major) and a_unit / b_unit the distance between
 // blocks of 64 rows (contraction length * 64 when k-blocked, 64 when row-major).
-template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR>
+template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS>
 __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
     int M, int N, int K, const float* __restrict__ sa_dev, const float* __restrict__ sb_dev, void* __restrict__ C,
@@ -360,7 +380,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     // and the accumulators start from zero).
     int a_slab = 0;  // slab of A of this step; step t+2 goes to the slab before it in the rotation
     constexpr bool EPI16 = C_DT != F8MI_FP32;
-    Epilogue16<EPI16 ? C_DT : F8MI_BF16> epi(m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
+    Epilogue16<EPI16 ? C_DT : F8MI_BF16, ODD_ROWS> epi(m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
     auto step = [&](auto parity, auto mode) __attribute__((always_inline)) {
         constexpr int P = decltype(parity)::value;
         constexpr bool FIRST = decltype(mode)::value == 3;
@@ -442,48 +462,50 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     if constexpr (EPI16) {
 #pragma unroll
         for (int tp = 0; tp < 4; tp++) epi.piece(acc, 7, tp);
+        epi.finish();
     } else {
         store_c_tile16_fp32(acc, m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
     }
 }
 
-template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR>
+template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS>
 static int launch16_4(dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt, int64_t ldb,
                       int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc,
                       const void* bias, int tiles_m, int tiles_n, int c_vec_ok) {
     static std::atomic<uint64_t> lds_allowed{0};
-    auto kern = gemm_nt_dma16_kernel<AF, BF, C_DT, ODD, A_TR, B_TR>;
+    auto kern = gemm_nt_dma16_kernel<AF, BF, C_DT, ODD, A_TR, B_TR, ODD_ROWS>;
     if (int rc = allow_big_lds(kern, DMA16_LDS, lds_allowed)) return rc;
     hipLaunchKernelGGL(kern, g, dim3(GEMM_THREADS), DMA16_LDS, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C,
                        ldc, bias, tiles_m, tiles_n, c_vec_ok);
     return check_hip(hipGetLastError(), "gemm (LDS-DMA, 16x16x128) kernel launch");
 }
 
-template <int AF, int BF, int C_DT, bool A_TR, bool B_TR>
+template <int AF, int BF, int C_DT, bool A_TR, bool B_TR, bool ODD_ROWS>
 static int launch16_3(dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt, int64_t ldb,
                       int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc,
                       const void* bias, int tiles_m, int tiles_n, int c_vec_ok) {
-    if ((K / 128) & 1) return launch16_4<AF, BF, C_DT, true, A_TR, B_TR>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    return launch16_4<AF, BF, C_DT, false, A_TR, B_TR>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if ((K / 128) & 1) return launch16_4<AF, BF, C_DT, true, A_TR, B_TR, ODD_ROWS>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    return launch16_4<AF, BF, C_DT, false, A_TR, B_TR, ODD_ROWS>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
 }
 
-template <int AF, int BF, bool A_TR, bool B_TR>
+template <int AF, int BF, bool A_TR, bool B_TR, bool ODD_ROWS>
 static int launch16_2(int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt,
                       int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc,
                       const void* bias, int tiles_m, int tiles_n, int c_vec_ok) {
-    if (c_dtype == F8MI_BF16) return launch16_3<AF, BF, F8MI_BF16, A_TR, B_TR>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    if (c_dtype == F8MI_FP16) return launch16_3<AF, BF, F8MI_FP16, A_TR, B_TR>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    return launch16_3<AF, BF, F8MI_FP32, A_TR, B_TR>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (c_dtype == F8MI_BF16) return launch16_3<AF, BF, F8MI_BF16, A_TR, B_TR, ODD_ROWS>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (c_dtype == F8MI_FP16) return launch16_3<AF, BF, F8MI_FP16, A_TR, B_TR, ODD_ROWS>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if constexpr (ODD_ROWS) { set_error("gemm: fp32 rows are never at odd multiples of two bytes"); return F8MI_ERR_INVALID_ARG; }
+    else return launch16_3<AF, BF, F8MI_FP32, A_TR, B_TR, false>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
 }
 
-template <bool A_TR, bool B_TR>
+template <bool A_TR, bool B_TR, bool ODD_ROWS = false>
 static int launch_gemm_dma16_t(int a_fmt, int b_fmt, int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
                       const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb,
                       void* C, int64_t ldc, const void* bias, int tiles_m, int tiles_n, int c_vec_ok) {
-    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E4M3FN) return launch16_2<0, 0, A_TR, B_TR>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    if (a_fmt == F8MI_E5M2 && b_fmt == F8MI_E4M3FN) return launch16_2<1, 0, A_TR, B_TR>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E5M2) return launch16_2<0, 1, A_TR, B_TR>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    return launch16_2<1, 1, A_TR, B_TR>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E4M3FN) return launch16_2<0, 0, A_TR, B_TR, ODD_ROWS>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (a_fmt == F8MI_E5M2 && b_fmt == F8MI_E4M3FN) return launch16_2<1, 0, A_TR, B_TR, ODD_ROWS>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E5M2) return launch16_2<0, 1, A_TR, B_TR, ODD_ROWS>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    return launch16_2<1, 1, A_TR, B_TR, ODD_ROWS>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
 }
 
 }  // namespace f8mi

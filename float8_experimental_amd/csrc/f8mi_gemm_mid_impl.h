@@ -81,7 +81,8 @@ __device__ __forceinline__ uint32_t mid_tr_voff(int instr, int64_t ld, int64_t u
     return (uint32_t)(row * ld + blk * unit) + (c & 3) * 16;
 }
 
-template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR>
+// ODD_ROWS: rows of C start at odd multiples of two bytes too (see ShiftedRows); a piece is then stored behind the next one.
+template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR, bool ODD_ROWS>
 __global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
     const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
     int M, int N, int K, const float* sa_dev, const float* sb_dev, void* __restrict__ C,
@@ -225,8 +226,16 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
     // even ones of the second, which turns a lane's 4 + 4 columns of two tiles into 8 neighbouring columns of one (lq
     // even: columns 4 lq .. + 7 of tile 2p, lq odd: 4 (lq - 1) .. + 7 of tile 2p + 1): one 16-byte store per lane, 64
     // contiguous bytes per row and instruction.
-    const bool interior = c_vec_ok && m0 + MID_TILE_M <= M && n0 + Cfg::TILE_N <= N;  // the same for every lane: nothing to check
+    ShiftedRows rows_shifted(C, ldc, m0 + wm * 64 + lm);
+    const bool whole = m0 + MID_TILE_M <= M && n0 + Cfg::TILE_N <= N;
+    const bool interior = c_vec_ok && whole;  // the same for every lane: nothing to check
     const int col_l = wcol0 + (lq & 1) * 16 + (lq >> 1) * 8;
+    auto store_held = [&](int ti, int tp) __attribute__((always_inline)) {
+        const int row = m0 + wm * 64 + ti * 16 + lm, col = col_l + tp * 32;
+        uint16_t* dst = (uint16_t*)C + (int64_t)row * ldc + col;
+        if (whole) rows_shifted.store(dst, true, tp == 0, tp == TJ / 2 - 1, 0, 0, M, N);
+        else rows_shifted.store(dst, false, tp == 0, tp == TJ / 2 - 1, row, col, M, N);
+    };
     auto store_piece = [&](int ti, int tp) __attribute__((always_inline)) {
         if constexpr (C_DT != F8MI_FP32) {
             const int te = 2 * tp, to = 2 * tp + 1;
@@ -236,6 +245,12 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
             const uint32_t y1 = pack2<C_DT>(acc[to][ti][2] * inv + bv[to][2], acc[to][ti][3] * inv + bv[to][3]);
             const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);  // every lane takes part
             const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
+            if constexpr (ODD_ROWS) {
+                if (tp > 0) store_held(ti, tp - 1);
+                else if (ti > 0) store_held(ti - 1, TJ / 2 - 1);
+                rows_shifted.hold(make_uint4(s0[0], s1[0], s0[1], s1[1]));
+                return;
+            }
             const int row = m0 + wm * 64 + ti * 16 + lm, col = col_l + tp * 32;
             uint16_t* dst = (uint16_t*)C + (int64_t)row * ldc + col;
             if (__builtin_expect(interior, 1)) {
@@ -341,15 +356,16 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
     } else {
 #pragma unroll
         for (int tp = 0; tp < TJ / 2; tp++) store_piece(3, tp);
+        if constexpr (ODD_ROWS) store_held(3, TJ / 2 - 1);
     }
 }
 
-template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR>
+template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR, bool ODD_ROWS>
 static int launch_mid4(hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt, int64_t ldb,
                        int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc, const void* bias,
                        int c_vec_ok, int k_splits) {
     static std::atomic<uint64_t> lds_allowed{0};
-    auto kern = gemm_mid_kernel<AF, BF, C_DT, TJ, A_TR, B_TR>;
+    auto kern = gemm_mid_kernel<AF, BF, C_DT, TJ, A_TR, B_TR, ODD_ROWS>;
     if (int rc = allow_big_lds(kern, MidCfg<TJ>::LDS, lds_allowed)) return rc;
     const int tiles_m = (M + MID_TILE_M - 1) / MID_TILE_M, tiles_n = (N + MidCfg<TJ>::TILE_N - 1) / MidCfg<TJ>::TILE_N;
     hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n), (unsigned)k_splits), dim3(GEMM_THREADS), MidCfg<TJ>::LDS, stream, A, lda, a_unit,
@@ -357,31 +373,32 @@ static int launch_mid4(hipStream_t stream, const uint8_t* A, int64_t lda, int64_
     return check_hip(hipGetLastError(), "gemm (128-row tiles) kernel launch");
 }
 
-template <int AF, int BF, int C_DT, bool A_TR, bool B_TR>
+template <int AF, int BF, int C_DT, bool A_TR, bool B_TR, bool ODD_ROWS>
 static int launch_mid3(bool wide, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt, int64_t ldb,
                        int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc, const void* bias,
                        int c_vec_ok, int k_splits) {
-    if (wide) return launch_mid4<AF, BF, C_DT, 8, A_TR, B_TR>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
-    return launch_mid4<AF, BF, C_DT, 4, A_TR, B_TR>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
+    if (wide) return launch_mid4<AF, BF, C_DT, 8, A_TR, B_TR, ODD_ROWS>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
+    return launch_mid4<AF, BF, C_DT, 4, A_TR, B_TR, ODD_ROWS>(stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
 }
 
-template <int AF, int BF, bool A_TR, bool B_TR>
+template <int AF, int BF, bool A_TR, bool B_TR, bool ODD_ROWS>
 static int launch_mid2(int c_dtype, bool wide, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt,
                        int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc,
                        const void* bias, int c_vec_ok, int k_splits) {
-    if (c_dtype == F8MI_BF16) return launch_mid3<AF, BF, F8MI_BF16, A_TR, B_TR>(wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
-    if (c_dtype == F8MI_FP16) return launch_mid3<AF, BF, F8MI_FP16, A_TR, B_TR>(wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
-    return launch_mid3<AF, BF, F8MI_FP32, A_TR, B_TR>(wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
+    if (c_dtype == F8MI_BF16) return launch_mid3<AF, BF, F8MI_BF16, A_TR, B_TR, ODD_ROWS>(wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
+    if (c_dtype == F8MI_FP16) return launch_mid3<AF, BF, F8MI_FP16, A_TR, B_TR, ODD_ROWS>(wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
+    if constexpr (ODD_ROWS) { set_error("gemm: fp32 rows are never at odd multiples of two bytes"); return F8MI_ERR_INVALID_ARG; }
+    else return launch_mid3<AF, BF, F8MI_FP32, A_TR, B_TR, false>(wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
 }
 
-template <bool A_TR, bool B_TR>
+template <bool A_TR, bool B_TR, bool ODD_ROWS = false>
 static int launch_mid1(int a_fmt, int b_fmt, int c_dtype, bool wide, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
                        const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C,
                        int64_t ldc, const void* bias, int c_vec_ok, int k_splits) {
-    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E4M3FN) return launch_mid2<0, 0, A_TR, B_TR>(c_dtype, wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
-    if (a_fmt == F8MI_E5M2 && b_fmt == F8MI_E4M3FN) return launch_mid2<1, 0, A_TR, B_TR>(c_dtype, wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
-    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E5M2) return launch_mid2<0, 1, A_TR, B_TR>(c_dtype, wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
-    return launch_mid2<1, 1, A_TR, B_TR>(c_dtype, wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
+    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E4M3FN) return launch_mid2<0, 0, A_TR, B_TR, ODD_ROWS>(c_dtype, wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
+    if (a_fmt == F8MI_E5M2 && b_fmt == F8MI_E4M3FN) return launch_mid2<1, 0, A_TR, B_TR, ODD_ROWS>(c_dtype, wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
+    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E5M2) return launch_mid2<0, 1, A_TR, B_TR, ODD_ROWS>(c_dtype, wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
+    return launch_mid2<1, 1, A_TR, B_TR, ODD_ROWS>(c_dtype, wide, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, c_vec_ok, k_splits);
 }
 
 }  // namespace f8mi

@@ -75,6 +75,61 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     }
 }
 
+// Stores of 2-byte outputs whose rows do not all start at a multiple of four bytes (an odd row pitch): the memory system takes a 16-byte
+// store apart unless it starts at one (4096 rows, 11007 columns over 4224: 151 us at pitches 11008, 11006 and 11004, 178 at 11007, now 157;
+// 2048 x 4095 over 4096 in 128-row tiles: 33 at an even pitch, 36 at this one).  A lane of such a row stores one column further to the left instead, its neighbour's last column and its own first seven.
+// In kernels of their own (ODD_ROWS, operands as they are): inside the others, not even taken, the code cost products of 2048 x 4096 x
+// 4096 between other kernels 2 us each.
+// Lanes hold 8 neighbouring columns of one row, the quarters lane / 16 = 0, 2, 1, 3 of a wave 32 of them one behind the other; the
+// pieces of 32 columns of one row are stored from left to right.
+inline bool rows_at_odd_addresses(const void* C, int64_t ldc, int c_dtype) { return c_dtype != F8MI_FP32 && ((ldc & 1) || ((uintptr_t)C & 2)); }
+struct ShiftedRows {
+    int shifted;      // 1: this lane's rows (16 apart) need it
+    uint32_t sel;     // bytes of {a word, the one before it} that make a stored word
+    int from;         // ds_bpermute address of the lane that holds the 8 columns before
+    uint4 held;       // the piece to be stored next
+    uint32_t prev;    // the last word before it
+
+    __device__ __forceinline__ ShiftedRows(const void* C, int64_t ldc, int row) {
+        const int lane = threadIdx.x & 63, lq = lane >> 4;
+        shifted = (((uintptr_t)C >> 1) + (uint64_t)row * (uint64_t)ldc) & 1;
+        sel = shifted ? 0x05040302u : 0x07060504u;
+        from = 4 * (lane + (lq == 0 ? 48 : lq == 1 ? 16 : -32));
+        held = make_uint4(0u, 0u, 0u, 0u);
+        prev = 0u;
+    }
+    // The lane's columns col .. + 7 of `row`, at dst, in two halves so that the exchange between lanes has the time of the next piece:
+    // `hold` takes them, `store` writes what is held.  Every lane takes part.  whole: row and columns lie inside C in every lane.
+    __device__ __forceinline__ void hold(uint4 w) {
+        const int lq = (threadIdx.x & 63) >> 4;
+        prev = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)(lq == 3 ? held.w : w.w));
+        held = w;
+    }
+    __device__ __forceinline__ void store(uint16_t* dst, bool whole, bool first, bool last, int row, int col, int M, int N) const {
+        const int lq = (threadIdx.x & 63) >> 4;
+        const uint32_t d0 = __builtin_amdgcn_perm(held.x, prev, sel), d1 = __builtin_amdgcn_perm(held.y, held.x, sel);
+        const uint32_t d2 = __builtin_amdgcn_perm(held.z, held.y, sel), d3 = __builtin_amdgcn_perm(held.w, held.z, sel);
+        const bool no_left = first && lq == 0 && shifted;  // the column before belongs to another wave
+        if (!whole && (row >= M || col >= N)) return;
+        if (!no_left && (whole || col + 8 - shifted <= N)) {
+            store16_any(dst - shifted, make_uint4(d0, d1, d2, d3));
+        } else if (no_left && (whole || col + 7 <= N)) {
+            dst[0] = (uint16_t)held.x;
+            store8_any(dst + 1, d1, d2);
+            *(u32_any*)(dst + 5) = d3;
+        } else {
+            const uint32_t v[4] = {held.x, held.y, held.z, held.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (col + i < N) dst[i] = (uint16_t)(v[i >> 1] >> (16 * (i & 1)));
+            if (shifted && !no_left) dst[-1] = (uint16_t)d0;
+            return;
+        }
+        // nobody to the right takes the last column
+        if (shifted && ((last && lq == 3) || (!whole && col + 8 == N)) && (whole || col + 8 <= N)) dst[7] = (uint16_t)(held.w >> 16);
+    }
+};
+
 // Scales a workgroup's 256 x 256 accumulators by 1 / (sa * sb), adds the bias, converts and writes C.
 // acc[tj][ti] is the 32 x 32 tile (row block ti, column block tj) of this wave's 128 x 128 quarter
 // as left by MFMA(first = Bt rows, second = A rows): lane holds row lane%32 and columns
@@ -184,6 +239,13 @@ static int allow_big_lds(K kern, int bytes, std::atomic<uint64_t>& done_mask) {
     return 0;
 }
 
+// Both for 2-byte outputs with rows at odd multiples of two bytes (f8mi_gemm_dma16_odd.hip, f8mi_gemm_mid_odd.hip).
+int launch_gemm_mid_odd(int a_fmt, int b_fmt, int c_dtype, bool wide, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
+                        const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C,
+                        int64_t ldc, const void* bias, int c_vec_ok);
+int launch_gemm_dma16_odd(int a_fmt, int b_fmt, int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
+                          const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb,
+                          void* C, int64_t ldc, const void* bias, int tiles_m, int tiles_n, int c_vec_ok);
 // The 16x16x128 kernel with Bt (nt) or both operands (tt) given transposed: memory holds [contraction][rows];
 // lda / ldb = bytes between contraction rows, a_unit / b_unit = bytes between blocks of 64 rows.
 // 128-row-tile kernels (f8mi_gemm_mid_impl.h) for outputs of few 256 x 256 tiles: K % 128 == 0, aligned operands.

@@ -725,6 +725,29 @@ def test_gemm_dma_kernel_shapes(nat, m, n, k, out_dt):
 # Few rows (m <= 256, k % 128 == 0, aligned): the kernel that streams Bt straight into the matrix cores and splits k
 # over the eight waves of a workgroup.  m around the 16-row tile edges, n ragged against the 32-column
 # workgroups, k from one step (seven idle waves) over nine (uneven split) to a long one.
+# Rows of C that start at odd multiples of two bytes (an odd pitch, or a C that starts at one): every column remainder of a lane's eight
+# and of a wave's 128, in tiles of 128 x 128, 128 x 256 and 256 x 256, against the same product in rows at multiples of four bytes.
+@pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,k,n", [(300, 384, n) for n in (1, 7, 8, 9, 63, 121, 127, 128, 129, 135, 255)] +
+                         [(2100, 512, n) for n in (2041, 2049)] + [(4099, 384, n) for n in (4611, 4625, 4735)] + [(8192, 512, 4095)])
+def test_gemm_rows_of_c_at_odd_addresses(nat, m, k, n, out_dt):
+    a, bt = (_rand_fp8((k // 64, rows, 64), torch.float8_e4m3fn, 50 + i, 4.0).to(DEV) for i, rows in enumerate((m, n)))
+    one, code = torch.ones((), device=DEV), nat._DT[out_dt]
+
+    def product(pitch, start):
+        buf = torch.full((m * pitch + start + 16,), 7.0, device=DEV, dtype=out_dt)
+        rc = nat.lib().f8mi_gemm_nt_kb(a.data_ptr(), 0, bt.data_ptr(), 0, m, n, k, one.data_ptr(), one.data_ptr(), buf.data_ptr() + 2 * start, code, pitch, None,
+                                       nat._stream(one))
+        assert rc == 0, nat.lib().f8mi_last_error()
+        c = buf[start:start + m * pitch].view(m, pitch)
+        assert (buf[:start] == 7).all() and (buf[start + m * pitch:] == 7).all() and (c[:, n:] == 7).all()
+        return c[:, :n]
+
+    want = product((n + 1) // 2 * 2, 0)
+    for pitch, start in {(n | 1, 0), (n | 1, 1), ((n + 1) // 2 * 2, 1), ((n + 4) | 1, 3)}:
+        assert torch.equal(product(pitch, start), want), (pitch, start)
+
+
 @pytest.mark.parametrize("m", [1, 5, 16, 17, 32, 33, 64, 65, 100, 128, 129, 200, 256])
 @pytest.mark.parametrize("n,k", [(7, 128), (32, 256), (200, 1152), (1000, 1024), (96, 8192)])
 def test_gemm_few_rows_shapes(nat, m, n, k):

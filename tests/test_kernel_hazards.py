@@ -14,7 +14,7 @@ import pytest
 
 from float8_experimental_amd import _build
 
-UNITS = ["f8mi_gemm_dma16.hip", "f8mi_gemm_dma16_nt.hip", "f8mi_gemm_dma16_tt.hip"]
+UNITS = ["f8mi_gemm_dma16.hip", "f8mi_gemm_dma16_nt.hip", "f8mi_gemm_dma16_tt.hip", "f8mi_gemm_dma16_odd.hip"]
 MID_UNITS = ["f8mi_gemm_mid.hip", "f8mi_gemm_mid_nt.hip", "f8mi_gemm_mid_tt.hip"]
 MIN_MFMAS = 8        # MFMAs issued after the producing one (each occupies the matrix core for 8 passes of 4 cycles) ...
 MIN_WAIT_STATES = 18  # ... or this many wait states of s_nop between the two
