@@ -309,7 +309,7 @@ def gemm_workspace(dev: torch.device, m: int, k: int, n: int = 0):
     return ws.data_ptr(), GEMM_WORKSPACE_BYTES
 
 
-PLAN_NAMES = {1: "tiles128_split_k", 2: "few_rows", 3: "tiles128", 4: "tiles256", 5: "tiles256_and_128", 6: "tiles256_mfma32",
+PLAN_NAMES = {1: "tiles128_split_k", 2: "few_rows", 3: "tiles128", 4: "tiles256", 5: "tiles256_and_128", 6: "tiles256_mfma32", 8: "tiles256x224",
               7: "staged"}
 
 

@@ -295,6 +295,18 @@ static RowSplit split_last_round(int64_t tiles_m, int64_t tiles_n, int64_t k) {
     return {rows_large, mid};
 }
 
+// 256 x 224 tiles instead of 256 x 256: where they fill their rounds so much better that less is paid for.  A round of them takes 0.9
+// of one of those.  us, 256 / 224 columns: 2048 x 14336 over 1024: 38.6 / 36.5, over 4096: 98.5 / 90.1, over 8192: 176.7 / 162.1 (448 tiles, 1.75
+// rounds, against 512); 2048 x 28672 over 4096: 188.6 / 174.2; 4096 x 6144 over 4096 (384, 448): 92.4 / 87.0; 5120 x 5120 over 5120: 110.0 /
+// 103.1; 8192 x 5120 over 4096 (640, 736): 136.9 / 131.9.
+constexpr int NARROW_N = 224;
+static bool narrow_tiles_pay(int64_t tiles_m, int64_t n, const RowSplit& split) {
+    const int64_t tiles_n = (n + BN - 1) / BN, narrow = tiles_m * ((n + NARROW_N - 1) / NARROW_N), per_round = 256;
+    const int64_t large = split.rows_large ? split.rows_large * tiles_n : tiles_m * tiles_n;
+    const double cost = (double)((large + per_round - 1) / per_round) + (split.rows_large ? (split.mid == 1 ? 0.4 : 0.65) : 0.0);
+    return narrow <= 0x7fffffff && 0.9 * (double)((narrow + per_round - 1) / per_round) < cost - 0.1;
+}
+
 // Which kernel computes an m x n x k product (codes: include/f8mi.h, F8MI_PLAN_*).  One function for both entry points,
 // so that row-major and k-blocked operands of one shape always take the same kernel and give the same bits.
 //   aligned, K % 128 == 0:  few 128-row tiles, a long k and a workspace (pick_k_splits) -> those tiles with k split over workgroups
@@ -302,11 +314,12 @@ static RowSplit split_last_round(int64_t tiles_m, int64_t tiles_n, int64_t k) {
 //                                                     -> few-row kernel (Bt streamed once per 128 rows, k split over waves)
 //                           up to 256 tiles of 128 x 128 / 128 x 256 -> those
 //                           K >= 384                  -> 256 x 256 tiles, 16x16x128 MFMA, LDS-DMA (the tile rows of a
-//                                                        sparse last round: 128-row tiles, see split_last_round)
+//                                                        sparse last round: 128-row tiles, see split_last_round), or
+//                                                        256 x 224 tiles (see narrow_tiles_pay)
 //   aligned, K % 64 == 0, K >= 384                    -> 256 x 256 tiles, 32x32x64 MFMA, LDS-DMA
 //   anything else (ragged K, unaligned, short K)      -> 256 x 256 tiles, register-staged
 struct GemmPlan { int kind; int parts; int mid; RowSplit split; };
-static GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, bool aligned, int64_t ws_bytes) {
+static GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, bool aligned, int64_t ws_bytes, bool odd_rows_of_c) {
     GemmPlan p{F8MI_PLAN_STAGED, 0, 0, {0, 0}};
     if (aligned) {
         if (const int parts = pick_k_splits(m, n, k, ws_bytes)) {
@@ -320,6 +333,7 @@ static GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, bool aligned, int64_t
         if (k % 128 == 0) {
             const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
             p.split = split_last_round(tiles_m, tiles_n, k);
+            if (!odd_rows_of_c && narrow_tiles_pay(tiles_m, n, p.split)) { p.kind = F8MI_PLAN_TILES256X224; return p; }
             p.kind = p.split.rows_large ? F8MI_PLAN_TILES256_AND_128 : F8MI_PLAN_TILES256;
             p.mid = p.split.mid;
             return p;
@@ -353,7 +367,7 @@ static int launch_transposed(bool a_transposed, int a_fmt, int b_fmt, int c_dtyp
 
 extern "C" int f8mi_gemm_plan(int64_t m, int64_t n, int64_t k, int aligned, int64_t workspace_bytes) {
     if (m <= 0 || n <= 0 || k < 0) return 0;
-    const GemmPlan p = gemm_plan(m, n, k, aligned != 0, workspace_bytes);
+    const GemmPlan p = gemm_plan(m, n, k, aligned != 0, workspace_bytes, n % 2 != 0);
     return p.kind | (p.parts << 8) | (p.mid << 16);
 }
 
@@ -386,7 +400,7 @@ extern "C" int f8mi_gemm_nt_ws(const void* a, int a_fmt, int64_t lda, const void
     const uint8_t* B = (const uint8_t*)bt;
     const int M = (int)m, N = (int)n, K = (int)k;
     const bool ws_ok = workspace && (uintptr_t)workspace % 16 == 0;
-    const GemmPlan plan = gemm_plan(m, n, k, aligned, ws_ok ? workspace_bytes : 0);
+    const GemmPlan plan = gemm_plan(m, n, k, aligned, ws_ok ? workspace_bytes : 0, rows_at_odd_addresses(c, ldc, c_dtype));
     switch (plan.kind) {
         case F8MI_PLAN_TILES128_SPLIT_K:
             return launch_gemm_mid_splitk(a_fmt, b_fmt, c_dtype, plan.mid == 2, plan.parts, (float*)workspace, stream, A, lda, 64, B, ldb, 64, M, N, K,
@@ -402,6 +416,11 @@ extern "C" int f8mi_gemm_nt_ws(const void* a, int a_fmt, int64_t lda, const void
                 return rc;
             return launch_gemm_mid(a_fmt, b_fmt, c_dtype, plan.mid == 2, stream, A + (int64_t)m1 * lda, lda, 64, B, ldb, 64, M - m1, N, K, scale_a_dev,
                                    scale_b_dev, (uint8_t*)c + (int64_t)m1 * ldc * csz, ldc, bias_dev, c_vec_ok);
+        }
+        case F8MI_PLAN_TILES256X224: {
+            const int64_t narrow_n = (n + NARROW_N - 1) / NARROW_N;
+            return launch_gemm_dma16_narrow(a_fmt, b_fmt, c_dtype, dim3((unsigned)(tiles_m * narrow_n)), stream, A, lda, 64, B, ldb, 64, M, N, K, scale_a_dev, scale_b_dev, c, ldc,
+                                            bias_dev, (int)tiles_m, (int)narrow_n, c_vec_ok);
         }
         case F8MI_PLAN_TILES256:
             return launch_gemm_dma16(a_fmt, b_fmt, c_dtype, g, stream, A, lda, 64, B, ldb, 64, M, N, K, scale_a_dev, scale_b_dev, c, ldc, bias_dev, (int)tiles_m, (int)tiles_n, c_vec_ok);
@@ -443,7 +462,7 @@ extern "C" int f8mi_gemm_nt_kb_ws(const void* a, int a_fmt, const void* bt, int 
     const int M = (int)m, N = (int)n, K = (int)k;
     const int64_t a_unit = m * 64, b_unit = n * 64;  // bytes between 64-deep blocks
     const bool ws_ok = workspace && (uintptr_t)workspace % 16 == 0;
-    const GemmPlan plan = gemm_plan(m, n, k, true, ws_ok ? workspace_bytes : 0);
+    const GemmPlan plan = gemm_plan(m, n, k, true, ws_ok ? workspace_bytes : 0, rows_at_odd_addresses(c, ldc, c_dtype));
     switch (plan.kind) {
         case F8MI_PLAN_TILES128_SPLIT_K:
             return launch_gemm_mid_splitk(a_fmt, b_fmt, c_dtype, plan.mid == 2, plan.parts, (float*)workspace, stream, A, 64, a_unit, B, 64, b_unit, M, N, K,
@@ -460,6 +479,11 @@ extern "C" int f8mi_gemm_nt_kb_ws(const void* a, int a_fmt, const void* bt, int 
                 return rc;
             return launch_gemm_mid(a_fmt, b_fmt, c_dtype, plan.mid == 2, stream, A + m1 * 64, 64, a_unit, B, 64, b_unit, (int)(m - m1), N, K, scale_a_dev,
                                    scale_b_dev, (uint8_t*)c + m1 * ldc * csz, ldc, bias_dev, c_vec_ok);
+        }
+        case F8MI_PLAN_TILES256X224: {
+            const int64_t narrow_n = (n + NARROW_N - 1) / NARROW_N;
+            return launch_gemm_dma16_narrow(a_fmt, b_fmt, c_dtype, dim3((unsigned)(tiles_m * narrow_n)), stream, A, 64, a_unit, B, 64, b_unit, M, N, K, scale_a_dev, scale_b_dev, c, ldc,
+                                            bias_dev, (int)tiles_m, (int)narrow_n, c_vec_ok);
         }
         default: break;
     }

@@ -11,7 +11,16 @@ constexpr int SLAB_BYTES = 256 * 128;   // one operand, one step
 constexpr int HALF_BYTES = 256 * 64;    // one 64-deep unit of it
 constexpr int NSLAB_A = 3, NSLAB_B = 2;
 constexpr int DMA16_LDS = (NSLAB_A + NSLAB_B) * SLAB_BYTES;  // 160 KB
-static_assert(DMA16_LDS >= EPI_BYTES, "the C staging tile reuses the slabs");
+
+// TJ = 16-column tiles per wave: 8 -> 256 x 256 workgroup tiles; 7 -> 256 x 224 (see narrow_tiles_pay), operands as they are and rows of
+// C at multiples of four bytes only.
+template <int TJ>
+struct LargeCfg {
+    static constexpr int TILE_N = 32 * TJ;
+    static constexpr int B_HALF = TILE_N * 64;  // one 64-deep unit of a slab of Bt
+    static constexpr int B_SLAB = 2 * B_HALF;
+    static constexpr int LDS = NSLAB_A * SLAB_BYTES + NSLAB_B * B_SLAB;
+};
 
 __device__ __forceinline__ void dma16b(const uint8_t* base, uint32_t voff, uint32_t lds_addr) {
     // M0 carries the LDS address; one wait state between the scalar write of M0 and its use
@@ -56,7 +65,7 @@ __device__ __forceinline__ float acc_read(float a) {
 // 4 (lq - 1) .. + 7 of tile 2p + 1) and one 16-byte store per lane writes 64 contiguous bytes of 16 rows.
 // (Staging the tile through LDS for 256-byte row segments takes the same time and needs the slabs to be free.)
 // ODD_ROWS: rows of C start at odd multiples of two bytes too (see ShiftedRows); a piece is then stored behind the next one.
-template <int C_DT, bool ODD_ROWS>
+template <int C_DT, bool ODD_ROWS, int TJ>
 struct Epilogue16 {
     int M, N, c_vec_ok, lq, row0, col0, wcol0;
     bool whole, interior;  // the 256 x 256 tile lies inside C; and its rows take 16-byte stores as they are (the same for every lane)
@@ -66,7 +75,7 @@ struct Epilogue16 {
     void* C;
     const void* bias;
     ShiftedRows rows_shifted;
-    float bv[8][4];
+    float bv[TJ][4];
 
     __device__ __forceinline__ Epilogue16(int m0, int n0, int M_, int N_, float inv_, void* C_, int64_t ldc_, const void* bias_,
                                           int c_vec_ok_)
@@ -74,17 +83,17 @@ struct Epilogue16 {
           rows_shifted(C_, ldc_, m0 + (int)(threadIdx.x >> 7) * 128 + (int)(threadIdx.x & 15)) {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         lq = lane >> 4;
-        wcol0 = n0 + (wave & 1) * 128;
+        wcol0 = n0 + (wave & 1) * (16 * TJ);
         row0 = m0 + (wave >> 1) * 128 + (lane & 15);
         col0 = wcol0 + (lq & 1) * 16 + (lq >> 1) * 8;  // of the lane's 8 columns in the first pair of tiles
-        whole = m0 + 256 <= M && n0 + 256 <= N;
+        whole = m0 + 256 <= M && n0 + 32 * TJ <= N;
         interior = c_vec_ok && whole;
         base = (uint16_t*)C + (int64_t)row0 * ldc + col0;
     }
 
     __device__ __forceinline__ void load_bias_row() {
 #pragma unroll
-        for (int tj = 0; tj < 8; tj++) {
+        for (int tj = 0; tj < TJ; tj++) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int col = wcol0 + tj * 16 + 4 * lq + r;
@@ -104,7 +113,7 @@ struct Epilogue16 {
 
     // rows ti*16 .. +15, columns tp*32 .. +31 of the wave's quarter (C_DT: bf16 or fp16); every lane must call it; pieces of a row of
     // tiles from left to right, rows from the top
-    __device__ __forceinline__ void piece(v4f (&acc)[8][8], int ti, int tp) {
+    __device__ __forceinline__ void piece(v4f (&acc)[TJ][8], int ti, int tp) {
         const int te = 2 * tp, to = 2 * tp + 1;
         float e[4], o[4];
 #pragma unroll
@@ -146,20 +155,47 @@ struct Epilogue16 {
             }
         }
     }
+
+    // the last column of tiles of an odd number, rows ti*16 .. +15: a lane's own 4 columns, 8 bytes
+    __device__ __forceinline__ void piece_last(v4f (&acc)[TJ][8], int ti) {
+        constexpr int tj = TJ - 1;
+        float e[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) e[r] = acc_read(acc[tj][ti][r]);
+        const uint32_t x0 = pack2<C_DT>(e[0] * inv + bv[tj][0], e[1] * inv + bv[tj][1]);
+        const uint32_t x1 = pack2<C_DT>(e[2] * inv + bv[tj][2], e[3] * inv + bv[tj][3]);
+        const int row = row0 + ti * 16, col = wcol0 + tj * 16 + 4 * lq;
+        uint16_t* dst = (uint16_t*)C + (int64_t)row * ldc + col;
+        if (__builtin_expect(interior, 1)) {
+            store8_any(dst, x0, x1);
+            return;
+        }
+        if (row < M && col < N) {
+            if (c_vec_ok && col + 4 <= N) {
+                store8_any(dst, x0, x1);
+            } else {
+                const uint32_t w[2] = {x0, x1};
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (col + i < N) dst[i] = (uint16_t)((w[i >> 1] >> (16 * (i & 1))) & 0xffffu);
+            }
+        }
+    }
 };
 
 // fp32 outputs: a lane's 4 columns are 16 bytes already
-__device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[8][8], int m0, int n0, int M, int N, float inv,
+template <int TJ>
+__device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[TJ][8], int m0, int n0, int M, int N, float inv,
                                                     void* __restrict__ C, int64_t ldc, const void* __restrict__ bias,
                                                     int c_vec_ok) {
     constexpr int C_DT = F8MI_FP32;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int lm = lane & 15, lq = lane >> 4;
-    const int wrow0 = m0 + wm * 128, wcol0 = n0 + wn * 128;
+    const int wrow0 = m0 + wm * 128, wcol0 = n0 + wn * (16 * TJ);
     float* Cf = (float*)C;
 #pragma unroll
-    for (int tj = 0; tj < 8; tj++) {
+    for (int tj = 0; tj < TJ; tj++) {
         const int col = wcol0 + tj * 16 + 4 * lq;
         float bv[4] = {0.f, 0.f, 0.f, 0.f};
         if (bias) {
@@ -192,11 +228,13 @@ __device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[8][8], int m0, in
 // are built with ds_read_b64_tr_b8.  For such an operand lda / ldb is the byte distance between contraction
 // rows (64 when k-blocked over `rows`, the row stride when row-major) and a_unit / b_unit the distance between
 // blocks of 64 rows (contraction length * 64 when k-blocked, 64 when row-major).
-template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS>
+template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ>
 __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
     int M, int N, int K, const float* __restrict__ sa_dev, const float* __restrict__ sb_dev, void* __restrict__ C,
     int64_t ldc, const void* __restrict__ bias, int tiles_m, int tiles_n, int c_vec_ok) {
+    static_assert(TJ == 8 || (TJ == 7 && !A_TR && !B_TR && !ODD_ROWS), "narrower tiles: operands as they are");
+    using Cfg = LargeCfg<TJ>;
     extern __shared__ __align__(16) uint8_t smem[];
     // lda / ldb: bytes from one operand row to the next; a_unit / b_unit: bytes from one 64-deep unit
     // to the next.  Row-major operands: (row stride, 64); k-blocked [K/64][rows][64]: (64, rows*64).
@@ -236,7 +274,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
         tm = first_m + (lid % width) % gsz;
         tn = (lid % width) / gsz;
     }
-    const int m0 = tm * BM, n0 = tn * BN;
+    const int m0 = tm * BM, n0 = tn * Cfg::TILE_N;
     // 1 / (sa * sb) for the epilogue, fetched now and kept in a scalar register: loaded after the main loop, the two
     // scales were a memory round trip with nothing to hide it
     const float inv = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(
@@ -258,7 +296,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     // Transposed operand: instruction j = wave*8 + d covers contraction rows 4j .. 4j+3 of the slab, 256 bytes
     // (16 slots) each; lane l fetches row 4j + l/16, the slot that belongs at position l%16: (l%16) ^ f(row).
     const uint32_t lds_u32 = (uint32_t)(uintptr_t)smem;
-    uint32_t a_voff[A_TR ? 8 : 4], b_voff[B_TR ? 8 : 4];
+    uint32_t a_voff[A_TR ? 8 : 4], b_voff[B_TR ? 8 : TJ == 8 ? 4 : TJ];
     const uint8_t* a_ptr;  // first byte of the next step to be fetched
     const uint8_t* b_ptr;
     int64_t a_step, b_step;  // bytes from one step's data to the next
@@ -292,12 +330,13 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
         b_ptr = Bt + (int64_t)(n0 / 64) * b_unit;
         b_step = 128 * ldb;
     } else {
+        // 256 rows: as for A; fewer: wave w takes TJ of the 2 TJ instructions of the half w / 2
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int r = (wave * 4 + i) * 16 + (lane >> 2);
+        for (int i = 0; i < (TJ == 8 ? 4 : TJ); i++) {
+            const int r = (TJ == 8 ? wave * 4 + i : (wave & 1) * TJ + i) * 16 + (lane >> 2);
             b_voff[i] = (uint32_t)(min(r, N - 1 - n0) * ldb) + (((lane & 3) ^ (lane >> 5)) << 4);
         }
-        b_ptr = Bt + (int64_t)n0 * ldb;
+        b_ptr = Bt + (int64_t)n0 * ldb + (TJ == 8 ? 0 : (wave >> 1) * b_unit);
         b_step = 2 * b_unit;
     }
     uint32_t a_dst = 0, b_dst = 0;  // LDS address of the slabs being refilled
@@ -309,8 +348,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     };
     auto issue_b = [&](int d) __attribute__((always_inline)) {
         if constexpr (B_TR) dma16b(b_ptr, b_voff[d], b_dst + (wave * 8 + d) * 1024);
-        else dma16b(d < 4 ? b_ptr : b_ptr + b_unit, b_voff[d & 3], b_dst + wave * 4096 + (d >> 2) * HALF_BYTES + (d & 3) * 1024);
-        if (d == 7) b_ptr += b_step;
+        else if constexpr (TJ == 8) dma16b(d < 4 ? b_ptr : b_ptr + b_unit, b_voff[d & 3], b_dst + wave * 4096 + (d >> 2) * HALF_BYTES + (d & 3) * 1024);
+        else dma16b(b_ptr, b_voff[d], b_dst + (wave * TJ + d) * 1024);
+        if (d == TJ - 1) b_ptr += b_step;
     };
 
     // ---- fragment addressing.
@@ -334,7 +374,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
         for (int x = 0; x < 8; x++) b_tr_off[x] = base + ((x ^ (tr_f & 7)) << 4);
     }
     const int a_frag_base = (wm * 128) * 64;
-    const int b_frag_base = (wn * 128) * 64;
+    const int b_frag_base = (wn * (16 * TJ)) * 64 + (fq >> 1) * (Cfg::B_HALF - HALF_BYTES);
     auto frag_a = [&](const uint8_t* slab, int ti) __attribute__((always_inline)) {
         if constexpr (A_TR) {
             return read_frag_tr(slab + a_tr_off[ti]);
@@ -352,9 +392,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
         }
     };
 
-    v4f acc[8][8];  // first written by step 0
+    v4f acc[TJ][8];  // first written by step 0
 
-    v8i fb[2][8];  // [step parity][n tile]
+    v8i fb[2][TJ];  // [step parity][n tile]
     v8i fa[2];     // rolling: group ti multiplies fa[ti & 1] while fa[(ti + 1) & 1] is being fetched
 
     // ---- prologue: steps 0 and 1 (A into slabs 0, 1; Bt into slabs 3, 4), wait for step 0,
@@ -362,16 +402,16 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
 #pragma unroll
     for (int s = 0; s < 2; s++) {
         a_dst = lds_u32 + s * SLAB_BYTES;
-        b_dst = lds_u32 + (NSLAB_A + s) * SLAB_BYTES;
+        b_dst = lds_u32 + NSLAB_A * SLAB_BYTES + s * Cfg::B_SLAB;
 #pragma unroll
         for (int d = 0; d < 8; d++) issue_a(d);
 #pragma unroll
-        for (int d = 0; d < 8; d++) issue_b(d);
+        for (int d = 0; d < TJ; d++) issue_b(d);
     }
-    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + TJ) : "memory");
     lds_barrier();
 #pragma unroll
-    for (int x = 0; x < 8; x++) fb[0][x] = frag_b(smem + NSLAB_A * SLAB_BYTES, x);
+    for (int x = 0; x < TJ; x++) fb[0][x] = frag_b(smem + NSLAB_A * SLAB_BYTES, x);
     fa[0] = frag_a(smem, 0);
     lds_barrier();
 
@@ -380,7 +420,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     // and the accumulators start from zero).
     int a_slab = 0;  // slab of A of this step; step t+2 goes to the slab before it in the rotation
     constexpr bool EPI16 = C_DT != F8MI_FP32;
-    Epilogue16<EPI16 ? C_DT : F8MI_BF16, ODD_ROWS> epi(m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
+    Epilogue16<EPI16 ? C_DT : F8MI_BF16, ODD_ROWS, TJ> epi(m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
     auto step = [&](auto parity, auto mode) __attribute__((always_inline)) {
         constexpr int P = decltype(parity)::value;
         constexpr bool FIRST = decltype(mode)::value == 3;
@@ -389,10 +429,10 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
         const int a_free = a_next + 1 == NSLAB_A ? 0 : a_next + 1;  // held step t-1
         const uint8_t* a_cur = smem + a_slab * SLAB_BYTES;
         const uint8_t* a_nxt = smem + a_next * SLAB_BYTES;
-        const uint8_t* b_nxt = smem + (NSLAB_A + (P ^ 1)) * SLAB_BYTES;
+        const uint8_t* b_nxt = smem + NSLAB_A * SLAB_BYTES + (P ^ 1) * Cfg::B_SLAB;
         if (MODE == 0) {
             a_dst = lds_u32 + a_free * SLAB_BYTES;
-            b_dst = lds_u32 + (NSLAB_A + P) * SLAB_BYTES;  // Bt of this step: already in registers
+            b_dst = lds_u32 + NSLAB_A * SLAB_BYTES + P * Cfg::B_SLAB;  // Bt of this step: already in registers
         }
         // Everything that is not an MFMA sits in a fixed slot between two MFMAs (each keeps the matrix
         // core busy for 32 cycles): one fragment (two 16-byte LDS reads) or one DMA at a time.
@@ -408,23 +448,35 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
                 asm volatile("s_barrier" ::: "memory");  // ... and so have everybody's; no LDS hazard here, so no wait on LDS reads
             }
 #pragma unroll
-            for (int tj = 0; tj < 8; tj++) {
+            for (int tj = 0; tj < TJ; tj++) {
                 if (tj == 0 && ti < 7) fa[(ti + 1) & 1] = frag_a(a_cur, ti + 1);
                 if (tj == 0 && ti == 7 && MODE < 2) fa[0] = frag_a(a_nxt, 0);
-                if (MODE < 2 && ti >= 6 && (tj & 1) == 1) fb[P ^ 1][(ti - 6) * 4 + (tj >> 1)] = frag_b(b_nxt, (ti - 6) * 4 + (tj >> 1));
+                if constexpr (TJ == 8) {
+                    if (MODE < 2 && ti >= 6 && (tj & 1) == 1) fb[P ^ 1][(ti - 6) * 4 + (tj >> 1)] = frag_b(b_nxt, (ti - 6) * 4 + (tj >> 1));
+                } else {  // four of the seven in the last but one row, three in the last
+                    if (MODE < 2 && ti == 6 && (tj == 1 || tj == 3 || tj >= 5)) fb[P ^ 1][tj == 6 ? 3 : tj >> 1] = frag_b(b_nxt, tj == 6 ? 3 : tj >> 1);
+                    if (MODE < 2 && ti == 7 && (tj & 1) == 1) fb[P ^ 1][4 + (tj >> 1)] = frag_b(b_nxt, 4 + (tj >> 1));
+                }
                 if (FIRST) mfma16_first<BF, AF>(acc[tj][ti], fb[P][tj], fa[ti & 1]);
                 else mfma16<BF, AF>(acc[tj][ti], fb[P][tj], fa[ti & 1]);
                 F8MI_SCHED_FENCE();
-                if (MODE == 2 && EPI16 && ti >= 1 && (tj & 1) == 1) {
-                    epi.piece(acc, ti - 1, tj >> 1);
+                // (seven tiles: a place later, and the last one in the row after, for the same distance from the MFMA that wrote it)
+                if (MODE == 2 && EPI16 && ti >= 1 && (TJ == 8 ? (tj & 1) == 1 : tj >= 2 && (tj & 1) == 0)) {
+                    epi.piece(acc, ti - 1, TJ == 8 ? tj >> 1 : (tj >> 1) - 1);
                     F8MI_SCHED_FENCE();
+                }
+                if constexpr (TJ == 7) {
+                    if (MODE == 2 && EPI16 && ti >= 2 && tj == 1) {
+                        epi.piece_last(acc, ti - 2);
+                        F8MI_SCHED_FENCE();
+                    }
                 }
                 if (MODE == 0 && (tj & 3) == 0) {
                     // 16 DMAs over the 64 MFMAs, one after every fourth: A slab first, then Bt.  (Packed into
                     // the first half of the step they cost 3 % more time: the four waves share one load unit.)
                     const int d = ti * 2 + (tj >> 2);
                     if (d < 8) issue_a(d);
-                    else issue_b(d - 8);
+                    else if (d - 8 < TJ) issue_b(d - 8);
                     F8MI_SCHED_FENCE();
                 }
             }
@@ -461,51 +513,55 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     if constexpr (EPI16) {
 #pragma unroll
-        for (int tp = 0; tp < 4; tp++) epi.piece(acc, 7, tp);
+        for (int tp = 0; tp < TJ / 2; tp++) epi.piece(acc, 7, tp);
+        if constexpr (TJ == 7) {
+            epi.piece_last(acc, 6);
+            epi.piece_last(acc, 7);
+        }
         epi.finish();
     } else {
         store_c_tile16_fp32(acc, m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
     }
 }
 
-template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS>
+template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ>
 static int launch16_4(dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt, int64_t ldb,
                       int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc,
                       const void* bias, int tiles_m, int tiles_n, int c_vec_ok) {
     static std::atomic<uint64_t> lds_allowed{0};
-    auto kern = gemm_nt_dma16_kernel<AF, BF, C_DT, ODD, A_TR, B_TR, ODD_ROWS>;
-    if (int rc = allow_big_lds(kern, DMA16_LDS, lds_allowed)) return rc;
-    hipLaunchKernelGGL(kern, g, dim3(GEMM_THREADS), DMA16_LDS, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C,
+    auto kern = gemm_nt_dma16_kernel<AF, BF, C_DT, ODD, A_TR, B_TR, ODD_ROWS, TJ>;
+    if (int rc = allow_big_lds(kern, LargeCfg<TJ>::LDS, lds_allowed)) return rc;
+    hipLaunchKernelGGL(kern, g, dim3(GEMM_THREADS), LargeCfg<TJ>::LDS, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C,
                        ldc, bias, tiles_m, tiles_n, c_vec_ok);
     return check_hip(hipGetLastError(), "gemm (LDS-DMA, 16x16x128) kernel launch");
 }
 
-template <int AF, int BF, int C_DT, bool A_TR, bool B_TR, bool ODD_ROWS>
+template <int AF, int BF, int C_DT, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ>
 static int launch16_3(dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt, int64_t ldb,
                       int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc,
                       const void* bias, int tiles_m, int tiles_n, int c_vec_ok) {
-    if ((K / 128) & 1) return launch16_4<AF, BF, C_DT, true, A_TR, B_TR, ODD_ROWS>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    return launch16_4<AF, BF, C_DT, false, A_TR, B_TR, ODD_ROWS>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if ((K / 128) & 1) return launch16_4<AF, BF, C_DT, true, A_TR, B_TR, ODD_ROWS, TJ>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    return launch16_4<AF, BF, C_DT, false, A_TR, B_TR, ODD_ROWS, TJ>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
 }
 
-template <int AF, int BF, bool A_TR, bool B_TR, bool ODD_ROWS>
+template <int AF, int BF, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ>
 static int launch16_2(int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit, const uint8_t* Bt,
                       int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb, void* C, int64_t ldc,
                       const void* bias, int tiles_m, int tiles_n, int c_vec_ok) {
-    if (c_dtype == F8MI_BF16) return launch16_3<AF, BF, F8MI_BF16, A_TR, B_TR, ODD_ROWS>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    if (c_dtype == F8MI_FP16) return launch16_3<AF, BF, F8MI_FP16, A_TR, B_TR, ODD_ROWS>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (c_dtype == F8MI_BF16) return launch16_3<AF, BF, F8MI_BF16, A_TR, B_TR, ODD_ROWS, TJ>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (c_dtype == F8MI_FP16) return launch16_3<AF, BF, F8MI_FP16, A_TR, B_TR, ODD_ROWS, TJ>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
     if constexpr (ODD_ROWS) { set_error("gemm: fp32 rows are never at odd multiples of two bytes"); return F8MI_ERR_INVALID_ARG; }
-    else return launch16_3<AF, BF, F8MI_FP32, A_TR, B_TR, false>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    else return launch16_3<AF, BF, F8MI_FP32, A_TR, B_TR, false, TJ>(g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
 }
 
-template <bool A_TR, bool B_TR, bool ODD_ROWS = false>
+template <bool A_TR, bool B_TR, bool ODD_ROWS = false, int TJ = 8>
 static int launch_gemm_dma16_t(int a_fmt, int b_fmt, int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
                       const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb,
                       void* C, int64_t ldc, const void* bias, int tiles_m, int tiles_n, int c_vec_ok) {
-    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E4M3FN) return launch16_2<0, 0, A_TR, B_TR, ODD_ROWS>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    if (a_fmt == F8MI_E5M2 && b_fmt == F8MI_E4M3FN) return launch16_2<1, 0, A_TR, B_TR, ODD_ROWS>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E5M2) return launch16_2<0, 1, A_TR, B_TR, ODD_ROWS>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
-    return launch16_2<1, 1, A_TR, B_TR, ODD_ROWS>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E4M3FN) return launch16_2<0, 0, A_TR, B_TR, ODD_ROWS, TJ>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (a_fmt == F8MI_E5M2 && b_fmt == F8MI_E4M3FN) return launch16_2<1, 0, A_TR, B_TR, ODD_ROWS, TJ>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    if (a_fmt == F8MI_E4M3FN && b_fmt == F8MI_E5M2) return launch16_2<0, 1, A_TR, B_TR, ODD_ROWS, TJ>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
+    return launch16_2<1, 1, A_TR, B_TR, ODD_ROWS, TJ>(c_dtype, g, stream, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa, sb, C, ldc, bias, tiles_m, tiles_n, c_vec_ok);
 }
 
 }  // namespace f8mi

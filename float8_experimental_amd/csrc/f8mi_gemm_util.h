@@ -246,6 +246,10 @@ int launch_gemm_mid_odd(int a_fmt, int b_fmt, int c_dtype, bool wide, hipStream_
 int launch_gemm_dma16_odd(int a_fmt, int b_fmt, int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
                           const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb,
                           void* C, int64_t ldc, const void* bias, int tiles_m, int tiles_n, int c_vec_ok);
+// Tiles of 256 x 224 (f8mi_gemm_dma16_narrow.hip), rows of C at multiples of four bytes or fp32.
+int launch_gemm_dma16_narrow(int a_fmt, int b_fmt, int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
+                             const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb,
+                             void* C, int64_t ldc, const void* bias, int tiles_m, int tiles_n, int c_vec_ok);
 // The 16x16x128 kernel with Bt (nt) or both operands (tt) given transposed: memory holds [contraction][rows];
 // lda / ldb = bytes between contraction rows, a_unit / b_unit = bytes between blocks of 64 rows.
 // 128-row-tile kernels (f8mi_gemm_mid_impl.h) for outputs of few 256 x 256 tiles: K % 128 == 0, aligned operands.

@@ -318,6 +318,7 @@ int f8mi_gemm_nt_kb_ws(const void* a, int a_fmt, const void* bt, int b_fmt, int6
 #define F8MI_PLAN_TILES256 4         /* 256 x 256 tiles, 16x16x128 MFMA, operands through LDS-DMA */
 #define F8MI_PLAN_TILES256_AND_128 5 /* the same for the tile rows of whole rounds, 128-row tiles for the rest */
 #define F8MI_PLAN_TILES256_MFMA32 6  /* 256 x 256 tiles, 32x32x64 MFMA (k % 128 == 64) */
+#define F8MI_PLAN_TILES256X224 8     /* 256 x 224 tiles, 16x16x128 MFMA, where they fill whole rounds better */
 #define F8MI_PLAN_STAGED 7           /* 256 x 256 tiles, register-staged (ragged or short k, unaligned operands) */
 int f8mi_gemm_plan(int64_t m, int64_t n, int64_t k, int aligned, int64_t workspace_bytes);
 

@@ -725,6 +725,26 @@ def test_gemm_dma_kernel_shapes(nat, m, n, k, out_dt):
 # Few rows (m <= 256, k % 128 == 0, aligned): the kernel that streams Bt straight into the matrix cores and splits k
 # over the eight waves of a workgroup.  m around the 16-row tile edges, n ragged against the 32-column
 # workgroups, k from one step (seven idle waves) over nine (uneven split) to a long one.
+# Tiles of 256 x 224: whole ones, a last column of tiles of 1, 111, 113 and 223 columns, ragged rows, an odd and an even number of steps,
+# every output type, against 128-row tiles (the same order of additions, hence the same bits) of both ends of the rows.
+@pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(2048, 14336, 512), (2000, 14112 + 2, 384), (2048, 14112 + 112, 384), (1801, 14112 + 114, 640), (2048, 14112 + 222, 512), (2047, 14332, 384)])
+def test_gemm_narrow_tiles_equal_128_row_tiles_bitwise(nat, m, n, k, out_dt):
+    assert nat.gemm_plan(m, n, k) == ("tiles256x224", 0, 0)
+    a, bt = _rand_fp8((m, k), torch.float8_e5m2, 61).to(DEV), _rand_fp8((n, k), torch.float8_e4m3fn, 62).to(DEV)
+    sa, sb = torch.tensor(3.0, device=DEV), torch.tensor(0.37, device=DEV)
+    bias = torch.linspace(-1, 1, n).to(out_dt).to(DEV)
+    for b in (None, bias):
+        buf = torch.full((m + 1, n), 7.0, device=DEV, dtype=out_dt)
+        got = nat.gemm_nt(a, sa, bt, sb, out_dt, bias=b, out=buf[:m])
+        assert (buf[m] == 7).all()
+        for rows in (slice(0, 272), slice(m - 300, m)):
+            for cols in (slice(0, 4096), slice(4096, 8192), slice(8192, 12288), slice(12288, n)):
+                assert nat.gemm_plan(rows.stop - rows.start, cols.stop - cols.start, k)[0] == "tiles128"
+                want = nat.gemm_nt(a[rows], sa, bt[cols], sb, out_dt, bias=None if b is None else b[cols].contiguous())
+                assert torch.equal(got[rows, cols], want), (rows, cols)
+
+
 # Rows of C that start at odd multiples of two bytes (an odd pitch, or a C that starts at one): every column remainder of a lane's eight
 # and of a wave's 128, in tiles of 128 x 128, 128 x 256 and 256 x 256, against the same product in rows at multiples of four bytes.
 @pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float16])
