@@ -91,16 +91,7 @@ struct Epilogue16 {
         base = (uint16_t*)C + (int64_t)row0 * ldc + col0;
     }
 
-    __device__ __forceinline__ void load_bias_row() {
-#pragma unroll
-        for (int tj = 0; tj < TJ; tj++) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int col = wcol0 + tj * 16 + 4 * lq + r;
-                bv[tj][r] = (bias && col < N) ? load_bias<C_DT>(bias, col) : 0.f;
-            }
-        }
-    }
+    __device__ __forceinline__ void load_bias_row() { load_bias_tiles<C_DT, TJ>(bv, bias, wcol0 + 4 * lq, N); }
 
     __device__ __forceinline__ void store_held(int ti, int tp) {
         uint16_t* dst = base + ((int64_t)(ti * 16) * ldc + tp * 32);

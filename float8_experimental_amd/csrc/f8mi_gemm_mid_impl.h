@@ -303,13 +303,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
         // everybody's DMAs of step s+1 have landed and everybody's reads of this step's stage are done
         if constexpr (MODE < 2) mid_wait_barrier<decltype(in_flight)::value * NDMA>();
         if constexpr (MODE == 2) {
-#pragma unroll
-            for (int tj = 0; tj < TJ; tj++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int col = wcol0 + tj * 16 + 4 * lq + e;
-                    bv[tj][e] = (bias && col < N) ? load_bias<C_DT>(bias, col) : 0.f;
-                }
+            load_bias_tiles<C_DT, TJ>(bv, bias, wcol0 + 4 * lq, N);
         }
         F8MI_SCHED_FENCE();
 #pragma unroll

@@ -62,6 +62,24 @@ __device__ __forceinline__ float load_bias(const void* bias, int col) {
     else return ((const float*)bias)[col];
 }
 
+// The bias of the columns col0 + 16 tj + e, zeros without one; columns past the end get the last one's, which nobody stores.  One
+// branch in all: with a test for each element the last step of a 128 x 256 tile began with 64 of them, bias or none (2048 tokens, 4096 -> 14336 with a
+// bias: 96.9 -> 93.5 us; a training step of 2048, 4096 -> 4096: 132 -> 131, of 8192, 4096 -> 14336 twice: 2333 -> 2315).
+template <int C_DT, int TJ>
+__device__ __forceinline__ void load_bias_tiles(float (&bv)[TJ][4], const void* bias, int col0, int N) {
+    if (bias) {
+#pragma unroll
+        for (int tj = 0; tj < TJ; tj++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) bv[tj][e] = load_bias<C_DT>(bias, min(col0 + 16 * tj + e, N - 1));
+    } else {
+#pragma unroll
+        for (int tj = 0; tj < TJ; tj++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) bv[tj][e] = 0.f;
+    }
+}
+
 // two fp32 -> two packed 2-byte outputs (round to nearest even)
 template <int C_DT>
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
