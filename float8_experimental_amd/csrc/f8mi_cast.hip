@@ -561,6 +561,11 @@ static int launch_cast_small(int fmt, hipStream_t stream, const void* x, int64_t
 constexpr int FLAT_THREADS = 1024;
 constexpr int FLAT_UNROLL = 8;  // 16-byte loads in flight per lane of the scan
 constexpr int64_t FLAT_MAX_BYTES = 512 << 10;
+// Past this many bytes the kernel that reads the tensor once (cast_dynamic_resident_kernel) is faster, where the stream has its words:
+// us, this / that: 32 x 4096 (256 KB): 5.5 / 5.8, 48 x 4096: 6.3 / 5.9, 16 x 14336 (448 KB): 7.2 / 6.3, 64 x 4096: 7.3 / 5.9.  Its tiles
+// have 64 rows: with fewer than a quarter of them it is left to this one.
+constexpr int64_t FLAT_BEST_BYTES = 320 << 10;
+constexpr int64_t FLAT_BEST_ROWS = 16;
 
 template <int DT, int FMT>
 __global__ __launch_bounds__(FLAT_THREADS) void cast_dynamic_flat_kernel(const uint8_t* __restrict__ x, uint32_t rows, uint32_t cols,
@@ -954,17 +959,18 @@ extern "C" int f8mi_cast_dynamic(const void* x, int64_t rows, int64_t cols, int6
         if (rc) return rc;
         return f8mi_cast_layout(x, rows, cols, ld, in_dtype, scale_dev, in_dtype, fp8_fmt, out, out_layout, out_t, out_t_layout, nullptr, stream_);
     }
-    if (out && !out_t && cols % 8 == 0 && (ld == cols || rows == 1) && n * (int64_t)esz <= FLAT_MAX_BYTES && out_t_layout >= F8MI_LAYOUT_ROWMAJOR &&
-        out_t_layout <= F8MI_LAYOUT_KBLOCK64_PAD128 && (out_layout == F8MI_LAYOUT_ROWMAJOR || (out_layout == F8MI_LAYOUT_KBLOCK64 && cols % 64 == 0))) {
+    const bool flat = out && !out_t && cols % 8 == 0 && (ld == cols || rows == 1) && n * (int64_t)esz <= FLAT_MAX_BYTES && out_t_layout >= F8MI_LAYOUT_ROWMAJOR &&
+                      out_t_layout <= F8MI_LAYOUT_KBLOCK64_PAD128 && (out_layout == F8MI_LAYOUT_ROWMAJOR || (out_layout == F8MI_LAYOUT_KBLOCK64 && cols % 64 == 0));
+    if (resident_tile_rows(rows, cols) && !(flat && (n * (int64_t)esz <= FLAT_BEST_BYTES || rows < FLAT_BEST_ROWS))) {
+        const int rc = f8mi_cast_dynamic_resident(x, rows, cols, ld, in_dtype, fp8_fmt, scale_dev, out, out_layout, out_t, out_t_layout, EXCHANGE_WAIT_TICKS, stream_);
+        if (rc != F8MI_ERR_UNSUPPORTED) return rc;
+    }
+    if (flat) {
         const int out_kb = out_layout == F8MI_LAYOUT_KBLOCK64;
         ProfScope prof(F8MI_K_CAST, (double)n * (esz + 1), stream);
         if (in_dtype == F8MI_BF16) return launch_cast_flat<F8MI_BF16>(fp8_fmt, stream, x, rows, cols, scale_dev, out, out_kb);
         if (in_dtype == F8MI_FP16) return launch_cast_flat<F8MI_FP16>(fp8_fmt, stream, x, rows, cols, scale_dev, out, out_kb);
         return launch_cast_flat<F8MI_FP32>(fp8_fmt, stream, x, rows, cols, scale_dev, out, out_kb);
-    }
-    if (resident_tile_rows(rows, cols)) {
-        const int rc = f8mi_cast_dynamic_resident(x, rows, cols, ld, in_dtype, fp8_fmt, scale_dev, out, out_layout, out_t, out_t_layout, EXCHANGE_WAIT_TICKS, stream_);
-        if (rc != F8MI_ERR_UNSUPPORTED) return rc;
     }
     // amax pass: per-workgroup maxima into the workspace; the cast's workgroups reduce them and derive the scale
     // themselves (no one-block finalize launch in between), workgroup 0 stores it to *scale_dev

@@ -557,6 +557,27 @@ def test_cast_dynamic_one_copy_equals_amax_scale_then_cast(nat, dt, shape):
                 assert same_bytes_mod_nan_sign(fp8_bytes(o), fp8_bytes(o_want)), (dt, shape, fmt, kb)
 
 
+# The line between the kernels that read such a tensor once and once a workgroup, on either side; captured, the latter again.
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("shape", [(40, 4096), (41, 4096), (15, 14336), (16, 14336), (20, 4096), (21, 4096), (15, 8192), (16, 8192), (64, 4096)])
+def test_cast_dynamic_either_side_of_the_flat_kernel(nat, dt, shape):
+    x = heavy(shape, TORCH_DT[dt], 33).to(DEV)
+    for fmt, (code, f8dt) in F8.items():
+        s_want = nat.amax_scale(x, f8dt, want_amax=False)[1]
+        for layout in (0, 1):
+            want = nat.cast(x, s_want, f8dt, out_kblock=layout)[0]
+            got, _, s = nat.cast_dynamic(x, f8dt, out_kblock=layout)
+            assert torch.equal(s, s_want) and torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q, _, sq = nat.cast_dynamic(x, torch.float8_e4m3fn)
+    for _ in range(3):
+        x.mul_(0.5)
+        graph.replay()
+        assert torch.equal(sq, nat.amax_scale(x, torch.float8_e4m3fn, want_amax=False)[1])
+        assert torch.equal(q.view(torch.uint8), nat.cast(x, sq, torch.float8_e4m3fn)[0].view(torch.uint8))
+
+
 # The one-launch cast of a tensor that the chip holds: a single tile, tiles of 64 rows and of 128, one row or column into the next tile,
 # the last size of either kind and the largest of all; nobody waits (every workgroup finds the maximum itself) or as shipped.
 @pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
