@@ -279,27 +279,105 @@ __device__ __forceinline__ void emit_tile(const Row8<DT> (&in)[H][4], uint32_t* 
 
 // An exchange of maxima inside a launch.  Whoever has one publishes a 64-bit word, {launch tag, maximum}, with an agent-scope store;
 // whoever needs them all reads the words with agent-scope loads until each carries the tag: the words are all there is to
-// exchange, so no fence is needed.  The tag is the host's count of such launches, never used twice, so a word of any other launch
+// exchange, so no fence is needed.  The tag is the host's count of such launches, so a word of any other launch
 // just reads as "not there yet" and nothing has to be cleared; the host keeps launches that may run at the same time (other
-// streams) on other words.  Nothing depends on the others being on the chip: a workgroup that has waited for wait_ticks of the 100
-// MHz clock finds the maximum itself by reading the whole tensor.  So every wave ends whatever else runs, and the result is the same
+// streams) on other words.  (The count has 32 bits: a word would be taken for a later launch's if exactly 2^32 launches had gone by
+// without one that wrote it.)  Nothing depends on the others being on the chip: a workgroup that has waited for wait_ticks of the 100
+// MHz clock reads the tiles whose words are missing itself.  So every wave ends whatever else runs, and the result is the same
 // bits either way.
 struct TaggedWords {
     uint64_t* words;  // null: no exchange
     uint32_t tag, wait_ticks;
 };
-constexpr uint32_t EXCHANGE_WAIT_TICKS = 200000;  // 2 ms: several rounds of the longest tiles of the GEMMs that may hold the CUs
+// Everybody collects, and waits for workgroups that may find no room.  60 us: the last tile of the largest tensor arrives after 10 - 20, with
+// as large a cast beside it after 40.  us a cast of 4096 x 4096 where two / three of them run at once on streams of their own, bf16: waits of
+// 20: 17 / 38, 50 - 500: 16 / 21 (in turn on one stream: 18); fp32: 20: 50 / 61, 50: 25 / 65, 120: 24 / 83, 500: 24 / 242 (in turn: 25).
+constexpr uint32_t EXCHANGE_WAIT_TICKS = 6000;
+// Only the workgroup started last collects: the others end whatever it does, and most of them have.
+constexpr uint32_t EXCHANGE_WAIT_TICKS_LAST = 200000;
 
 __device__ __forceinline__ void publish_word(const TaggedWords& e, uint32_t i, uint32_t m) {
     __hip_atomic_store(&e.words[i], (uint64_t)e.tag << 32 | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The maximum of the first n words and of every lane's m, the same in all lanes of the workgroup.  Every lane asks for BATCH words at
-// a time, from the last ones (which come last) down: one round trip to memory (0.7 us) for each batch.  With every workgroup
-// collecting, BATCH is 1: more words polled at a time hold up the loads that are waited for (4096 x 4096 bf16: 18.9 us, with four 24.7).
-template <int DT, int BATCH>
-__device__ __forceinline__ uint32_t collect_words(const TaggedWords& e, uint32_t n, uint32_t m, uint32_t (&red)[CAST_THREADS / 64], const void* x,
-                                                  int64_t rows, int64_t cols, int64_t ld) {
+// One tensor of a launch, as the kernels take it.
+struct CastJob {
+    const void* x;
+    int64_t rows, cols, ld;
+    uint8_t *out, *out_t;
+    uint32_t tiles_x, tiles_y;
+    int out_kb, out_t_kb;      // F8MI_LAYOUT_* code of the respective output
+    const float* scale_dev;    // the scale, given beforehand; else
+    float* scale_out;          // where the one found here goes,
+    const uint32_t* amax_ws;   // found from the amax_nblocks maxima in amax_ws (the resident kernel: from the tensor itself)
+    int amax_nblocks;
+    float* amax_out;           // fused amax: its value, through
+    uint32_t* amax_spread;     // these words, or
+    TaggedWords tagged;        // an exchange
+};
+
+// The maximum of the tensor's nb tiles of 64 H rows for a workgroup that has waited long enough: words that are there are taken, the
+// tiles of those that are not are read, one after the other, each followed by another look at the words.  Workgroups start at
+// different words and pick different tiles, and what one finds it publishes, so that together they read each missing tile about once
+// (4096 x 4096, nobody waits at all: bf16 25 us for 16, fp32 53 for 24; when each of them read the whole tensor: 13.8 ms, bf16).  Every turn settles a word
+// that was not: at most one for each word, whatever happens to the words meanwhile.  W words a tile; several: nobody else looks.
+constexpr int RED_WORDS = CAST_THREADS / 64 + 1;
+template <int DT, int H, int W>
+__device__ __forceinline__ uint32_t collect_late(const CastJob& j, uint32_t bid, uint32_t nb, uint32_t* red) {
+    const uint32_t t = threadIdx.x, wave = t >> 6, n = nb * W;
+    const uint32_t first = (bid * 0x9e3779b1u) % n;
+    uint32_t m = 0;
+    for (uint32_t k = 0; k < n; k += CAST_THREADS) {
+        const bool mine = k + t < n;
+        const uint32_t i = first + k + t < n ? first + k + t : first + k + t - n;
+        bool settled = !mine;
+        for (uint32_t turn = bid;; turn++) {
+            if (!settled) {
+                const uint64_t w = __hip_atomic_load(&j.tagged.words[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((uint32_t)(w >> 32) == j.tagged.tag) {
+                    m = max(m, (uint32_t)w);
+                    settled = true;
+                }
+            }
+            const uint64_t missing = __ballot(!settled);
+            __syncthreads();  // everybody has read `red`
+            if ((t & 63) == 0) red[wave] = (uint32_t)__popcll(missing);
+            __syncthreads();
+            const uint32_t total = red[0] + red[1] + red[2] + red[3];
+            if (!total) break;
+            uint32_t rank = (uint32_t)__popcll(missing & ((1ull << (t & 63)) - 1));
+            for (uint32_t v = 0; v < wave; v++) rank += red[v];
+            if (!settled && rank == (turn * 0x85ebca6bu >> 8) % total) red[4] = i / W;
+            __syncthreads();
+            const uint32_t tile = red[4];
+            if (mine && i / W == tile) settled = true;
+            int ty, tx;
+            cast_tile_of(tile, nb, j.tiles_x, j.tiles_y, ty, tx);
+            Row8<DT> in[H][4];
+            load_tile<DT, H>(in, j.x, (int64_t)ty * (64 * H), (int64_t)tx * CAST_TILE, j.rows, j.cols, j.ld);
+            const uint32_t found = wave_max_u32(absmax_tile<DT, H>(in));
+            m = max(m, found);
+            if constexpr (W == 1) {
+                __syncthreads();  // everybody has read `red`
+                if ((t & 63) == 0) red[wave] = found;
+                __syncthreads();
+                if (t == 0) publish_word(j.tagged, tile, max(max(red[0], red[1]), max(red[2], red[3])));
+            }
+        }
+    }
+    m = wave_max_u32(m);
+    __syncthreads();
+    if ((t & 63) == 0) red[wave] = m;
+    __syncthreads();
+    return max(max(red[0], red[1]), max(red[2], red[3]));
+}
+
+// Whether all n words were there in time; m: their maximum and every lane's, the same in all lanes of the workgroup.
+// Every lane asks for BATCH words at a time, from the last ones (which come last) down: one round trip to memory (0.7 us) for each
+// batch.  With every workgroup collecting, BATCH is 1: more words polled at a time hold up the loads that are waited for (4096 x 4096
+// bf16: 18.9 us, with four 24.7).
+template <int BATCH>
+__device__ __forceinline__ bool collect_words(const TaggedWords& e, uint32_t n, uint32_t& m, uint32_t* red) {
     const int t = threadIdx.x;
     const uint64_t start = wall_clock64();
     constexpr uint32_t STEP = BATCH * CAST_THREADS, LATE = 0x80000000u;  // no maximum has the top bit
@@ -325,42 +403,12 @@ __device__ __forceinline__ uint32_t collect_words(const TaggedWords& e, uint32_t
     if ((t & 63) == 0) red[t >> 6] = m;
     __syncthreads();
     m = max(max(red[0], red[1]), max(red[2], red[3]));
-    if (m & LATE) {
-        m = 0;
-        for (int64_t r = 0; r < (ld ? rows : 1); r++)
-            for (int64_t c = 8 * t; c < cols; c += 8 * CAST_THREADS) {
-                Row8<DT> v;
-                load_row8<DT>(v, x, r, c, rows, cols, ld);
-                m = absmax_row<DT>(v, m);
-            }
-        m = wave_max_u32(absmax_done<DT>(m));
-        __syncthreads();  // everybody has read `red`
-        if ((t & 63) == 0) red[t >> 6] = m;
-        __syncthreads();
-        m = max(max(red[0], red[1]), max(red[2], red[3]));
-    }
-    return m;
+    return !(m & LATE);
 }
-
-// One tensor of a launch, as the kernels take it.
-struct CastJob {
-    const void* x;
-    int64_t rows, cols, ld;
-    uint8_t *out, *out_t;
-    uint32_t tiles_x, tiles_y;
-    int out_kb, out_t_kb;      // F8MI_LAYOUT_* code of the respective output
-    const float* scale_dev;    // the scale, given beforehand; else
-    float* scale_out;          // where the one found here goes,
-    const uint32_t* amax_ws;   // found from the amax_nblocks maxima in amax_ws (the resident kernel: from the tensor itself)
-    int amax_nblocks;
-    float* amax_out;           // fused amax: its value, through
-    uint32_t* amax_spread;     // these words, or
-    TaggedWords tagged;        // an exchange
-};
 
 // Workgroup `bid` of the `nb` that cast the tensor.
 template <int DT, int PROD, int FMT, bool TAGGED>
-__device__ __forceinline__ void cast_body(const CastJob& j, uint32_t bid, uint32_t nb, uint32_t* tileT, uint32_t (&red)[CAST_THREADS / 64]) {
+__device__ __forceinline__ void cast_body(const CastJob& j, uint32_t bid, uint32_t nb, uint32_t* tileT, uint32_t* red) {
     const void* const x = j.x;
     const int64_t rows = j.rows, cols = j.cols, ld = j.ld;
     float* const amax_out = j.amax_out;
@@ -424,7 +472,7 @@ __device__ __forceinline__ void cast_body(const CastJob& j, uint32_t bid, uint32
         m = wave_max_u32(m);
         if ((t & 63) == 0) publish_word(j.tagged, bid * (CAST_THREADS / 64) + (t >> 6), m);
         if (bid == nb - 1) {
-            m = collect_words<DT, 8>(j.tagged, nb * (CAST_THREADS / 64), m, red, x, rows, cols, ld);
+            if (!collect_words<8>(j.tagged, nb * (CAST_THREADS / 64), m, red)) m = collect_late<DT, 2, CAST_THREADS / 64>(j, bid, nb, red);
             if (t == 0) *amax_out = abs_bits_to_float(m, DT);
         }
     } else if (amax_out && j.amax_spread) {
@@ -455,7 +503,7 @@ __device__ __forceinline__ void cast_body(const CastJob& j, uint32_t bid, uint32
 template <int DT, int PROD, int FMT, bool TAGGED>
 __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(CastJob j) {
     __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];  // [column][row/4] dwords, swizzled
-    __shared__ uint32_t red[CAST_THREADS / 64];
+    __shared__ uint32_t red[RED_WORDS];
     cast_body<DT, PROD, FMT, TAGGED>(j, blockIdx.x, gridDim.x, tileT, red);
 }
 
@@ -463,7 +511,7 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(CastJob j) {
 template <int DTA, int DTB, int FMT, bool TAGGED>
 __global__ __launch_bounds__(CAST_THREADS) void cast_pair_kernel(CastJob a, CastJob b, uint32_t nb_a) {
     __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];
-    __shared__ uint32_t red[CAST_THREADS / 64];
+    __shared__ uint32_t red[RED_WORDS];
     if (blockIdx.x < nb_a) cast_body<DTA, TAGGED ? F8MI_FP32 : DTA, FMT, TAGGED>(a, blockIdx.x, nb_a, tileT, red);
     else cast_body<DTB, TAGGED ? F8MI_FP32 : DTB, FMT, TAGGED>(b, blockIdx.x - nb_a, gridDim.x - nb_a, tileT, red);
 }
@@ -629,18 +677,19 @@ static int launch_cast_flat(int fmt, hipStream_t stream, const void* x, int64_t 
 // workgroup loads its tile (64 H rows x 128 columns) into registers, publishes the tile's maximum, collects everybody's and casts
 // what it holds.  The two kernels it replaces read the tensor twice and pay a launch and a ramp more.
 //
-// All workgroups fit on the chip at once (see resident_tile_rows), but nothing depends on it.
+// Alone on the chip all workgroups are there at once (see resident_tile_rows).  Beside other streams' kernels they may not be: whoever
+// waits for too long reads the missing tiles itself (see collect_late).  The kernel keeps nothing for that path in registers.
 //
 // us a call, back to back, inputs cold, amax and cast / this one: one copy, bf16, 512 x 1024: 8.8 / 6.4, 2048 x 2048: 10.6 / 9.0, 2726 x 934
 // (padded): 16.1 / 10.7, 2048 x 4096: 14.3 / 11.5, 4096 x 4096: 20.5 / 17.6; both copies, 4096 x 4096: 21.8 / 19.3; fp32,
 // 512 x 1024: 9.9 / 6.4, 4096 x 4096: 30.7 / 24.3.  (Twice as many tiles, all that eight workgroups a CU hold: 8192 x 4096 34.7 / 31.3 -- but then
-// one workgroup that finds no room, beside another stream's kernel, keeps all the others waiting: not taken.)  Inside a launch of 4096 x 4096 bf16 (1024 workgroups): the last tile has arrived after 9.5
+// any other kernel on the chip makes all of them late: not taken.)  Inside a launch of 4096 x 4096 bf16 (1024 workgroups): the last tile has arrived after 9.5
 // us, everybody has everybody's maximum after 11.3 (2 us is what a word takes to memory and back, 512 x 1024 waits as long), the
 // last byte is stored after 15.  Loads in smaller batches, other tile shapes and linear tile orders all took the same or longer.
 constexpr int RESIDENT_TILES = 1024;  // workgroups at most
 
 template <int DT, int FMT, int H>
-__device__ __forceinline__ void resident_body(const CastJob& j, uint32_t bid, uint32_t nb, uint32_t* tileT, uint32_t (&red)[2][CAST_THREADS / 64]) {
+__device__ __forceinline__ void resident_body(const CastJob& j, uint32_t bid, uint32_t nb, uint32_t* tileT, uint32_t* red) {
     const int t = threadIdx.x;
     int ty, tx;
     cast_tile_of(bid, nb, j.tiles_x, j.tiles_y, ty, tx);
@@ -648,10 +697,16 @@ __device__ __forceinline__ void resident_body(const CastJob& j, uint32_t bid, ui
     Row8<DT> in[H][4];
     load_tile<DT, H>(in, j.x, r0, c0, j.rows, j.cols, j.ld);
     uint32_t m = wave_max_u32(absmax_tile<DT, H>(in));
-    if ((t & 63) == 0) red[0][t >> 6] = m;
+    if ((t & 63) == 0) red[t >> 6] = m;
     __syncthreads();
-    if (t == 0) publish_word(j.tagged, bid, max(max(red[0][0], red[0][1]), max(red[0][2], red[0][3])));
-    m = collect_words<DT, 1>(j.tagged, nb, m, red[1], j.x, j.rows, j.cols, j.ld);
+    if (t == 0) publish_word(j.tagged, bid, max(max(red[0], red[1]), max(red[2], red[3])));
+    if (!collect_words<1>(j.tagged, nb, m, red + CAST_THREADS / 64)) {
+        m = collect_late<DT, H, 1>(j, bid, nb, red);
+        // The tile again: held meanwhile, it or its addresses would cost every launch registers, and a CU a workgroup.
+        int64_t again = r0;
+        asm volatile("" : "+s"(again));
+        load_tile<DT, H>(in, j.x, again, c0, j.rows, j.cols, j.ld);
+    }
     const float amax = abs_bits_to_float(m, DT), scale = amax_to_scale_dev(amax, DT, FMT, DT == F8MI_FP16);
     if (bid == 0 && t == 0) *j.scale_out = scale;
     emit_tile<DT, DT, FMT, H>(in, tileT, scale, within_range<FMT>(amax, scale), r0, c0, j.rows, j.cols, j.out, j.out_t, j.out_kb, j.out_t_kb);
@@ -660,7 +715,7 @@ __device__ __forceinline__ void resident_body(const CastJob& j, uint32_t bid, ui
 template <int DT, int FMT, int H>
 __global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_kernel(CastJob j) {
     __shared__ uint32_t tileT[32 * 64 * H];
-    __shared__ uint32_t red[2][CAST_THREADS / 64];
+    __shared__ uint32_t red[2 * CAST_THREADS / 64];
     resident_body<DT, FMT, H>(j, blockIdx.x, gridDim.x, tileT, red);
 }
 
@@ -668,7 +723,7 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_kernel(Cas
 template <int DTA, int DTB, int FMT, int H>
 __global__ __launch_bounds__(CAST_THREADS) void cast_dynamic_resident_pair_kernel(CastJob a, CastJob b, uint32_t nb_a) {
     __shared__ uint32_t tileT[32 * 64 * H];
-    __shared__ uint32_t red[2][CAST_THREADS / 64];
+    __shared__ uint32_t red[2 * CAST_THREADS / 64];
     if (blockIdx.x < nb_a) resident_body<DTA, FMT, H>(a, blockIdx.x, nb_a, tileT, red);
     else resident_body<DTB, FMT, H>(b, blockIdx.x - nb_a, gridDim.x - nb_a, tileT, red);
 }
@@ -872,7 +927,7 @@ extern "C" int f8mi_cast_delayed(const void* x, int64_t rows, int64_t cols, int6
     if (!workspace || (uintptr_t)workspace % 4 != 0) { set_error("f8mi_cast_delayed: null or misaligned workspace"); return F8MI_ERR_INVALID_ARG; }
     AmaxSource src{};
     if (rows > 0 && cols > 0 && one_launch_delayed(rows, cols))
-        if (const int rc = begin_exchange((hipStream_t)stream, EXCHANGE_WAIT_TICKS, src.tagged)) return rc;
+        if (const int rc = begin_exchange((hipStream_t)stream, EXCHANGE_WAIT_TICKS_LAST, src.tagged)) return rc;
     if (src.tagged.words)
         return cast_layout_impl(x, rows, cols, ld, in_dtype, scale_dev, F8MI_FP32, fp8_fmt, out, out_layout, out_t, out_t_layout, amax_dev,
                                 (hipStream_t)stream, src);
@@ -885,7 +940,8 @@ extern "C" int f8mi_cast_delayed(const void* x, int64_t rows, int64_t cols, int6
 namespace f8mi {
 
 // Rows of the tiles that the one-launch cast gives a tensor, 0: it does not take it.  At most four workgroups a CU (RESIDENT_TILES on
-// 256): it holds eight of them (five of 128 rows of fp32), so that all are there at once also beside other streams' kernels.
+// 256) of the eight that it holds, seven of 128 rows, five of 128 rows of fp32: a launch that is alone has them all there at once, with
+// room for a small one beside it.
 static int resident_tile_rows(int64_t rows, int64_t cols) {
     const int64_t tx = (cols + CAST_TILE - 1) / CAST_TILE, ty = (rows + CAST_TILE - 1) / CAST_TILE, most = std::min(RESIDENT_TILES, 4 * cu_count());
     if (ty > most || tx > most) return 0;
@@ -1098,7 +1154,7 @@ extern "C" int f8mi_cast_delayed_pair(const f8mi_cast_job* a, const f8mi_cast_jo
     if (!a || !b) { set_error("f8mi_cast_delayed_pair: null job"); return F8MI_ERR_INVALID_ARG; }
     if (pair_ok(*a, *b) && a->amax_dev && b->amax_dev && one_launch_delayed((tiles_of(*a) + tiles_of(*b)) * CAST_TILE, CAST_TILE)) {
         TaggedWords tagged;
-        if (const int rc = begin_exchange(stream, EXCHANGE_WAIT_TICKS, tagged)) return rc;
+        if (const int rc = begin_exchange(stream, EXCHANGE_WAIT_TICKS_LAST, tagged)) return rc;
         if (tagged.words) {
             CastJob ja = kernel_job(*a, CAST_TILE), jb = kernel_job(*b, CAST_TILE);
             ja.scale_dev = a->scale_dev;

@@ -637,6 +637,47 @@ def test_cast_dynamic_resident_on_several_streams_and_what_it_refuses(nat):
         assert torch.equal(q.view(torch.uint8), nat.cast(xs[0], sq, torch.float8_e4m3fn)[0].view(torch.uint8))
 
 
+def test_cast_dynamic_resident_costs_little_when_workgroups_are_late(nat):
+    """Three launches of 1024 workgroups at once are more than the chip holds, so each waits for workgroups that have no room until
+    the others' end: they read the missing tiles, and not the whole tensor each (1.4 - 2.4 ms for three casts that take 0.08 in turn).
+    The same where nobody waits for anybody (13.8 ms)."""
+    import time
+
+    for dt in (torch.bfloat16, torch.float32):
+        streams = [torch.cuda.Stream() for _ in range(3)]
+        xs = [heavy((4096, 4096), dt, 90 + i).to(DEV) for i in range(3)]
+        want = [nat.cast(x, nat.amax_scale(x, torch.float8_e4m3fn, want_amax=False)[1], torch.float8_e4m3fn)[0].view(torch.uint8) for x in xs]
+        outs = [torch.empty(4096, 4096, device=DEV, dtype=torch.uint8) for _ in xs]
+        scales = [torch.empty((), device=DEV) for _ in xs]
+
+        def cast(i, stream, ticks=None):
+            args = (xs[i].data_ptr(), 4096, 4096, 4096, nat._DT[dt], 0, scales[i].data_ptr(), outs[i].data_ptr(), 0, None, 0)
+            if ticks is None:
+                rc = nat.lib().f8mi_cast_dynamic(*args, nat.workspace(xs[i].device).data_ptr(), stream.cuda_stream)
+            else:
+                rc = nat.lib().f8mi_cast_dynamic_resident(*args, ticks, stream.cuda_stream)
+            assert rc == 0, nat.lib().f8mi_last_error()
+
+        def fastest(calls):  # of six rounds: one may be interrupted
+            best = 1e9
+            for _ in range(6):
+                torch.cuda.synchronize()
+                begin = time.perf_counter()
+                calls()
+                torch.cuda.synchronize()
+                best = min(best, time.perf_counter() - begin)
+            return best
+
+        in_turn = fastest(lambda: [cast(i, streams[0]) for _ in range(20) for i in range(3)])
+        at_once = fastest(lambda: [cast(i, streams[i]) for _ in range(20) for i in range(3)])
+        assert at_once < 4 * in_turn, (dt, in_turn, at_once)
+        for o, w in zip(outs, want):
+            assert torch.equal(o, w)
+            o.zero_()
+        assert fastest(lambda: [cast(i, streams[0], 0) for i in range(3)]) < 3e-3
+        assert all(torch.equal(o, w) for o, w in zip(outs, want))
+
+
 # Two tensors in one call: tiny, tiles of 64 and of 128 rows, the most that one launch takes together (1024 tiles, delayed 2048) and one row
 # more, one or both too large for it, ragged and row-strided.
 @pytest.mark.parametrize("dts", ["bf16 bf16", "fp16 fp16", "fp32 fp32", "bf16 fp32", "fp16 fp32", "fp32 bf16"])

@@ -109,6 +109,18 @@ def test_few_row_kernels_of_one_step_per_wave_leave_room_for_two_workgroups(tmp_
     assert len(sizes) >= len(vgprs) and not any(sizes)
 
 
+def test_one_launch_casts_leave_room_beside_them(tmp_path):
+    """At most four workgroups a CU of a cast that holds its tensor on the chip, out of the eight, with 128-row tiles seven (fp32
+    five) that its registers allow: one register too many, and a launch that is alone has workgroups without room."""
+    text = "\n".join(_asm("f8mi_cast.hip", str(tmp_path)))
+    kernels = re.findall(r"\.amdhsa_kernel \S*cast_dynamic_resident_(?:pair_)?kernelILi(\S+?)EEv.*?\.amdhsa_private_segment_fixed_size (\d+).*?\.amdhsa_next_free_vgpr (\d+)", text, re.S)
+    assert len(kernels) == 3 * 2 * 2 + 5 * 2
+    for name, scratch, vgprs in kernels:
+        codes = [int(v) for v in re.findall(r"\d+", name.replace("ELi", " "))]
+        workgroups = 8 if codes[-1] == 1 else 5 if 2 in codes[:-2] else 7
+        assert int(scratch) == 0 and int(vgprs) <= 512 // workgroups // 8 * 8, (name, vgprs)
+
+
 def test_few_row_linear_keeps_to_its_registers(tmp_path):
     """Two workgroups a CU leave a lane 128 registers; the activations take up to 64 of them and the weights in flight the
     rest: no instantiation may spill."""
