@@ -807,6 +807,16 @@ __global__ __launch_bounds__(SPREAD_WORDS) void cast_spread_finalize_kernel(uint
     }
 }
 
+// LDS that a cast asks for without using it, to be held to six workgroups a CU instead of the eight (fp32: four instead of five) that its
+// registers allow, where its tiles number two rounds of them or more.  More of them at a time write more rows and columns at a time than
+// the memory takes at full rate.  us, eight / six, bf16: 8192 x 4096 22.7 / 23.3, 12288 x 4096 32.0 / 32.0, 8192 x 14336 71.7 / 69.3, 28672 x 8192 140 /
+// 138; with both copies 29.7 / 30.1, 42.7 / 42.1, 97.7 / 95.2, 187 / 182; fp32 with both, five / four: 8192 x 4096 43.8 / 43.4, 28672 x 8192 290 / 285.
+constexpr unsigned UNUSED_LDS_16 = 10 << 10, UNUSED_LDS_32 = 20 << 10;
+static unsigned unused_lds(int in_dtype, int64_t tiles) {
+    const bool wide = in_dtype == F8MI_FP32;
+    return tiles >= (wide ? 8 : 12) * (int64_t)cu_count() ? (wide ? UNUSED_LDS_32 : UNUSED_LDS_16) : 0u;
+}
+
 template <int DT, int PROD, int FMT>
 static int launch_cast2(dim3 g, hipStream_t stream, const CastJob& j) {
     if constexpr (PROD == F8MI_FP32) {  // what delayed scaling computes in
@@ -815,7 +825,7 @@ static int launch_cast2(dim3 g, hipStream_t stream, const CastJob& j) {
             return check_hip(hipGetLastError(), "cast kernel launch");
         }
     }
-    hipLaunchKernelGGL((cast_kernel<DT, PROD, FMT, false>), g, dim3(CAST_THREADS), 0, stream, j);
+    hipLaunchKernelGGL((cast_kernel<DT, PROD, FMT, false>), g, dim3(CAST_THREADS), unused_lds(DT, g.x), stream, j);
     return check_hip(hipGetLastError(), "cast kernel launch");
 }
 
@@ -1088,7 +1098,8 @@ static int launch_cast_pair1(int tile_rows, hipStream_t stream, const CastJob& a
     if constexpr (!TAGGED) {
         if (tile_rows == 64) hipLaunchKernelGGL((cast_dynamic_resident_pair_kernel<DTA, DTB, F8MI_E4M3FN, 1>), g, t, 0, stream, a, b, nb_a);
         else if (tile_rows == 128) hipLaunchKernelGGL((cast_dynamic_resident_pair_kernel<DTA, DTB, F8MI_E4M3FN, 2>), g, t, 0, stream, a, b, nb_a);
-        else hipLaunchKernelGGL((cast_pair_kernel<DTA, DTB, F8MI_E4M3FN, false>), g, t, 0, stream, a, b, nb_a);
+        // (unequal types: five workgroups a CU, and no fewer is faster)
+        else hipLaunchKernelGGL((cast_pair_kernel<DTA, DTB, F8MI_E4M3FN, false>), g, t, DTA == DTB ? unused_lds(DTA, g.x) : 0u, stream, a, b, nb_a);
     } else {
         hipLaunchKernelGGL((cast_pair_kernel<DTA, DTB, F8MI_E4M3FN, true>), g, t, 0, stream, a, b, nb_a);
     }
