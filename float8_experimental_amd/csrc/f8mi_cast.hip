@@ -760,7 +760,10 @@ static std::atomic<uint32_t> g_exchange_tag{0};
 static int begin_exchange(hipStream_t stream, uint32_t wait_ticks, TaggedWords& e) {
     e = TaggedWords{nullptr, 0, wait_ticks};
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (check_hip(hipStreamIsCapturing(stream, &capture), "hipStreamIsCapturing")) return F8MI_ERR_HIP;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {  // of the default stream, say, while a blocking one is captured: launches are taken
+        (void)hipGetLastError();
+        return F8MI_OK;
+    }
     if (capture != hipStreamCaptureStatusNone) return F8MI_OK;
     int dev = 0;
     if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return F8MI_ERR_HIP;

@@ -108,3 +108,41 @@ def test_delayed_scaling_step_with_sync_replays_bitwise(f8):
             assert torch.equal(a, b), it
         for (name, b1), (_, b2) in zip(model.named_buffers(), twin.named_buffers()):
             assert torch.equal(b1, b2), (it, name)
+
+
+def test_default_stream_is_served_while_a_blocking_stream_is_captured(f8):
+    """The runtime refuses to say whether the default stream is being captured while a stream that synchronises with it is; launches
+    on it are taken all the same, and so are the casts, as before and after the capture and on the captured stream."""
+    import ctypes
+
+    from float8_experimental_amd import _native as nat
+
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    x = torch.randn(1024, 1024, device=DEV).bfloat16()
+    scale = torch.tensor([3.0], device=DEV)
+    want, _, s_want = nat.cast_dynamic(x, torch.float8_e4m3fn)
+    want_delayed = nat.cast(x, scale, torch.float8_e4m3fn, product_dtype=torch.float32)[0]
+    got, s = torch.zeros_like(want), torch.zeros_like(s_want)
+    got_delayed, amax = torch.zeros_like(want), torch.zeros(1, device=DEV)
+    args = x.data_ptr(), 1024, 1024, 1024, 0
+    ws, delayed_ws = nat.workspace(x.device).data_ptr(), nat.delayed_workspace(x.device).data_ptr()
+
+    def casts(stream):
+        return (nat.lib().f8mi_cast_dynamic(*args, 0, s.data_ptr(), got.data_ptr(), 0, None, 0, ws, stream),
+                nat.lib().f8mi_cast_delayed(*args, scale.data_ptr(), 0, got_delayed.data_ptr(), 0, None, 0, amax.data_ptr(), delayed_ws, stream))
+
+    torch.cuda.synchronize()
+    for mode in (1, 2):  # thread-local, relaxed
+        stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 0) == 0
+        assert hip.hipStreamBeginCapture(stream, mode) == 0
+        answers = casts(None), casts(stream)
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        assert answers == ((0, 0), (0, 0)), nat.lib().f8mi_last_error()
+        assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)) and torch.equal(s, s_want)
+        assert torch.equal(got_delayed.view(torch.uint8), want_delayed.view(torch.uint8)) and amax.item() == x.abs().max().item()
+        for t in (got.view(torch.uint8), s, got_delayed.view(torch.uint8), amax):
+            t.zero_()
