@@ -745,16 +745,27 @@ static T* device_array(const void* symbol, std::atomic<T*> (&known)[STATIC_MAX_D
     return (T*)addr;
 }
 
-// The words of the exchanges: a set for each of the first EXCHANGE_STREAMS streams that use one, so that launches which may run at
-// the same time do not share any (sharing would be slow, not wrong).  Later streams take the kernels that need no exchange, and so do
-// streams that are being captured: a captured launch would use its tag again on every replay.  A stream handle that comes back for a
-// new stream finds the old one's set: its work is done.
+// The words of the exchanges: a set for each of the last EXCHANGE_STREAMS streams to use one for the first time, so that launches which
+// may run at the same time do not share any (sharing would be slow, not wrong).  A further stream takes over the set that was given
+// out first, whose stream may be gone; if it is not, it gets another with its next launch.  Streams that are being captured have none: a captured launch would
+// use its tag again on every replay.  A stream handle that comes back for a new stream finds the old one's set: its work is done.
 constexpr int EXCHANGE_STREAMS = 64;
 constexpr int EXCHANGE_WORDS = 8192;
 static __device__ __align__(256) uint64_t exchange_words[EXCHANGE_STREAMS][EXCHANGE_WORDS];
 static std::atomic<uint64_t*> g_exchange_words[STATIC_MAX_DEVICES];
 static std::atomic<uintptr_t> g_exchange_streams[STATIC_MAX_DEVICES][EXCHANGE_STREAMS];
+static std::atomic<uint32_t> g_exchange_given[STATIC_MAX_DEVICES];
 static std::atomic<uint32_t> g_exchange_tag{0};
+
+static int exchange_set(int dev, hipStream_t stream) {
+    static thread_local char own;  // one handle stands for every thread's own stream
+    const uintptr_t key = stream == hipStreamPerThread ? (uintptr_t)&own : (uintptr_t)stream + 1;  // the default stream is a null handle
+    for (int i = 0; i < EXCHANGE_STREAMS; i++)
+        if (g_exchange_streams[dev][i].load(std::memory_order_relaxed) == key) return i;
+    const int i = (int)(g_exchange_given[dev].fetch_add(1, std::memory_order_relaxed) % EXCHANGE_STREAMS);
+    g_exchange_streams[dev][i].store(key, std::memory_order_relaxed);
+    return i;
+}
 
 // Words and a tag for one launch on `stream`; words null: none to be had.  An error code if the runtime reports one.
 static int begin_exchange(hipStream_t stream, uint32_t wait_ticks, TaggedWords& e) {
@@ -769,16 +780,9 @@ static int begin_exchange(hipStream_t stream, uint32_t wait_ticks, TaggedWords& 
     if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return F8MI_ERR_HIP;
     uint64_t* base = device_array(HIP_SYMBOL(exchange_words), g_exchange_words, "exchange_words");
     if (!base) return F8MI_ERR_HIP;
-    const uintptr_t key = (uintptr_t)stream + 1;  // the default stream is a null handle
-    for (int i = 0; i < EXCHANGE_STREAMS; i++) {
-        uintptr_t have = g_exchange_streams[dev][i].load(std::memory_order_relaxed);
-        if (!have && g_exchange_streams[dev][i].compare_exchange_strong(have, key, std::memory_order_relaxed)) have = key;
-        if (have != key) continue;
-        e.words = base + (size_t)i * EXCHANGE_WORDS;
-        e.tag = g_exchange_tag.fetch_add(1, std::memory_order_relaxed) + 1;
-        if (!e.tag) e.tag = g_exchange_tag.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 is what the words start with
-        break;
-    }
+    e.words = base + (size_t)exchange_set(dev, stream) * EXCHANGE_WORDS;
+    e.tag = g_exchange_tag.fetch_add(1, std::memory_order_relaxed) + 1;
+    if (!e.tag) e.tag = g_exchange_tag.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 is what the words start with
     return F8MI_OK;
 }
 
@@ -987,7 +991,7 @@ extern "C" int f8mi_cast_dynamic_resident(const void* x, int64_t rows, int64_t c
     if (!tile_rows) { set_error("f8mi_cast_dynamic_resident: %lld x %lld is more than the chip holds", (long long)rows, (long long)cols); return F8MI_ERR_UNSUPPORTED; }
     TaggedWords tagged;
     if (const int rc = begin_exchange(stream, wait_ticks, tagged)) return rc;
-    if (!tagged.words) { set_error("f8mi_cast_dynamic_resident: the stream is being captured, or %d others use it", EXCHANGE_STREAMS); return F8MI_ERR_UNSUPPORTED; }
+    if (!tagged.words) { set_error("f8mi_cast_dynamic_resident: the stream is being captured"); return F8MI_ERR_UNSUPPORTED; }
     const int out_kb = out ? out_layout : F8MI_LAYOUT_ROWMAJOR, out_t_kb = out_t ? out_t_layout : F8MI_LAYOUT_ROWMAJOR;
     // whole 128 x 128 tiles, as the padded layouts are
     const uint32_t tiles_x = (uint32_t)((cols + CAST_TILE - 1) / CAST_TILE), tiles_y = (uint32_t)((rows + CAST_TILE - 1) / CAST_TILE) * (CAST_TILE / tile_rows);

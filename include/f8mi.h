@@ -237,8 +237,7 @@ int f8mi_cast_dynamic_static(const void* x, int64_t rows, int64_t cols, int64_t 
  * on a device of fewer than 256 CUs).  f8mi_cast_dynamic takes it by itself; the same bits.  The workgroups exchange their
  * maxima inside the launch; one that has waited wait_ticks of the 100 MHz clock for the others reads the tiles itself whose
  * maxima are missing, so the launch ends and is right whatever else runs (wait_ticks 0: nobody waits).  Refused with
- * F8MI_ERR_UNSUPPORTED, nothing queued: larger tensors, a stream that is being captured, more than 64 streams of one
- * device. */
+ * F8MI_ERR_UNSUPPORTED, nothing queued: larger tensors, a stream that is being captured. */
 int f8mi_cast_dynamic_resident(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, int fp8_fmt,
                                float* scale_dev, uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout,
                                uint32_t wait_ticks, void* stream);

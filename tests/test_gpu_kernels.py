@@ -637,6 +637,51 @@ def test_cast_dynamic_resident_on_several_streams_and_what_it_refuses(nat):
         assert torch.equal(q.view(torch.uint8), nat.cast(xs[0], sq, torch.float8_e4m3fn)[0].view(torch.uint8))
 
 
+def test_cast_dynamic_resident_serves_every_stream(nat):
+    """64 streams of a device have words of their own; those of streams that are gone go to new ones.  One handle is a stream of its
+    own in every thread."""
+    import ctypes
+    import threading
+
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    x = heavy((1024, 1024), torch.bfloat16, 35).to(DEV)
+    want = nat.cast(x, nat.amax_scale(x, torch.float8_e4m3fn, want_amax=False)[1], torch.float8_e4m3fn)[0].view(torch.uint8)
+    torch.cuda.synchronize()
+
+    def cast(out, scale, stream):
+        rc = nat.lib().f8mi_cast_dynamic_resident(x.data_ptr(), 1024, 1024, 1024, 0, 0, scale.data_ptr(), out.data_ptr(), 0, None, 0, 200000, stream)
+        assert rc == 0, nat.lib().f8mi_last_error()
+
+    outs = [torch.zeros_like(want) for _ in range(8)]
+    scales = [torch.zeros((), device=DEV) for _ in outs]
+    for _ in range(3):
+        streams = [ctypes.c_void_p() for _ in range(40)]
+        for stream in streams:
+            assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0
+        for i, stream in enumerate(streams):
+            cast(outs[i % 8], scales[i % 8], stream)
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, want) for o in outs)
+        for o in outs:
+            o.zero_()
+        torch.cuda.synchronize()
+        assert all(hip.hipStreamDestroy(stream) == 0 for stream in streams)
+
+    def work(i):
+        torch.cuda.set_device(0)
+        for _ in range(50):
+            cast(outs[i], scales[i], ctypes.c_void_p(2))  # hipStreamPerThread
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for o in outs[:4])
+
+
 def test_cast_dynamic_resident_costs_little_when_workgroups_are_late(nat):
     """Three launches of 1024 workgroups at once are more than the chip holds, so each waits for workgroups that have no room until
     the others' end: they read the missing tiles, and not the whole tensor each (1.4 - 2.4 ms for three casts that take 0.08 in turn).
