@@ -85,6 +85,15 @@ __device__ __forceinline__ float elem(const Row8<DT>& r, int i) {
     }
 }
 
+// Nothing of the row that is worked out before this is kept for what comes after it: on one side of a branch it keeps the compiler from
+// unpacking the rows, which both sides do, ahead of it (16-bit cast with its maximum collected: 73 registers and six workgroups a CU, with
+// this 61 and eight; 8192 x 4096 with both copies 31.2 -> 30.1 us).  Not fp32, where nothing is unpacked: five workgroups instead of four were slower.
+template <int DT>
+__device__ __forceinline__ void set_apart(Row8<DT>& r) {
+#pragma unroll
+    for (uint32_t& w : r.w) asm("" : "+v"(w));
+}
+
 // Folds the eight elements of a row into a running maximum.  16-bit types: `m` holds two 16-bit maxima side by side
 // (see absmax16x2); absmax_done merges them.
 template <int DT>
@@ -219,7 +228,11 @@ __device__ __forceinline__ void emit_tile(const Row8<DT> (&in)[H][4], uint32_t* 
             for (int j = 0; j < 4; j++) cast_row8<DT, PROD, FMT, true>(in[h][j], scale, lo[j], hi[j]);
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) cast_row8<DT, PROD, FMT, false>(in[h][j], scale, lo[j], hi[j]);
+            for (int j = 0; j < 4; j++) {
+                Row8<DT> r = in[h][j];
+                if constexpr (DT != F8MI_FP32) set_apart(r);
+                cast_row8<DT, PROD, FMT, false>(r, scale, lo[j], hi[j]);
+            }
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -316,15 +329,15 @@ struct CastJob {
     TaggedWords tagged;        // an exchange
 };
 
-// The maximum of the tensor's nb tiles of 64 H rows for a workgroup that has waited long enough: words that are there are taken, the
+// The maximum of the tensor's n tiles of 64 H rows for a workgroup that has waited long enough: words that are there are taken, the
 // tiles of those that are not are read, one after the other, each followed by another look at the words.  Workgroups start at
 // different words and pick different tiles, and what one finds it publishes, so that together they read each missing tile about once
 // (4096 x 4096, nobody waits at all: bf16 25 us for 16, fp32 53 for 24; when each of them read the whole tensor: 13.8 ms, bf16).  Every turn settles a word
-// that was not: at most one for each word, whatever happens to the words meanwhile.  W words a tile; several: nobody else looks.
-constexpr int RED_WORDS = CAST_THREADS / 64 + 1;
-template <int DT, int H, int W>
-__device__ __forceinline__ uint32_t collect_late(const CastJob& j, uint32_t bid, uint32_t nb, uint32_t* red) {
-    const uint32_t t = threadIdx.x, wave = t >> 6, n = nb * W;
+// that was not: at most one for each word, whatever happens to the words meanwhile.  red: five words.
+template <int DT, int H>
+__device__ __forceinline__ uint32_t collect_late(const CastJob& j, uint32_t bid, uint32_t n, uint32_t* red) {
+    const uint32_t t = threadIdx.x, wave = t >> 6;
+    constexpr int ROWS = 4;  // loads at a time
     const uint32_t first = (bid * 0x9e3779b1u) % n;
     uint32_t m = 0;
     for (uint32_t k = 0; k < n; k += CAST_THREADS) {
@@ -347,27 +360,52 @@ __device__ __forceinline__ uint32_t collect_late(const CastJob& j, uint32_t bid,
             if (!total) break;
             uint32_t rank = (uint32_t)__popcll(missing & ((1ull << (t & 63)) - 1));
             for (uint32_t v = 0; v < wave; v++) rank += red[v];
-            if (!settled && rank == (turn * 0x85ebca6bu >> 8) % total) red[4] = i / W;
+            if (!settled && rank == (turn * 0x85ebca6bu >> 8) % total) red[4] = i;
             __syncthreads();
             const uint32_t tile = red[4];
-            if (mine && i / W == tile) settled = true;
+            if (mine && i == tile) settled = true;
             int ty, tx;
-            cast_tile_of(tile, nb, j.tiles_x, j.tiles_y, ty, tx);
-            Row8<DT> in[H][4];
-            load_tile<DT, H>(in, j.x, (int64_t)ty * (64 * H), (int64_t)tx * CAST_TILE, j.rows, j.cols, j.ld);
-            const uint32_t found = wave_max_u32(absmax_tile<DT, H>(in));
-            m = max(m, found);
-            if constexpr (W == 1) {
-                __syncthreads();  // everybody has read `red`
-                if ((t & 63) == 0) red[wave] = found;
-                __syncthreads();
-                if (t == 0) publish_word(j.tagged, tile, max(max(red[0], red[1]), max(red[2], red[3])));
+            cast_tile_of(tile, n, j.tiles_x, j.tiles_y, ty, tx);
+            uint32_t found = 0;
+#pragma unroll 1
+            for (int r0 = t >> 4; r0 < 64 * H; r0 += 16 * ROWS) {
+                Row8<DT> in[ROWS];
+#pragma unroll
+                for (int r = 0; r < ROWS; r++)
+                    load_row8<DT>(in[r], j.x, (int64_t)ty * (64 * H) + r0 + 16 * r, (int64_t)tx * CAST_TILE + 8 * (t & 15), j.rows, j.cols, j.ld);
+#pragma unroll
+                for (int r = 0; r < ROWS; r++) found = absmax_row<DT>(in[r], found);
             }
+            found = wave_max_u32(absmax_done<DT>(found));
+            m = max(m, found);
+            __syncthreads();  // everybody has read `red`
+            if ((t & 63) == 0) red[wave] = found;
+            __syncthreads();
+            if (t == 0) publish_word(j.tagged, tile, max(max(red[0], red[1]), max(red[2], red[3])));
         }
     }
     m = wave_max_u32(m);
     __syncthreads();
     if ((t & 63) == 0) red[wave] = m;
+    __syncthreads();
+    return max(max(red[0], red[1]), max(red[2], red[3]));
+}
+
+// The same where only this workgroup collects, and the others, who wait for nobody, have left their words unless they were held up for
+// as long as that: the whole tensor, in little code.
+template <int DT>
+__device__ __forceinline__ uint32_t collect_alone(const CastJob& j, uint32_t* red) {
+    const int t = threadIdx.x;
+    uint32_t m = 0;
+    for (int64_t r = 0; r < (j.ld ? j.rows : 1); r++)
+        for (int64_t c = 8 * t; c < j.cols; c += 8 * CAST_THREADS) {
+            Row8<DT> v;
+            load_row8<DT>(v, j.x, r, c, j.rows, j.cols, j.ld);
+            m = absmax_row<DT>(v, m);
+        }
+    m = wave_max_u32(absmax_done<DT>(m));
+    __syncthreads();  // everybody has read `red`
+    if ((t & 63) == 0) red[t >> 6] = m;
     __syncthreads();
     return max(max(red[0], red[1]), max(red[2], red[3]));
 }
@@ -472,7 +510,7 @@ __device__ __forceinline__ void cast_body(const CastJob& j, uint32_t bid, uint32
         m = wave_max_u32(m);
         if ((t & 63) == 0) publish_word(j.tagged, bid * (CAST_THREADS / 64) + (t >> 6), m);
         if (bid == nb - 1) {
-            if (!collect_words<8>(j.tagged, nb * (CAST_THREADS / 64), m, red)) m = collect_late<DT, 2, CAST_THREADS / 64>(j, bid, nb, red);
+            if (__builtin_expect(!collect_words<8>(j.tagged, nb * (CAST_THREADS / 64), m, red), 0)) m = collect_alone<DT>(j, red);
             if (t == 0) *amax_out = abs_bits_to_float(m, DT);
         }
     } else if (amax_out && j.amax_spread) {
@@ -503,7 +541,7 @@ __device__ __forceinline__ void cast_body(const CastJob& j, uint32_t bid, uint32
 template <int DT, int PROD, int FMT, bool TAGGED>
 __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(CastJob j) {
     __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];  // [column][row/4] dwords, swizzled
-    __shared__ uint32_t red[RED_WORDS];
+    __shared__ uint32_t red[CAST_THREADS / 64];
     cast_body<DT, PROD, FMT, TAGGED>(j, blockIdx.x, gridDim.x, tileT, red);
 }
 
@@ -511,7 +549,7 @@ __global__ __launch_bounds__(CAST_THREADS) void cast_kernel(CastJob j) {
 template <int DTA, int DTB, int FMT, bool TAGGED>
 __global__ __launch_bounds__(CAST_THREADS) void cast_pair_kernel(CastJob a, CastJob b, uint32_t nb_a) {
     __shared__ uint32_t tileT[CAST_TILE * CAST_TILE / 4];
-    __shared__ uint32_t red[RED_WORDS];
+    __shared__ uint32_t red[CAST_THREADS / 64];
     if (blockIdx.x < nb_a) cast_body<DTA, TAGGED ? F8MI_FP32 : DTA, FMT, TAGGED>(a, blockIdx.x, nb_a, tileT, red);
     else cast_body<DTB, TAGGED ? F8MI_FP32 : DTB, FMT, TAGGED>(b, blockIdx.x - nb_a, gridDim.x - nb_a, tileT, red);
 }
@@ -700,8 +738,8 @@ __device__ __forceinline__ void resident_body(const CastJob& j, uint32_t bid, ui
     if ((t & 63) == 0) red[t >> 6] = m;
     __syncthreads();
     if (t == 0) publish_word(j.tagged, bid, max(max(red[0], red[1]), max(red[2], red[3])));
-    if (!collect_words<1>(j.tagged, nb, m, red + CAST_THREADS / 64)) {
-        m = collect_late<DT, H, 1>(j, bid, nb, red);
+    if (__builtin_expect(!collect_words<1>(j.tagged, nb, m, red + CAST_THREADS / 64), 0)) {
+        m = collect_late<DT, H>(j, bid, nb, red);
         // The tile again: held meanwhile, it or its addresses would cost every launch registers, and a CU a workgroup.
         int64_t again = r0;
         asm volatile("" : "+s"(again));
@@ -823,7 +861,6 @@ static unsigned unused_lds(int in_dtype, int64_t tiles) {
     const bool wide = in_dtype == F8MI_FP32;
     return tiles >= (wide ? 8 : 12) * (int64_t)cu_count() ? (wide ? UNUSED_LDS_32 : UNUSED_LDS_16) : 0u;
 }
-
 template <int DT, int PROD, int FMT>
 static int launch_cast2(dim3 g, hipStream_t stream, const CastJob& j) {
     if constexpr (PROD == F8MI_FP32) {  // what delayed scaling computes in
@@ -957,8 +994,8 @@ extern "C" int f8mi_cast_delayed(const void* x, int64_t rows, int64_t cols, int6
 namespace f8mi {
 
 // Rows of the tiles that the one-launch cast gives a tensor, 0: it does not take it.  At most four workgroups a CU (RESIDENT_TILES on
-// 256) of the eight that it holds, seven of 128 rows, five of 128 rows of fp32: a launch that is alone has them all there at once, with
-// room for a small one beside it.
+// 256) of the eight that it holds, five of 128 rows of fp32: a launch that is alone has them all there at once, with room for another
+// beside it (fp32: for a small one).
 static int resident_tile_rows(int64_t rows, int64_t cols) {
     const int64_t tx = (cols + CAST_TILE - 1) / CAST_TILE, ty = (rows + CAST_TILE - 1) / CAST_TILE, most = std::min(RESIDENT_TILES, 4 * cu_count());
     if (ty > most || tx > most) return 0;

@@ -118,14 +118,22 @@ def casts(tmp_path_factory):
 
 
 def test_one_launch_casts_leave_room_beside_them(casts):
-    """At most four workgroups a CU of a cast that holds its tensor on the chip, out of the eight, with 128-row tiles seven (fp32
-    five) that its registers allow: one register too many, and a launch that is alone has workgroups without room."""
+    """At most four workgroups a CU of a cast that holds its tensor on the chip, out of the eight (fp32 with 128-row tiles: five) that
+    its registers allow: a few registers too many, and a launch that is alone has workgroups without room."""
     kernels = [k for k in casts if "resident" in k[0]]
     assert len(kernels) == 3 * 2 * 2 + 5 * 2
     for name, codes, _, scratch, vgprs in kernels:
         types = codes[:2] if "pair" in name else codes[:1]
-        workgroups = 8 if codes[-1] == 1 else 5 if 2 in types else 7
+        workgroups = 5 if codes[-1] == 2 and 2 in types else 8
         assert scratch == 0 and vgprs <= 512 // workgroups // 8 * 8, (name, codes, vgprs)
+
+
+def test_16_bit_casts_that_collect_their_maximum_hold_as_many_workgroups_as_those_that_do_not(casts):
+    """Eight a CU: 2048 tiles, the most that one launch collects for, all fit at once."""
+    kernels = [k for k in casts if k[0] in ("cast_kernel", "cast_pair_kernel") and k[1][-1] == 1 and 2 not in (k[1][:2] if "pair" in k[0] else k[1][:1])]
+    assert len(kernels) == 2 * 2 + 2
+    for name, codes, _, scratch, vgprs in kernels:
+        assert scratch == 0 and vgprs <= 64, (name, codes, vgprs)
 
 
 def test_casts_of_many_tiles_run_with_the_workgroups_they_are_held_to(casts):
