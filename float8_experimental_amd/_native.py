@@ -49,6 +49,7 @@ EXPORTS = (
     "f8mi_cast_dynamic_resident",
     "f8mi_cast_dynamic_pair",
     "f8mi_cast_delayed_pair",
+    "f8mi_cast_one_launch",
     "f8mi_linear_few_rows",
     "f8mi_gemm_weight_only",
     "f8mi_dequant",
@@ -122,6 +123,8 @@ def lib() -> C.CDLL:
         for pair in (L.f8mi_cast_dynamic_pair, L.f8mi_cast_delayed_pair):
             pair.restype = i32
             pair.argtypes = [vp, vp, vp, vp]
+        L.f8mi_cast_one_launch.restype = i32
+        L.f8mi_cast_one_launch.argtypes = [vp, vp, i32, C.c_uint32, vp]
         L.f8mi_gemm_nt_kb.restype = i32
         L.f8mi_gemm_nt_kb.argtypes = [vp, i32, vp, i32, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp]
         L.f8mi_gemm_kb_ex.restype = i32

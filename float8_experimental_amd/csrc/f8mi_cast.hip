@@ -974,17 +974,28 @@ static bool one_launch_delayed(int64_t rows, int64_t cols) {
 }
 }  // namespace f8mi
 
+// F8MI_ERR_UNSUPPORTED, and nothing queued: not in one launch.
+static int cast_delayed_one_launch(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, const float* scale_dev, int fp8_fmt, uint8_t* out,
+                                   int out_layout, uint8_t* out_t, int out_t_layout, float* amax_dev, uint32_t wait_ticks, hipStream_t stream) {
+    if (rows <= 0 || cols <= 0 || !one_launch_delayed(rows, cols)) return F8MI_ERR_UNSUPPORTED;
+    AmaxSource src{};
+    if (const int rc = begin_exchange(stream, wait_ticks, src.tagged)) return rc;
+    if (!src.tagged.words) return F8MI_ERR_UNSUPPORTED;
+    return cast_layout_impl(x, rows, cols, ld, in_dtype, scale_dev, F8MI_FP32, fp8_fmt, out, out_layout, out_t, out_t_layout, amax_dev, stream, src);
+}
+
 extern "C" int f8mi_cast_delayed(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, const float* scale_dev, int fp8_fmt,
                                  uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout, float* amax_dev, void* workspace,
                                  void* stream) {
     if (!amax_dev) { set_error("f8mi_cast_delayed: null amax"); return F8MI_ERR_INVALID_ARG; }
     if (!workspace || (uintptr_t)workspace % 4 != 0) { set_error("f8mi_cast_delayed: null or misaligned workspace"); return F8MI_ERR_INVALID_ARG; }
+    {
+        const int rc = cast_delayed_one_launch(x, rows, cols, ld, in_dtype, scale_dev, fp8_fmt, out, out_layout, out_t, out_t_layout, amax_dev,
+                                               EXCHANGE_WAIT_TICKS_LAST, (hipStream_t)stream);
+        // (a cast that is refused for its layouts is refused again below, with the same message)
+        if (rc != F8MI_ERR_UNSUPPORTED) return rc;
+    }
     AmaxSource src{};
-    if (rows > 0 && cols > 0 && one_launch_delayed(rows, cols))
-        if (const int rc = begin_exchange((hipStream_t)stream, EXCHANGE_WAIT_TICKS_LAST, src.tagged)) return rc;
-    if (src.tagged.words)
-        return cast_layout_impl(x, rows, cols, ld, in_dtype, scale_dev, F8MI_FP32, fp8_fmt, out, out_layout, out_t, out_t_layout, amax_dev,
-                                (hipStream_t)stream, src);
     src.spread = (uint32_t*)workspace;
     const std::lock_guard<std::mutex> guard(f8mi::delayed_lock(workspace));
     return cast_layout_impl(x, rows, cols, ld, in_dtype, scale_dev, F8MI_FP32, fp8_fmt, out, out_layout, out_t, out_t_layout, amax_dev,
@@ -1158,33 +1169,61 @@ static int launch_cast_pair(int dt_a, int dt_b, int tile_rows, hipStream_t strea
     return launch_cast_pair1<F8MI_FP32, F8MI_FP32, TAGGED>(tile_rows, stream, a, b);
 }
 
+
+// Both casts in the launch that exchanges maxima.  F8MI_ERR_UNSUPPORTED, and nothing queued: not in one.
+static int cast_dynamic_pair_one_launch(const f8mi_cast_job& a, const f8mi_cast_job& b, uint32_t wait_ticks, hipStream_t stream) {
+    const int tile_rows = resident_tile_rows((tiles_of(a) + tiles_of(b)) * CAST_TILE, CAST_TILE);
+    if (!tile_rows) return F8MI_ERR_UNSUPPORTED;
+    TaggedWords tagged;
+    if (const int rc = begin_exchange(stream, wait_ticks, tagged)) return rc;
+    if (!tagged.words) return F8MI_ERR_UNSUPPORTED;
+    CastJob ja = kernel_job(a, tile_rows), jb = kernel_job(b, tile_rows);
+    ja.scale_out = a.scale_dev;
+    jb.scale_out = b.scale_dev;
+    ja.tagged = jb.tagged = tagged;
+    jb.tagged.words += ja.tiles_x * ja.tiles_y;
+    ProfScope prof(F8MI_K_CAST, job_bytes(a) + job_bytes(b), stream);
+    return launch_cast_pair<false>(a.in_dtype, b.in_dtype, tile_rows, stream, ja, jb);
+}
+static int cast_delayed_pair_one_launch(const f8mi_cast_job& a, const f8mi_cast_job& b, uint32_t wait_ticks, hipStream_t stream) {
+    if (!a.amax_dev || !b.amax_dev || !one_launch_delayed((tiles_of(a) + tiles_of(b)) * CAST_TILE, CAST_TILE)) return F8MI_ERR_UNSUPPORTED;
+    TaggedWords tagged;
+    if (const int rc = begin_exchange(stream, wait_ticks, tagged)) return rc;
+    if (!tagged.words) return F8MI_ERR_UNSUPPORTED;
+    CastJob ja = kernel_job(a, CAST_TILE), jb = kernel_job(b, CAST_TILE);
+    ja.scale_dev = a.scale_dev;
+    jb.scale_dev = b.scale_dev;
+    ja.amax_out = a.amax_dev;
+    jb.amax_out = b.amax_dev;
+    ja.tagged = jb.tagged = tagged;
+    jb.tagged.words += ja.tiles_x * ja.tiles_y * (CAST_THREADS / 64);
+    ProfScope prof(F8MI_K_CAST, job_bytes(a) + job_bytes(b), stream);
+    return launch_cast_pair<true>(a.in_dtype, b.in_dtype, 0, stream, ja, jb);
+}
+
 }  // namespace f8mi
+
+extern "C" int f8mi_cast_one_launch(const f8mi_cast_job* a, const f8mi_cast_job* b, int delayed, uint32_t wait_ticks, void* stream_) {
+    hipStream_t stream = (hipStream_t)stream_;
+    if (!a || !pair_ok(*a, b ? *b : *a) || (delayed && (!a->amax_dev || (b && !b->amax_dev)))) { set_error("f8mi_cast_one_launch: bad job"); return F8MI_ERR_INVALID_ARG; }
+    int rc;
+    if (b) rc = delayed ? cast_delayed_pair_one_launch(*a, *b, wait_ticks, stream) : cast_dynamic_pair_one_launch(*a, *b, wait_ticks, stream);
+    else if (delayed) rc = cast_delayed_one_launch(a->x, a->rows, a->cols, a->ld, a->in_dtype, a->scale_dev, F8MI_E4M3FN, a->out, a->out_layout, a->out_t, a->out_t_layout, a->amax_dev, wait_ticks, stream);
+    else return f8mi_cast_dynamic_resident(a->x, a->rows, a->cols, a->ld, a->in_dtype, F8MI_E4M3FN, a->scale_dev, a->out, a->out_layout, a->out_t, a->out_t_layout, wait_ticks, stream_);
+    if (rc == F8MI_ERR_UNSUPPORTED) set_error("f8mi_cast_one_launch: more tiles than one launch takes, or a stream that is being captured");
+    return rc;
+}
 
 extern "C" int f8mi_cast_dynamic_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream_) {
     hipStream_t stream = (hipStream_t)stream_;
     if (!a || !b) { set_error("f8mi_cast_dynamic_pair: null job"); return F8MI_ERR_INVALID_ARG; }
     if (workspace && (uintptr_t)workspace % 16 == 0 && pair_ok(*a, *b)) {
-        const int64_t tiles_a = tiles_of(*a), tiles_b = tiles_of(*b);
-        CastJob ja, jb;
-        if (const int tile_rows = resident_tile_rows((tiles_a + tiles_b) * CAST_TILE, CAST_TILE)) {
-            TaggedWords tagged;
-            if (const int rc = begin_exchange(stream, EXCHANGE_WAIT_TICKS, tagged)) return rc;
-            if (tagged.words) {
-                ja = kernel_job(*a, tile_rows);
-                jb = kernel_job(*b, tile_rows);
-                ja.scale_out = a->scale_dev;
-                jb.scale_out = b->scale_dev;
-                ja.tagged = jb.tagged = tagged;
-                jb.tagged.words += ja.tiles_x * ja.tiles_y;
-                ProfScope prof(F8MI_K_CAST, job_bytes(*a) + job_bytes(*b), stream);
-                return launch_cast_pair<false>(a->in_dtype, b->in_dtype, tile_rows, stream, ja, jb);
-            }
-        }
+        const int one = cast_dynamic_pair_one_launch(*a, *b, EXCHANGE_WAIT_TICKS, stream);
+        if (one != F8MI_ERR_UNSUPPORTED) return one;
         // one of them too large for a launch of its own: both through the two launches it takes
         if (two_launches_pay(*a, *b) && a->ld && b->ld &&
             amax_pair_ok(a->x, a->rows, a->cols, a->ld, b->x, b->rows, b->cols, b->ld)) {
-            ja = kernel_job(*a, CAST_TILE);
-            jb = kernel_job(*b, CAST_TILE);
+            CastJob ja = kernel_job(*a, CAST_TILE), jb = kernel_job(*b, CAST_TILE);
             ja.scale_out = a->scale_dev;
             jb.scale_out = b->scale_dev;
             ja.amax_ws = (const uint32_t*)workspace;
@@ -1207,20 +1246,9 @@ extern "C" int f8mi_cast_dynamic_pair(const f8mi_cast_job* a, const f8mi_cast_jo
 extern "C" int f8mi_cast_delayed_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream_) {
     hipStream_t stream = (hipStream_t)stream_;
     if (!a || !b) { set_error("f8mi_cast_delayed_pair: null job"); return F8MI_ERR_INVALID_ARG; }
-    if (pair_ok(*a, *b) && a->amax_dev && b->amax_dev && one_launch_delayed((tiles_of(*a) + tiles_of(*b)) * CAST_TILE, CAST_TILE)) {
-        TaggedWords tagged;
-        if (const int rc = begin_exchange(stream, EXCHANGE_WAIT_TICKS_LAST, tagged)) return rc;
-        if (tagged.words) {
-            CastJob ja = kernel_job(*a, CAST_TILE), jb = kernel_job(*b, CAST_TILE);
-            ja.scale_dev = a->scale_dev;
-            jb.scale_dev = b->scale_dev;
-            ja.amax_out = a->amax_dev;
-            jb.amax_out = b->amax_dev;
-            ja.tagged = jb.tagged = tagged;
-            jb.tagged.words += ja.tiles_x * ja.tiles_y * (CAST_THREADS / 64);
-            ProfScope prof(F8MI_K_CAST, job_bytes(*a) + job_bytes(*b), stream);
-            return launch_cast_pair<true>(a->in_dtype, b->in_dtype, 0, stream, ja, jb);
-        }
+    if (pair_ok(*a, *b)) {
+        const int rc = cast_delayed_pair_one_launch(*a, *b, EXCHANGE_WAIT_TICKS_LAST, stream);
+        if (rc != F8MI_ERR_UNSUPPORTED) return rc;
     }
     for (const f8mi_cast_job* j : {a, b})
         if (const int rc = f8mi_cast_delayed(j->x, j->rows, j->cols, j->ld, j->in_dtype, j->scale_dev, F8MI_E4M3FN, j->out, j->out_layout, j->out_t, j->out_t_layout, j->amax_dev,

@@ -259,6 +259,10 @@ typedef struct f8mi_cast_job {
 int f8mi_cast_dynamic_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream);
 /* f8mi_cast_delayed of `a`, then of `b`, both to e4m3, in one launch up to 2048 tiles together. */
 int f8mi_cast_delayed_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream);
+/* The one launch of these two, or, with b null, of f8mi_cast_dynamic_resident and of f8mi_cast_delayed (to e4m3), by itself, with wait_ticks as
+ * there (in a delayed cast one workgroup collects, and reads the whole tensor when it gives up).  F8MI_ERR_UNSUPPORTED, nothing
+ * queued, where they do not take it. */
+int f8mi_cast_one_launch(const f8mi_cast_job* a, const f8mi_cast_job* b, int delayed, uint32_t wait_ticks, void* stream);
 
 /* A whole linear of at most 16 rows and F8MI_FEW_ROWS_ELEMS activations in one kernel: c[m][n] = sum_k x8[m][k] * w[n][k]
  * / (scale_x * scale_w) (+ bias[n]) with x8 the saturated e4m3 cast of x, which every workgroup makes for itself.  The same

@@ -3,6 +3,7 @@
 Bars: amax, scales and fp8 bytes bit-exact (NaN codes may differ in the sign
 bit); GEMM within a stated tolerance of the emulated fp32 product.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -640,7 +641,6 @@ def test_cast_dynamic_resident_on_several_streams_and_what_it_refuses(nat):
 def test_cast_dynamic_resident_serves_every_stream(nat):
     """64 streams of a device have words of their own; those of streams that are gone go to new ones.  One handle is a stream of its
     own in every thread."""
-    import ctypes
     import threading
 
     with open("/proc/self/maps") as f:
@@ -723,18 +723,64 @@ def test_cast_dynamic_resident_costs_little_when_workgroups_are_late(nat):
         assert all(torch.equal(o, w) for o, w in zip(outs, want))
 
 
+class CastJob(ctypes.Structure):  # f8mi_cast_job
+    _fields_ = ([("x", ctypes.c_void_p)] + [(f, ctypes.c_int64) for f in ("rows", "cols", "ld")] + [(f, ctypes.c_void_p) for f in ("scale", "out", "out_t", "amax")] +
+                [(f, ctypes.c_int) for f in ("dtype", "layout", "layout_t")])
+
+
+# The casts that exchange maxima in their launch, where nobody waits for anybody: the collecting workgroups find the maximum themselves, which
+# has to be the same.  One tile, edges in both directions, several tiles a window of words; row-strided and repeated rows; NaN, infinity.
+@pytest.mark.parametrize("dts", ["bf16 bf16", "fp16 fp16", "fp32 fp32", "bf16 fp32", "fp16 fp32"])
+@pytest.mark.parametrize("shapes", [((1, 1), (1, 1)), ((129, 257), (64, 130)), ((1000, 3001), (513, 1031)), ((2048, 4096), (4096, 2048))])
+def test_one_launch_casts_that_do_not_wait(nat, dts, shapes):
+    f8dt = torch.float8_e4m3fn
+    base = [heavy(s, TORCH_DT[d], 60 + i).to(DEV) for i, (s, d) in enumerate(zip(shapes, dts.split()))]
+    special = [x.clone() for x in base]
+    special[0].view(-1)[-1], special[1].view(-1)[0] = float("nan"), float("-inf")
+    strided = [torch.zeros(x.shape[0], x.shape[1] + 5, device=DEV, dtype=x.dtype)[:, 3:x.shape[1] + 3].copy_(x) for x in base]
+    repeated = [x[-1:].expand(x.shape) for x in base]
+    for xs in (base, special, strided, repeated):
+        for delayed in (False, True):
+            want = []
+            for x, s in zip(xs, (3.0, 700.0)):
+                amax, s_dyn = nat.amax_scale(x.contiguous(), f8dt)
+                scale = torch.tensor([s], device=DEV) if delayed else s_dyn
+                q, qt = nat.cast(x.contiguous(), scale, f8dt, product_dtype=torch.float32 if delayed else None, want_out_t=True, out_kblock=2, out_t_kblock=2)
+                want.append((q, qt, scale, amax))
+            for which in ((0,), (1,), (0, 1)):
+                jobs, got = (CastJob * 2)(), []
+                for i in which:
+                    x, job = xs[i], jobs[i]
+                    q, qt = (torch.zeros_like(t.view(torch.uint8)) for t in want[i][:2])
+                    scale, amax = want[i][2].clone() if delayed else torch.zeros((), device=DEV), torch.full((1,), -1.0, device=DEV)
+                    got.append((q, qt, scale, amax))
+                    job.x, job.rows, job.cols, job.ld, job.dtype = x.data_ptr(), *x.shape, x.stride(0), nat._DT[x.dtype]
+                    job.scale, job.amax, job.layout, job.layout_t, job.out, job.out_t = scale.data_ptr(), amax.data_ptr(), 2, 2, q.data_ptr(), qt.data_ptr()
+                rc = nat.lib().f8mi_cast_one_launch(ctypes.byref(jobs[which[0]]), ctypes.byref(jobs[1]) if len(which) == 2 else None, int(delayed), 0, nat._stream(xs[0]))
+                assert rc == 0, nat.lib().f8mi_last_error()
+                for i, (q, qt, scale, amax) in zip(which, got):
+                    assert same_bytes_mod_nan_sign(fp8_bytes(q), fp8_bytes(want[i][0])) and same_bytes_mod_nan_sign(fp8_bytes(qt), fp8_bytes(want[i][1])), (which, delayed)
+                    assert torch.equal(scale, want[i][2]) or (torch.isnan(scale).all() and torch.isnan(want[i][2]).all())
+                    assert not delayed or amax.item() == want[i][3].item() or (math.isnan(amax.item()) and math.isnan(want[i][3].item()))
+
+
+def test_one_launch_casts_refuse_what_is_larger(nat):
+    x = torch.zeros(8193, 4096, device=DEV, dtype=torch.bfloat16)
+    out, s, amax = torch.zeros(8193, 4096, device=DEV, dtype=torch.uint8), torch.ones(1, device=DEV), torch.zeros(1, device=DEV)
+    job = CastJob(x.data_ptr(), 8193, 4096, 4096, s.data_ptr(), out.data_ptr(), None, amax.data_ptr(), 0, 0, 0)
+    small = CastJob(x.data_ptr(), 64, 4096, 4096, s.data_ptr(), out.data_ptr(), None, amax.data_ptr(), 0, 0, 0)
+    call = lambda *a: nat.lib().f8mi_cast_one_launch(*(ctypes.byref(j) if j else None for j in a[:2]), a[2], 0, nat._stream(x))
+    assert [call(job, None, 0), call(job, None, 1), call(small, job, 0), call(small, job, 1)] == [-2] * 4
+    small.amax = None
+    assert call(small, None, 0) == 0 and call(small, None, 1) == -1 and call(None, None, 0) == -1
+
+
 # Two tensors in one call: tiny, tiles of 64 and of 128 rows, the most that one launch takes together (1024 tiles, delayed 2048) and one row
 # more, one or both too large for it, ragged and row-strided.
 @pytest.mark.parametrize("dts", ["bf16 bf16", "fp16 fp16", "fp32 fp32", "bf16 fp32", "fp16 fp32", "fp32 bf16"])
 @pytest.mark.parametrize("shapes", [((1, 1), (1, 1)), ((64, 128), (65, 129)), ((512, 1024), (1024, 1024)), ((2048, 2048), (6144, 2048)), ((2049, 2048), (6144, 2048)),
                                     ((8192, 2048), (8193, 1024)), ((8192, 4096), (300, 4096)), ((4099, 4097), (1001, 4097)), ((4099, 4096), (4480, 4096))])
 def test_cast_of_two_tensors_equals_two_casts(nat, dts, shapes):
-    import ctypes as C
-
-    class Job(C.Structure):
-        _fields_ = ([("x", C.c_void_p)] + [(f, C.c_int64) for f in ("rows", "cols", "ld")] + [(f, C.c_void_p) for f in ("scale", "out", "out_t", "amax")] +
-                    [(f, C.c_int) for f in ("dtype", "layout", "layout_t")])
-
     f8dt, tdts = torch.float8_e4m3fn, [TORCH_DT[d] for d in dts.split()]
     base = [heavy(s, t, 40 + i).to(DEV) for i, (s, t) in enumerate(zip(shapes, tdts))]
     nan = [x.clone() for x in base]
@@ -745,7 +791,7 @@ def test_cast_of_two_tensors_equals_two_casts(nat, dts, shapes):
             for delayed in (False, True):
                 scales = [torch.tensor([s], device=DEV) if delayed else torch.zeros((), device=DEV) for s in (3.0, 700.0)]
                 amaxes, outs, want = [torch.full((1,), -1.0, device=DEV) for _ in xs], [], []
-                jobs = (Job * 2)()
+                jobs = (CastJob * 2)()
                 for x, s, a, job in zip(xs, scales, amaxes, jobs):
                     wa = torch.zeros((1,), device=DEV)
                     if delayed:
@@ -760,9 +806,9 @@ def test_cast_of_two_tensors_equals_two_casts(nat, dts, shapes):
                     job.scale, job.amax, job.layout, job.layout_t = s.data_ptr(), a.data_ptr(), layout, layout
                     job.out, job.out_t = o[0].data_ptr(), o[1].data_ptr() if both else None
                 if delayed:
-                    rc = nat.lib().f8mi_cast_delayed_pair(C.byref(jobs[0]), C.byref(jobs[1]), nat.delayed_workspace(xs[0].device).data_ptr(), nat._stream(xs[0]))
+                    rc = nat.lib().f8mi_cast_delayed_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), nat.delayed_workspace(xs[0].device).data_ptr(), nat._stream(xs[0]))
                 else:
-                    rc = nat.lib().f8mi_cast_dynamic_pair(C.byref(jobs[0]), C.byref(jobs[1]), nat.workspace(xs[0].device).data_ptr(), nat._stream(xs[0]))
+                    rc = nat.lib().f8mi_cast_dynamic_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), nat.workspace(xs[0].device).data_ptr(), nat._stream(xs[0]))
                 assert rc == 0, nat.lib().f8mi_last_error()
                 for (w, wt, ws, wa), o, s, a in zip(want, outs, scales, amaxes):
                     assert same_bytes_mod_nan_sign(fp8_bytes(o[0]), fp8_bytes(w)), (dts, shapes, layout, delayed)
