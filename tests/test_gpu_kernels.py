@@ -301,9 +301,10 @@ def test_cast_kblocked_refused_by_the_library_when_not_a_multiple_of_64(nat):
 
 @pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
 def test_delayed_cast_with_workspace_equals_the_cast_without(nat, dt):
-    """f8mi_cast_delayed folds the amax into the 1024 words of its workspace and a second launch reduces them: same bytes
-    and the same amax as f8mi_cast_layout with amax_dev, the oracle's amax (NaN, inf, all-zero and all-negative-zero
-    tensors included), and the workspace is all zero again after every call -- also on the next, smaller call."""
+    """f8mi_cast_delayed folds the amax of more than 2048 tiles into the 1024 words of its workspace and a second launch reduces them;
+    up to 2048 its launch collects the amax and leaves the workspace alone: same bytes and the same amax as
+    f8mi_cast_layout with amax_dev, the oracle's amax (NaN, inf, all-zero and all-negative-zero tensors included), and the
+    workspace is all zero again after every call -- also on the next call with a smaller amax, of either kind."""
     co, to = _oracles()
     L = nat.lib()
     assert L.f8mi_delayed_workspace_bytes() == 4096
@@ -315,6 +316,10 @@ def test_delayed_cast_with_workspace_equals_the_cast_without(nat, dt):
     inf = heavy((129, 257), TORCH_DT[dt], 7)
     inf[5, 5] = float("-inf")
     cases += [nan, inf]
+    big = heavy((65, 4096), TORCH_DT[dt], 8).repeat(127, 1)  # 65 x 32 tiles: the workspace
+    nan_big = big.clone()
+    nan_big[5000, 17] = float("nan")
+    cases = [nan_big, big, big[:8193] * 0.25, torch.zeros_like(big), big] + cases
     ws = nat.delayed_workspace(torch.device(DEV))
     for x in cases:
         xd = x.to(DEV)

@@ -827,19 +827,20 @@ def test_native_host_path_leaves_what_it_does_not_take_to_the_step_by_step_funct
         assert bad is None
 
 
-def test_delayed_casts_of_two_threads_on_one_stream_keep_their_maxima_apart(f8):
-    """Cast and finalize of one call are two launches over words that calls on one stream share: another thread's cast must not
-    come between them."""
+@pytest.mark.parametrize("shape,calls", [((64, 128), 2000), ((8193, 4096), 100)])
+def test_delayed_casts_of_two_threads_on_one_stream_keep_their_maxima_apart(f8, shape, calls):
+    """Past 2048 tiles cast and finalize of one call are two launches over words that calls on one stream share: another thread's cast
+    must not come between them.  Up to there, calls on one stream share the words that their launches exchange maxima in."""
     import threading
 
     from float8_experimental_amd import _native
 
-    calls, scale = 2000, torch.ones(1, device=DEV)
+    scale = torch.ones(1, device=DEV)
     amaxes = {v: torch.zeros(calls, device=DEV) for v in (1.0, 300.0)}
     start = threading.Barrier(2)
 
     def work(v):
-        x = torch.full((64, 128), v, device=DEV, dtype=torch.bfloat16)
+        x = torch.full(shape, v, device=DEV, dtype=torch.bfloat16)
         out = amaxes[v]
         start.wait()
         for i in range(calls):
