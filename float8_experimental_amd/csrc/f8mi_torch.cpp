@@ -140,7 +140,7 @@ struct Call {
     };
     void cast_two(const Cast& a, const Cast& b) const {
         const bool delayed = a.s.amax.defined() && b.s.amax.defined(), dynamic = !a.s.scale.defined() && !b.s.scale.defined();
-        if (!(delayed && L.cast_delayed_pair) && !(dynamic && L.cast_dynamic_pair)) {
+        if (!delayed && !dynamic) {
             for (const Cast* c : {&a, &b}) cast(c->x, c->s, F8MI_E4M3FN, true, c->row_layout, c->want_tr, c->tr_layout, c->row, c->tr, c->scale);
             return;
         }
@@ -367,9 +367,8 @@ PyObject* load(PyObject*, PyObject* args) {
     get(L.linear_few_rows, "f8mi_linear_few_rows");
     get(L.last_error, "f8mi_last_error");
     get(L.gemm_plan, "f8mi_gemm_plan");
-    // (a library may be without these: the calls they stand for are made one by one then)
-    L.cast_dynamic_pair = reinterpret_cast<decltype(L.cast_dynamic_pair)>(dlsym(h, "f8mi_cast_dynamic_pair"));
-    L.cast_delayed_pair = reinterpret_cast<decltype(L.cast_delayed_pair)>(dlsym(h, "f8mi_cast_delayed_pair"));
+    get(L.cast_dynamic_pair, "f8mi_cast_dynamic_pair");
+    get(L.cast_delayed_pair, "f8mi_cast_delayed_pair");
     if (missing) {
         L.gemm_plan = nullptr;
         return PyErr_Format(PyExc_ImportError, "%s does not export %s", path, missing);

@@ -866,6 +866,8 @@ int f8mi_gemm_plan(int64_t m, int64_t n, int64_t k, int a, int64_t w) { return 0
 int f8mi_cast_dynamic(void) { return slow(); }
 int f8mi_cast_layout(void) { return slow(); }
 int f8mi_cast_delayed(void) { return slow(); }
+int f8mi_cast_dynamic_pair(void) { return slow(); }
+int f8mi_cast_delayed_pair(void) { return slow(); }
 int f8mi_gemm_nt_ws(void) { return slow(); }
 int f8mi_gemm_nt_kb_ws(void) { return slow(); }
 int f8mi_gemm_kb_ex(void) { return slow(); }
