@@ -649,9 +649,10 @@ constexpr int FLAT_UNROLL = 8;  // 16-byte loads in flight per lane of the scan
 constexpr int64_t FLAT_MAX_BYTES = 512 << 10;
 // Past this many bytes the kernel that reads the tensor once (cast_dynamic_resident_kernel) is faster, where the stream has its words:
 // us, this / that: 32 x 4096 (256 KB): 5.5 / 5.8, 48 x 4096: 6.3 / 5.9, 16 x 14336 (448 KB): 7.2 / 6.3, 64 x 4096: 7.3 / 5.9.  Its tiles
-// have 64 rows: with fewer than a quarter of them it is left to this one.
+// have 64 rows, so that few rows are many tiles of mostly nothing: bf16, 8 rows 320 KB 6.44 / 7.31, 448 KB 7.55 / 7.57; 10 rows 6.44 / 6.46, 384 KB 6.66 /
+// 7.11; 12 rows 320 KB 6.52 / 6.38, 384 KB 6.62 / 6.45, 512 KB 7.77 / 7.30; fp32, 4 rows 320 KB 6.34 / 7.20, 8 rows 6.37 / 6.22, 12 rows 6.46 / 6.01.
 constexpr int64_t FLAT_BEST_BYTES = 320 << 10;
-constexpr int64_t FLAT_BEST_ROWS = 16;
+constexpr int64_t FLAT_BEST_ROWS = 12;
 
 template <int DT, int FMT>
 __global__ __launch_bounds__(FLAT_THREADS) void cast_dynamic_flat_kernel(const uint8_t* __restrict__ x, uint32_t rows, uint32_t cols,

@@ -565,7 +565,7 @@ def test_cast_dynamic_one_copy_equals_amax_scale_then_cast(nat, dt, shape):
 
 # The line between the kernels that read such a tensor once and once a workgroup, on either side; captured, the latter again.
 @pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
-@pytest.mark.parametrize("shape", [(40, 4096), (41, 4096), (15, 14336), (16, 14336), (20, 4096), (21, 4096), (15, 8192), (16, 8192), (64, 4096)])
+@pytest.mark.parametrize("shape", [(40, 4096), (41, 4096), (15, 14336), (16, 14336), (20, 4096), (21, 4096), (15, 8192), (16, 8192), (64, 4096), (11, 20480), (12, 20480)])
 def test_cast_dynamic_either_side_of_the_flat_kernel(nat, dt, shape):
     x = heavy(shape, TORCH_DT[dt], 33).to(DEV)
     for fmt, (code, f8dt) in F8.items():
