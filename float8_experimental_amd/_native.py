@@ -318,7 +318,8 @@ PLAN_NAMES = {1: "tiles128_split_k", 2: "few_rows", 3: "tiles128", 4: "tiles256"
 
 def gemm_plan(m: int, n: int, k: int, aligned: bool = True, split_k: bool = True):
     """(kernel name, parts of k, 0 / 1 / 2 for none / 128 x 128 / 128 x 256 tiles) the library picks for an m x n x k
-    product, as gemm_nt / gemm_nt_kb call it (``split_k``: with the scratch buffer they pass).  Needs no GPU."""
+    product into a dense 16-bit output, as gemm_nt / gemm_nt_kb call it (``split_k``: with the scratch buffer they pass).  Needs no
+    GPU."""
     ws = GEMM_WORKSPACE_BYTES if split_k and m >= _GEMM_WS_MIN_ROWS and k >= _GEMM_WS_MIN_K else 0
     code = lib().f8mi_gemm_plan(m, n, k, int(aligned), ws)
     return PLAN_NAMES.get(code & 0xff), (code >> 8) & 0xff, (code >> 16) & 0xff

@@ -127,7 +127,8 @@ __global__ __launch_bounds__(AMAX_THREADS) void amax_dense_kernel(const void* __
     amax_dense_body<DT, NT>(x, n, ws, blockIdx.x, gridDim.x, red);
 }
 
-// Two tensors in one launch, the first nb_a blocks for the first.
+// Two tensors in one launch, the first nb_a blocks for the first.  Non-temporal loads at every size, as the shipped rule for one tensor has
+// them (F8MI_AMAX_PLAIN_LOADS_MAX_BYTES is 0 and does not reach here).
 template <int DTA, int DTB>
 __global__ __launch_bounds__(AMAX_THREADS) void amax_dense_pair_kernel(const void* __restrict__ xa, int64_t na, uint32_t* __restrict__ ws_a, uint32_t nb_a,
                                                                        const void* __restrict__ xb, int64_t nb, uint32_t* __restrict__ ws_b) {

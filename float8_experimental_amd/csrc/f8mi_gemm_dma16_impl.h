@@ -10,7 +10,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int SLAB_BYTES = 256 * 128;   // one operand, one step
 constexpr int HALF_BYTES = 256 * 64;    // one 64-deep unit of it
 constexpr int NSLAB_A = 3, NSLAB_B = 2;
-constexpr int DMA16_LDS = (NSLAB_A + NSLAB_B) * SLAB_BYTES;  // 160 KB
 
 // TJ = 16-column tiles per wave: 8 -> 256 x 256 workgroup tiles; 7 -> 256 x 224 (see narrow_tiles_pay), operands as they are and rows of
 // C at multiples of four bytes only.

@@ -299,7 +299,7 @@ int f8mi_gemm_nt_kb(const void* a, int a_fmt, const void* bt, int b_fmt, int64_t
  * hundred rows and a long contraction, which would otherwise leave most CUs idle: partial sums go to the workspace
  * and a second kernel adds them in a fixed order (deterministic; another summation order than without the split,
  * so the two agree within the accumulation tolerance, not bit for bit).  Which path runs depends on (m, n, k),
- * alignment and workspace_bytes only; F8MI_GEMM_WORKSPACE_BYTES is enough for every case that is ever split.
+ * alignment (of the operands and of C's rows) and workspace_bytes only; F8MI_GEMM_WORKSPACE_BYTES is enough for every case that is ever split.
  * With workspace NULL they are f8mi_gemm_nt / f8mi_gemm_nt_kb.  No counterpart in the reference (torch._scaled_mm
  * hides hipBLASLt's own workspace, float8_python_api.py:24-64). */
 #define F8MI_GEMM_WORKSPACE_BYTES (32ll << 20)
@@ -311,7 +311,8 @@ int f8mi_gemm_nt_kb_ws(const void* a, int a_fmt, const void* bt, int b_fmt, int6
                        const void* bias_dev, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Which kernel f8mi_gemm_nt(_ws) / f8mi_gemm_nt_kb(_ws) would run for an m x n x k product (no GPU needed; for tests,
- * logs and benchmarks).  `aligned`: operands and row strides are 16-byte aligned (k-blocked operands always are);
+ * logs and benchmarks) into a dense 16-bit C.  (Where n is odd, an fp32 C, or one whose rows all start at multiples of four
+ * bytes, may take F8MI_PLAN_TILES256X224 instead of 256 x 256 tiles: the same bits.)  `aligned`: operands and row strides are 16-byte aligned (k-blocked operands always are);
  * workspace_bytes: 0 without a workspace.  Returns a F8MI_PLAN_* code in bits 0-7, the number of parts k is split
  * into in bits 8-15 and, where 128-row tiles take part, 1 (128 x 128) or 2 (128 x 256) in bits 16-23; 0 for an
  * empty product.  No counterpart in the reference. */

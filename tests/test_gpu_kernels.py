@@ -880,10 +880,7 @@ def test_gemm_dma_kernel_shapes(nat, m, n, k, out_dt):
     _gemm_check(nat, m, n, k, "e5m2", "e4m3", out_dt, seed=m + n + k, bias=(m % 2 == 0))
 
 
-# Few rows (m <= 256, k % 128 == 0, aligned): the kernel that streams Bt straight into the matrix cores and splits k
-# over the eight waves of a workgroup.  m around the 16-row tile edges, n ragged against the 32-column
-# workgroups, k from one step (seven idle waves) over nine (uneven split) to a long one.
-# Tiles of 256 x 224: whole ones, a last column of tiles of 1, 111, 113 and 223 columns, ragged rows, an odd and an even number of steps,
+# Tiles of 256 x 224: whole ones, a last column of tiles of 2, 112, 114, 220 and 222 columns, ragged rows, an odd and an even number of steps,
 # every output type, against 128-row tiles (the same order of additions, hence the same bits) of both ends of the rows.
 @pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("m,n,k", [(2048, 14336, 512), (2000, 14112 + 2, 384), (2048, 14112 + 112, 384), (1801, 14112 + 114, 640), (2048, 14112 + 222, 512), (2047, 14332, 384)])
@@ -901,6 +898,28 @@ def test_gemm_narrow_tiles_equal_128_row_tiles_bitwise(nat, m, n, k, out_dt):
                 assert nat.gemm_plan(rows.stop - rows.start, cols.stop - cols.start, k)[0] == "tiles128"
                 want = nat.gemm_nt(a[rows], sa, bt[cols], sb, out_dt, bias=None if b is None else b[cols].contiguous())
                 assert torch.equal(got[rows, cols], want), (rows, cols)
+
+
+# An odd number of columns: 1, 111, 113 and 223 in the last column of tiles.  The plan answers for a dense 16-bit C, whose odd rows are for the
+# large tiles; fp32, and 16-bit rows at an even pitch, take these.
+@pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(2048, 14112 + 1, 384), (2000, 14112 + 111, 512), (1801, 14112 + 113, 640), (2048, 14112 + 223, 384)])
+def test_gemm_narrow_tiles_of_odd_columns(nat, m, n, k, out_dt):
+    assert nat.gemm_plan(m, n + 1, k)[0] == "tiles256x224" and nat.gemm_plan(m, n, k)[0] == "tiles256"
+    pitch = n if out_dt == torch.float32 else n + 1
+    a, bt = _rand_fp8((m, k), torch.float8_e4m3fn, 63).to(DEV), _rand_fp8((n, k), torch.float8_e5m2, 64).to(DEV)
+    sa, sb = torch.tensor(3.0, device=DEV), torch.tensor(0.37, device=DEV)
+    bias = torch.linspace(-1, 1, n).to(out_dt).to(DEV)
+    for b in (None, bias):
+        buf = torch.full((m + 1, pitch), 7.0, device=DEV, dtype=out_dt)
+        rc = nat.lib().f8mi_gemm_nt(a.data_ptr(), 0, k, bt.data_ptr(), 1, k, m, n, k, sa.data_ptr(), sb.data_ptr(), buf.data_ptr(), nat._DT[out_dt], pitch,
+                                    None if b is None else b.data_ptr(), nat._stream(a))
+        assert rc == 0, nat.lib().f8mi_last_error()
+        assert (buf[m] == 7).all() and (buf[:m, n:] == 7).all()
+        for rows in (slice(0, 272), slice(m - 300, m)):
+            for cols in (slice(0, 4096), slice(4096, 8192), slice(8192, 12288), slice(12288, n)):
+                want = nat.gemm_nt(a[rows], sa, bt[cols], sb, out_dt, bias=None if b is None else b[cols].contiguous())
+                assert torch.equal(buf[rows, cols], want), (rows, cols)
 
 
 # Rows of C that start at odd multiples of two bytes (an odd pitch, or a C that starts at one): every column remainder of a lane's eight
@@ -926,6 +945,9 @@ def test_gemm_rows_of_c_at_odd_addresses(nat, m, k, n, out_dt):
         assert torch.equal(product(pitch, start), want), (pitch, start)
 
 
+# Few rows (m <= 256, k % 128 == 0, aligned): the kernel that streams Bt straight into the matrix cores and splits k
+# over the eight waves of a workgroup.  m around the 16-row tile edges, n ragged against the 32-column
+# workgroups, k from one step (seven idle waves) over nine (uneven split) to a long one.
 @pytest.mark.parametrize("m", [1, 5, 16, 17, 32, 33, 64, 65, 100, 128, 129, 200, 256])
 @pytest.mark.parametrize("n,k", [(7, 128), (32, 256), (200, 1152), (1000, 1024), (96, 8192)])
 def test_gemm_few_rows_shapes(nat, m, n, k):
