@@ -199,6 +199,28 @@ def test_cast_fp32_bit_patterns(nat, fmt):
 
 @pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+def test_cast_bit_patterns_within_the_largest_code(nat, dt, fmt):
+    """The same where no wave needs the clamp, as it takes other instructions: every 16-bit pattern, and fp32 patterns of every
+    exponent, whose product stays below the largest code, under scales from tiny to large; products in either type."""
+    _, tdt = F8[fmt]
+    if dt == "fp32":
+        rng = np.random.default_rng(7)
+        bits = np.concatenate([np.arange(0, 2**32, 16381, dtype=np.uint64).astype(np.uint32), rng.integers(0, 2**32, size=256 * 1024, dtype=np.uint64).astype(np.uint32)])
+        every = torch.from_numpy(bits.view(np.float32).copy())
+    else:
+        every = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(TORCH_DT[dt])
+    for s in (1.0, -1.0, 0.37, 1234.5, 2.0**-30, 2.0**20):
+        sc = torch.tensor(s, dtype=torch.float32)
+        x = every[(every.float() * s).abs() <= (440.0 if fmt == "e4m3" else 56000.0)]
+        x = torch.nn.functional.pad(x, (0, -x.numel() % 256)).reshape(-1, 256)
+        for delayed in (False, True):
+            out, out_t = nat.cast(x.to(DEV), sc.to(DEV), tdt, product_dtype=torch.float32 if delayed else TORCH_DT[dt], want_out_t=True)
+            assert np.array_equal(fp8_bytes(out), np.asarray(_ref_cast(x, sc, tdt, delayed)).reshape(x.shape)), (s, delayed)
+            assert np.array_equal(fp8_bytes(out_t), fp8_bytes(out).T)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
 def test_cast_of_tiles_around_the_largest_code(nat, dt, fmt):
     """A wave leaves the clamp out where its products stay below the middle past the largest code: one magnitude a tile, below, at
     and above that line, of either sign, under scales of either sign, and tiles of it with one larger, infinite or NaN element."""
