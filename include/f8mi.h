@@ -192,8 +192,10 @@ int f8mi_cast_layout(const void* x, int64_t rows, int64_t cols, int64_t ld, int 
  * (float8_scaling_utils.py:65-96: amax_buffer.fill_(tensor_to_amax(x)), then the cast with the stale scale).
  * Same bytes and the same amax as f8mi_cast_layout with amax_dev; what differs is how the amax leaves the cast kernel:
  * there every workgroup compares with *amax_dev at its end (and holds its LDS and wave slots for that round trip:
- * 6 - 20 us per tensor of 128 MB - 1.8 GB), here every wave folds its maximum into one of 1024 words of `workspace`
- * with an atomic that returns nothing, and a one-workgroup launch reduces the words (4 us).
+ * 6 - 20 us per tensor of 128 MB - 1.8 GB).  Here, up to 2048 tiles of 128 x 128 and unless the stream is being captured, every wave
+ * leaves its maximum in a word of the library's own, and the workgroup started last collects them; beyond, every wave
+ * folds it into one of 1024 words of `workspace` with an atomic that returns nothing, and a one-workgroup launch reduces
+ * the words (4 us).
  *   workspace   f8mi_delayed_workspace_bytes() of device memory, 4-byte aligned, ALL ZERO before the first call that
  *               uses it; every call leaves it all zero again when its work completes.  Not to be shared by calls that
  *               can overlap in time (one per stream), and not the workspace of f8mi_amax_scale, whose contents are
@@ -207,8 +209,9 @@ int f8mi_cast_delayed(const void* x, int64_t rows, int64_t cols, int64_t ld, int
  * product in x's dtype -- hp_tensor_to_float8_dynamic (float8_scaling_utils.py:33-62: tensor_to_scale, then
  * hp_tensor_and_scale_to_float8 with the 0-dim scale).  *scale_dev receives the scale.  A tensor of at most
  * 32 K elements goes through one launch of one workgroup (a few rows of activations: the launches cost more
- * than the work), a dense one of at most 512 KB of which one copy is asked for through one launch of several, anything
- * larger through the two kernels above; the results are the same bits either way.
+ * than the work), a dense one of at most 320 KB (of few rows: 512 KB) of which one copy is asked for through one launch of
+ * several, anything else of at most 1024 tiles of 128 x 128 through f8mi_cast_dynamic_resident unless the stream is being
+ * captured, and the rest through the two kernels above; the results are the same bits either way.
  * `workspace` as for f8mi_amax_scale. */
 int f8mi_cast_dynamic(const void* x, int64_t rows, int64_t cols, int64_t ld, int in_dtype, int fp8_fmt, float* scale_dev,
                       uint8_t* out, int out_layout, uint8_t* out_t, int out_t_layout, void* workspace, void* stream);
