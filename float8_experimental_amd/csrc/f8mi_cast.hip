@@ -726,6 +726,8 @@ static int launch_cast_flat(int fmt, hipStream_t stream, const void* x, int64_t 
 // us, everybody has everybody's maximum after 11.3 (2 us is what a word takes to memory and back, 512 x 1024 waits as long), the
 // last byte is stored after 15.  Loads in smaller batches, other tile shapes and linear tile orders all took the same or longer.
 constexpr int RESIDENT_TILES = 1024;  // workgroups at most
+// of two 16-bit tensors together, six workgroups a CU: see pair_tile_rows
+constexpr int RESIDENT_PAIR_TILES = 1536;
 
 template <int DT, int FMT, int H>
 __device__ __forceinline__ void resident_body(const CastJob& j, uint32_t bid, uint32_t nb, uint32_t* tileT, uint32_t* red) {
@@ -1171,9 +1173,19 @@ static int launch_cast_pair(int dt_a, int dt_b, int tile_rows, hipStream_t strea
 }
 
 
+// Rows of the tiles that both get in one launch, 0: not in one.  Two 16-bit tensors may have half as many tiles again as one tensor: in two
+// launches each of them waits for its own words, together once.  us, two launches / one: 2048 x 4096 with 3072 x 4096 (1280 tiles) 25.9 /
+// 21.0, with 4096 x 4096 (1536) 29.1 / 24.1, both copies 33.1 / 26.7; 3000 x 3000 with 3100 x 3000, both copies 30.0 / 22.3; 1024 x 4096 with 5120 x 4096
+// (two launches, one of them for the maxima) 26.0 / 24.3.  Six workgroups of eight leave other kernels a quarter of the chip.  Two such pairs on streams of
+// their own at the same time: 23.7 / 23.0 a pair, but three: 24 / 47 (some wait for the others' places).  fp32 has room for five.
+static int pair_tile_rows(const f8mi_cast_job& a, const f8mi_cast_job& b) {
+    const int64_t tiles = tiles_of(a) + tiles_of(b);
+    if (const int rows = resident_tile_rows(tiles * CAST_TILE, CAST_TILE)) return rows;
+    return b.in_dtype != F8MI_FP32 && tiles <= std::min(RESIDENT_PAIR_TILES, 6 * cu_count()) ? CAST_TILE : 0;
+}
 // Both casts in the launch that exchanges maxima.  F8MI_ERR_UNSUPPORTED, and nothing queued: not in one.
 static int cast_dynamic_pair_one_launch(const f8mi_cast_job& a, const f8mi_cast_job& b, uint32_t wait_ticks, hipStream_t stream) {
-    const int tile_rows = resident_tile_rows((tiles_of(a) + tiles_of(b)) * CAST_TILE, CAST_TILE);
+    const int tile_rows = pair_tile_rows(a, b);
     if (!tile_rows) return F8MI_ERR_UNSUPPORTED;
     TaggedWords tagged;
     if (const int rc = begin_exchange(stream, wait_ticks, tagged)) return rc;

@@ -844,6 +844,13 @@ def test_cast_of_two_tensors_equals_two_casts(nat, dts, shapes):
                     assert torch.equal(a, wa) or (torch.isnan(a).all() and torch.isnan(wa).all())
 
 
+# 16-bit pairs past what one tensor may have: ragged, the most tiles one launch takes together (1536) and a row more.
+@pytest.mark.parametrize("dts", ["bf16 bf16", "fp16 fp16", "bf16 fp32"])
+@pytest.mark.parametrize("shapes", [((3000, 3000), (3100, 3001)), ((2048, 4096), (4096, 4096)), ((2049, 4096), (4096, 4096))])
+def test_cast_of_two_tensors_of_up_to_six_tiles_a_cu(nat, dts, shapes):
+    test_cast_of_two_tensors_equals_two_casts(nat, dts, shapes)
+
+
 def _rand_fp8(shape, tdt, seed, scale=1.0):
     g = torch.Generator().manual_seed(seed)
     v = torch.randn(shape, generator=g) * scale
