@@ -56,6 +56,7 @@ EXPORTS = (
     "f8mi_gemm_nt",
     "f8mi_gemm_nt_kb",
     "f8mi_gemm_kb_ex",
+    "f8mi_gemm_pair",
     "f8mi_gemm_ex",
     "f8mi_sync",
     "f8mi_sync_host",
@@ -129,6 +130,8 @@ def lib() -> C.CDLL:
         L.f8mi_gemm_nt_kb.argtypes = [vp, i32, vp, i32, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp]
         L.f8mi_gemm_kb_ex.restype = i32
         L.f8mi_gemm_kb_ex.argtypes = [vp, i32, i32, vp, i32, i32, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp]
+        L.f8mi_gemm_pair.restype = i32
+        L.f8mi_gemm_pair.argtypes = [vp, vp, i32, vp]
         L.f8mi_gemm_ex.restype = i32
         L.f8mi_gemm_ex.argtypes = [vp, i32, i32, i64, vp, i32, i32, i64, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp]
         L.f8mi_gemm_nt.restype = i32

@@ -27,7 +27,7 @@
 #include <cstdlib>
 #include <cstring>
 
-#include "f8mi_gemm_util.h"
+#include "f8mi_gemm_pair.h"
 
 namespace f8mi {
 
@@ -544,4 +544,133 @@ extern "C" int f8mi_gemm_ex(const void* a, int a_fmt, int a_transposed, int64_t 
     // a row-major matrix read transposed: row stride between contraction rows, 64 bytes between blocks of 64 rows
     return launch_transposed(a_transposed != 0, a_fmt, b_fmt, c_dtype, stream, (const uint8_t*)a, lda, 64, (const uint8_t*)bt, ldb, 64, m, n, k, scale_a_dev,
                              scale_b_dev, c, ldc, bias_dev, c_vec_ok);
+}
+
+// ---- two products in one launch
+
+// What one of them needs of the kernels that take two, checked like f8mi_gemm_kb_ex; false: one by one.
+static bool pair_side(const f8mi_gemm_job& j, GemmSide* s) {
+    if (j.m <= 0 || j.n <= 0 || j.k < 384 || j.k % 128 != 0 || j.m > 0x7fffffff || j.n > 0x7fffffff || j.k * 64 * 4 > 0x7fffffffLL || j.ldc < j.n) return false;
+    if (j.a_fmt != F8MI_E5M2 || j.b_fmt != F8MI_E4M3FN || j.c_dtype < 0 || j.c_dtype > 2) return false;
+    if (!j.a || !j.bt || !j.c || !j.scale_a_dev || !j.scale_b_dev || (uintptr_t)j.a % 16 != 0 || (uintptr_t)j.bt % 16 != 0) return false;
+    if ((j.a_transposed && (!j.b_transposed || j.m % 64 != 0)) || (j.b_transposed && j.n % 64 != 0)) return false;
+    const int c_vec_ok = (uintptr_t)j.c % (j.c_dtype == F8MI_FP32 ? 4 : 2) == 0;
+    *s = {(const uint8_t*)j.a, 64, j.a_transposed ? j.k * 64 : j.m * 64, (const uint8_t*)j.bt, 64, j.b_transposed ? j.k * 64 : j.n * 64, (int)j.m, (int)j.n, (int)j.k,
+          j.scale_a_dev, j.scale_b_dev, j.c, j.ldc, 0, 0, c_vec_ok};
+    return true;
+}
+
+static int gemm_job(const f8mi_gemm_job& j, void* stream) {
+    if (j.a_transposed || j.b_transposed)
+        return f8mi_gemm_kb_ex(j.a, j.a_fmt, j.a_transposed, j.bt, j.b_fmt, j.b_transposed, j.m, j.n, j.k, j.scale_a_dev, j.scale_b_dev, j.c, j.c_dtype, j.ldc, nullptr, stream);
+    return f8mi_gemm_nt_kb_ws(j.a, j.a_fmt, j.bt, j.b_fmt, j.m, j.n, j.k, j.scale_a_dev, j.scale_b_dev, j.c, j.c_dtype, j.ldc, nullptr, j.workspace, j.workspace_bytes, stream);
+}
+
+// Estimates in us behind the choice between one launch and two, and of its tiles: every tile of a kind takes a constant and a step's
+// time per 128 of k (128 x 256 tiles an eighth more where they do not all run at once: their operands come faster than the L2 gives them), a
+// launch 2.6 us by itself, and 256 workgroups run at a time, those of the longer contraction first.  Fitted to 620 pairs of products of 384 -
+// 16384 tokens and 512 - 28672 features, both kinds of operands, timed in every form: the choice is within 0.5 % of the best one in the mean,
+// 1.195 times as fast as two launches, and slower than those by more than 2 % in four cases (7 % in one: 6144 tokens, 1408 -> 2176).
+struct PairTiles { int rows, cols; double us, step_us, crowded; };
+constexpr PairTiles PAIR_TILES[4] = {{}, {128, 128, 2.2, 0.48, 1.0}, {128, 256, 3.4, 0.64, 1.125}, {256, 256, 5.9, 1.13, 1.0}};
+constexpr double PAIR_LAUNCH_US = 2.6;
+constexpr int64_t PAIR_WORKGROUPS = 256;
+static int64_t tiles_of(const PairTiles& t, int64_t m, int64_t n) { return (m + t.rows - 1) / t.rows * ((n + t.cols - 1) / t.cols); }
+static double tile_us(const PairTiles& t, int64_t k, bool crowded) { return t.us + t.step_us * (crowded ? t.crowded : 1.0) * (double)(k / 128); }
+
+static double pair_us(const PairTiles& t, const f8mi_gemm_job& a, const f8mi_gemm_job& b) {
+    const f8mi_gemm_job &lng = a.k >= b.k ? a : b, &shrt = a.k >= b.k ? b : a;
+    const int64_t n_long = tiles_of(t, lng.m, lng.n), n_short = tiles_of(t, shrt.m, shrt.n);
+    const bool crowded = n_long + n_short > PAIR_WORKGROUPS;
+    const double us_long = tile_us(t, lng.k, crowded), us_short = tile_us(t, shrt.k, crowded);
+    const int64_t rounds = n_long / PAIR_WORKGROUPS, late = n_long % PAIR_WORKGROUPS;
+    // when the workgroups without and with a tile of the long ones' last round are free, and which of them take the short ones
+    double early_us = us_long * (double)rounds, late_us = us_long * (double)(rounds + 1), end = late ? late_us : early_us;
+    for (int64_t left = n_short; left > 0;) {
+        const bool early = early_us <= late_us || late == 0;
+        double& t_free = early ? early_us : late_us;
+        left -= early ? PAIR_WORKGROUPS - late : late;
+        t_free += us_short;
+        if (t_free > end) end = t_free;
+    }
+    return PAIR_LAUNCH_US + end;
+}
+
+// A product by itself, on the kernels that gemm_plan and launch_transposed choose; 0: on kernels whose sums are in another order or that
+// are none of these.
+static double single_us(const f8mi_gemm_job& j) {
+    const double rounds_us = tile_us(PAIR_TILES[3], j.k, false);
+    const auto rounds = [](int64_t tiles) { return (double)((tiles + PAIR_WORKGROUPS - 1) / PAIR_WORKGROUPS); };
+    const int64_t tiles_m = (j.m + BM - 1) / BM, tiles_n = (j.n + BN - 1) / BN;
+    GemmPlan p{F8MI_PLAN_TILES256, 0, use_mid_tiles(j.m, j.n, j.k), {0, 0}};
+    if (j.b_transposed) {
+        if (p.mid) p.kind = F8MI_PLAN_TILES128;
+        else p.split = split_last_round(tiles_m, tiles_n, j.k);
+        if (p.split.rows_large) { p.kind = F8MI_PLAN_TILES256_AND_128; p.mid = p.split.mid; }
+    } else {
+        const bool ws_ok = j.workspace && (uintptr_t)j.workspace % 16 == 0;
+        p = gemm_plan(j.m, j.n, j.k, true, ws_ok ? j.workspace_bytes : 0, rows_at_odd_addresses(j.c, j.ldc, j.c_dtype));
+    }
+    switch (p.kind) {
+        case F8MI_PLAN_TILES128: return PAIR_LAUNCH_US + tile_us(PAIR_TILES[p.mid], j.k, false);
+        case F8MI_PLAN_TILES256: return PAIR_LAUNCH_US + rounds_us * rounds(tiles_m * tiles_n);
+        case F8MI_PLAN_TILES256X224: return PAIR_LAUNCH_US + 0.9 * rounds_us * rounds(tiles_m * ((j.n + NARROW_N - 1) / NARROW_N));
+        case F8MI_PLAN_TILES256_AND_128: return 2.0 * PAIR_LAUNCH_US + rounds_us * rounds(p.split.rows_large * tiles_n) + tile_us(PAIR_TILES[p.mid], j.k, false);
+        default: return 0.0;
+    }
+}
+
+// The tiles of one launch, or F8MI_PAIR_BY_SIZE for two launches.  Many rounds of 256 x 256 tiles leave nothing to gain, and small tiles
+// nothing past four rounds.
+static int pair_tiles(const f8mi_gemm_job& a, const f8mi_gemm_job& b) {
+    if (tiles_of(PAIR_TILES[F8MI_PAIR_TILES256], a.m, a.n) + tiles_of(PAIR_TILES[F8MI_PAIR_TILES256], b.m, b.n) > 16 * PAIR_WORKGROUPS) return F8MI_PAIR_BY_SIZE;
+    const double us_a = single_us(a), us_b = single_us(b);
+    if (us_a == 0.0 || us_b == 0.0) return F8MI_PAIR_BY_SIZE;
+    double best_us = 0.96 * (us_a + us_b);  // the estimates are not better than that
+    int best = F8MI_PAIR_BY_SIZE;
+    for (int kind = F8MI_PAIR_TILES128; kind <= F8MI_PAIR_TILES256; kind++) {
+        const PairTiles& t = PAIR_TILES[kind];
+        if (kind != F8MI_PAIR_TILES256 && tiles_of(t, a.m, a.n) + tiles_of(t, b.m, b.n) > 4 * PAIR_WORKGROUPS) continue;
+        const double us = pair_us(t, a, b);
+        if (us < best_us) { best_us = us; best = kind; }
+    }
+    return best;
+}
+
+extern "C" int f8mi_gemm_pair(const f8mi_gemm_job* a, const f8mi_gemm_job* b, int tiles, void* stream) {
+    if (!a || !b) { set_error("f8mi_gemm_pair: null pointer"); return F8MI_ERR_INVALID_ARG; }
+    if (tiles < F8MI_PAIR_BY_SIZE || tiles > F8MI_PAIR_TILES256) { set_error("f8mi_gemm_pair: unknown tiles %d", tiles); return F8MI_ERR_INVALID_ARG; }
+    GemmPair pair;
+    const bool tr = a->b_transposed != 0;
+    bool ok = pair_side(*a, &pair.s[0]) && pair_side(*b, &pair.s[1]) && a->c_dtype == b->c_dtype && !a->a_transposed && (a->b_transposed != 0) == (b->b_transposed != 0) &&
+              (b->a_transposed != 0) == tr;
+    int kind = tiles;
+    bool odd_rows = false;
+    if (ok) {
+        const bool odd[2] = {rows_at_odd_addresses(a->c, a->ldc, a->c_dtype), rows_at_odd_addresses(b->c, b->ldc, b->c_dtype)};
+        odd_rows = odd[0] && odd[1] && pair.s[0].c_vec_ok && pair.s[1].c_vec_ok;
+        if (!tr && odd[0] != odd[1]) ok = false;
+        if (tr) odd_rows = false;
+        if (kind == F8MI_PAIR_BY_SIZE) kind = pair_tiles(*a, *b);
+    }
+    if (ok && kind != F8MI_PAIR_BY_SIZE) {
+        const int rows = kind == F8MI_PAIR_TILES256 ? 256 : 128, cols = kind == F8MI_PAIR_TILES128 ? 128 : 256;
+        int64_t total = 0;
+        for (GemmSide& s : pair.s) {
+            const int64_t tm = ((int64_t)s.M + rows - 1) / rows, tn = ((int64_t)s.N + cols - 1) / cols;
+            total += tm * tn;
+            s.tiles_m = (int)tm;
+            s.tiles_n = (int)tn;
+        }
+        if (total > 0x7fffffff) ok = false;
+    }
+    if (ok && kind != F8MI_PAIR_BY_SIZE) {
+        ProfScope prof(F8MI_K_GEMM, 2.0 * ((double)a->m * (double)a->n * (double)a->k + (double)b->m * (double)b->n * (double)b->k), (hipStream_t)stream);
+        const bool second_first = b->k > a->k;  // the longer ones first: the last round is then of short ones
+        if (kind == F8MI_PAIR_TILES256) return launch_gemm_pair_large(tr, odd_rows, a->c_dtype, (hipStream_t)stream, pair, second_first);
+        return launch_gemm_pair_mid(tr, odd_rows, kind == F8MI_PAIR_TILES128X256, a->c_dtype, (hipStream_t)stream, pair, second_first);
+    }
+    if (tiles != F8MI_PAIR_BY_SIZE) { set_error("f8mi_gemm_pair: not built for these two products"); return F8MI_ERR_UNSUPPORTED; }
+    if (int rc = gemm_job(*a, stream)) return rc;
+    return gemm_job(*b, stream);
 }

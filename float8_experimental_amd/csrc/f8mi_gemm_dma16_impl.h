@@ -218,9 +218,10 @@ __device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[TJ][8], int m0, i
 // are built with ds_read_b64_tr_b8.  For such an operand lda / ldb is the byte distance between contraction
 // rows (64 when k-blocked over `rows`, the row stride when row-major) and a_unit / b_unit the distance between
 // blocks of 64 rows (contraction length * 64 when k-blocked, 64 when row-major).
+// Workgroup `lid` of the `npid` that compute this product.
 template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ>
-__global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
-    const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
+__device__ __forceinline__ void gemm_dma16_tile(
+    int lid, const int npid, const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
     int M, int N, int K, const float* __restrict__ sa_dev, const float* __restrict__ sb_dev, void* __restrict__ C,
     int64_t ldc, const void* __restrict__ bias, int tiles_m, int tiles_n, int c_vec_ok) {
     static_assert(TJ == 8 || (TJ == 7 && !A_TR && !B_TR && !ODD_ROWS), "narrower tiles: operands as they are");
@@ -230,8 +231,6 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     // to the next.  Row-major operands: (row stride, 64); k-blocked [K/64][rows][64]: (64, rows*64).
 
     // ---- which tile (same walk as the other kernels)
-    int lid = blockIdx.x;
-    const int npid = gridDim.x;
 #if F8MI_WALK_XCD_CHUNK == 0
     lid = xcd_contiguous_id(lid, npid);
 #else
@@ -512,6 +511,15 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
     } else {
         store_c_tile16_fp32(acc, m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
     }
+}
+
+template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ>
+__global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_dma16_kernel(
+    const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
+    int M, int N, int K, const float* __restrict__ sa_dev, const float* __restrict__ sb_dev, void* __restrict__ C,
+    int64_t ldc, const void* __restrict__ bias, int tiles_m, int tiles_n, int c_vec_ok) {
+    gemm_dma16_tile<AF, BF, C_DT, ODD, A_TR, B_TR, ODD_ROWS, TJ>(blockIdx.x, gridDim.x, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa_dev, sb_dev, C,
+                                                                 ldc, bias, tiles_m, tiles_n, c_vec_ok);
 }
 
 template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ>

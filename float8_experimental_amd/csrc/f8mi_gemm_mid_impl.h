@@ -81,11 +81,12 @@ __device__ __forceinline__ uint32_t mid_tr_voff(int instr, int64_t ld, int64_t u
     return (uint32_t)(row * ld + blk * unit) + (c & 3) * 16;
 }
 
+// Workgroup `bid` of the `grid` that compute this product (or one part of its k).
 // ODD_ROWS: rows of C start at odd multiples of two bytes too (see ShiftedRows); a piece is then stored behind the next one.
 template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR, bool ODD_ROWS>
-__global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
-    const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
-    int M, int N, int K, const float* sa_dev, const float* sb_dev, void* __restrict__ C,
+__device__ __forceinline__ void gemm_mid_tile(
+    const int bid, const int grid, const int split, const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt,
+    int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa_dev, const float* sb_dev, void* __restrict__ C,
     int64_t ldc, const void* __restrict__ bias, int tiles_m, int tiles_n, int c_vec_ok, int k_splits) {
     using Cfg = MidCfg<TJ>;
     constexpr int NSTAGE = Cfg::NSTAGE, NDMA = Cfg::NDMA;
@@ -93,14 +94,13 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
     // consecutive workgroup ids go to the 8 XCDs round-robin; re-deal them so that one XCD (one L2) gets a contiguous
     // run of the tile order, which walks bands of eight tile rows column by column: the 32 workgroups of an XCD then
     // hold a patch of 8 x 4 neighbouring tiles, the fewest operand panels through that L2
-    const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
+    const int lid = xcd_contiguous_id(bid, grid);
     const int band = lid / (8 * tiles_n), in_band = lid % (8 * tiles_n);
     const int band_rows = min(tiles_m - band * 8, 8);
     const int tm = band * 8 + in_band % band_rows, tn = in_band / band_rows;
     const int m0 = tm * MID_TILE_M, n0 = tn * Cfg::TILE_N;
-    // k_splits > 1 (host: fp32 output, no bias): blockIdx.y takes the y-th part of k and writes its partial sums,
-    // unscaled, to the y-th M x ldc slab of C; a second kernel adds the slabs in a fixed order.
-    const int split = blockIdx.y;
+    // k_splits > 1 (host: fp32 output, no bias): takes the split-th part of k and writes its partial sums,
+    // unscaled, to the split-th M x ldc slab of C; a second kernel adds the slabs in a fixed order.
     const int K_part = K / k_splits;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -352,6 +352,15 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
         for (int tp = 0; tp < TJ / 2; tp++) store_piece(3, tp);
         if constexpr (ODD_ROWS) store_held(3, TJ / 2 - 1);
     }
+}
+
+template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR, bool ODD_ROWS>
+__global__ __launch_bounds__(GEMM_THREADS) void gemm_mid_kernel(
+    const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
+    int M, int N, int K, const float* sa_dev, const float* sb_dev, void* __restrict__ C,
+    int64_t ldc, const void* __restrict__ bias, int tiles_m, int tiles_n, int c_vec_ok, int k_splits) {
+    gemm_mid_tile<AF, BF, C_DT, TJ, A_TR, B_TR, ODD_ROWS>(blockIdx.x, gridDim.x, blockIdx.y, A, lda, a_unit, Bt, ldb, b_unit, M, N, K, sa_dev, sb_dev, C,
+                                                          ldc, bias, tiles_m, tiles_n, c_vec_ok, k_splits);
 }
 
 template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR, bool ODD_ROWS>

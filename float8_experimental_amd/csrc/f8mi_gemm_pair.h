@@ -1,0 +1,41 @@
+// Two products in one launch (the backward of a linear: grad_input and grad_weight): what the host rule and the kernels share.
+//
+// One after the other, each product fills the chip and drains it again, and the workgroups of its last round leave the rest of the CUs idle.
+// In one launch the tiles of the second start where those of the first end, those of the longer contraction first.  Both products have the
+// same work, so a product of few tiles that each take long runs beside one of many that do not.  us, one after the other / together (tokens,
+// in -> out features; tiles): 512, 1024 -> 1024: 12.3 / 7.1 (128 x 128); 384, 2048 -> 5120: 27.3 / 18.0 (128 x 128); 1664, 3328 -> 2560: 40.3 /
+// 31.7 (128 x 256); 2048, 4096 -> 4096: 60.5 / 56.7 (256 x 256); 3584, 2816 -> 11648: 196.7 / 166.9; 2981, 2989 -> 8117: 158 / 125; 4096, 4096
+// -> 4096, one full round each: 101.3 / 99.4; 8192, 4096 -> 14336: 617 / 630, where the rule in f8mi_gemm.hip stays with two.
+// The tiles are the ones that a product by itself runs on (f8mi_gemm_dma16_impl.h, f8mi_gemm_mid_impl.h): the same bits.
+#pragma once
+#include "f8mi_gemm_util.h"
+
+namespace f8mi {
+
+// One product: the arguments of its kernel by itself.
+struct GemmSide {
+    const uint8_t* A;
+    int64_t lda, a_unit;
+    const uint8_t* Bt;
+    int64_t ldb, b_unit;
+    int M, N, K;
+    const float *sa, *sb;
+    void* C;
+    int64_t ldc;
+    int tiles_m, tiles_n;
+    int c_vec_ok;
+};
+
+__host__ __device__ inline int workgroups(const GemmSide& s) { return s.tiles_m * s.tiles_n; }
+// Both, as a kernel takes them: the side is looked up by its index, one set of scalar registers for either (as two arguments their fields
+// are all loaded up front, and 90 scalar registers spilled).
+struct GemmPair {
+    GemmSide s[2];
+};
+// A e5m2, Bt e4m3 on both sides.  transposed: s[0] reads its Bt transposed, s[1] both its operands; else both sides read them as they are.
+// second_first: the workgroups of s[1] come first.  odd_rows: rows of C at odd multiples of two bytes (not with transposed).
+int launch_gemm_pair_large(bool transposed, bool odd_rows, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+int launch_gemm_pair_large_tr(int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+int launch_gemm_pair_mid(bool transposed, bool odd_rows, bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+
+}  // namespace f8mi

@@ -1,0 +1,12 @@
+// Two products in one launch on 256 x 256 tiles: Bt of one read transposed, both operands of the other.
+#include "f8mi_gemm_pair_large_impl.h"
+
+namespace f8mi {
+
+int launch_gemm_pair_large_tr(int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first) {
+    if (c_dtype == F8MI_FP32) return launch_pair_large<F8MI_FP32, true, false>(stream, pair, second_first);
+    if (c_dtype == F8MI_FP16) return launch_pair_large<F8MI_FP16, true, false>(stream, pair, second_first);
+    return launch_pair_large<F8MI_BF16, true, false>(stream, pair, second_first);
+}
+
+}  // namespace f8mi

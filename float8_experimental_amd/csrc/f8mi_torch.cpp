@@ -31,6 +31,7 @@ struct Lib {
     decltype(&f8mi_gemm_nt_ws) gemm_nt_ws;
     decltype(&f8mi_gemm_nt_kb_ws) gemm_nt_kb_ws;
     decltype(&f8mi_gemm_kb_ex) gemm_kb_ex;
+    decltype(&f8mi_gemm_pair) gemm_pair;
     decltype(&f8mi_gemm_plan) gemm_plan;
     decltype(&f8mi_linear_few_rows) linear_few_rows;
     decltype(&f8mi_last_error) last_error;
@@ -162,19 +163,23 @@ struct Call {
         }
     }
 
+    // scratch for a product that is split over k
+    at::Tensor split_workspace(int64_t m, int64_t n, int64_t k, int layout, int64_t& bytes) const {
+        bytes = 0;
+        if (m < 17 || k < 2048 || (layout == F8MI_LAYOUT_ROWMAJOR && k % 16 != 0)) return {};  // below these none is
+        const int plan = L.gemm_plan(m, n, k, 1, F8MI_GEMM_WORKSPACE_BYTES);
+        if ((plan & 0xff) != F8MI_PLAN_TILES128_SPLIT_K) return {};
+        bytes = (int64_t)((plan >> 8) & 0xff) * m * n * 4;
+        return make({bytes / 4}, at::kFloat);
+    }
+
     // a [m][k] times bt [n][k] in the layout, both contracting over kc (before padding)
     at::Tensor gemm(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& bt, const at::Tensor& sb, int layout, int64_t m, int64_t n,
                     int64_t kc, at::ScalarType out, const at::Tensor& bias = {}) const {
-        at::Tensor c = make({m, n}, out), ws;
+        const at::Tensor c = make({m, n}, out);
         const int64_t k = padded(kc, layout);
         int64_t ws_bytes = 0;
-        if (m >= 17 && k >= 2048 && (layout != F8MI_LAYOUT_ROWMAJOR || k % 16 == 0)) {  // below these no product is split over k
-            const int plan = L.gemm_plan(m, n, k, 1, F8MI_GEMM_WORKSPACE_BYTES);
-            if ((plan & 0xff) == F8MI_PLAN_TILES128_SPLIT_K) {
-                ws_bytes = (int64_t)((plan >> 8) & 0xff) * m * n * 4;
-                ws = make({ws_bytes / 4}, at::kFloat);
-            }
-        }
+        const at::Tensor ws = split_workspace(m, n, k, layout, ws_bytes);
         void* pws = ws_bytes ? ws.data_ptr() : nullptr;
         const float *pa = (const float*)sa.data_ptr(), *pb = (const float*)sb.data_ptr();
         const int fa = fp8_code(a.scalar_type()), fb = fp8_code(bt.scalar_type()), dt = dtype_code(out);
@@ -191,6 +196,30 @@ struct Call {
         check(L.gemm_kb_ex(a.data_ptr(), fp8_code(a.scalar_type()), a_tr, bt.data_ptr(), fp8_code(bt.scalar_type()), 1, m, n, k, (const float*)sa.data_ptr(),
                            (const float*)sb.data_ptr(), c.data_ptr(), dtype_code(out), n, nullptr, stream), "f8mi_gemm_kb_ex");
         return c;
+    }
+
+    // One product of a library call that computes two, of k-blocked operands.
+    struct Product {
+        const at::Tensor &a, &sa, &bt, &sb;
+        bool a_tr, b_tr;
+        int layout;
+        int64_t m, n, kc;
+        at::Tensor& c;
+    };
+    void gemm_two(const Product& p, const Product& q, at::ScalarType out) const {
+        f8mi_gemm_job jobs[2];
+        at::Tensor ws[2];
+        int i = 0;
+        for (const Product* g : {&p, &q}) {
+            const int64_t k = padded(g->kc, g->layout);
+            int64_t bytes = 0;
+            if (!g->b_tr) ws[i] = split_workspace(g->m, g->n, k, g->layout, bytes);
+            g->c = make({g->m, g->n}, out);
+            jobs[i] = {g->a.data_ptr(), g->bt.data_ptr(), fp8_code(g->a.scalar_type()), fp8_code(g->bt.scalar_type()), g->a_tr, g->b_tr, g->m, g->n, k,
+                       (const float*)g->sa.data_ptr(), (const float*)g->sb.data_ptr(), g->c.data_ptr(), g->n, dtype_code(out), bytes ? ws[i].data_ptr() : nullptr, bytes};
+            i++;
+        }
+        check(L.gemm_pair(&jobs[0], &jobs[1], F8MI_PAIR_BY_SIZE, stream), "f8mi_gemm_pair");
     }
 };
 
@@ -278,17 +307,28 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             if (fp8_code(t->scalar_type()) < 0 || !t->is_contiguous() || t->sizes() != copy_sizes(rows, kc, layout)) Py_RETURN_NONE;
         }
         at::Tensor g8, g8t, sg, dx, dw;
-        {
-            const WithoutGil no_gil;
+        const auto compute = [&] {
             if (one_copy) {
                 c.cast(dy, go, F8MI_E5M2, true, F8MI_LAYOUT_KBLOCK64, false, 0, g8, g8t, sg);
+                if (need_dx && need_dw && L.gemm_pair) {
+                    c.gemm_two({g8, sg, ws, sw, false, true, F8MI_LAYOUT_KBLOCK64, m, k, n, dx}, {g8, sg, xs, sx, true, true, F8MI_LAYOUT_KBLOCK64, n, k, m, dw}, dy.scalar_type());
+                    return;
+                }
                 if (need_dx) dx = c.gemm_tr(g8, false, sg, ws, sw, m, k, n, dy.scalar_type());
                 if (need_dw) dw = c.gemm_tr(g8, true, sg, xs, sx, n, k, m, dy.scalar_type());
             } else {
                 c.cast(dy, go, F8MI_E5M2, need_dx, kb_dx, need_dw, kb_dw, g8, g8t, sg);
+                if (need_dx && need_dw && kb_dx != F8MI_LAYOUT_ROWMAJOR && kb_dw != F8MI_LAYOUT_ROWMAJOR && L.gemm_pair) {
+                    c.gemm_two({g8, sg, ws, sw, false, false, kb_dx, m, k, n, dx}, {g8t, sg, xs, sx, false, false, kb_dw, n, k, m, dw}, dy.scalar_type());
+                    return;
+                }
                 if (need_dx) dx = c.gemm(g8, sg, ws, sw, kb_dx, m, k, n, dy.scalar_type());
                 if (need_dw) dw = c.gemm(g8t, sg, xs, sx, kb_dw, n, k, m, dy.scalar_type());
             }
+        };
+        {
+            const WithoutGil no_gil;
+            compute();
         }
         return wrap_all(dx, dw);
     });
@@ -369,6 +409,7 @@ PyObject* load(PyObject*, PyObject* args) {
     get(L.gemm_plan, "f8mi_gemm_plan");
     get(L.cast_dynamic_pair, "f8mi_cast_dynamic_pair");
     get(L.cast_delayed_pair, "f8mi_cast_delayed_pair");
+    L.gemm_pair = reinterpret_cast<decltype(L.gemm_pair)>(dlsym(h, "f8mi_gemm_pair"));  // without it the products go one by one
     if (missing) {
         L.gemm_plan = nullptr;
         return PyErr_Format(PyExc_ImportError, "%s does not export %s", path, missing);

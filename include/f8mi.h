@@ -342,6 +342,30 @@ int f8mi_gemm_kb_ex(const void* a, int a_fmt, int a_transposed, const void* bt, 
                     int64_t n, int64_t k, const float* scale_a_dev, const float* scale_b_dev, void* c, int c_dtype,
                     int64_t ldc, const void* bias_dev, void* stream);
 
+/* One product of a call that computes two: the arguments of f8mi_gemm_kb_ex without a bias and, for operands that are both given as they
+ * are, the workspace of f8mi_gemm_nt_kb_ws. */
+typedef struct f8mi_gemm_job {
+    const void *a, *bt;
+    int a_fmt, b_fmt, a_transposed, b_transposed;
+    int64_t m, n, k;
+    const float *scale_a_dev, *scale_b_dev;
+    void* c;
+    int64_t ldc;
+    int c_dtype;
+    void* workspace;
+    int64_t workspace_bytes;
+} f8mi_gemm_job;
+
+/* Two independent products, as the backward of a linear has them (a: grad_input, b: grad_weight): in one launch where that pays,
+ * else one after the other; the same bits.  One launch takes e5m2 times e4m3 with k % 128 == 0 and k >= 384, both pairs of operands as
+ * they are, or a with bt transposed and b with both.  tiles: F8MI_PAIR_BY_SIZE, or (for tests and measurements) the tiles of one
+ * launch, F8MI_ERR_UNSUPPORTED with nothing queued where it does not take them. */
+#define F8MI_PAIR_BY_SIZE 0
+#define F8MI_PAIR_TILES128 1
+#define F8MI_PAIR_TILES128X256 2
+#define F8MI_PAIR_TILES256 3
+int f8mi_gemm_pair(const f8mi_gemm_job* a, const f8mi_gemm_job* b, int tiles, void* stream);
+
 /* f8mi_gemm_nt on ROW-MAJOR fp8 operands either of which may be given transposed, so that the fp8 transposes
  * preprocess_addmm makes for torch._scaled_mm's layout rule (a row-major, b column-major: float8_ops.py:131-155, the
  * .t().contiguous().t() of :150-153) need not be made: the matrix-core kernel transposes on the way from LDS to the

@@ -1041,6 +1041,48 @@ def test_gemm_mid_tile_kernel_reads_transposed_operands(nat, m, n, k, mid, out_d
     assert torch.equal(nat.gemm_kb_ex(turned(a), True, sa, turned(bt), True, sb, out_dt, bias=bias), want)
 
 
+class GemmJob(ctypes.Structure):  # f8mi_gemm_job
+    _fields_ = ([(f, ctypes.c_void_p) for f in ("a", "bt")] + [(f, ctypes.c_int) for f in ("a_fmt", "b_fmt", "a_tr", "b_tr")] +
+                [(f, ctypes.c_int64) for f in ("m", "n", "k")] + [(f, ctypes.c_void_p) for f in ("sa", "sb", "c")] +
+                [("ldc", ctypes.c_int64), ("dtype", ctypes.c_int), ("ws", ctypes.c_void_p), ("ws_bytes", ctypes.c_int64)])
+
+
+# Both products of a backward in one launch, on each of its tiles and by the rule: grad_input (tokens x features) and grad_weight of one gradient,
+# operands read transposed (multiples of 128) or as they are (any size); one tile and edges of tiles, odd and even step counts on either
+# side, which of the two is longer, more than one round of workgroups, more than eight tile rows.
+@pytest.mark.parametrize("tokens,k,n", [(384, 384, 384), (512, 1024, 1024), (640, 384, 1152), (1408, 512, 640), (2432, 1280, 4864), (2304, 4096, 512),
+                                        (385, 391, 413), (700, 1001, 391), (1025, 515, 4099), (4133, 739, 862)])
+@pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float16, torch.float32])
+def test_gemm_pair_equals_the_products_one_by_one(nat, tokens, k, n, out_dt):
+    g = _rand_fp8((tokens, n), torch.float8_e5m2, tokens + n, 4.0).to(DEV)
+    w = _rand_fp8((n, k), torch.float8_e4m3fn, n + k, 4.0).to(DEV)
+    x = _rand_fp8((tokens, k), torch.float8_e4m3fn, tokens + k, 4.0).to(DEV)
+    sg, sw, sx = (torch.tensor(s, device=DEV) for s in (2.0, 0.25, 0.5))
+    transposed = tokens % 128 == 0 and k % 128 == 0 and n % 128 == 0
+    turned = lambda t: t.view(torch.uint8).t().contiguous().view(t.dtype)
+    pad = lambda v: -(-v // 128) * 128
+    forms = [(False, [_to_kb_padded(t)[0] for t in (g, turned(w), turned(g), turned(x))])]
+    if transposed:
+        forms.append((True, [_to_kb(g), _to_kb(w), _to_kb(g), _to_kb(x)]))
+    for tr, (a0, b0, a1, b1) in forms:
+        shapes = (tokens, k, pad(n)), (n, k, pad(tokens))
+        if tr:
+            want = [nat.gemm_kb_ex(a0, False, sg, b0, True, sw, out_dt), nat.gemm_kb_ex(a1, True, sg, b1, True, sx, out_dt)]
+        else:
+            want = [nat.gemm_nt_kb(a0, sg, b0, sw, out_dt, split_k=False), nat.gemm_nt_kb(a1, sg, b1, sx, out_dt, split_k=False)]
+        jobs, got = (GemmJob * 2)(), [torch.empty_like(t) for t in want]
+        for job, a, b, sb, (rows, cols, kc), c, a_tr in zip(jobs, (a0, a1), (b0, b1), (sw, sx), shapes, got, (0, int(tr))):
+            job.a, job.bt, job.a_fmt, job.b_fmt, job.a_tr, job.b_tr = a.data_ptr(), b.data_ptr(), nat.E5M2, nat.E4M3FN, a_tr, int(tr)
+            job.m, job.n, job.k, job.sa, job.sb, job.c, job.ldc, job.dtype = rows, cols, kc, sg.data_ptr(), sb.data_ptr(), c.data_ptr(), cols, nat._DT[out_dt]
+        for tiles in (0, 1, 2, 3):
+            for t in got:
+                t.fill_(float("nan"))
+            assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), tiles, nat._stream(g)) == 0, nat.lib().f8mi_last_error()
+            assert all(torch.equal(a, b) for a, b in zip(got, want)), (tr, tiles)
+        jobs[1].b_fmt = nat.E5M2  # what one launch does not take is two by the rule, and refused by name
+        assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), 3, nat._stream(g)) == nat.ERR_UNSUPPORTED
+
+
 # Few rows: one to three 128-deep steps per wave and one more or less of them, on each block of rows and both widths.
 @pytest.mark.parametrize("m,n,k", [(m, n, k) for m, n in ((1, 1000), (16, 4104), (17, 40), (32, 1000), (33, 40), (64, 1000))
                                    for k in (128, 896, 1024, 1152, 2048, 2176, 3200) if m <= 16 or k > 128])
