@@ -57,6 +57,9 @@ EXPORTS = (
     "f8mi_gemm_nt_kb",
     "f8mi_gemm_kb_ex",
     "f8mi_gemm_pair",
+    "f8mi_gemm_kb_bias",
+    "f8mi_column_sum",
+    "f8mi_column_sum_workspace_bytes",
     "f8mi_gemm_ex",
     "f8mi_sync",
     "f8mi_sync_host",
@@ -132,6 +135,12 @@ def lib() -> C.CDLL:
         L.f8mi_gemm_kb_ex.argtypes = [vp, i32, i32, vp, i32, i32, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp]
         L.f8mi_gemm_pair.restype = i32
         L.f8mi_gemm_pair.argtypes = [vp, vp, i32, vp]
+        L.f8mi_gemm_kb_bias.restype = i32
+        L.f8mi_gemm_kb_bias.argtypes = [vp, vp, i64, i64, i64, fp, fp, vp, i32, i64, vp, i32, i64, vp]
+        L.f8mi_column_sum.restype = i32
+        L.f8mi_column_sum.argtypes = [vp, i64, i64, i64, i32, vp, i32, vp, i64, vp]
+        L.f8mi_column_sum_workspace_bytes.restype = i64
+        L.f8mi_column_sum_workspace_bytes.argtypes = [i64, i64, i32]
         L.f8mi_gemm_ex.restype = i32
         L.f8mi_gemm_ex.argtypes = [vp, i32, i32, i64, vp, i32, i32, i64, i64, i64, i64, fp, fp, vp, i32, i64, vp, vp]
         L.f8mi_gemm_nt.restype = i32
@@ -497,29 +506,33 @@ def linear_layouts(m: int, k: int, n: int):
     return False, kblock_layout(k), kblock_layout(n), kblock_layout(m)
 
 
-def linear_forward(x: torch.Tensor, weight: torch.Tensor, layouts, need_dx: bool, need_dw: bool, delayed_x, delayed_w, weight_scale):
+def linear_forward(x: torch.Tensor, weight: torch.Tensor, layouts, need_dx: bool, need_dw: bool, delayed_x, delayed_w, weight_scale,
+                   bias: Optional[torch.Tensor] = None):
     """Casts and product of the fused Float8Linear's forward as one native call: (y, copy of x for backward, copy of the
     weight for backward, scale of x, scale of the weight); None for arguments that the step-by-step functions have to
-    take (or refuse).  ``delayed_x`` / ``delayed_w``: (amax, scale) buffers of a tensor with delayed scaling."""
+    take (or refuse).  ``delayed_x`` / ``delayed_w``: (amax, scale) buffers of a tensor with delayed scaling.  ``bias`` is
+    added to the rounded product, as a pass of its own would."""
     if not x.is_cuda:
         return None
     _check_device(x.device)
     idx = torch._C._cuda_getDevice()
     ws = delayed_workspace(x.device) if delayed_x is not None or delayed_w is not None else None
     return ext().linear_forward(x, weight, *layouts, need_dx, need_dw, delayed_x, delayed_w, weight_scale,
-                                None if ws is None else ws.data_ptr(), idx, torch._C._cuda_getCurrentRawStream(idx))
+                                None if ws is None else ws.data_ptr(), idx, torch._C._cuda_getCurrentRawStream(idx), bias)
 
 
-def linear_backward(dy: torch.Tensor, x_saved, w_saved, x_scale, w_scale, k: int, layouts, need_dx: bool, need_dw: bool, delayed_dy):
+def linear_backward(dy: torch.Tensor, x_saved, w_saved, x_scale, w_scale, k: int, layouts, need_dx: bool, need_dw: bool, delayed_dy,
+                    bias_dtype: Optional[torch.dtype] = None):
     """Cast and products of the fused Float8Linear's backward as one native call: (grad_input, grad_weight), or None (see
-    ``linear_forward``)."""
+    ``linear_forward``).  With ``bias_dtype`` also the gradient of the bias, in that type."""
     if not dy.is_cuda:
         return None
     idx = torch._C._cuda_getDevice()
     ws = delayed_workspace(dy.device) if delayed_dy is not None else None
     one_copy, _, kb_dx, kb_dw = layouts
     return ext().linear_backward(dy, x_saved, w_saved, x_scale, w_scale, k, one_copy, kb_dx, kb_dw, need_dx, need_dw, delayed_dy,
-                                 None if ws is None else ws.data_ptr(), idx, torch._C._cuda_getCurrentRawStream(idx))
+                                 None if ws is None else ws.data_ptr(), idx, torch._C._cuda_getCurrentRawStream(idx),
+                                 None if bias_dtype is None else _DT[bias_dtype])
 
 
 def inference_linear(x: torch.Tensor, weight: torch.Tensor, n: int, layout: int, weight_scale: torch.Tensor,

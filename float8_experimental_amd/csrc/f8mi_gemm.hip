@@ -674,3 +674,32 @@ extern "C" int f8mi_gemm_pair(const f8mi_gemm_job* a, const f8mi_gemm_job* b, in
     if (int rc = gemm_job(*a, stream)) return rc;
     return gemm_job(*b, stream);
 }
+
+// ---- a product whose bias is added to the rounded result
+
+extern "C" int f8mi_gemm_kb_bias(const void* a, const void* bt, int64_t m, int64_t n, int64_t k, const float* scale_a_dev, const float* scale_b_dev, void* c,
+                                 int c_dtype, int64_t ldc, const void* bias_dev, int bias_dtype, int64_t workspace_bytes, void* stream_) {
+    hipStream_t stream = (hipStream_t)stream_;
+    if (m < 0 || n < 0 || k < 0 || ldc < n) { set_error("f8mi_gemm_kb_bias: bad shape m=%lld n=%lld k=%lld ldc=%lld", (long long)m, (long long)n, (long long)k, (long long)ldc); return F8MI_ERR_INVALID_ARG; }
+    if (c_dtype < 0 || c_dtype > 2 || (bias_dtype != c_dtype && bias_dtype != F8MI_FP32)) { set_error("f8mi_gemm_kb_bias: unknown dtype code, or a bias neither of C's type nor fp32"); return F8MI_ERR_INVALID_ARG; }
+    if (m == 0 || n == 0) return F8MI_OK;
+    if (!a || !bt || !c || !scale_a_dev || !scale_b_dev || !bias_dev) { set_error("f8mi_gemm_kb_bias: null pointer"); return F8MI_ERR_INVALID_ARG; }
+    const int csz = c_dtype == F8MI_FP32 ? 4 : 2;
+    if (k % 128 != 0 || k < 384 || (uintptr_t)a % 16 != 0 || (uintptr_t)bt % 16 != 0 || (uintptr_t)c % csz != 0 || m > 0x7fffffff || n > 0x7fffffff || k > 0x7fffffff - BK) { set_error("f8mi_gemm_kb_bias: k %% 128 == 0, k >= 384 and aligned operands"); return F8MI_ERR_UNSUPPORTED; }
+    const int64_t tiles_m = (m + BM - 1) / BM, narrow_n = (n + NARROW_N - 1) / NARROW_N;
+    if (tiles_m * narrow_n > 0x7fffffff) { set_error("f8mi_gemm_kb_bias: too many tiles"); return F8MI_ERR_UNSUPPORTED; }
+    const GemmPlan plan = gemm_plan(m, n, k, true, workspace_bytes, rows_at_odd_addresses(c, ldc, c_dtype));
+    const bool two = plan.kind == F8MI_PLAN_TILES256_AND_128;
+    if (!two && plan.kind != F8MI_PLAN_TILES128 && plan.kind != F8MI_PLAN_TILES256 && plan.kind != F8MI_PLAN_TILES256X224) { set_error("f8mi_gemm_kb_bias: a product of other kernels"); return F8MI_ERR_UNSUPPORTED; }
+    ProfScope prof(F8MI_K_GEMM, 2.0 * (double)m * (double)n * (double)k, stream);
+    const uint8_t *A = (const uint8_t*)a, *B = (const uint8_t*)bt;
+    const int bias_fp32 = bias_dtype == F8MI_FP32;
+    const int64_t m1 = two ? plan.split.rows_large * BM : plan.kind == F8MI_PLAN_TILES128 ? 0 : m;  // rows of large tiles
+    if (m1 > 0) {
+        const int cols = plan.kind == F8MI_PLAN_TILES256X224 ? NARROW_N : BN;
+        if (int rc = launch_gemm_biased(true, cols, c_dtype, stream, A, m * 64, B, n * 64, (int)m1, (int)n, (int)k, scale_a_dev, scale_b_dev, c, ldc, bias_dev, bias_fp32, 1)) return rc;
+    }
+    if (m1 == m) return F8MI_OK;
+    return launch_gemm_biased(false, plan.mid == 2 ? 256 : 128, c_dtype, stream, A + m1 * 64, m * 64, B, n * 64, (int)(m - m1), (int)n, (int)k, scale_a_dev, scale_b_dev,
+                              (uint8_t*)c + m1 * ldc * csz, ldc, bias_dev, bias_fp32, 1);
+}

@@ -64,7 +64,7 @@ __device__ __forceinline__ float acc_read(float a) {
 // 4 (lq - 1) .. + 7 of tile 2p + 1) and one 16-byte store per lane writes 64 contiguous bytes of 16 rows.
 // (Staging the tile through LDS for 256-byte row segments takes the same time and needs the slabs to be free.)
 // ODD_ROWS: rows of C start at odd multiples of two bytes too (see ShiftedRows); a piece is then stored behind the next one.
-template <int C_DT, bool ODD_ROWS, int TJ>
+template <int C_DT, bool ODD_ROWS, int TJ, bool BIAS_AFTER>
 struct Epilogue16 {
     int M, N, c_vec_ok, lq, row0, col0, wcol0;
     bool whole, interior;  // the 256 x 256 tile lies inside C; and its rows take 16-byte stores as they are (the same for every lane)
@@ -73,12 +73,13 @@ struct Epilogue16 {
     int64_t ldc;
     void* C;
     const void* bias;
+    int bias_fp32;
     ShiftedRows rows_shifted;
     float bv[TJ][4];
 
     __device__ __forceinline__ Epilogue16(int m0, int n0, int M_, int N_, float inv_, void* C_, int64_t ldc_, const void* bias_,
-                                          int c_vec_ok_)
-        : M(M_), N(N_), c_vec_ok(c_vec_ok_), inv(inv_), ldc(ldc_), C(C_), bias(bias_),
+                                          int bias_fp32_, int c_vec_ok_)
+        : M(M_), N(N_), c_vec_ok(c_vec_ok_), inv(inv_), ldc(ldc_), C(C_), bias(bias_), bias_fp32(bias_fp32_),
           rows_shifted(C_, ldc_, m0 + (int)(threadIdx.x >> 7) * 128 + (int)(threadIdx.x & 15)) {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         lq = lane >> 4;
@@ -90,7 +91,10 @@ struct Epilogue16 {
         base = (uint16_t*)C + (int64_t)row0 * ldc + col0;
     }
 
-    __device__ __forceinline__ void load_bias_row() { load_bias_tiles<C_DT, TJ>(bv, bias, wcol0 + 4 * lq, N); }
+    __device__ __forceinline__ void load_bias_row() {
+        if constexpr (BIAS_AFTER) load_rounded_bias_tiles<C_DT, TJ>(bv, bias, bias_fp32, wcol0 + 4 * lq, N);
+        else load_bias_tiles<C_DT, TJ>(bv, bias, wcol0 + 4 * lq, N);
+    }
 
     __device__ __forceinline__ void store_held(int ti, int tp) {
         uint16_t* dst = base + ((int64_t)(ti * 16) * ldc + tp * 32);
@@ -110,10 +114,10 @@ struct Epilogue16 {
         for (int r = 0; r < 4; r++) e[r] = acc_read(acc[te][ti][r]);
 #pragma unroll
         for (int r = 0; r < 4; r++) o[r] = acc_read(acc[to][ti][r]);
-        const uint32_t x0 = pack2<C_DT>(e[0] * inv + bv[te][0], e[1] * inv + bv[te][1]);
-        const uint32_t x1 = pack2<C_DT>(e[2] * inv + bv[te][2], e[3] * inv + bv[te][3]);
-        const uint32_t y0 = pack2<C_DT>(o[0] * inv + bv[to][0], o[1] * inv + bv[to][1]);
-        const uint32_t y1 = pack2<C_DT>(o[2] * inv + bv[to][2], o[3] * inv + bv[to][3]);
+        const uint32_t x0 = finish2<C_DT, BIAS_AFTER>(e[0], e[1], inv, bv[te][0], bv[te][1]);
+        const uint32_t x1 = finish2<C_DT, BIAS_AFTER>(e[2], e[3], inv, bv[te][2], bv[te][3]);
+        const uint32_t y0 = finish2<C_DT, BIAS_AFTER>(o[0], o[1], inv, bv[to][0], bv[to][1]);
+        const uint32_t y1 = finish2<C_DT, BIAS_AFTER>(o[2], o[3], inv, bv[to][2], bv[to][3]);
         const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);
         const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
         if constexpr (ODD_ROWS) {
@@ -152,8 +156,8 @@ struct Epilogue16 {
         float e[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) e[r] = acc_read(acc[tj][ti][r]);
-        const uint32_t x0 = pack2<C_DT>(e[0] * inv + bv[tj][0], e[1] * inv + bv[tj][1]);
-        const uint32_t x1 = pack2<C_DT>(e[2] * inv + bv[tj][2], e[3] * inv + bv[tj][3]);
+        const uint32_t x0 = finish2<C_DT, BIAS_AFTER>(e[0], e[1], inv, bv[tj][0], bv[tj][1]);
+        const uint32_t x1 = finish2<C_DT, BIAS_AFTER>(e[2], e[3], inv, bv[tj][2], bv[tj][3]);
         const int row = row0 + ti * 16, col = wcol0 + tj * 16 + 4 * lq;
         uint16_t* dst = (uint16_t*)C + (int64_t)row * ldc + col;
         if (__builtin_expect(interior, 1)) {
@@ -174,7 +178,7 @@ struct Epilogue16 {
 };
 
 // fp32 outputs: a lane's 4 columns are 16 bytes already
-template <int TJ>
+template <int TJ, bool BIAS_AFTER>
 __device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[TJ][8], int m0, int n0, int M, int N, float inv,
                                                     void* __restrict__ C, int64_t ldc, const void* __restrict__ bias,
                                                     int c_vec_ok) {
@@ -199,7 +203,7 @@ __device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[TJ][8], int m0, i
             if (row >= M || col >= N) continue;
             float v[4];
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = acc_read(acc[tj][ti][r]) * inv + bv[r];
+            for (int r = 0; r < 4; r++) v[r] = finish_fp32<BIAS_AFTER>(acc_read(acc[tj][ti][r]), inv, bv[r]);
             float* dst = Cf + (int64_t)row * ldc + col;
             if (c_vec_ok && col + 4 <= N) {
                 store16_any(dst, make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])));
@@ -219,11 +223,11 @@ __device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[TJ][8], int m0, i
 // rows (64 when k-blocked over `rows`, the row stride when row-major) and a_unit / b_unit the distance between
 // blocks of 64 rows (contraction length * 64 when k-blocked, 64 when row-major).
 // Workgroup `lid` of the `npid` that compute this product.
-template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ>
+template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ, bool BIAS_AFTER = false>
 __device__ __forceinline__ void gemm_dma16_tile(
     int lid, const int npid, const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt, int64_t ldb, int64_t b_unit,
     int M, int N, int K, const float* __restrict__ sa_dev, const float* __restrict__ sb_dev, void* __restrict__ C,
-    int64_t ldc, const void* __restrict__ bias, int tiles_m, int tiles_n, int c_vec_ok) {
+    int64_t ldc, const void* __restrict__ bias, int tiles_m, int tiles_n, int c_vec_ok, int bias_fp32 = 0) {
     static_assert(TJ == 8 || (TJ == 7 && !A_TR && !B_TR && !ODD_ROWS), "narrower tiles: operands as they are");
     using Cfg = LargeCfg<TJ>;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -409,7 +413,7 @@ __device__ __forceinline__ void gemm_dma16_tile(
     // and the accumulators start from zero).
     int a_slab = 0;  // slab of A of this step; step t+2 goes to the slab before it in the rotation
     constexpr bool EPI16 = C_DT != F8MI_FP32;
-    Epilogue16<EPI16 ? C_DT : F8MI_BF16, ODD_ROWS, TJ> epi(m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
+    Epilogue16<EPI16 ? C_DT : F8MI_BF16, ODD_ROWS, TJ, BIAS_AFTER> epi(m0, n0, M, N, inv, C, ldc, bias, bias_fp32, c_vec_ok);
     auto step = [&](auto parity, auto mode) __attribute__((always_inline)) {
         constexpr int P = decltype(parity)::value;
         constexpr bool FIRST = decltype(mode)::value == 3;
@@ -509,7 +513,7 @@ __device__ __forceinline__ void gemm_dma16_tile(
         }
         epi.finish();
     } else {
-        store_c_tile16_fp32(acc, m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
+        store_c_tile16_fp32<TJ, BIAS_AFTER>(acc, m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
     }
 }
 

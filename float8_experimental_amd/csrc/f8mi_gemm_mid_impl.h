@@ -83,11 +83,11 @@ __device__ __forceinline__ uint32_t mid_tr_voff(int instr, int64_t ld, int64_t u
 
 // Workgroup `bid` of the `grid` that compute this product (or one part of its k).
 // ODD_ROWS: rows of C start at odd multiples of two bytes too (see ShiftedRows); a piece is then stored behind the next one.
-template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR, bool ODD_ROWS>
+template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR, bool ODD_ROWS, bool BIAS_AFTER = false>
 __device__ __forceinline__ void gemm_mid_tile(
     const int bid, const int grid, const int split, const uint8_t* __restrict__ A, int64_t lda, int64_t a_unit, const uint8_t* __restrict__ Bt,
     int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa_dev, const float* sb_dev, void* __restrict__ C,
-    int64_t ldc, const void* __restrict__ bias, int tiles_m, int tiles_n, int c_vec_ok, int k_splits) {
+    int64_t ldc, const void* __restrict__ bias, int tiles_m, int tiles_n, int c_vec_ok, int k_splits, int bias_fp32 = 0) {
     using Cfg = MidCfg<TJ>;
     constexpr int NSTAGE = Cfg::NSTAGE, NDMA = Cfg::NDMA;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -239,10 +239,10 @@ __device__ __forceinline__ void gemm_mid_tile(
     auto store_piece = [&](int ti, int tp) __attribute__((always_inline)) {
         if constexpr (C_DT != F8MI_FP32) {
             const int te = 2 * tp, to = 2 * tp + 1;
-            const uint32_t x0 = pack2<C_DT>(acc[te][ti][0] * inv + bv[te][0], acc[te][ti][1] * inv + bv[te][1]);
-            const uint32_t x1 = pack2<C_DT>(acc[te][ti][2] * inv + bv[te][2], acc[te][ti][3] * inv + bv[te][3]);
-            const uint32_t y0 = pack2<C_DT>(acc[to][ti][0] * inv + bv[to][0], acc[to][ti][1] * inv + bv[to][1]);
-            const uint32_t y1 = pack2<C_DT>(acc[to][ti][2] * inv + bv[to][2], acc[to][ti][3] * inv + bv[to][3]);
+            const uint32_t x0 = finish2<C_DT, BIAS_AFTER>(acc[te][ti][0], acc[te][ti][1], inv, bv[te][0], bv[te][1]);
+            const uint32_t x1 = finish2<C_DT, BIAS_AFTER>(acc[te][ti][2], acc[te][ti][3], inv, bv[te][2], bv[te][3]);
+            const uint32_t y0 = finish2<C_DT, BIAS_AFTER>(acc[to][ti][0], acc[to][ti][1], inv, bv[to][0], bv[to][1]);
+            const uint32_t y1 = finish2<C_DT, BIAS_AFTER>(acc[to][ti][2], acc[to][ti][3], inv, bv[to][2], bv[to][3]);
             const auto s0 = __builtin_amdgcn_permlane16_swap(x0, y0, false, false);  // every lane takes part
             const auto s1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
             if constexpr (ODD_ROWS) {
@@ -278,7 +278,7 @@ __device__ __forceinline__ void gemm_mid_tile(
                 if (row >= M || col >= N) continue;
                 float v[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = acc[tj][ti][e] * inv + bv[tj][e];
+                for (int e = 0; e < 4; e++) v[e] = finish_fp32<BIAS_AFTER>(acc[tj][ti][e], inv, bv[tj][e]);
                 float* dst = (float*)C + ((int64_t)split * M + row) * ldc + col;
                 if (c_vec_ok && col + 4 <= N) {
                     store16_any(dst, make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])));
@@ -303,7 +303,8 @@ __device__ __forceinline__ void gemm_mid_tile(
         // everybody's DMAs of step s+1 have landed and everybody's reads of this step's stage are done
         if constexpr (MODE < 2) mid_wait_barrier<decltype(in_flight)::value * NDMA>();
         if constexpr (MODE == 2) {
-            load_bias_tiles<C_DT, TJ>(bv, bias, wcol0 + 4 * lq, N);
+            if constexpr (BIAS_AFTER) load_rounded_bias_tiles<C_DT, TJ>(bv, bias, bias_fp32, wcol0 + 4 * lq, N);
+            else load_bias_tiles<C_DT, TJ>(bv, bias, wcol0 + 4 * lq, N);
         }
         F8MI_SCHED_FENCE();
 #pragma unroll

@@ -93,6 +93,51 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     }
 }
 
+template <int C_DT>
+__device__ __forceinline__ void unpack2(uint32_t w, float& a, float& b) {
+    if constexpr (C_DT == F8MI_BF16) {
+        a = __uint_as_float(w << 16);
+        b = __uint_as_float(w & 0xffff0000u);
+    } else {
+        a = fp16_bits_to_float(w & 0xffffu);
+        b = fp16_bits_to_float(w >> 16);
+    }
+}
+
+// Two accumulators to two packed 2-byte outputs.  BIAS_AFTER: the product is rounded to the output's type, then the bias (of that type) is
+// added and the sum rounded again, as `x @ w.t() + bias` does; else the bias is added before the only rounding.
+template <int C_DT, bool BIAS_AFTER>
+__device__ __forceinline__ uint32_t finish2(float a, float b, float inv, float bias_a, float bias_b) {
+    if constexpr (!BIAS_AFTER) {
+        return pack2<C_DT>(a * inv + bias_a, b * inv + bias_b);
+    } else {
+        float x, y;
+        unpack2<C_DT>(pack2<C_DT>(a * inv + 0.f, b * inv + 0.f), x, y);  // + 0: a product of -0 is 0, as without a bias
+        return pack2<C_DT>(x + bias_a, y + bias_b);
+    }
+}
+template <bool BIAS_AFTER>
+__device__ __forceinline__ float finish_fp32(float a, float inv, float bias) {
+    if constexpr (BIAS_AFTER) return __fadd_rn(__fmaf_rn(a, inv, 0.f), bias);
+    else return a * inv + bias;
+}
+
+// load_bias_tiles for BIAS_AFTER: a bias of C's type, or an fp32 one rounded to it.
+template <int C_DT, int TJ>
+__device__ __forceinline__ void load_rounded_bias_tiles(float (&bv)[TJ][4], const void* bias, int bias_fp32, int col0, int N) {
+    if (C_DT == F8MI_FP32 || !bias_fp32) {
+        load_bias_tiles<C_DT, TJ>(bv, bias, col0, N);
+        return;
+    }
+    load_bias_tiles<F8MI_FP32, TJ>(bv, bias, col0, N);
+    if constexpr (C_DT != F8MI_FP32) {
+#pragma unroll
+        for (int tj = 0; tj < TJ; tj++)
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) unpack2<C_DT>(pack2<C_DT>(bv[tj][e], bv[tj][e + 1]), bv[tj][e], bv[tj][e + 1]);
+    }
+}
+
 // Stores of 2-byte outputs whose rows do not all start at a multiple of four bytes (an odd row pitch): the memory system takes a 16-byte
 // store apart unless it starts at one (4096 rows, 11007 columns over 4224: 151 us at pitches 11008, 11006 and 11004, 178 at 11007, now 157;
 // 2048 x 4095 over 4096 in 128-row tiles: 33 at an even pitch, 36 at this one).  A lane of such a row stores one column further to the left instead, its neighbour's last column and its own first seven.
@@ -264,6 +309,10 @@ int launch_gemm_mid_odd(int a_fmt, int b_fmt, int c_dtype, bool wide, hipStream_
 int launch_gemm_dma16_odd(int a_fmt, int b_fmt, int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
                           const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb,
                           void* C, int64_t ldc, const void* bias, int tiles_m, int tiles_n, int c_vec_ok);
+// Both, large and 128-row tiles, with the bias added to the rounded product (f8mi_gemm_biased.hip): operands as they are, e4m3.
+// large: tiles of 256 x `cols` (256, 224); else 128 x cols (128, 256).
+int launch_gemm_biased(bool large, int cols, int c_dtype, hipStream_t stream, const uint8_t* A, int64_t a_unit, const uint8_t* Bt, int64_t b_unit, int M, int N,
+                       int K, const float* sa, const float* sb, void* C, int64_t ldc, const void* bias, int bias_fp32, int c_vec_ok);
 // Tiles of 256 x 224 (f8mi_gemm_dma16_narrow.hip), rows of C at multiples of four bytes or fp32.
 int launch_gemm_dma16_narrow(int a_fmt, int b_fmt, int c_dtype, dim3 g, hipStream_t stream, const uint8_t* A, int64_t lda, int64_t a_unit,
                              const uint8_t* Bt, int64_t ldb, int64_t b_unit, int M, int N, int K, const float* sa, const float* sb,

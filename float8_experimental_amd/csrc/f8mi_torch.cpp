@@ -31,7 +31,11 @@ struct Lib {
     decltype(&f8mi_gemm_nt_ws) gemm_nt_ws;
     decltype(&f8mi_gemm_nt_kb_ws) gemm_nt_kb_ws;
     decltype(&f8mi_gemm_kb_ex) gemm_kb_ex;
+    // null in a library without them: two products one by one, a bias and its gradient by torch
     decltype(&f8mi_gemm_pair) gemm_pair;
+    decltype(&f8mi_gemm_kb_bias) gemm_kb_bias;
+    decltype(&f8mi_column_sum) column_sum;
+    decltype(&f8mi_column_sum_workspace_bytes) column_sum_workspace_bytes;
     decltype(&f8mi_gemm_plan) gemm_plan;
     decltype(&f8mi_linear_few_rows) linear_few_rows;
     decltype(&f8mi_last_error) last_error;
@@ -190,6 +194,34 @@ struct Call {
             check(L.gemm_nt_kb_ws(a.data_ptr(), fa, bt.data_ptr(), fb, m, n, k, pa, pb, c.data_ptr(), dt, n, pbias, pws, ws_bytes, stream), "f8mi_gemm_nt_kb_ws");
         return c;
     }
+    // y = x8 w8^T (in the type of x), plus the bias added to the rounded product
+    at::Tensor gemm_biased(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& bt, const at::Tensor& sb, int layout, int64_t m, int64_t n,
+                           int64_t kc, at::ScalarType out, const at::Tensor& bias) const {
+        const int64_t k = padded(kc, layout);
+        if (layout != F8MI_LAYOUT_ROWMAJOR && L.gemm_kb_bias && (bias.scalar_type() == out || bias.scalar_type() == at::kFloat)) {
+            const at::Tensor c = make({m, n}, out);
+            const int rc = L.gemm_kb_bias(a.data_ptr(), bt.data_ptr(), m, n, k, (const float*)sa.data_ptr(), (const float*)sb.data_ptr(), c.data_ptr(),
+                                          dtype_code(out), n, bias.data_ptr(), dtype_code(bias.scalar_type()), F8MI_GEMM_WORKSPACE_BYTES, stream);
+            if (rc != F8MI_ERR_UNSUPPORTED) {
+                check(rc, "f8mi_gemm_kb_bias");
+                return c;
+            }
+        }
+        return gemm(a, sa, bt, sb, layout, m, n, kc, out).add_(bias.to(out));
+    }
+
+    // the gradient of a bias: the columns of dy summed, in dy's type, then in that of the bias
+    at::Tensor column_sum(const at::Tensor& dy, at::ScalarType bias_type) const {
+        if (!L.column_sum || !L.column_sum_workspace_bytes) return dy.sum(0).to(bias_type);
+        const int64_t rows = dy.size(0), cols = dy.size(1);
+        const int dt = dtype_code(dy.scalar_type());
+        const int64_t bytes = L.column_sum_workspace_bytes(rows, cols, dt);
+        const at::Tensor out = make({cols}, bias_type), ws = bytes ? make({bytes / 4}, at::kFloat) : at::Tensor();
+        check(L.column_sum(dy.data_ptr(), rows, cols, dy.stride(0), dt, out.data_ptr(), dtype_code(bias_type), bytes ? ws.data_ptr() : nullptr, bytes, stream),
+              "f8mi_column_sum");
+        return out;
+    }
+
     at::Tensor gemm_tr(const at::Tensor& a, bool a_tr, const at::Tensor& sa, const at::Tensor& bt, const at::Tensor& sb, int64_t m, int64_t n,
                        int64_t k, at::ScalarType out) const {
         at::Tensor c = make({m, n}, out);
@@ -250,9 +282,9 @@ PyObject* guarded(F body) {
     }
     END_HANDLE_TH_ERRORS
 }
-bool expect(Py_ssize_t got, Py_ssize_t want, const char* name) {
+bool expect(Py_ssize_t got, Py_ssize_t want, const char* name, int optional = 0) {
     if (!L.gemm_plan) PyErr_SetString(PyExc_RuntimeError, "f8mi_torch: load() has not been called");
-    else if (got != want) PyErr_Format(PyExc_TypeError, "%s takes %zd arguments, got %zd", name, want, got);
+    else if (got < want || got > want + optional) PyErr_Format(PyExc_TypeError, "%s takes %zd arguments, got %zd", name, want, got);
     else return true;
     return false;
 }
@@ -260,22 +292,26 @@ int as_int(PyObject* o) { return (int)PyLong_AsLong(o); }
 void* as_ptr(PyObject* o) { return o == Py_None ? nullptr : PyLong_AsVoidPtr(o); }
 
 // linear_forward(x [m, k], weight [n, k], one_copy, kb_fwd, kb_dx, kb_dw, need_dx, need_dw, delayed_x, delayed_w, weight_scale,
-//                delayed_workspace, device, stream) -> (y, saved of x, saved of weight, scale of x, scale of weight) or None
+//                delayed_workspace, device, stream, bias = None) -> (y, saved of x, saved of weight, scale of x, scale of weight) or None
 PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
-    if (!expect(n_args, 14, "linear_forward")) return nullptr;
+    if (!expect(n_args, 14, "linear_forward", 1)) return nullptr;
     return guarded([&]() -> PyObject* {
         const Call c{as_ptr(a[13]), as_int(a[12]), as_ptr(a[11])};
         const at::Tensor x = matrix(a[0], c.device), w = matrix(a[1], c.device);
         Scaling in, we;
         if (!x.defined() || !w.defined() || x.size(1) != w.size(1) || !in.parse(Py_None, a[8], c.device) || !we.parse(a[10], a[9], c.device)) Py_RETURN_NONE;
         if ((in.amax.defined() || we.amax.defined()) && !c.delayed_ws) Py_RETURN_NONE;
+        const bool with_bias = n_args > 14 && a[14] != Py_None;
+        const at::Tensor bias = with_bias ? plain(a[14], c.device) : at::Tensor();
+        if (with_bias && (!bias.defined() || dtype_code(bias.scalar_type()) < 0 || bias.dim() != 1 || bias.size(0) != w.size(0) || !bias.is_contiguous())) Py_RETURN_NONE;
         const bool one_copy = as_int(a[2]), need_dx = as_int(a[6]), need_dw = as_int(a[7]);
         const int kb_fwd = as_int(a[3]), kb_dx = as_int(a[4]), kb_dw = as_int(a[5]);
         at::Tensor y, x8, x8t, sx, w8, w8t, sw;
         {
             const WithoutGil no_gil;
             c.cast_two({x, in, !one_copy && need_dw, kb_fwd, kb_dw, x8, x8t, sx}, {w, we, !one_copy && need_dx, kb_fwd, kb_dx, w8, w8t, sw});
-            y = c.gemm(x8, sx, w8, sw, kb_fwd, x.size(0), w.size(0), x.size(1), x.scalar_type());
+            if (with_bias) y = c.gemm_biased(x8, sx, w8, sw, kb_fwd, x.size(0), w.size(0), x.size(1), x.scalar_type(), bias);
+            else y = c.gemm(x8, sx, w8, sw, kb_fwd, x.size(0), w.size(0), x.size(1), x.scalar_type());
         }
         if (one_copy) return wrap_all(y, x8, w8, sx, sw);
         return wrap_all(y, x8t, w8t, sx, sw);
@@ -283,9 +319,10 @@ PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 }
 
 // linear_backward(dy [m, n], saved of x, saved of weight, scale of x, scale of weight, k, one_copy, kb_dx, kb_dw, need_dx, need_dw,
-//                 delayed_dy, delayed_workspace, device, stream) -> (grad of x [m, k], grad of weight [n, k]) or None
+//                 delayed_dy, delayed_workspace, device, stream, type of the bias = None) -> (grad of x [m, k], grad of weight [n, k]
+//                 and, with such a type, grad of the bias [n]) or None
 PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
-    if (!expect(n_args, 15, "linear_backward")) return nullptr;
+    if (!expect(n_args, 15, "linear_backward", 1)) return nullptr;
     return guarded([&]() -> PyObject* {
         const Call c{as_ptr(a[14]), as_int(a[13]), as_ptr(a[12])};
         const at::Tensor dy = matrix(a[0], c.device);
@@ -306,8 +343,12 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             const int layout = one_copy ? F8MI_LAYOUT_KBLOCK64 : t == &xs ? kb_dw : kb_dx;
             if (fp8_code(t->scalar_type()) < 0 || !t->is_contiguous() || t->sizes() != copy_sizes(rows, kc, layout)) Py_RETURN_NONE;
         }
-        at::Tensor g8, g8t, sg, dx, dw;
+        const bool need_db = n_args > 15 && a[15] != Py_None;
+        const int bias_dt = need_db ? as_int(a[15]) : F8MI_FP32;
+        const at::ScalarType bias_type = bias_dt == F8MI_BF16 ? at::kBFloat16 : bias_dt == F8MI_FP16 ? at::kHalf : at::kFloat;
+        at::Tensor g8, g8t, sg, dx, dw, db;
         const auto compute = [&] {
+            if (need_db) db = c.column_sum(dy, bias_type);
             if (one_copy) {
                 c.cast(dy, go, F8MI_E5M2, true, F8MI_LAYOUT_KBLOCK64, false, 0, g8, g8t, sg);
                 if (need_dx && need_dw && L.gemm_pair) {
@@ -330,6 +371,7 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             const WithoutGil no_gil;
             compute();
         }
+        if (need_db) return wrap_all(dx, dw, db);
         return wrap_all(dx, dw);
     });
 }
@@ -409,7 +451,11 @@ PyObject* load(PyObject*, PyObject* args) {
     get(L.gemm_plan, "f8mi_gemm_plan");
     get(L.cast_dynamic_pair, "f8mi_cast_dynamic_pair");
     get(L.cast_delayed_pair, "f8mi_cast_delayed_pair");
-    L.gemm_pair = reinterpret_cast<decltype(L.gemm_pair)>(dlsym(h, "f8mi_gemm_pair"));  // without it the products go one by one
+    const auto get_if_there = [&](auto& f, const char* name) { f = reinterpret_cast<std::decay_t<decltype(f)>>(dlsym(h, name)); };
+    get_if_there(L.gemm_pair, "f8mi_gemm_pair");
+    get_if_there(L.gemm_kb_bias, "f8mi_gemm_kb_bias");
+    get_if_there(L.column_sum, "f8mi_column_sum");
+    get_if_there(L.column_sum_workspace_bytes, "f8mi_column_sum_workspace_bytes");
     if (missing) {
         L.gemm_plan = nullptr;
         return PyErr_Format(PyExc_ImportError, "%s does not export %s", path, missing);

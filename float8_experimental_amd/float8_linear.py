@@ -35,6 +35,8 @@ from .float8_tensor import (
 from .float8_utils import e4m3_dtype, e5m2_dtype
 
 _KINDS = ("input", "weight", "grad_output")
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+_HP_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 
 
 @torch._dynamo.allow_in_graph
@@ -103,7 +105,8 @@ def _gemm(a8, sa, b8, sb, out_dtype, kb: bool):
 
 
 class _float8_linear_fn(torch.autograd.Function):
-    """y = x W^T with every matmul of forward and backward in fp8 (no bias).
+    """y = x W^T (+ bias) with every matmul of forward and backward in fp8.  A bias is added to the product rounded to its
+    type, and its gradient is the column sum of dY in that type, as ``x @ w.t() + bias`` has them.
 
     Each of the three GEMMs contracts a different dimension (in_features, out_features, tokens).
     When all three are multiples of 128 (and at least 384) each tensor is cast ONCE, k-blocked over
@@ -116,7 +119,7 @@ class _float8_linear_fn(torch.autograd.Function):
     """
 
     @staticmethod
-    def forward(ctx, x, weight, mod, is_amax_initialized):
+    def forward(ctx, x, weight, mod, is_amax_initialized, bias=None):
         k = x.shape[-1]
         x2 = x.reshape(-1, k)
         m, n = x2.shape[0], weight.shape[0]
@@ -128,10 +131,11 @@ class _float8_linear_fn(torch.autograd.Function):
         ctx.is_amax_initialized = is_amax_initialized
         ctx.x_shape = x.shape
         ctx.layouts = None
+        ctx.bias_dtype = None if bias is None else bias.dtype
         if not emulate and not emulate_bw and (is_amax_initialized or not mod.has_any_delayed_scaling):
             layouts = _native.linear_layouts(m, k, n)
             done = _native.linear_forward(x2, weight, layouts, need_dx, need_dw, mod._delayed_pair("input"), mod._delayed_pair("weight"),
-                                          mod._precomputed_weight_scale)
+                                          mod._precomputed_weight_scale, bias)
             if done is not None:
                 y, xs, ws, sx, sw = done
                 ctx.layouts = layouts
@@ -159,6 +163,8 @@ class _float8_linear_fn(torch.autograd.Function):
                 y = _gemm(x8, sx, w8, sw, x.dtype, kb_fwd)
             ctx.kb = (kb_dx, kb_dw)
             ctx.save_for_backward(x8t, w8t, sx, sw)
+        if bias is not None:
+            y = y + bias.to(y.dtype)
         return y.reshape(*x.shape[:-1], n)
 
     @staticmethod
@@ -166,14 +172,23 @@ class _float8_linear_fn(torch.autograd.Function):
         mod = ctx.mod
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         dy2 = dy.reshape(-1, dy.shape[-1])
-        dx = dw = None
+        dx = dw = db = None
+        need_db = ctx.needs_input_grad[4]
+        if need_db and (torch.is_grad_enabled() or not (need_dx or need_dw)):  # with create_graph: a sum that has a gradient itself
+            db = dy2.sum(0).to(ctx.bias_dtype)
+            need_db = False
+        if not (need_dx or need_dw):
+            return None, None, None, None, db
         saved = ctx.saved_tensors  # once: non-reentrant checkpointing refuses to unpack a tensor a second time
-        if ctx.layouts is not None and (need_dx or need_dw):
+        if ctx.layouts is not None:
             done = _native.linear_backward(dy2, *saved, ctx.x_shape[-1], ctx.layouts, need_dx, need_dw,
-                                           mod._delayed_pair("grad_output"))
+                                           mod._delayed_pair("grad_output"), ctx.bias_dtype if need_db else None)
             if done is not None:
-                dx, dw = done
-                return dx if dx is None or len(ctx.x_shape) == 2 else dx.reshape(ctx.x_shape), dw, None, None
+                dx, dw, *native_db = done
+                return (dx if dx is None or len(ctx.x_shape) == 2 else dx.reshape(ctx.x_shape), dw, None, None,
+                        native_db[0] if need_db else db)
+        if need_db:
+            db = dy2.sum(0).to(ctx.bias_dtype)
         dlg = mod._delayed_buffers("grad_output")
         if ctx.kb is None:  # one copy per tensor: x8 [K/64, M, 64], w8 [K/64, N, 64], g8 [N/64, M, 64]
             x8, w8, sx, sw = saved
@@ -182,7 +197,7 @@ class _float8_linear_fn(torch.autograd.Function):
                 dx = _native.gemm_kb_ex(g8, False, sg, w8, True, sw, dy.dtype).reshape(ctx.x_shape)
             if need_dw:  # grad_weight = dY^T @ x: both read transposed
                 dw = _native.gemm_kb_ex(g8, True, sg, x8, True, sx, dy.dtype)
-            return dx, dw, None, None
+            return dx, dw, None, None, db
         x8t, w8t, sx, sw = saved
         kb_dx, kb_dw = ctx.kb
         g8, g8t, sg = _cast_for_gemm(dy2, e5m2_dtype, dlg, ctx.is_amax_initialized, need_dx, need_dw, kb_dx, kb_dw)
@@ -198,7 +213,7 @@ class _float8_linear_fn(torch.autograd.Function):
                 dw = torch.ops.aten.mm_float8_emulated(g8t, sg, x8t.t(), sx, dy.dtype)
             else:
                 dw = _gemm(g8t, sg, x8t, sx, dy.dtype, kb_dw)
-        return dx, dw, None, None
+        return dx, dw, None, None, db
 
 
 class Float8Linear(torch.nn.Linear):
@@ -410,12 +425,20 @@ class Float8Linear(torch.nn.Linear):
             # pre-cast operands: only the composed path knows how to pass them through
             return self._forward_composed_body(input)
         x = self._autocast_input(input)
-        output = _float8_linear_fn.apply(x, self.weight, self, self.is_amax_initialized)
-        if self.bias is not None:
-            output = output + self.bias.to(output.dtype)
+        bias = self.bias
+        inside = bias is not None and self._bias_inside(x, bias)
+        output = _float8_linear_fn.apply(x, self.weight, self, self.is_amax_initialized, bias if inside else None)
+        if bias is not None and not inside:
+            output = output + bias.to(output.dtype)
         if self.has_any_delayed_scaling:
             self.float8_post_forward()
         return output
+
+    def _bias_inside(self, x: torch.Tensor, bias: torch.Tensor) -> bool:
+        """True where the fused function takes the bias along: plain tensors on the GPU and nothing that would have to see the
+        addition as an operation of its own (subclasses, forward-mode derivatives, which the function has none of)."""
+        return (type(x) in _PLAIN and type(bias) in _PLAIN and x.is_cuda and bias.is_cuda and bias.shape == self.weight.shape[:1]
+                and bias.dtype in _HP_DTYPES and not self.config.emulate and torch.autograd.forward_ad._current_level < 0)
 
     def _forward_composed_body(self, input):
         input_fp8 = self.cast_input_to_float8(input, self.is_amax_initialized)

@@ -342,6 +342,19 @@ int f8mi_gemm_kb_ex(const void* a, int a_fmt, int a_transposed, const void* bt, 
                     int64_t n, int64_t k, const float* scale_a_dev, const float* scale_b_dev, void* c, int c_dtype,
                     int64_t ldc, const void* bias_dev, void* stream);
 
+/* f8mi_gemm_nt_kb of two e4m3 operands with the bias added to the finished product: rounded to C's type, the bias (of that type, or fp32
+ * and rounded to it) added, the sum rounded again, the bits of the product followed by a pass that adds the bias.  k % 128 == 0 and the
+ * products that f8mi_gemm_plan gives to 128-row, 256 x 256 or 256 x 224 tiles, workspace_bytes as there; F8MI_ERR_UNSUPPORTED, nothing
+ * queued, for all others. */
+int f8mi_gemm_kb_bias(const void* a, const void* bt, int64_t m, int64_t n, int64_t k, const float* scale_a_dev, const float* scale_b_dev,
+                      void* c, int c_dtype, int64_t ldc, const void* bias_dev, int bias_dtype, int64_t workspace_bytes, void* stream);
+
+/* out[j] = the sum of column j of x [rows][cols] (rows `ld` elements apart, unit column stride): fp32 sums in a fixed order, rounded to
+ * x's type and stored in out_dtype: the gradient of a bias.  workspace: f8mi_column_sum_workspace_bytes (0: none needed). */
+int f8mi_column_sum(const void* x, int64_t rows, int64_t cols, int64_t ld, int dtype, void* out, int out_dtype, void* workspace,
+                    int64_t workspace_bytes, void* stream);
+int64_t f8mi_column_sum_workspace_bytes(int64_t rows, int64_t cols, int dtype);
+
 /* One product of a call that computes two: the arguments of f8mi_gemm_kb_ex without a bias and, for operands that are both given as they
  * are, the workspace of f8mi_gemm_nt_kb_ws. */
 typedef struct f8mi_gemm_job {

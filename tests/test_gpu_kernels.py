@@ -1083,6 +1083,54 @@ def test_gemm_pair_equals_the_products_one_by_one(nat, tokens, k, n, out_dt):
         assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), 3, nat._stream(g)) == nat.ERR_UNSUPPORTED
 
 
+# A bias added to the rounded product, on each of the tiles that take it: 128 x 128, 128 x 256, 256 x 256 with and without a sparse last round,
+# 256 x 224, odd and even step counts and rows of C; refused where the product runs on other kernels.
+@pytest.mark.parametrize("m,n,k,plan", [(300, 200, 512, "tiles128"), (257, 511, 384, "tiles128"), (2048, 4000, 640, "tiles128"), (2040, 3999, 384, "tiles128"),
+                                        (4096, 4096, 384, "tiles256"), (4090, 4095, 512, "tiles256"), (4352, 4095, 640, "tiles256_and_128"),
+                                        (2048, 14336, 512, "tiles256x224"), (2000, 14300, 384, "tiles256x224"), (16, 512, 512, None), (64, 2048, 8192, None)])
+@pytest.mark.parametrize("out_dt,bias_dt", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float16, torch.float32),
+                                            (torch.float16, torch.float16), (torch.float32, torch.float32)])
+def test_gemm_adds_a_bias_to_the_rounded_product(nat, m, n, k, plan, out_dt, bias_dt):
+    a, bt = (_rand_fp8((r, k), torch.float8_e4m3fn, r + k + i, 4.0).to(DEV) for i, r in enumerate((m, n)))
+    sa, sb = torch.tensor(2.0, device=DEV), torch.tensor(0.25, device=DEV)
+    bias = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 3).to(bias_dt).to(DEV)
+    c, ka, kbt = torch.full((m, n), float("nan"), device=DEV, dtype=out_dt), _to_kb(a), _to_kb(bt)
+    call = lambda dt: nat.lib().f8mi_gemm_kb_bias(ka.data_ptr(), kbt.data_ptr(), m, n, k, sa.data_ptr(), sb.data_ptr(), c.data_ptr(), nat._DT[out_dt], n,
+                                                  bias.data_ptr(), dt, nat.GEMM_WORKSPACE_BYTES, nat._stream(a))
+    if plan is None:
+        assert call(nat._DT[bias_dt]) == nat.ERR_UNSUPPORTED
+        return
+    assert nat.gemm_plan(m, n, k)[0] == plan
+    assert call(nat._DT[bias_dt]) == 0, nat.lib().f8mi_last_error()
+    want = nat.gemm_nt_kb(ka, sa, kbt, sb, out_dt) + bias.to(out_dt)
+    assert torch.equal(c, want)
+
+
+# One row and one workgroup's rows with one more or less; columns that leave a lane some of its eight or four; several chunks; rows at any
+# distance and alignment.  Any order of fp32 additions is within rows * 2^-24 of the sum of the magnitudes; then the rounding to x's type (half an
+# ulp: 2^-8 of a number with 8 bits, 2^-11, 2^-24) and to the bias's.
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (31, 512), (32, 513), (33, 256), (129, 1031), (4096, 4096), (4099, 11007), (20000, 24), (700, 70001)])
+@pytest.mark.parametrize("dt,out_dt", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float16, torch.float32), (torch.float32, torch.float32),
+                                       (torch.float32, torch.bfloat16)])
+def test_column_sum(nat, rows, cols, dt, out_dt):
+    base = heavy((rows, cols + 5), torch.float32, rows + cols).clamp(-100, 100).to(dt).to(DEV)
+    for x in (base[:, :cols].contiguous(), base[:, 3:cols + 3]):
+        need = nat.lib().f8mi_column_sum_workspace_bytes(rows, cols, nat._DT[dt])
+        ws, out = torch.empty(max(need // 4, 1), device=DEV), torch.full((cols,), float("nan"), device=DEV, dtype=out_dt)
+        call = lambda t: nat.lib().f8mi_column_sum(t.data_ptr(), rows, cols, t.stride(0), nat._DT[dt], out.data_ptr(), nat._DT[out_dt], ws.data_ptr(), need, nat._stream(t))
+        assert call(x) == 0, nat.lib().f8mi_last_error()
+        want, half = x.double().sum(0), {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11, torch.float32: 2.0**-24}
+        bound = rows * 2.0**-24 * x.double().abs().sum(0)
+        bound = bound + (want.abs() + bound) * (half[dt] + half[out_dt] * 1.01) + 2.0**-24  # (fp16: half of its smallest number)
+        assert ((out.double() - want).abs() <= bound).all()
+        again = out.clone()
+        assert call(x) == 0 and torch.equal(out, again)  # a fixed order
+    x = base[:, :cols].clone()
+    x[rows // 2, cols // 2], x[0, 0] = float("inf"), float("nan")
+    assert call(x) == 0 and torch.isnan(out[0]) and (cols == 1 or out[cols // 2] == float("inf") or cols // 2 == 0)
+    assert call(x) == 0 and torch.isfinite(out).sum() == cols - len({0, cols // 2})
+
+
 # Few rows: one to three 128-deep steps per wave and one more or less of them, on each block of rows and both widths.
 @pytest.mark.parametrize("m,n,k", [(m, n, k) for m, n in ((1, 1000), (16, 4104), (17, 40), (32, 1000), (33, 40), (64, 1000))
                                    for k in (128, 896, 1024, 1152, 2048, 2176, 3200) if m <= 16 or k > 128])

@@ -930,3 +930,69 @@ def test_native_host_path_refuses_saved_copies_of_another_shape(f8, m, k, n):
         y = mod(x)
     with pytest.raises(Exception):
         y.backward(torch.randn_like(y))
+
+
+@pytest.mark.parametrize("m,k,n", [(512, 1024, 1024), (300, 520, 1000), (2048, 512, 14336), (4, 512, 512)])
+@pytest.mark.parametrize("scaling", ["dynamic", "delayed"])
+@pytest.mark.parametrize("dtype,bias_dtype,autocast", [(torch.bfloat16, torch.bfloat16, False), (torch.float32, torch.float32, True),
+                                                       (torch.float32, torch.float32, False), (torch.float16, torch.float32, False)])
+def test_bias_inside_the_fused_function_equals_the_addition_outside(f8, monkeypatch, m, k, n, scaling, dtype, bias_dtype, autocast):
+    """The same output bits and gradients as the product without a bias, ``+ bias``, and its gradient by autograd (whose sum has another
+    order: within m * 2^-24 of the magnitudes and one rounding of the output's type)."""
+    kind = f8.CastConfig(scaling_type=f8.ScalingType.DELAYED if scaling == "delayed" else f8.ScalingType.DYNAMIC)
+    config = f8.Float8LinearConfig(cast_config_input=kind, cast_config_weight=kind, cast_config_grad_output=kind)
+    g = torch.Generator().manual_seed(m + n)
+    act = torch.bfloat16 if autocast else dtype
+    w, b = (torch.randn(n, k, generator=g) / 30).to(dtype).to(DEV), torch.randn(n, generator=g).to(bias_dtype).to(DEV)
+    x0, dy = torch.randn(2, m // 2, k, generator=g).to(act).to(DEV), (torch.randn(2, m // 2, n, generator=g) / 100).to(act).to(DEV)
+
+    def step(inside, frozen=()):
+        lin = torch.nn.Linear(k, n, device=DEV, dtype=dtype)
+        lin.weight, lin.bias = torch.nn.Parameter(w.clone()), torch.nn.Parameter(b.clone())
+        mod = f8.convert_to_float8_training(torch.nn.Sequential(lin), config=config)
+        if not inside:
+            monkeypatch.setattr(f8.Float8Linear, "_bias_inside", lambda self, x, bias: False)
+        out = []
+        for it in range(2):
+            if it and scaling == "delayed":
+                f8.sync_float8_amax_and_scale_history(mod)
+            x = x0.clone().requires_grad_("x" not in frozen)
+            mod[0].weight.requires_grad_("w" not in frozen)
+            mod.zero_grad()
+            with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+                y = mod(x)
+            y.backward(dy)
+            out += [y.detach(), x.grad, mod[0].weight.grad] + [t.clone() for t in mod.buffers()]
+            grad = mod[0].bias.grad
+        monkeypatch.undo()
+        return out, grad
+
+    for frozen in ((), ("x",), ("x", "w")):
+        (got, got_db), (want, want_db) = step(True, frozen), step(False, frozen)
+        assert len(got) == len(want) and all(p is q is None or torch.equal(p, q) for p, q in zip(got, want))
+        assert got_db.dtype == want_db.dtype == bias_dtype and got_db.shape == want_db.shape
+        exact, ulp = dy.double().sum((0, 1)), {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11, torch.float32: 2.0**-24}[act]
+        bound = m * 2.0**-24 * dy.double().abs().sum((0, 1))
+        assert ((got_db.double() - exact).abs() <= bound + (exact.abs() + bound) * ulp + 2.0**-24).all()
+
+
+def test_bias_gradient_with_create_graph_has_a_gradient_itself(f8):
+    mod = f8.convert_to_float8_training(torch.nn.Sequential(torch.nn.Linear(512, 512, device=DEV, dtype=torch.bfloat16)))
+    y = mod(torch.randn(64, 512, device=DEV, dtype=torch.bfloat16))
+    dy = torch.randn_like(y).requires_grad_()
+    (db,) = torch.autograd.grad(y, mod[0].bias, dy, create_graph=True)
+    (ddy,) = torch.autograd.grad(db.sum(), dy)
+    assert torch.equal(ddy, torch.ones_like(dy))
+
+
+def test_bias_with_a_forward_mode_derivative_is_added_outside(f8):
+    """As before: the fused function has no forward-mode derivative, the addition of a bias has."""
+    import torch.autograd.forward_ad as fwd
+
+    mod = f8.convert_to_float8_training(torch.nn.Sequential(torch.nn.Linear(512, 256, device=DEV, dtype=torch.bfloat16)))
+    bias = mod[0].bias.detach()
+    del mod[0].bias
+    with fwd.dual_level(), torch.no_grad():
+        mod[0].bias = fwd.make_dual(bias, torch.ones_like(bias))
+        y, tangent = fwd.unpack_dual(mod(torch.randn(64, 512, device=DEV, dtype=torch.bfloat16)))
+        assert torch.equal(tangent, torch.ones_like(y))
