@@ -52,7 +52,7 @@ __device__ __forceinline__ float acc_read(float a) {
     return v;
 }
 
-// The epilogue: scales the 8 x 8 tiles of 16 x 16 accumulators, adds the bias, converts and writes C.
+// The epilogue: scales the 8 x 8 (TJ x 8) tiles of 16 x 16 accumulators, adds the bias, converts and writes C.
 // acc[tj][ti] as left by MFMA(first = Bt rows, second = A rows): lane holds row ti*16 + lane%16
 // and the four columns tj*16 + 4*(lane/16) + e of its wave's 128 x 128 quarter.
 //
@@ -63,12 +63,16 @@ __device__ __forceinline__ float acc_read(float a) {
 // every lane holds 8 neighbouring columns (lq even: columns 4 lq .. 4 lq + 7 of tile 2p; lq odd: columns
 // 4 (lq - 1) .. + 7 of tile 2p + 1) and one 16-byte store per lane writes 64 contiguous bytes of 16 rows.
 // (Staging the tile through LDS for 256-byte row segments takes the same time and needs the slabs to be free.)
+// A piece of an fp32 C is a lane's own four columns of either tile, two 16-byte stores (us, all of the tile written
+// behind the last MFMA / piece by piece: 4096 x 4096 over 4096 54.8 / 51.4, 8192 x 4096 over 1024 47.9 / 40.7, 8192 x 14336 over 4096 404 / 358,
+// 4099 x 11007 over 4224 186 / 150).
 // ODD_ROWS: rows of C start at odd multiples of two bytes too (see ShiftedRows); a piece is then stored behind the next one.
 template <int C_DT, bool ODD_ROWS, int TJ, bool BIAS_AFTER>
 struct Epilogue16 {
     int M, N, c_vec_ok, lq, row0, col0, wcol0;
     bool whole, interior;  // the 256 x 256 tile lies inside C; and its rows take 16-byte stores as they are (the same for every lane)
     uint16_t* base;  // of the lane's first piece: a piece's address is this plus an offset that is the same for every lane
+    float* base32;   // the same of an fp32 C
     float inv;
     int64_t ldc;
     void* C;
@@ -89,10 +93,12 @@ struct Epilogue16 {
         whole = m0 + 256 <= M && n0 + 32 * TJ <= N;
         interior = c_vec_ok && whole;
         base = (uint16_t*)C + (int64_t)row0 * ldc + col0;
+        base32 = (float*)C + (int64_t)row0 * ldc + wcol0 + 4 * lq;
     }
 
     __device__ __forceinline__ void load_bias_row() {
-        if constexpr (BIAS_AFTER) load_rounded_bias_tiles<C_DT, TJ>(bv, bias, bias_fp32, wcol0 + 4 * lq, N);
+        if constexpr (c_is_fp32(C_DT)) load_bias_tiles<F8MI_FP32, TJ>(bv, bias, wcol0 + 4 * lq, N);
+        else if constexpr (BIAS_AFTER) load_rounded_bias_tiles<C_DT, TJ>(bv, bias, bias_fp32, wcol0 + 4 * lq, N);
         else load_bias_tiles<C_DT, TJ>(bv, bias, wcol0 + 4 * lq, N);
     }
 
@@ -105,7 +111,7 @@ struct Epilogue16 {
         if constexpr (ODD_ROWS) store_held(7, 3);
     }
 
-    // rows ti*16 .. +15, columns tp*32 .. +31 of the wave's quarter (C_DT: bf16 or fp16); every lane must call it; pieces of a row of
+    // rows ti*16 .. +15, columns tp*32 .. +31 of the wave's quarter; every lane must call it; pieces of a row of
     // tiles from left to right, rows from the top
     __device__ __forceinline__ void piece(v4f (&acc)[TJ][8], int ti, int tp) {
         const int te = 2 * tp, to = 2 * tp + 1;
@@ -114,6 +120,13 @@ struct Epilogue16 {
         for (int r = 0; r < 4; r++) e[r] = acc_read(acc[te][ti][r]);
 #pragma unroll
         for (int r = 0; r < 4; r++) o[r] = acc_read(acc[to][ti][r]);
+        if constexpr (c_is_fp32(C_DT)) {
+            const int r = row0 + ti * 16, c = wcol0 + te * 16 + 4 * lq;
+            float* dst = base32 + ((int64_t)(ti * 16) * ldc + tp * 32);
+            store_fp32x4(dst, finish4<C_DT, BIAS_AFTER>(e, inv, bv[te]), interior, c_vec_ok, r, c, M, N);
+            store_fp32x4(dst + 16, finish4<C_DT, BIAS_AFTER>(o, inv, bv[to]), interior, c_vec_ok, r, c + 16, M, N);
+            return;
+        }
         const uint32_t x0 = finish2<C_DT, BIAS_AFTER>(e[0], e[1], inv, bv[te][0], bv[te][1]);
         const uint32_t x1 = finish2<C_DT, BIAS_AFTER>(e[2], e[3], inv, bv[te][2], bv[te][3]);
         const uint32_t y0 = finish2<C_DT, BIAS_AFTER>(o[0], o[1], inv, bv[to][0], bv[to][1]);
@@ -156,6 +169,11 @@ struct Epilogue16 {
         float e[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) e[r] = acc_read(acc[tj][ti][r]);
+        if constexpr (c_is_fp32(C_DT)) {
+            store_fp32x4(base32 + ((int64_t)(ti * 16) * ldc + tj * 16), finish4<C_DT, BIAS_AFTER>(e, inv, bv[tj]), interior, c_vec_ok, row0 + ti * 16,
+                         wcol0 + tj * 16 + 4 * lq, M, N);
+            return;
+        }
         const uint32_t x0 = finish2<C_DT, BIAS_AFTER>(e[0], e[1], inv, bv[tj][0], bv[tj][1]);
         const uint32_t x1 = finish2<C_DT, BIAS_AFTER>(e[2], e[3], inv, bv[tj][2], bv[tj][3]);
         const int row = row0 + ti * 16, col = wcol0 + tj * 16 + 4 * lq;
@@ -176,45 +194,6 @@ struct Epilogue16 {
         }
     }
 };
-
-// fp32 outputs: a lane's 4 columns are 16 bytes already
-template <int TJ, bool BIAS_AFTER>
-__device__ __forceinline__ void store_c_tile16_fp32(v4f (&acc)[TJ][8], int m0, int n0, int M, int N, float inv,
-                                                    void* __restrict__ C, int64_t ldc, const void* __restrict__ bias,
-                                                    int c_vec_ok) {
-    constexpr int C_DT = F8MI_FP32;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int lm = lane & 15, lq = lane >> 4;
-    const int wrow0 = m0 + wm * 128, wcol0 = n0 + wn * (16 * TJ);
-    float* Cf = (float*)C;
-#pragma unroll
-    for (int tj = 0; tj < TJ; tj++) {
-        const int col = wcol0 + tj * 16 + 4 * lq;
-        float bv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (bias) {
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-                if (col + r < N) bv[r] = load_bias<C_DT>(bias, col + r);
-        }
-#pragma unroll
-        for (int ti = 0; ti < 8; ti++) {
-            const int row = wrow0 + ti * 16 + lm;
-            if (row >= M || col >= N) continue;
-            float v[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = finish_fp32<BIAS_AFTER>(acc_read(acc[tj][ti][r]), inv, bv[r]);
-            float* dst = Cf + (int64_t)row * ldc + col;
-            if (c_vec_ok && col + 4 <= N) {
-                store16_any(dst, make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])));
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-                    if (col + r < N) dst[r] = v[r];
-            }
-        }
-    }
-}
 
 // ODD (from the host): the number of steps K/128 is odd.
 // A_TR / B_TR: the operand is given "transposed": its memory holds the matrix [contraction][rows] (the layout
@@ -412,8 +391,7 @@ __device__ __forceinline__ void gemm_dma16_tile(
     // step's start with step t+2); 1: last but one (nothing left to fetch); 2: last step; 3: step 0 (as 0,
     // and the accumulators start from zero).
     int a_slab = 0;  // slab of A of this step; step t+2 goes to the slab before it in the rotation
-    constexpr bool EPI16 = C_DT != F8MI_FP32;
-    Epilogue16<EPI16 ? C_DT : F8MI_BF16, ODD_ROWS, TJ, BIAS_AFTER> epi(m0, n0, M, N, inv, C, ldc, bias, bias_fp32, c_vec_ok);
+    Epilogue16<C_DT, ODD_ROWS, TJ, BIAS_AFTER> epi(m0, n0, M, N, inv, C, ldc, bias, bias_fp32, c_vec_ok);
     auto step = [&](auto parity, auto mode) __attribute__((always_inline)) {
         constexpr int P = decltype(parity)::value;
         constexpr bool FIRST = decltype(mode)::value == 3;
@@ -431,7 +409,7 @@ __device__ __forceinline__ void gemm_dma16_tile(
         // core busy for 32 cycles): one fragment (two 16-byte LDS reads) or one DMA at a time.
         // The last step has neither; there the finished row of accumulator tiles (ti - 1: its last MFMA was issued
         // eight MFMAs before the first read) is scaled, converted and stored under the MFMAs of row ti.
-        if (MODE == 2 && EPI16) epi.load_bias_row();
+        if (MODE == 2) epi.load_bias_row();
 #pragma unroll
         for (int ti = 0; ti < 8; ti++) {
             if (ti == 6 && MODE < 2) {
@@ -454,12 +432,12 @@ __device__ __forceinline__ void gemm_dma16_tile(
                 else mfma16<BF, AF>(acc[tj][ti], fb[P][tj], fa[ti & 1]);
                 F8MI_SCHED_FENCE();
                 // (seven tiles: a place later, and the last one in the row after, for the same distance from the MFMA that wrote it)
-                if (MODE == 2 && EPI16 && ti >= 1 && (TJ == 8 ? (tj & 1) == 1 : tj >= 2 && (tj & 1) == 0)) {
+                if (MODE == 2 && ti >= 1 && (TJ == 8 ? (tj & 1) == 1 : tj >= 2 && (tj & 1) == 0)) {
                     epi.piece(acc, ti - 1, TJ == 8 ? tj >> 1 : (tj >> 1) - 1);
                     F8MI_SCHED_FENCE();
                 }
                 if constexpr (TJ == 7) {
-                    if (MODE == 2 && EPI16 && ti >= 2 && tj == 1) {
+                    if (MODE == 2 && ti >= 2 && tj == 1) {
                         epi.piece_last(acc, ti - 2);
                         F8MI_SCHED_FENCE();
                     }
@@ -504,17 +482,13 @@ __device__ __forceinline__ void gemm_dma16_tile(
     // the last MFMAs are still in the pipeline (8 passes): keep the accumulator reads away from them.  (No DMA is
     // outstanding: the last but one step waited for all of them.)
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-    if constexpr (EPI16) {
 #pragma unroll
-        for (int tp = 0; tp < TJ / 2; tp++) epi.piece(acc, 7, tp);
-        if constexpr (TJ == 7) {
-            epi.piece_last(acc, 6);
-            epi.piece_last(acc, 7);
-        }
-        epi.finish();
-    } else {
-        store_c_tile16_fp32<TJ, BIAS_AFTER>(acc, m0, n0, M, N, inv, C, ldc, bias, c_vec_ok);
+    for (int tp = 0; tp < TJ / 2; tp++) epi.piece(acc, 7, tp);
+    if constexpr (TJ == 7) {
+        epi.piece_last(acc, 6);
+        epi.piece_last(acc, 7);
     }
+    epi.finish();
 }
 
 template <int AF, int BF, int C_DT, bool ODD, bool A_TR, bool B_TR, bool ODD_ROWS, int TJ>

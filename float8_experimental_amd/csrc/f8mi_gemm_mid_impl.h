@@ -230,6 +230,7 @@ __device__ __forceinline__ void gemm_mid_tile(
     const bool whole = m0 + MID_TILE_M <= M && n0 + Cfg::TILE_N <= N;
     const bool interior = c_vec_ok && whole;  // the same for every lane: nothing to check
     const int col_l = wcol0 + (lq & 1) * 16 + (lq >> 1) * 8;
+    float* const base32 = (float*)C + ((int64_t)split * M + m0 + wm * 64 + lm) * ldc + wcol0 + 4 * lq;  // of the lane's first piece of an fp32 C
     auto store_held = [&](int ti, int tp) __attribute__((always_inline)) {
         const int row = m0 + wm * 64 + ti * 16 + lm, col = col_l + tp * 32;
         uint16_t* dst = (uint16_t*)C + (int64_t)row * ldc + col;
@@ -237,8 +238,16 @@ __device__ __forceinline__ void gemm_mid_tile(
         else rows_shifted.store(dst, false, tp == 0, tp == TJ / 2 - 1, row, col, M, N);
     };
     auto store_piece = [&](int ti, int tp) __attribute__((always_inline)) {
-        if constexpr (C_DT != F8MI_FP32) {
-            const int te = 2 * tp, to = 2 * tp + 1;
+        const int te = 2 * tp, to = 2 * tp + 1;
+        if constexpr (c_is_fp32(C_DT)) {  // a lane's 4 columns are 16 bytes already
+            const int row = m0 + wm * 64 + ti * 16 + lm, col = wcol0 + te * 16 + 4 * lq;
+            float* dst = base32 + ((int64_t)(ti * 16) * ldc + tp * 32);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const float v[4] = {acc[te + h][ti][0], acc[te + h][ti][1], acc[te + h][ti][2], acc[te + h][ti][3]};
+                store_fp32x4(dst + 16 * h, finish4<C_DT, BIAS_AFTER>(v, inv, bv[te + h]), interior, c_vec_ok, row, col + 16 * h, M, N);
+            }
+        } else {
             const uint32_t x0 = finish2<C_DT, BIAS_AFTER>(acc[te][ti][0], acc[te][ti][1], inv, bv[te][0], bv[te][1]);
             const uint32_t x1 = finish2<C_DT, BIAS_AFTER>(acc[te][ti][2], acc[te][ti][3], inv, bv[te][2], bv[te][3]);
             const uint32_t y0 = finish2<C_DT, BIAS_AFTER>(acc[to][ti][0], acc[to][ti][1], inv, bv[to][0], bv[to][1]);
@@ -267,30 +276,6 @@ __device__ __forceinline__ void gemm_mid_tile(
             }
         }
     };
-    // fp32 outputs: a lane's 4 columns are 16 bytes already
-    auto store_fp32 = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int tj = 0; tj < TJ; tj++) {
-            const int col = wcol0 + tj * 16 + 4 * lq;
-#pragma unroll
-            for (int ti = 0; ti < 4; ti++) {
-                const int row = m0 + wm * 64 + ti * 16 + lm;
-                if (row >= M || col >= N) continue;
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = finish_fp32<BIAS_AFTER>(acc[tj][ti][e], inv, bv[tj][e]);
-                float* dst = (float*)C + ((int64_t)split * M + row) * ldc + col;
-                if (c_vec_ok && col + 4 <= N) {
-                    store16_any(dst, make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (col + e < N) dst[e] = v[e];
-                }
-            }
-        }
-    };
-
     int cur = 0;  // stage of step s
     // One step: its products, between them the reads of the next step's fragments and the DMAs of the step NSTAGE
     // ahead into the stage whose fragments every wave holds by now.  IN_FLIGHT: steps that may still be in flight once
@@ -303,7 +288,8 @@ __device__ __forceinline__ void gemm_mid_tile(
         // everybody's DMAs of step s+1 have landed and everybody's reads of this step's stage are done
         if constexpr (MODE < 2) mid_wait_barrier<decltype(in_flight)::value * NDMA>();
         if constexpr (MODE == 2) {
-            if constexpr (BIAS_AFTER) load_rounded_bias_tiles<C_DT, TJ>(bv, bias, bias_fp32, wcol0 + 4 * lq, N);
+            if constexpr (c_is_fp32(C_DT)) load_bias_tiles<F8MI_FP32, TJ>(bv, bias, wcol0 + 4 * lq, N);
+            else if constexpr (BIAS_AFTER) load_rounded_bias_tiles<C_DT, TJ>(bv, bias, bias_fp32, wcol0 + 4 * lq, N);
             else load_bias_tiles<C_DT, TJ>(bv, bias, wcol0 + 4 * lq, N);
         }
         F8MI_SCHED_FENCE();
@@ -323,7 +309,7 @@ __device__ __forceinline__ void gemm_mid_tile(
                         else if (f < TJ + 4) fa[P ^ 1][f - TJ] = frag_a(st, f - TJ);
                     }
                     F8MI_SCHED_FENCE();
-                } else if (C_DT != F8MI_FP32 && ti >= 1 && (tj & 1)) {  // the finished row of tiles, under this row's products
+                } else if (ti >= 1 && (tj & 1)) {  // the finished row of tiles, under this row's products
                     F8MI_SCHED_FENCE();
                     store_piece(ti - 1, tj >> 1);
                     F8MI_SCHED_FENCE();
@@ -346,13 +332,9 @@ __device__ __forceinline__ void gemm_mid_tile(
     if (steps >= 2) step(c1, c1, c0);
     step(c0, c2, c0);
 
-    if constexpr (C_DT == F8MI_FP32) {
-        store_fp32();
-    } else {
 #pragma unroll
-        for (int tp = 0; tp < TJ / 2; tp++) store_piece(3, tp);
-        if constexpr (ODD_ROWS) store_held(3, TJ / 2 - 1);
-    }
+    for (int tp = 0; tp < TJ / 2; tp++) store_piece(3, tp);
+    if constexpr (ODD_ROWS) store_held(3, TJ / 2 - 1);
 }
 
 template <int AF, int BF, int C_DT, int TJ, bool A_TR, bool B_TR, bool ODD_ROWS>

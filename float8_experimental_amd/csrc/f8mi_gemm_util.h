@@ -55,6 +55,12 @@ __device__ __forceinline__ v8i read_frag_tr(const uint8_t* p) {
 // different slots.
 __device__ __forceinline__ int tr_swizzle(int k) { return (k & 7) | (((k >> 5) & 1) << 3); }
 
+// Types of C: F8MI_BF16, F8MI_FP16, F8MI_FP32, and fp32 that holds the 16-bit result (include/f8mi.h).
+constexpr __host__ __device__ bool c_is_fp32(int c_dtype) { return c_dtype >= F8MI_FP32; }
+constexpr __host__ __device__ int c_rounded_to(int c_dtype) {
+    return c_dtype == F8MI_BF16_IN_FP32 ? F8MI_BF16 : c_dtype == F8MI_FP16_IN_FP32 ? F8MI_FP16 : c_dtype;
+}
+
 template <int C_DT>
 __device__ __forceinline__ float load_bias(const void* bias, int col) {
     if constexpr (C_DT == F8MI_BF16) return bf16_bits_to_float(((const uint16_t*)bias)[col]);
@@ -116,10 +122,34 @@ __device__ __forceinline__ uint32_t finish2(float a, float b, float inv, float b
         return pack2<C_DT>(x + bias_a, y + bias_b);
     }
 }
-template <bool BIAS_AFTER>
-__device__ __forceinline__ float finish_fp32(float a, float inv, float bias) {
-    if constexpr (BIAS_AFTER) return __fadd_rn(__fmaf_rn(a, inv, 0.f), bias);
-    else return a * inv + bias;
+// Four neighbouring columns of an fp32 C.
+template <int C_DT, bool BIAS_AFTER>
+__device__ __forceinline__ uint4 finish4(const float (&a)[4], float inv, const float (&bias)[4]) {
+    constexpr int R = c_rounded_to(C_DT);
+    float v[4];
+    if constexpr (R != F8MI_FP32) {
+        unpack2<R>(pack2<R>(a[0] * inv + bias[0], a[1] * inv + bias[1]), v[0], v[1]);
+        unpack2<R>(pack2<R>(a[2] * inv + bias[2], a[3] * inv + bias[3]), v[2], v[3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = BIAS_AFTER ? __fadd_rn(__fmaf_rn(a[i], inv, 0.f), bias[i]) : a[i] * inv + bias[i];
+    }
+    return make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3]));
+}
+// ... and their store, at dst = C[row][col].  whole: all four lie inside C and it takes 16-byte stores (the same for every lane).
+__device__ __forceinline__ void store_fp32x4(float* dst, uint4 v, bool whole, int c_vec_ok, int row, int col, int M, int N) {
+    if (__builtin_expect(whole, 1)) {
+        store16_any(dst, v);
+    } else if (row < M && col < N) {
+        if (c_vec_ok && col + 4 <= N) {
+            store16_any(dst, v);
+        } else {
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (col + i < N) ((uint32_t*)dst)[i] = w[i];
+        }
+    }
 }
 
 // load_bias_tiles for BIAS_AFTER: a bias of C's type, or an fp32 one rounded to it.
@@ -145,7 +175,7 @@ __device__ __forceinline__ void load_rounded_bias_tiles(float (&bv)[TJ][4], cons
 // 4096 between other kernels 2 us each.
 // Lanes hold 8 neighbouring columns of one row, the quarters lane / 16 = 0, 2, 1, 3 of a wave 32 of them one behind the other; the
 // pieces of 32 columns of one row are stored from left to right.
-inline bool rows_at_odd_addresses(const void* C, int64_t ldc, int c_dtype) { return c_dtype != F8MI_FP32 && ((ldc & 1) || ((uintptr_t)C & 2)); }
+inline bool rows_at_odd_addresses(const void* C, int64_t ldc, int c_dtype) { return !c_is_fp32(c_dtype) && ((ldc & 1) || ((uintptr_t)C & 2)); }
 struct ShiftedRows {
     int shifted;      // 1: this lane's rows (16 apart) need it
     uint32_t sel;     // bytes of {a word, the one before it} that make a stored word

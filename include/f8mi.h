@@ -355,6 +355,11 @@ int f8mi_column_sum(const void* x, int64_t rows, int64_t cols, int64_t ld, int d
                     int64_t workspace_bytes, void* stream);
 int64_t f8mi_column_sum_workspace_bytes(int64_t rows, int64_t cols, int dtype);
 
+/* Types of C beside those of tensors, for f8mi_gemm_job: fp32 that holds the product rounded to the 16-bit type, the bits of such a product
+ * followed by a conversion (the gradient of an fp32 weight under autocast). */
+#define F8MI_BF16_IN_FP32 3
+#define F8MI_FP16_IN_FP32 4
+
 /* One product of a call that computes two: the arguments of f8mi_gemm_kb_ex without a bias and, for operands that are both given as they
  * are, the workspace of f8mi_gemm_nt_kb_ws. */
 typedef struct f8mi_gemm_job {
