@@ -522,9 +522,10 @@ def linear_forward(x: torch.Tensor, weight: torch.Tensor, layouts, need_dx: bool
 
 
 def linear_backward(dy: torch.Tensor, x_saved, w_saved, x_scale, w_scale, k: int, layouts, need_dx: bool, need_dw: bool, delayed_dy,
-                    bias_dtype: Optional[torch.dtype] = None):
+                    bias_dtype: Optional[torch.dtype] = None, fp32_weight: bool = False):
     """Cast and products of the fused Float8Linear's backward as one native call: (grad_input, grad_weight), or None (see
-    ``linear_forward``).  With ``bias_dtype`` also the gradient of the bias, in that type."""
+    ``linear_forward``).  With ``bias_dtype`` also the gradient of the bias, in that type.  The gradient of an fp32 weight may
+    come in fp32, with the values that dy's type holds: what a conversion behind the product makes of it."""
     if not dy.is_cuda:
         return None
     idx = torch._C._cuda_getDevice()
@@ -532,7 +533,7 @@ def linear_backward(dy: torch.Tensor, x_saved, w_saved, x_scale, w_scale, k: int
     one_copy, _, kb_dx, kb_dw = layouts
     return ext().linear_backward(dy, x_saved, w_saved, x_scale, w_scale, k, one_copy, kb_dx, kb_dw, need_dx, need_dw, delayed_dy,
                                  None if ws is None else ws.data_ptr(), idx, torch._C._cuda_getCurrentRawStream(idx),
-                                 None if bias_dtype is None else _DT[bias_dtype])
+                                 None if bias_dtype is None else _DT[bias_dtype], fp32_weight)
 
 
 def inference_linear(x: torch.Tensor, weight: torch.Tensor, n: int, layout: int, weight_scale: torch.Tensor,

@@ -551,13 +551,54 @@ extern "C" int f8mi_gemm_ex(const void* a, int a_fmt, int a_transposed, int64_t 
 // What one of them needs of the kernels that take two, checked like f8mi_gemm_kb_ex; false: one by one.
 static bool pair_side(const f8mi_gemm_job& j, GemmSide* s) {
     if (j.m <= 0 || j.n <= 0 || j.k < 384 || j.k % 128 != 0 || j.m > 0x7fffffff || j.n > 0x7fffffff || j.k * 64 * 4 > 0x7fffffffLL || j.ldc < j.n) return false;
-    if (j.a_fmt != F8MI_E5M2 || j.b_fmt != F8MI_E4M3FN || j.c_dtype < 0 || j.c_dtype > 2) return false;
+    if (j.a_fmt != F8MI_E5M2 || j.b_fmt != F8MI_E4M3FN || j.c_dtype < 0 || j.c_dtype > F8MI_FP16_IN_FP32) return false;
     if (!j.a || !j.bt || !j.c || !j.scale_a_dev || !j.scale_b_dev || (uintptr_t)j.a % 16 != 0 || (uintptr_t)j.bt % 16 != 0) return false;
     if ((j.a_transposed && (!j.b_transposed || j.m % 64 != 0)) || (j.b_transposed && j.n % 64 != 0)) return false;
-    const int c_vec_ok = (uintptr_t)j.c % (j.c_dtype == F8MI_FP32 ? 4 : 2) == 0;
+    const int c_vec_ok = (uintptr_t)j.c % (c_is_fp32(j.c_dtype) ? 4 : 2) == 0;
     *s = {(const uint8_t*)j.a, 64, j.a_transposed ? j.k * 64 : j.m * 64, (const uint8_t*)j.bt, 64, j.b_transposed ? j.k * 64 : j.n * 64, (int)j.m, (int)j.n, (int)j.k,
           j.scale_a_dev, j.scale_b_dev, j.c, j.ldc, 0, 0, c_vec_ok};
     return true;
+}
+
+// A kernel by itself for a job: rows_large rows on tiles of 256 x cols_large, the rest on tiles of 128 x cols_mid.  False: other kernels, whose
+// sums are in another order or that are none of these.
+struct TileChoice { int64_t rows_large; int cols_large, cols_mid; };
+static bool tile_choice(const f8mi_gemm_job& j, TileChoice* t) {
+    const int64_t tiles_m = (j.m + BM - 1) / BM, tiles_n = (j.n + BN - 1) / BN;
+    GemmPlan p{F8MI_PLAN_TILES256, 0, use_mid_tiles(j.m, j.n, j.k), {0, 0}};
+    if (j.b_transposed) {  // as in launch_transposed
+        if (p.mid) p.kind = F8MI_PLAN_TILES128;
+        else p.split = split_last_round(tiles_m, tiles_n, j.k);
+        if (p.split.rows_large) { p.kind = F8MI_PLAN_TILES256_AND_128; p.mid = p.split.mid; }
+    } else {
+        const bool ws_ok = j.workspace && (uintptr_t)j.workspace % 16 == 0;
+        p = gemm_plan(j.m, j.n, j.k, true, ws_ok ? j.workspace_bytes : 0, rows_at_odd_addresses(j.c, j.ldc, j.c_dtype));
+    }
+    const int cols_mid = p.mid == 2 ? 256 : 128;
+    switch (p.kind) {
+        case F8MI_PLAN_TILES128: *t = {0, 0, cols_mid}; return true;
+        case F8MI_PLAN_TILES256: *t = {j.m, BN, 0}; return true;
+        case F8MI_PLAN_TILES256X224: *t = {j.m, NARROW_N, 0}; return true;
+        case F8MI_PLAN_TILES256_AND_128: *t = {p.split.rows_large * BM, BN, cols_mid}; return true;
+        default: return false;
+    }
+}
+
+static bool is_wide(const f8mi_gemm_job& j) { return j.c_dtype > F8MI_FP32; }
+static int gemm_wide_job(const f8mi_gemm_job& j, const GemmSide& s, const TileChoice& t, hipStream_t stream) {
+    const bool tr = j.b_transposed != 0;
+    ProfScope prof(F8MI_K_GEMM, 2.0 * (double)j.m * (double)j.n * (double)j.k, stream);
+    GemmSide part = s;
+    if (t.rows_large > 0) {
+        part.M = (int)t.rows_large;
+        if (int rc = launch_gemm_wide(tr, true, t.cols_large, j.c_dtype, stream, part)) return rc;
+    }
+    if (t.rows_large == j.m) return F8MI_OK;
+    part = s;
+    part.M = (int)(j.m - t.rows_large);
+    part.A += tr ? t.rows_large / 64 * s.a_unit : t.rows_large * s.lda;
+    part.C = (float*)s.C + t.rows_large * s.ldc;
+    return launch_gemm_wide(tr, false, t.cols_mid, j.c_dtype, stream, part);
 }
 
 static int gemm_job(const f8mi_gemm_job& j, void* stream) {
@@ -596,28 +637,17 @@ static double pair_us(const PairTiles& t, const f8mi_gemm_job& a, const f8mi_gem
     return PAIR_LAUNCH_US + end;
 }
 
-// A product by itself, on the kernels that gemm_plan and launch_transposed choose; 0: on kernels whose sums are in another order or that
-// are none of these.
+// A product by itself; 0: on kernels that one launch of two does not have.
 static double single_us(const f8mi_gemm_job& j) {
-    const double rounds_us = tile_us(PAIR_TILES[3], j.k, false);
-    const auto rounds = [](int64_t tiles) { return (double)((tiles + PAIR_WORKGROUPS - 1) / PAIR_WORKGROUPS); };
-    const int64_t tiles_m = (j.m + BM - 1) / BM, tiles_n = (j.n + BN - 1) / BN;
-    GemmPlan p{F8MI_PLAN_TILES256, 0, use_mid_tiles(j.m, j.n, j.k), {0, 0}};
-    if (j.b_transposed) {
-        if (p.mid) p.kind = F8MI_PLAN_TILES128;
-        else p.split = split_last_round(tiles_m, tiles_n, j.k);
-        if (p.split.rows_large) { p.kind = F8MI_PLAN_TILES256_AND_128; p.mid = p.split.mid; }
-    } else {
-        const bool ws_ok = j.workspace && (uintptr_t)j.workspace % 16 == 0;
-        p = gemm_plan(j.m, j.n, j.k, true, ws_ok ? j.workspace_bytes : 0, rows_at_odd_addresses(j.c, j.ldc, j.c_dtype));
+    TileChoice t;
+    if (!tile_choice(j, &t)) return 0.0;
+    double us = 0.0;
+    if (t.rows_large > 0) {
+        const int64_t tiles = (t.rows_large + BM - 1) / BM * ((j.n + t.cols_large - 1) / t.cols_large), rounds = (tiles + PAIR_WORKGROUPS - 1) / PAIR_WORKGROUPS;
+        us += PAIR_LAUNCH_US + (t.cols_large == BN ? 1.0 : 0.9) * (double)rounds * tile_us(PAIR_TILES[F8MI_PAIR_TILES256], j.k, false);
     }
-    switch (p.kind) {
-        case F8MI_PLAN_TILES128: return PAIR_LAUNCH_US + tile_us(PAIR_TILES[p.mid], j.k, false);
-        case F8MI_PLAN_TILES256: return PAIR_LAUNCH_US + rounds_us * rounds(tiles_m * tiles_n);
-        case F8MI_PLAN_TILES256X224: return PAIR_LAUNCH_US + 0.9 * rounds_us * rounds(tiles_m * ((j.n + NARROW_N - 1) / NARROW_N));
-        case F8MI_PLAN_TILES256_AND_128: return 2.0 * PAIR_LAUNCH_US + rounds_us * rounds(p.split.rows_large * tiles_n) + tile_us(PAIR_TILES[p.mid], j.k, false);
-        default: return 0.0;
-    }
+    if (t.rows_large < j.m) us += PAIR_LAUNCH_US + tile_us(PAIR_TILES[t.cols_mid == 256 ? F8MI_PAIR_TILES128X256 : F8MI_PAIR_TILES128], j.k, false);
+    return us;
 }
 
 // The tiles of one launch, or F8MI_PAIR_BY_SIZE for two launches.  Many rounds of 256 x 256 tiles leave nothing to gain, and small tiles
@@ -641,16 +671,15 @@ extern "C" int f8mi_gemm_pair(const f8mi_gemm_job* a, const f8mi_gemm_job* b, in
     if (!a || !b) { set_error("f8mi_gemm_pair: null pointer"); return F8MI_ERR_INVALID_ARG; }
     if (tiles < F8MI_PAIR_BY_SIZE || tiles > F8MI_PAIR_TILES256) { set_error("f8mi_gemm_pair: unknown tiles %d", tiles); return F8MI_ERR_INVALID_ARG; }
     GemmPair pair;
-    const bool tr = a->b_transposed != 0;
-    bool ok = pair_side(*a, &pair.s[0]) && pair_side(*b, &pair.s[1]) && a->c_dtype == b->c_dtype && !a->a_transposed && (a->b_transposed != 0) == (b->b_transposed != 0) &&
-              (b->a_transposed != 0) == tr;
+    const bool tr = a->b_transposed != 0, side_a = pair_side(*a, &pair.s[0]), side_b = pair_side(*b, &pair.s[1]);
+    const int type_b = is_wide(*b) ? c_rounded_to(b->c_dtype) : b->c_dtype;
+    bool ok = side_a && side_b && a->c_dtype == type_b && !a->a_transposed && (b->b_transposed != 0) == tr && (b->a_transposed != 0) == tr;
     int kind = tiles;
     bool odd_rows = false;
     if (ok) {
         const bool odd[2] = {rows_at_odd_addresses(a->c, a->ldc, a->c_dtype), rows_at_odd_addresses(b->c, b->ldc, b->c_dtype)};
-        odd_rows = odd[0] && odd[1] && pair.s[0].c_vec_ok && pair.s[1].c_vec_ok;
-        if (!tr && odd[0] != odd[1]) ok = false;
-        if (tr) odd_rows = false;
+        odd_rows = !tr && odd[0] && pair.s[0].c_vec_ok && pair.s[1].c_vec_ok;
+        if (!tr && odd[0] != odd[1] && !is_wide(*b)) ok = false;
         if (kind == F8MI_PAIR_BY_SIZE) kind = pair_tiles(*a, *b);
     }
     if (ok && kind != F8MI_PAIR_BY_SIZE) {
@@ -667,12 +696,17 @@ extern "C" int f8mi_gemm_pair(const f8mi_gemm_job* a, const f8mi_gemm_job* b, in
     if (ok && kind != F8MI_PAIR_BY_SIZE) {
         ProfScope prof(F8MI_K_GEMM, 2.0 * ((double)a->m * (double)a->n * (double)a->k + (double)b->m * (double)b->n * (double)b->k), (hipStream_t)stream);
         const bool second_first = b->k > a->k;  // the longer ones first: the last round is then of short ones
-        if (kind == F8MI_PAIR_TILES256) return launch_gemm_pair_large(tr, odd_rows, a->c_dtype, (hipStream_t)stream, pair, second_first);
-        return launch_gemm_pair_mid(tr, odd_rows, kind == F8MI_PAIR_TILES128X256, a->c_dtype, (hipStream_t)stream, pair, second_first);
+        if (kind == F8MI_PAIR_TILES256) return launch_gemm_pair_large(tr, odd_rows, is_wide(*b), a->c_dtype, (hipStream_t)stream, pair, second_first);
+        return launch_gemm_pair_mid(tr, odd_rows, is_wide(*b), kind == F8MI_PAIR_TILES128X256 ? 256 : 128, a->c_dtype, (hipStream_t)stream, pair, second_first);
     }
     if (tiles != F8MI_PAIR_BY_SIZE) { set_error("f8mi_gemm_pair: not built for these two products"); return F8MI_ERR_UNSUPPORTED; }
+    TileChoice choice{};
+    if (is_wide(*a) || (is_wide(*b) && (!side_b || (b->a_transposed != 0) != (b->b_transposed != 0) || !tile_choice(*b, &choice)))) {
+        set_error("f8mi_gemm_pair: a 16-bit result in fp32 is built for the second product, e5m2 times e4m3 on tile kernels");
+        return F8MI_ERR_UNSUPPORTED;
+    }
     if (int rc = gemm_job(*a, stream)) return rc;
-    return gemm_job(*b, stream);
+    return is_wide(*b) ? gemm_wide_job(*b, pair.s[1], choice, (hipStream_t)stream) : gemm_job(*b, stream);
 }
 
 // ---- a product whose bias is added to the rounded result

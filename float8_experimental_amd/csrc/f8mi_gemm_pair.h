@@ -33,9 +33,14 @@ struct GemmPair {
     GemmSide s[2];
 };
 // A e5m2, Bt e4m3 on both sides.  transposed: s[0] reads its Bt transposed, s[1] both its operands; else both sides read them as they are.
-// second_first: the workgroups of s[1] come first.  odd_rows: rows of C at odd multiples of two bytes (not with transposed).
-int launch_gemm_pair_large(bool transposed, bool odd_rows, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
-int launch_gemm_pair_large_tr(int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
-int launch_gemm_pair_mid(bool transposed, bool odd_rows, bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+// second_first: the workgroups of s[1] come first.
+// odd_rows: rows of C at odd multiples of two bytes (not with transposed; of s[0] only where s[1] is wide).
+// wide: C of s[1] is fp32 that holds values of c_dtype (bf16, fp16).
+int launch_gemm_pair_large(bool transposed, bool odd_rows, bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+int launch_gemm_pair_large_tr(bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+int launch_gemm_pair_mid(bool transposed, bool odd_rows, bool wide, int cols, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+// One product with such a C (f8mi_gemm_wide.hip): e5m2 times e4m3, both operands as they are or both transposed; large: tiles of 256 x cols
+// (256, or, operands as they are, 224), else 128 x cols (128, 256).
+int launch_gemm_wide(bool transposed, bool large, int cols, int c_dtype, hipStream_t stream, const GemmSide& s);
 
 }  // namespace f8mi

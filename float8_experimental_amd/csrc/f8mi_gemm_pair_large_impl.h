@@ -15,21 +15,22 @@ __device__ __forceinline__ void gemm_pair_large_side(int id, const GemmSide& s) 
                                                                     nullptr, s.tiles_m, s.tiles_n, s.c_vec_ok);
 }
 
-template <int C_DT, bool TR, bool ODD_ROWS>
+// C_Q: the type of the second product's C.
+template <int C_DT, int C_Q, bool TR, bool ODD_ROWS>
 __global__ __launch_bounds__(GEMM_THREADS) void gemm_pair_large_kernel(const GemmPair pair, int second_first) {
     const int bid = blockIdx.x, first = workgroups(pair.s[second_first]);
     const int which = (bid >= first) ^ second_first;
     const int id = bid >= first ? bid - first : bid;
     const GemmSide s = pair.s[which];
-    if constexpr (!TR) gemm_pair_large_side<C_DT, false, false, ODD_ROWS>(id, s);
-    else if (which) gemm_pair_large_side<C_DT, true, true, ODD_ROWS>(id, s);
-    else gemm_pair_large_side<C_DT, false, true, ODD_ROWS>(id, s);
+    if constexpr (!TR && C_DT == C_Q) gemm_pair_large_side<C_DT, false, false, ODD_ROWS>(id, s);
+    else if (which) gemm_pair_large_side<C_Q, TR, TR, ODD_ROWS && !c_is_fp32(C_Q)>(id, s);
+    else gemm_pair_large_side<C_DT, false, TR, ODD_ROWS>(id, s);
 }
 
-template <int C_DT, bool TR, bool ODD_ROWS>
+template <int C_DT, int C_Q, bool TR, bool ODD_ROWS>
 static int launch_pair_large(hipStream_t stream, const GemmPair& pair, bool second_first) {
     static std::atomic<uint64_t> lds_allowed{0};
-    auto kern = gemm_pair_large_kernel<C_DT, TR, ODD_ROWS>;
+    auto kern = gemm_pair_large_kernel<C_DT, C_Q, TR, ODD_ROWS>;
     if (int rc = allow_big_lds(kern, LargeCfg<8>::LDS, lds_allowed)) return rc;
     hipLaunchKernelGGL(kern, dim3((unsigned)(workgroups(pair.s[0]) + workgroups(pair.s[1]))), dim3(GEMM_THREADS), LargeCfg<8>::LDS, stream, pair, (int)second_first);
     return check_hip(hipGetLastError(), "gemm (two products, 256 x 256 tiles) kernel launch");

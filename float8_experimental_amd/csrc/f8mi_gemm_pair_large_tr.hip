@@ -3,10 +3,14 @@
 
 namespace f8mi {
 
-int launch_gemm_pair_large_tr(int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first) {
-    if (c_dtype == F8MI_FP32) return launch_pair_large<F8MI_FP32, true, false>(stream, pair, second_first);
-    if (c_dtype == F8MI_FP16) return launch_pair_large<F8MI_FP16, true, false>(stream, pair, second_first);
-    return launch_pair_large<F8MI_BF16, true, false>(stream, pair, second_first);
+int launch_gemm_pair_large_tr(bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first) {
+    if (c_dtype == F8MI_FP32) return launch_pair_large<F8MI_FP32, F8MI_FP32, true, false>(stream, pair, second_first);
+    if (c_dtype == F8MI_FP16) {
+        if (wide) return launch_pair_large<F8MI_FP16, F8MI_FP16_IN_FP32, true, false>(stream, pair, second_first);
+        return launch_pair_large<F8MI_FP16, F8MI_FP16, true, false>(stream, pair, second_first);
+    }
+    if (wide) return launch_pair_large<F8MI_BF16, F8MI_BF16_IN_FP32, true, false>(stream, pair, second_first);
+    return launch_pair_large<F8MI_BF16, F8MI_BF16, true, false>(stream, pair, second_first);
 }
 
 }  // namespace f8mi

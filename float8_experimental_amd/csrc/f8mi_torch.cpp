@@ -238,7 +238,8 @@ struct Call {
         int64_t m, n, kc;
         at::Tensor& c;
     };
-    void gemm_two(const Product& p, const Product& q, at::ScalarType out) const {
+    // wide: the second result in fp32, rounded to `out` as the first
+    void gemm_two(const Product& p, const Product& q, at::ScalarType out, bool wide) const {
         f8mi_gemm_job jobs[2];
         at::Tensor ws[2];
         int i = 0;
@@ -246,12 +247,15 @@ struct Call {
             const int64_t k = padded(g->kc, g->layout);
             int64_t bytes = 0;
             if (!g->b_tr) ws[i] = split_workspace(g->m, g->n, k, g->layout, bytes);
-            g->c = make({g->m, g->n}, out);
+            const bool fp32 = wide && g == &q;
+            g->c = make({g->m, g->n}, fp32 ? at::kFloat : out);
             jobs[i] = {g->a.data_ptr(), g->bt.data_ptr(), fp8_code(g->a.scalar_type()), fp8_code(g->bt.scalar_type()), g->a_tr, g->b_tr, g->m, g->n, k,
-                       (const float*)g->sa.data_ptr(), (const float*)g->sb.data_ptr(), g->c.data_ptr(), g->n, dtype_code(out), bytes ? ws[i].data_ptr() : nullptr, bytes};
+                       (const float*)g->sa.data_ptr(), (const float*)g->sb.data_ptr(), g->c.data_ptr(), g->n, !fp32 ? dtype_code(out) : out == at::kHalf ? F8MI_FP16_IN_FP32 : F8MI_BF16_IN_FP32, bytes ? ws[i].data_ptr() : nullptr, bytes};
             i++;
         }
-        check(L.gemm_pair(&jobs[0], &jobs[1], F8MI_PAIR_BY_SIZE, stream), "f8mi_gemm_pair");
+        const int rc = L.gemm_pair(&jobs[0], &jobs[1], F8MI_PAIR_BY_SIZE, stream);
+        if (wide && rc == F8MI_ERR_UNSUPPORTED) return gemm_two(p, q, out, false);  // the caller converts it
+        check(rc, "f8mi_gemm_pair");
     }
 };
 
@@ -319,10 +323,11 @@ PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 }
 
 // linear_backward(dy [m, n], saved of x, saved of weight, scale of x, scale of weight, k, one_copy, kb_dx, kb_dw, need_dx, need_dw,
-//                 delayed_dy, delayed_workspace, device, stream, type of the bias = None) -> (grad of x [m, k], grad of weight [n, k]
-//                 and, with such a type, grad of the bias [n]) or None
+//                 delayed_dy, delayed_workspace, device, stream, type of the bias = None, fp32 weight = False) -> (grad of x [m, k], grad of
+//                 weight [n, k] and, with such a type, grad of the bias [n]) or None.  The gradient of an fp32 weight comes in fp32 where a
+//                 kernel stores it so, with the values of dy's type; else in that type.
 PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
-    if (!expect(n_args, 15, "linear_backward", 1)) return nullptr;
+    if (!expect(n_args, 15, "linear_backward", 2)) return nullptr;
     return guarded([&]() -> PyObject* {
         const Call c{as_ptr(a[14]), as_int(a[13]), as_ptr(a[12])};
         const at::Tensor dy = matrix(a[0], c.device);
@@ -344,6 +349,7 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             if (fp8_code(t->scalar_type()) < 0 || !t->is_contiguous() || t->sizes() != copy_sizes(rows, kc, layout)) Py_RETURN_NONE;
         }
         const bool need_db = n_args > 15 && a[15] != Py_None;
+        const bool wide = n_args > 16 && as_int(a[16]) && dy.scalar_type() != at::kFloat;
         const int bias_dt = need_db ? as_int(a[15]) : F8MI_FP32;
         const at::ScalarType bias_type = bias_dt == F8MI_BF16 ? at::kBFloat16 : bias_dt == F8MI_FP16 ? at::kHalf : at::kFloat;
         at::Tensor g8, g8t, sg, dx, dw, db;
@@ -352,7 +358,7 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             if (one_copy) {
                 c.cast(dy, go, F8MI_E5M2, true, F8MI_LAYOUT_KBLOCK64, false, 0, g8, g8t, sg);
                 if (need_dx && need_dw && L.gemm_pair) {
-                    c.gemm_two({g8, sg, ws, sw, false, true, F8MI_LAYOUT_KBLOCK64, m, k, n, dx}, {g8, sg, xs, sx, true, true, F8MI_LAYOUT_KBLOCK64, n, k, m, dw}, dy.scalar_type());
+                    c.gemm_two({g8, sg, ws, sw, false, true, F8MI_LAYOUT_KBLOCK64, m, k, n, dx}, {g8, sg, xs, sx, true, true, F8MI_LAYOUT_KBLOCK64, n, k, m, dw}, dy.scalar_type(), wide);
                     return;
                 }
                 if (need_dx) dx = c.gemm_tr(g8, false, sg, ws, sw, m, k, n, dy.scalar_type());
@@ -360,7 +366,7 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             } else {
                 c.cast(dy, go, F8MI_E5M2, need_dx, kb_dx, need_dw, kb_dw, g8, g8t, sg);
                 if (need_dx && need_dw && kb_dx != F8MI_LAYOUT_ROWMAJOR && kb_dw != F8MI_LAYOUT_ROWMAJOR && L.gemm_pair) {
-                    c.gemm_two({g8, sg, ws, sw, false, false, kb_dx, m, k, n, dx}, {g8t, sg, xs, sx, false, false, kb_dw, n, k, m, dw}, dy.scalar_type());
+                    c.gemm_two({g8, sg, ws, sw, false, false, kb_dx, m, k, n, dx}, {g8t, sg, xs, sx, false, false, kb_dw, n, k, m, dw}, dy.scalar_type(), wide);
                     return;
                 }
                 if (need_dx) dx = c.gemm(g8, sg, ws, sw, kb_dx, m, k, n, dy.scalar_type());

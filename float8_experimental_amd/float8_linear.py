@@ -131,6 +131,7 @@ class _float8_linear_fn(torch.autograd.Function):
         ctx.is_amax_initialized = is_amax_initialized
         ctx.x_shape = x.shape
         ctx.layouts = None
+        ctx.fp32_weight = weight.dtype is torch.float32
         ctx.bias_dtype = None if bias is None else bias.dtype
         if not emulate and not emulate_bw and (is_amax_initialized or not mod.has_any_delayed_scaling):
             layouts = _native.linear_layouts(m, k, n)
@@ -182,7 +183,7 @@ class _float8_linear_fn(torch.autograd.Function):
         saved = ctx.saved_tensors  # once: non-reentrant checkpointing refuses to unpack a tensor a second time
         if ctx.layouts is not None:
             done = _native.linear_backward(dy2, *saved, ctx.x_shape[-1], ctx.layouts, need_dx, need_dw,
-                                           mod._delayed_pair("grad_output"), ctx.bias_dtype if need_db else None)
+                                           mod._delayed_pair("grad_output"), ctx.bias_dtype if need_db else None, ctx.fp32_weight)
             if done is not None:
                 dx, dw, *native_db = done
                 return (dx if dx is None or len(ctx.x_shape) == 2 else dx.reshape(ctx.x_shape), dw, None, None,

@@ -355,7 +355,7 @@ int f8mi_column_sum(const void* x, int64_t rows, int64_t cols, int64_t ld, int d
                     int64_t workspace_bytes, void* stream);
 int64_t f8mi_column_sum_workspace_bytes(int64_t rows, int64_t cols, int dtype);
 
-/* Types of C beside those of tensors, for f8mi_gemm_job: fp32 that holds the product rounded to the 16-bit type, the bits of such a product
+/* Types of C beside those of tensors, for the second product of f8mi_gemm_pair beside a first one of the 16-bit type: fp32 that holds the product rounded to the 16-bit type, the bits of such a product
  * followed by a conversion (the gradient of an fp32 weight under autocast). */
 #define F8MI_BF16_IN_FP32 3
 #define F8MI_FP16_IN_FP32 4
@@ -377,7 +377,8 @@ typedef struct f8mi_gemm_job {
 /* Two independent products, as the backward of a linear has them (a: grad_input, b: grad_weight): in one launch where that pays,
  * else one after the other; the same bits.  One launch takes e5m2 times e4m3 with k % 128 == 0 and k >= 384, both pairs of operands as
  * they are, or a with bt transposed and b with both.  tiles: F8MI_PAIR_BY_SIZE, or (for tests and measurements) the tiles of one
- * launch, F8MI_ERR_UNSUPPORTED with nothing queued where it does not take them. */
+ * launch, F8MI_ERR_UNSUPPORTED with nothing queued where it does not take them.  The same for a 16-bit result in fp32 that runs on other
+ * kernels than tiles. */
 #define F8MI_PAIR_BY_SIZE 0
 #define F8MI_PAIR_TILES128 1
 #define F8MI_PAIR_TILES128X256 2

@@ -1083,6 +1083,46 @@ def test_gemm_pair_equals_the_products_one_by_one(nat, tokens, k, n, out_dt):
         assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), 3, nat._stream(g)) == nat.ERR_UNSUPPORTED
 
 
+# grad_weight's 16-bit result stored in fp32, beside grad_input in one launch on each of the tiles and by itself (a first product that one launch
+# does not take): 128 x 128, 128 x 256, 256 x 256 with and without a sparse last round, 256 x 224; odd and even step counts, odd rows of grad_input.
+@pytest.mark.parametrize("tokens,k,n", [(384, 1024, 512), (512, 4096, 2048), (384, 4096, 4096), (512, 4096, 4352), (384, 14336, 2048), (512, 513, 700),
+                                        (500, 4095, 2100), (390, 14301, 2000)])
+@pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float16])
+def test_gemm_pair_stores_a_16_bit_gradient_in_fp32(nat, tokens, k, n, out_dt):
+    g = _rand_fp8((tokens, n), torch.float8_e5m2, tokens + n, 4.0).to(DEV)
+    w = _rand_fp8((n, k), torch.float8_e4m3fn, n + k, 4.0).to(DEV)
+    x = _rand_fp8((tokens, k), torch.float8_e4m3fn, tokens + k, 4.0).to(DEV)
+    sg, sw, sx = (torch.tensor(s, device=DEV) for s in (2.0, 0.25, 0.5))
+    turned = lambda t: t.view(torch.uint8).t().contiguous().view(t.dtype)
+    pad = lambda v: -(-v // 128) * 128
+    forms = [(0, [_to_kb_padded(t)[0] for t in (g, turned(w), turned(g), turned(x))])]
+    if tokens % 128 == 0 and k % 128 == 0 and n % 128 == 0:
+        forms.append((1, [_to_kb(g), _to_kb(w), _to_kb(g), _to_kb(x)]))
+    for tr, (a0, b0, a1, b1) in forms:
+        if tr:
+            want = [nat.gemm_kb_ex(a0, False, sg, b0, True, sw, out_dt), nat.gemm_kb_ex(a1, True, sg, b1, True, sx, out_dt)]
+        else:
+            want = [nat.gemm_nt_kb(a0, sg, b0, sw, out_dt, split_k=False), nat.gemm_nt_kb(a1, sg, b1, sx, out_dt, split_k=False)]
+        want[1] = want[1].float()
+        jobs, got = (GemmJob * 2)(), [torch.empty_like(t) for t in want]
+        wide = 3 if out_dt is torch.bfloat16 else 4  # F8MI_BF16_IN_FP32, F8MI_FP16_IN_FP32
+        for job, a, b, sb, (rows, cols, kc), c, a_tr, dt in zip(jobs, (a0, a1), (b0, b1), (sw, sx), ((tokens, k, pad(n)), (n, k, pad(tokens))), got, (0, tr),
+                                                                (nat._DT[out_dt], wide)):
+            job.a, job.bt, job.a_fmt, job.b_fmt, job.a_tr, job.b_tr = a.data_ptr(), b.data_ptr(), nat.E5M2, nat.E4M3FN, a_tr, tr
+            job.m, job.n, job.k, job.sa, job.sb, job.c, job.ldc, job.dtype = rows, cols, kc, sg.data_ptr(), sb.data_ptr(), c.data_ptr(), cols, dt
+        for tiles in (0, 1, 2, 3, None):
+            for t in got:
+                t.fill_(float("nan"))
+            if tiles is None:
+                jobs[0].b_fmt = nat.E5M2
+            assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), tiles or 0, nat._stream(g)) == 0, nat.lib().f8mi_last_error()
+            assert (tiles is None or torch.equal(got[0], want[0])) and torch.equal(got[1], want[1]), (tr, tiles)
+        jobs[1].b_fmt = nat.E5M2  # no such kernel: refused, and nothing queued
+        got[0].fill_(0.0)
+        assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), 0, nat._stream(g)) == nat.ERR_UNSUPPORTED
+        assert not got[0].any()
+
+
 # A bias added to the rounded product, on each of the tiles that take it: 128 x 128, 128 x 256, 256 x 256 with and without a sparse last round,
 # 256 x 224, odd and even step counts and rows of C; refused where the product runs on other kernels.
 @pytest.mark.parametrize("m,n,k,plan", [(300, 200, 512, "tiles128"), (257, 511, 384, "tiles128"), (2048, 4000, 640, "tiles128"), (2040, 3999, 384, "tiles128"),

@@ -167,14 +167,13 @@ def test_128_row_tile_kernels_keep_both_fragment_sets_in_registers(listings, uni
     assert sizes and not any(sizes)
 
 
-def test_kernels_of_two_products_or_with_a_bias_keep_to_the_same_rules(tmp_path):
-    """The tile bodies inside kernels that compute two products or add a bias to the rounded one: the distance of every accumulator read, M0
+def test_kernels_of_two_products_with_a_bias_or_a_wide_result_keep_to_the_same_rules(tmp_path):
+    """The tile bodies inside kernels that compute two products, add a bias to the rounded one or store it in fp32: the distance of every accumulator read, M0
     before every LDS-DMA, no scratch.  A body of 256 x 256 tiles reads each of its 256 accumulator registers once (256 x 224: 224): two bodies
-    (parity of the step count) in a pair of products that take their operands as they are, four where one reads one and the other both
-    transposed.  The 128-row bodies are the compiler's own MFMAs."""
-    units = {"f8mi_gemm_pair_large.hip": (5, 0, 2), "f8mi_gemm_pair_large_tr.hip": (3, 0, 4), "f8mi_gemm_pair_mid.hip": (0, 16, 0),
-             "f8mi_gemm_biased.hip": (16, 10, 1)}  # kernels of large tiles, of 128-row tiles, bodies of one of the former
-    with ThreadPoolExecutor(max_workers=4) as ex:
+    (parity of the step count) in a pair of products that take their operands as they are to outputs of one type, four in the other pairs.  The 128-row bodies are the compiler's own MFMAs."""
+    units = {"f8mi_gemm_pair_large.hip": (9, 0, None), "f8mi_gemm_pair_large_tr.hip": (5, 0, 4), "f8mi_gemm_pair_mid.hip": (0, 28, 0),
+             "f8mi_gemm_biased.hip": (16, 10, 1), "f8mi_gemm_wide.hip": (12, 8, 1)}  # kernels of large tiles, of 128-row tiles, bodies of one of the former
+    with ThreadPoolExecutor(max_workers=5) as ex:
         texts = dict(zip(units, ex.map(lambda u: _asm(u, str(tmp_path)), units)))
     for unit, (large, mid, bodies) in units.items():
         lines = texts[unit]
@@ -206,5 +205,7 @@ def test_kernels_of_two_products_or_with_a_bias_keep_to_the_same_rules(tmp_path)
                     at_mfma, at_line = written[int(m.group(1))]
                     nops = sum(int(n) + 1 for n in re.findall(r"s_nop (\d+)", "\n".join(lines[at_line + 1:i])))
                     assert n_mfma - at_mfma >= MIN_MFMAS or nops >= MIN_WAIT_STATES, f"{unit}:{i + 1}"
-            assert n_reads == (224 if "ELi7E" in name else 256) * bodies, (unit, name, n_reads)
+            types = re.search(r"large_kernelILi(\d)ELi(\d)E", name)
+            want = bodies if bodies else 2 if types.group(1) == types.group(2) else 4
+            assert n_reads == (224 if "ELi7E" in name else 256) * want, (unit, name, n_reads)
         assert seen == {True: large, False: mid}
