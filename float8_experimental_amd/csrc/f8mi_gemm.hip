@@ -556,7 +556,7 @@ static bool pair_side(const f8mi_gemm_job& j, GemmSide* s) {
     if ((j.a_transposed && (!j.b_transposed || j.m % 64 != 0)) || (j.b_transposed && j.n % 64 != 0)) return false;
     const int c_vec_ok = (uintptr_t)j.c % (c_is_fp32(j.c_dtype) ? 4 : 2) == 0;
     *s = {(const uint8_t*)j.a, 64, j.a_transposed ? j.k * 64 : j.m * 64, (const uint8_t*)j.bt, 64, j.b_transposed ? j.k * 64 : j.n * 64, (int)j.m, (int)j.n, (int)j.k,
-          j.scale_a_dev, j.scale_b_dev, j.c, j.ldc, 0, 0, c_vec_ok};
+          j.scale_a_dev, j.scale_b_dev, j.c, j.ldc, 0, 0, c_vec_ok, 0};
     return true;
 }
 
@@ -607,23 +607,25 @@ static int gemm_job(const f8mi_gemm_job& j, void* stream) {
     return f8mi_gemm_nt_kb_ws(j.a, j.a_fmt, j.bt, j.b_fmt, j.m, j.n, j.k, j.scale_a_dev, j.scale_b_dev, j.c, j.c_dtype, j.ldc, nullptr, j.workspace, j.workspace_bytes, stream);
 }
 
-// Estimates in us behind the choice between one launch and two, and of its tiles: every tile of a kind takes a constant and a step's
-// time per 128 of k (128 x 256 tiles an eighth more where they do not all run at once: their operands come faster than the L2 gives them), a
-// launch 2.6 us by itself, and 256 workgroups run at a time, those of the longer contraction first.  Fitted to 620 pairs of products of 384 -
-// 16384 tokens and 512 - 28672 features, both kinds of operands, timed in every form: the choice is within 0.5 % of the best one in the mean,
-// 1.195 times as fast as two launches, and slower than those by more than 2 % in four cases (7 % in one: 6144 tokens, 1408 -> 2176).
+// Estimates in us behind the choice between one launch and two, and of the tiles of either product: a tile of a kind takes a constant and a
+// step's time per 128 of k (more where all CUs run them), a launch 2.25 us by itself, and 256 workgroups run at a time, those
+// of the longer tiles first.  Fitted to 425 pairs of products of 384 - 16384 tokens and 512 - 28672 features, both kinds of operands, timed as two
+// launches and in each of the nine pairs of tiles: with the choice they are 1.19 times as fast as two launches (always the best: 1.21; the
+// same tiles on both sides only: 1.15), and slower by more than 2 % in fourteen cases (8 % in the worst: 6656 tokens, 1920 -> 5504).
 struct PairTiles { int rows, cols; double us, step_us, crowded; };
-constexpr PairTiles PAIR_TILES[4] = {{}, {128, 128, 2.2, 0.48, 1.0}, {128, 256, 3.4, 0.64, 1.125}, {256, 256, 5.9, 1.13, 1.0}};
-constexpr double PAIR_LAUNCH_US = 2.6;
+constexpr PairTiles PAIR_TILES[4] = {{}, {128, 128, 2.05, 0.447, 1.13}, {128, 256, 3.48, 0.636, 1.12}, {256, 256, 6.34, 1.06, 1.09}};
+constexpr double PAIR_LAUNCH_US = 2.25;
 constexpr int64_t PAIR_WORKGROUPS = 256;
 static int64_t tiles_of(const PairTiles& t, int64_t m, int64_t n) { return (m + t.rows - 1) / t.rows * ((n + t.cols - 1) / t.cols); }
-static double tile_us(const PairTiles& t, int64_t k, bool crowded) { return t.us + t.step_us * (crowded ? t.crowded : 1.0) * (double)(k / 128); }
+// ... where `tiles` are computed in all
+static double tile_us(const PairTiles& t, int64_t k, int64_t tiles) { return t.us + t.step_us * (tiles >= PAIR_WORKGROUPS ? t.crowded : 1.0) * (double)(k / 128); }
 
-static double pair_us(const PairTiles& t, const f8mi_gemm_job& a, const f8mi_gemm_job& b) {
-    const f8mi_gemm_job &lng = a.k >= b.k ? a : b, &shrt = a.k >= b.k ? b : a;
-    const int64_t n_long = tiles_of(t, lng.m, lng.n), n_short = tiles_of(t, shrt.m, shrt.n);
-    const bool crowded = n_long + n_short > PAIR_WORKGROUPS;
-    const double us_long = tile_us(t, lng.k, crowded), us_short = tile_us(t, shrt.k, crowded);
+static double pair_us(const PairTiles& ta, const f8mi_gemm_job& a, const PairTiles& tb, const f8mi_gemm_job& b, bool* b_first) {
+    const int64_t n_a = tiles_of(ta, a.m, a.n), n_b = tiles_of(tb, b.m, b.n);
+    const double us_a = tile_us(ta, a.k, n_a + n_b), us_b = tile_us(tb, b.k, n_a + n_b);
+    *b_first = us_b > us_a;  // the longer ones first: the last round is then of short ones
+    const int64_t n_long = *b_first ? n_b : n_a, n_short = *b_first ? n_a : n_b;
+    const double us_long = *b_first ? us_b : us_a, us_short = *b_first ? us_a : us_b;
     const int64_t rounds = n_long / PAIR_WORKGROUPS, late = n_long % PAIR_WORKGROUPS;
     // when the workgroups without and with a tile of the long ones' last round are free, and which of them take the short ones
     double early_us = us_long * (double)rounds, late_us = us_long * (double)(rounds + 1), end = late ? late_us : early_us;
@@ -644,9 +646,12 @@ static double single_us(const f8mi_gemm_job& j) {
     double us = 0.0;
     if (t.rows_large > 0) {
         const int64_t tiles = (t.rows_large + BM - 1) / BM * ((j.n + t.cols_large - 1) / t.cols_large), rounds = (tiles + PAIR_WORKGROUPS - 1) / PAIR_WORKGROUPS;
-        us += PAIR_LAUNCH_US + (t.cols_large == BN ? 1.0 : 0.9) * (double)rounds * tile_us(PAIR_TILES[F8MI_PAIR_TILES256], j.k, false);
+        us += PAIR_LAUNCH_US + (t.cols_large == BN ? 1.0 : 0.9) * (double)rounds * tile_us(PAIR_TILES[F8MI_PAIR_TILES256], j.k, tiles);
     }
-    if (t.rows_large < j.m) us += PAIR_LAUNCH_US + tile_us(PAIR_TILES[t.cols_mid == 256 ? F8MI_PAIR_TILES128X256 : F8MI_PAIR_TILES128], j.k, false);
+    if (t.rows_large < j.m) {
+        const PairTiles& mid = PAIR_TILES[t.cols_mid == 256 ? F8MI_PAIR_TILES128X256 : F8MI_PAIR_TILES128];
+        us += PAIR_LAUNCH_US + tile_us(mid, j.k, tiles_of(mid, j.m - t.rows_large, j.n));
+    }
     return us;
 }
 
@@ -658,18 +663,22 @@ static int pair_tiles(const f8mi_gemm_job& a, const f8mi_gemm_job& b) {
     if (us_a == 0.0 || us_b == 0.0) return F8MI_PAIR_BY_SIZE;
     double best_us = 0.96 * (us_a + us_b);  // the estimates are not better than that
     int best = F8MI_PAIR_BY_SIZE;
-    for (int kind = F8MI_PAIR_TILES128; kind <= F8MI_PAIR_TILES256; kind++) {
-        const PairTiles& t = PAIR_TILES[kind];
-        if (kind != F8MI_PAIR_TILES256 && tiles_of(t, a.m, a.n) + tiles_of(t, b.m, b.n) > 4 * PAIR_WORKGROUPS) continue;
-        const double us = pair_us(t, a, b);
-        if (us < best_us) { best_us = us; best = kind; }
+    for (int ka = F8MI_PAIR_TILES128; ka <= F8MI_PAIR_TILES256; ka++) {
+        if (ka != F8MI_PAIR_TILES256 && tiles_of(PAIR_TILES[ka], a.m, a.n) > 4 * PAIR_WORKGROUPS) continue;
+        for (int kb = F8MI_PAIR_TILES128; kb <= F8MI_PAIR_TILES256; kb++) {
+            if (kb != F8MI_PAIR_TILES256 && tiles_of(PAIR_TILES[kb], b.m, b.n) > 4 * PAIR_WORKGROUPS) continue;
+            bool b_first;
+            const double us = pair_us(PAIR_TILES[ka], a, PAIR_TILES[kb], b, &b_first);
+            if (us < best_us) { best_us = us; best = F8MI_PAIR_TILES(ka, kb); }
+        }
     }
     return best;
 }
 
 extern "C" int f8mi_gemm_pair(const f8mi_gemm_job* a, const f8mi_gemm_job* b, int tiles, void* stream) {
     if (!a || !b) { set_error("f8mi_gemm_pair: null pointer"); return F8MI_ERR_INVALID_ARG; }
-    if (tiles < F8MI_PAIR_BY_SIZE || tiles > F8MI_PAIR_TILES256) { set_error("f8mi_gemm_pair: unknown tiles %d", tiles); return F8MI_ERR_INVALID_ARG; }
+    const auto known = [](int kind) { return kind >= F8MI_PAIR_TILES128 && kind <= F8MI_PAIR_TILES256; };
+    if (tiles != F8MI_PAIR_BY_SIZE && (!known(tiles & 3) || !known(tiles >> 2))) { set_error("f8mi_gemm_pair: unknown tiles %d", tiles); return F8MI_ERR_INVALID_ARG; }
     GemmPair pair;
     const bool tr = a->b_transposed != 0, side_a = pair_side(*a, &pair.s[0]), side_b = pair_side(*b, &pair.s[1]);
     const int type_b = is_wide(*b) ? c_rounded_to(b->c_dtype) : b->c_dtype;
@@ -683,10 +692,12 @@ extern "C" int f8mi_gemm_pair(const f8mi_gemm_job* a, const f8mi_gemm_job* b, in
         if (kind == F8MI_PAIR_BY_SIZE) kind = pair_tiles(*a, *b);
     }
     if (ok && kind != F8MI_PAIR_BY_SIZE) {
-        const int rows = kind == F8MI_PAIR_TILES256 ? 256 : 128, cols = kind == F8MI_PAIR_TILES128 ? 128 : 256;
+        pair.s[0].tiles = kind & 3;
+        pair.s[1].tiles = kind >> 2;
         int64_t total = 0;
         for (GemmSide& s : pair.s) {
-            const int64_t tm = ((int64_t)s.M + rows - 1) / rows, tn = ((int64_t)s.N + cols - 1) / cols;
+            const PairTiles& t = PAIR_TILES[s.tiles];
+            const int64_t tm = ((int64_t)s.M + t.rows - 1) / t.rows, tn = ((int64_t)s.N + t.cols - 1) / t.cols;
             total += tm * tn;
             s.tiles_m = (int)tm;
             s.tiles_n = (int)tn;
@@ -695,9 +706,9 @@ extern "C" int f8mi_gemm_pair(const f8mi_gemm_job* a, const f8mi_gemm_job* b, in
     }
     if (ok && kind != F8MI_PAIR_BY_SIZE) {
         ProfScope prof(F8MI_K_GEMM, 2.0 * ((double)a->m * (double)a->n * (double)a->k + (double)b->m * (double)b->n * (double)b->k), (hipStream_t)stream);
-        const bool second_first = b->k > a->k;  // the longer ones first: the last round is then of short ones
-        if (kind == F8MI_PAIR_TILES256) return launch_gemm_pair_large(tr, odd_rows, is_wide(*b), a->c_dtype, (hipStream_t)stream, pair, second_first);
-        return launch_gemm_pair_mid(tr, odd_rows, is_wide(*b), kind == F8MI_PAIR_TILES128X256 ? 256 : 128, a->c_dtype, (hipStream_t)stream, pair, second_first);
+        bool b_first;
+        pair_us(PAIR_TILES[pair.s[0].tiles], *a, PAIR_TILES[pair.s[1].tiles], *b, &b_first);
+        return launch_gemm_pair(tr, odd_rows, is_wide(*b), a->c_dtype, (hipStream_t)stream, pair, b_first);
     }
     if (tiles != F8MI_PAIR_BY_SIZE) { set_error("f8mi_gemm_pair: not built for these two products"); return F8MI_ERR_UNSUPPORTED; }
     TileChoice choice{};

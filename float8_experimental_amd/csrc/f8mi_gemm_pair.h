@@ -5,7 +5,8 @@
 // same work, so a product of few tiles that each take long runs beside one of many that do not.  us, one after the other / together (tokens,
 // in -> out features; tiles): 512, 1024 -> 1024: 12.3 / 7.1 (128 x 128); 384, 2048 -> 5120: 27.3 / 18.0 (128 x 128); 1664, 3328 -> 2560: 40.3 /
 // 31.7 (128 x 256); 2048, 4096 -> 4096: 60.5 / 56.7 (256 x 256); 3584, 2816 -> 11648: 196.7 / 166.9; 2981, 2989 -> 8117: 158 / 125; 4096, 4096
-// -> 4096, one full round each: 101.3 / 99.4; 8192, 4096 -> 14336: 617 / 630, where the rule in f8mi_gemm.hip stays with two.
+// -> 4096, one full round each: 101.3 / 99.4; 8192, 4096 -> 14336: 617 / 630, where the rule in f8mi_gemm.hip stays with two.  Tiles of the
+// first and of the second product, two of one kind / of their own: 7040, 2560 -> 512: 36.4 / 24.6; 512, 6400 -> 15232: 145.6 / 128.8; 1209, 1408 -> 6144: 29.5 / 23.6.
 // The tiles are the ones that a product by itself runs on (f8mi_gemm_dma16_impl.h, f8mi_gemm_mid_impl.h): the same bits.
 #pragma once
 #include "f8mi_gemm_util.h"
@@ -24,6 +25,7 @@ struct GemmSide {
     int64_t ldc;
     int tiles_m, tiles_n;
     int c_vec_ok;
+    int tiles;  // F8MI_PAIR_TILES128, _TILES128X256 or _TILES256
 };
 
 __host__ __device__ inline int workgroups(const GemmSide& s) { return s.tiles_m * s.tiles_n; }
@@ -36,9 +38,10 @@ struct GemmPair {
 // second_first: the workgroups of s[1] come first.
 // odd_rows: rows of C at odd multiples of two bytes (not with transposed; of s[0] only where s[1] is wide).
 // wide: C of s[1] is fp32 that holds values of c_dtype (bf16, fp16).
-int launch_gemm_pair_large(bool transposed, bool odd_rows, bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
-int launch_gemm_pair_large_tr(bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
-int launch_gemm_pair_mid(bool transposed, bool odd_rows, bool wide, int cols, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+int launch_gemm_pair(bool transposed, bool odd_rows, bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+int launch_gemm_pair_tr(bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+int launch_gemm_pair_odd(bool wide, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
+int launch_gemm_pair_wide(bool transposed, int c_dtype, hipStream_t stream, const GemmPair& pair, bool second_first);
 // One product with such a C (f8mi_gemm_wide.hip): e5m2 times e4m3, both operands as they are or both transposed; large: tiles of 256 x cols
 // (256, or, operands as they are, 224), else 128 x cols (128, 256).
 int launch_gemm_wide(bool transposed, bool large, int cols, int c_dtype, hipStream_t stream, const GemmSide& s);

@@ -376,13 +376,14 @@ typedef struct f8mi_gemm_job {
 
 /* Two independent products, as the backward of a linear has them (a: grad_input, b: grad_weight): in one launch where that pays,
  * else one after the other; the same bits.  One launch takes e5m2 times e4m3 with k % 128 == 0 and k >= 384, both pairs of operands as
- * they are, or a with bt transposed and b with both.  tiles: F8MI_PAIR_BY_SIZE, or (for tests and measurements) the tiles of one
- * launch, F8MI_ERR_UNSUPPORTED with nothing queued where it does not take them.  The same for a 16-bit result in fp32 that runs on other
+ * they are, or a with bt transposed and b with both.  tiles: F8MI_PAIR_BY_SIZE, or (for tests and measurements) those of a and of b in one
+ * launch, F8MI_PAIR_TILES(a, b), F8MI_ERR_UNSUPPORTED with nothing queued where it does not take them.  The same for a 16-bit result in fp32 that runs on other
  * kernels than tiles. */
 #define F8MI_PAIR_BY_SIZE 0
 #define F8MI_PAIR_TILES128 1
 #define F8MI_PAIR_TILES128X256 2
 #define F8MI_PAIR_TILES256 3
+#define F8MI_PAIR_TILES(a, b) ((a) | (b) << 2)
 int f8mi_gemm_pair(const f8mi_gemm_job* a, const f8mi_gemm_job* b, int tiles, void* stream);
 
 /* f8mi_gemm_nt on ROW-MAJOR fp8 operands either of which may be given transposed, so that the fp8 transposes

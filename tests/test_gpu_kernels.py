@@ -1074,13 +1074,13 @@ def test_gemm_pair_equals_the_products_one_by_one(nat, tokens, k, n, out_dt):
         for job, a, b, sb, (rows, cols, kc), c, a_tr in zip(jobs, (a0, a1), (b0, b1), (sw, sx), shapes, got, (0, int(tr))):
             job.a, job.bt, job.a_fmt, job.b_fmt, job.a_tr, job.b_tr = a.data_ptr(), b.data_ptr(), nat.E5M2, nat.E4M3FN, a_tr, int(tr)
             job.m, job.n, job.k, job.sa, job.sb, job.c, job.ldc, job.dtype = rows, cols, kc, sg.data_ptr(), sb.data_ptr(), c.data_ptr(), cols, nat._DT[out_dt]
-        for tiles in (0, 1, 2, 3):
+        for tiles in (0, *(p | q << 2 for p in (1, 2, 3) for q in (1, 2, 3))):
             for t in got:
                 t.fill_(float("nan"))
             assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), tiles, nat._stream(g)) == 0, nat.lib().f8mi_last_error()
             assert all(torch.equal(a, b) for a, b in zip(got, want)), (tr, tiles)
         jobs[1].b_fmt = nat.E5M2  # what one launch does not take is two by the rule, and refused by name
-        assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), 3, nat._stream(g)) == nat.ERR_UNSUPPORTED
+        assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), 15, nat._stream(g)) == nat.ERR_UNSUPPORTED
 
 
 # grad_weight's 16-bit result stored in fp32, beside grad_input in one launch on each of the tiles and by itself (a first product that one launch
@@ -1110,7 +1110,7 @@ def test_gemm_pair_stores_a_16_bit_gradient_in_fp32(nat, tokens, k, n, out_dt):
                                                                 (nat._DT[out_dt], wide)):
             job.a, job.bt, job.a_fmt, job.b_fmt, job.a_tr, job.b_tr = a.data_ptr(), b.data_ptr(), nat.E5M2, nat.E4M3FN, a_tr, tr
             job.m, job.n, job.k, job.sa, job.sb, job.c, job.ldc, job.dtype = rows, cols, kc, sg.data_ptr(), sb.data_ptr(), c.data_ptr(), cols, dt
-        for tiles in (0, 1, 2, 3, None):
+        for tiles in (0, *(p | q << 2 for p in (1, 2, 3) for q in (1, 2, 3)), None):
             for t in got:
                 t.fill_(float("nan"))
             if tiles is None:

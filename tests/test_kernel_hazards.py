@@ -168,14 +168,16 @@ def test_128_row_tile_kernels_keep_both_fragment_sets_in_registers(listings, uni
 
 
 def test_kernels_of_two_products_with_a_bias_or_a_wide_result_keep_to_the_same_rules(tmp_path):
-    """The tile bodies inside kernels that compute two products, add a bias to the rounded one or store it in fp32: the distance of every accumulator read, M0
-    before every LDS-DMA, no scratch.  A body of 256 x 256 tiles reads each of its 256 accumulator registers once (256 x 224: 224): two bodies
-    (parity of the step count) in a pair of products that take their operands as they are to outputs of one type, four in the other pairs.  The 128-row bodies are the compiler's own MFMAs."""
-    units = {"f8mi_gemm_pair_large.hip": (9, 0, None), "f8mi_gemm_pair_large_tr.hip": (5, 0, 4), "f8mi_gemm_pair_mid.hip": (0, 28, 0),
-             "f8mi_gemm_biased.hip": (16, 10, 1), "f8mi_gemm_wide.hip": (12, 8, 1)}  # kernels of large tiles, of 128-row tiles, bodies of one of the former
-    with ThreadPoolExecutor(max_workers=5) as ex:
+    """The tile bodies inside kernels that compute two products, add a bias to the rounded one or store it in fp32: the distance of every
+    accumulator read, M0 before every LDS-DMA, no scratch.  A body of 256 x 256 tiles reads each of its 256 accumulator registers once (256 x
+    224: 224); a kernel of two products has two such bodies (parity of the step count) where one serves both, else four, beside 128-row bodies,
+    whose MFMAs are the compiler's own: only hand-written instructions are looked at, and between those of a body nothing else writes
+    accumulators."""
+    units = {"f8mi_gemm_pair.hip": (3, 0), "f8mi_gemm_pair_tr.hip": (3, 0), "f8mi_gemm_pair_wide.hip": (4, 0), "f8mi_gemm_pair_odd.hip": (4, 0),
+             "f8mi_gemm_biased.hip": (16, 10), "f8mi_gemm_wide.hip": (12, 8)}  # kernels with and without bodies of large tiles
+    with ThreadPoolExecutor(max_workers=6) as ex:
         texts = dict(zip(units, ex.map(lambda u: _asm(u, str(tmp_path)), units)))
-    for unit, (large, mid, bodies) in units.items():
+    for unit, (large, mid) in units.items():
         lines = texts[unit]
         assert not any("scratch_store" in l or "scratch_load" in l for l in lines)
         assert [int(x) for x in re.findall(r"; ScratchSize: (\d+)", "\n".join(lines))] == [0] * (large + mid)
@@ -189,23 +191,31 @@ def test_kernels_of_two_products_with_a_bias_or_a_wide_result_keep_to_the_same_r
                 name, start = m.group(1), end
             if not re.match(r"\.Lfunc_end\d+:", line):
                 continue
-            seen["large" in name] += 1
-            if "large" not in name:
+            has_large = "mid_kernel" not in name
+            seen[has_large] += 1
+            if not has_large:
                 continue
-            written, n_mfma, n_reads = {}, 0, 0
+            want = 224 if "ELi7E" in name else 256
+            written, n_mfma, n_reads, by_hand = {}, 0, 0, False
             for i in range(start, end):
+                by_hand = "#ASMSTART" in lines[i] or (by_hand and "#ASMEND" not in lines[i])
+                if not by_hand:
+                    if written and "v_accvgpr_" in lines[i]:
+                        assert "v_accvgpr_read" in lines[i] or n_reads % want == 0, f"{unit}:{i + 1}: inside a body"
+                    continue
                 m = re.search(r"v_mfma_\S+ a\[(\d+):(\d+)\]", lines[i])
                 if m:
                     n_mfma += 1
                     written.update((r, (n_mfma, i)) for r in range(int(m.group(1)), int(m.group(2)) + 1))
-                assert "v_accvgpr_write" not in lines[i] and "v_accvgpr_mov" not in lines[i]
                 m = re.search(r"v_accvgpr_read_b32 v\d+, a(\d+)", lines[i])
                 if m:
                     n_reads += 1
                     at_mfma, at_line = written[int(m.group(1))]
                     nops = sum(int(n) + 1 for n in re.findall(r"s_nop (\d+)", "\n".join(lines[at_line + 1:i])))
                     assert n_mfma - at_mfma >= MIN_MFMAS or nops >= MIN_WAIT_STATES, f"{unit}:{i + 1}"
-            types = re.search(r"large_kernelILi(\d)ELi(\d)E", name)
-            want = bodies if bodies else 2 if types.group(1) == types.group(2) else 4
-            assert n_reads == (224 if "ELi7E" in name else 256) * want, (unit, name, n_reads)
+                    if n_reads % want == 0:
+                        written = {}
+            types = re.search(r"gemm_pair_kernelILi(\d)ELi(\d)ELb(\d)E", name)
+            bodies = 1 if types is None else 2 if types.group(1) == types.group(2) and types.group(3) == "0" else 4
+            assert n_reads == want * bodies, (unit, name, n_reads)
         assert seen == {True: large, False: mid}
