@@ -240,6 +240,40 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bufs_x=None, bufs_w=None, bufs
     return y.reshape(*x.shape[:-1], weight.shape[0])
 
 
+@torch.library.custom_op("f8mi::column_sum", mutates_args=())
+def column_sum(dy2: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """The gradient of a bias, as the eager layer computes it."""
+    return _native.column_sum(dy2, dtype)
+
+
+@column_sum.register_fake
+def _(dy2, dtype):
+    return torch.empty(dy2.shape[1], dtype=dtype, device=dy2.device)
+
+
+def _column_sum_context(ctx, inputs, output):
+    ctx.dy = inputs[0].shape, inputs[0].dtype
+
+
+column_sum.register_autograd(lambda ctx, g: (g.to(ctx.dy[1]).expand(ctx.dy[0]), None), setup_context=_column_sum_context)
+
+
+class _AddBias(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, y, bias):
+        ctx.bias_dtype = bias.dtype
+        return y + bias.to(y.dtype)
+
+    @staticmethod
+    def backward(ctx, gy):
+        return gy, column_sum(gy.reshape(-1, gy.shape[-1]), ctx.bias_dtype) if ctx.needs_input_grad[1] else None
+
+
+def add_bias(y: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
+    """``y + bias.to(y.dtype)`` whose gradient of the bias has the bits of the eager layer's."""
+    return _AddBias.apply(y, bias)
+
+
 def linear_dynamic(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """``linear`` with all three tensors dynamically scaled."""
     return linear(x, weight)

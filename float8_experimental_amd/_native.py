@@ -536,6 +536,21 @@ def linear_backward(dy: torch.Tensor, x_saved, w_saved, x_scale, w_scale, k: int
                                  None if bias_dtype is None else _DT[bias_dtype], fp32_weight)
 
 
+def column_sum(dy: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """The columns of ``dy`` [m, n] summed, rounded to its type, in ``dtype``: the gradient of a bias.  In the order of
+    f8mi_column_sum, as ``linear_backward`` has it, wherever its kernel reads ``dy`` as it is; else torch's sum."""
+    m, n = dy.shape
+    if not (dy.is_cuda and dy.dtype in _DT and dtype in _DT and m > 0 and n > 0 and dy.stride(1) == 1 and dy.stride(0) >= n):
+        return dy.sum(0).to(dtype)
+    _check_device(dy.device)
+    need = lib().f8mi_column_sum_workspace_bytes(m, n, _DT[dy.dtype])
+    ws = torch.empty(need // 4, dtype=torch.float32, device=dy.device)
+    out = torch.empty(n, dtype=dtype, device=dy.device)
+    rc = lib().f8mi_column_sum(dy.data_ptr(), m, n, dy.stride(0), _DT[dy.dtype], out.data_ptr(), _DT[dtype], ws.data_ptr() if need else None, need, _stream(dy))
+    _check(rc, "f8mi_column_sum")
+    return out
+
+
 def inference_linear(x: torch.Tensor, weight: torch.Tensor, n: int, layout: int, weight_scale: torch.Tensor,
                      static_scale: Optional[torch.Tensor], bias: Optional[torch.Tensor]):
     """Activation cast and product of an inference linear as one native call; None as for ``linear_forward``."""

@@ -175,10 +175,12 @@ class _float8_linear_fn(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1])
         dx = dw = db = None
         need_db = ctx.needs_input_grad[4]
-        if need_db and (torch.is_grad_enabled() or not (need_dx or need_dw)):  # with create_graph: a sum that has a gradient itself
+        if need_db and torch.is_grad_enabled():  # with create_graph: a sum that has a gradient itself
             db = dy2.sum(0).to(ctx.bias_dtype)
             need_db = False
         if not (need_dx or need_dw):
+            if need_db:
+                db = _native.column_sum(dy2, ctx.bias_dtype)
             return None, None, None, None, db
         saved = ctx.saved_tensors  # once: non-reentrant checkpointing refuses to unpack a tensor a second time
         if ctx.layouts is not None:
@@ -189,7 +191,7 @@ class _float8_linear_fn(torch.autograd.Function):
                 return (dx if dx is None or len(ctx.x_shape) == 2 else dx.reshape(ctx.x_shape), dw, None, None,
                         native_db[0] if need_db else db)
         if need_db:
-            db = dy2.sum(0).to(ctx.bias_dtype)
+            db = _native.column_sum(dy2, ctx.bias_dtype)
         dlg = mod._delayed_buffers("grad_output")
         if ctx.kb is None:  # one copy per tensor: x8 [K/64, M, 64], w8 [K/64, N, 64], g8 [N/64, M, 64]
             x8, w8, sx, sw = saved
@@ -412,7 +414,7 @@ class Float8Linear(torch.nn.Linear):
 
         output = linear(self._autocast_input(input), self.weight, bufs("input"), bufs("weight"), bufs("grad_output"))
         if self.bias is not None:
-            output = output + self.bias.to(output.dtype)
+            output = self._add_bias(output, self.bias)
         return output
 
     @torch._dynamo.disable
@@ -441,13 +443,21 @@ class Float8Linear(torch.nn.Linear):
         return (type(x) in _PLAIN and type(bias) in _PLAIN and x.is_cuda and bias.is_cuda and bias.shape == self.weight.shape[:1]
                 and bias.dtype in _HP_DTYPES and not self.config.emulate and torch.autograd.forward_ad._current_level < 0)
 
+    def _add_bias(self, output: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
+        """The addition outside the fused function; its gradient in the same order of sums where that function would take it."""
+        if not self._bias_inside(output, bias):
+            return output + bias.to(output.dtype)
+        from ._custom_ops import add_bias
+
+        return add_bias(output, bias)
+
     def _forward_composed_body(self, input):
         input_fp8 = self.cast_input_to_float8(input, self.is_amax_initialized)
         weight_fp8 = self.cast_weight_to_float8(self.weight, self.is_amax_initialized)
         output = manual_float8_matmul.apply(input_fp8, weight_fp8.t())
         output = self.cast_output_to_float8_in_bw(output)
         if self.bias is not None:
-            output = output + self.bias.to(output.dtype)
+            output = self._add_bias(output, self.bias)
         if self.has_any_delayed_scaling:
             self.float8_post_forward()
         return output

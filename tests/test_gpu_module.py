@@ -978,11 +978,12 @@ def test_bias_inside_the_fused_function_equals_the_addition_outside(f8, monkeypa
 
 def test_bias_gradient_with_create_graph_has_a_gradient_itself(f8):
     mod = f8.convert_to_float8_training(torch.nn.Sequential(torch.nn.Linear(512, 512, device=DEV, dtype=torch.bfloat16)))
-    y = mod(torch.randn(64, 512, device=DEV, dtype=torch.bfloat16))
-    dy = torch.randn_like(y).requires_grad_()
-    (db,) = torch.autograd.grad(y, mod[0].bias, dy, create_graph=True)
-    (ddy,) = torch.autograd.grad(db.sum(), dy)
-    assert torch.equal(ddy, torch.ones_like(dy))
+    for forward in (mod, mod[0].forward_composed):
+        y = forward(torch.randn(64, 512, device=DEV, dtype=torch.bfloat16))
+        dy = torch.randn_like(y).requires_grad_()
+        (db,) = torch.autograd.grad(y, mod[0].bias, dy, create_graph=True)
+        (ddy,) = torch.autograd.grad(db.sum(), dy)
+        assert torch.equal(ddy, torch.ones_like(dy))
 
 
 def test_bias_with_a_forward_mode_derivative_is_added_outside(f8):
