@@ -3,8 +3,9 @@
 
 The reference strings the layer together from four autograd functions and a tensor
 subclass (cast x, cast W, matmul, cast dY in backward).  Here the whole layer is ONE
-autograd function around five kernel launches per direction: amax+scale and
-cast per tensor, and one matrix-core GEMM per product.  Where the sizes allow it each
+autograd function around a few kernel launches per direction: amax + scale and cast of
+a tensor (of both of the forward together), the forward's matrix-core GEMM, which adds the
+bias, and the backward's two, in one launch where that pays.  Where the sizes allow it each
 tensor has ONE fp8 copy and the backward GEMMs read it transposed; otherwise the
 transposed fp8 copies are written by the cast kernels while the data is in registers,
 and only those are kept for backward.
@@ -174,7 +175,7 @@ class _float8_linear_fn(torch.autograd.Function):
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         dy2 = dy.reshape(-1, dy.shape[-1])
         dx = dw = db = None
-        need_db = ctx.needs_input_grad[4]
+        need_db = ctx.bias_dtype is not None and ctx.needs_input_grad[4]
         if need_db and torch.is_grad_enabled():  # with create_graph: a sum that has a gradient itself
             db = dy2.sum(0).to(ctx.bias_dtype)
             need_db = False
