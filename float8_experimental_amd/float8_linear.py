@@ -38,6 +38,7 @@ from .float8_utils import e4m3_dtype, e5m2_dtype
 _KINDS = ("input", "weight", "grad_output")
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _HP_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
+_unsafe_view = torch.ops.aten._unsafe_view.default
 
 
 @torch._dynamo.allow_in_graph
@@ -105,6 +106,12 @@ def _gemm(a8, sa, b8, sb, out_dtype, kb: bool):
     return _native.gemm_nt_kb(a8, sa, b8, sb, out_dtype) if kb else _native.gemm_nt(a8, sa, b8, sb, out_dtype)
 
 
+def _output(y: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """The product y [m, n] in the shape of the input x.  Not as a view: autograd refuses to let a caller change a view made inside a
+    function in place (``relu_(layer(x))``, ``y += residual``)."""
+    return y if x.dim() == 2 else _unsafe_view(y, (*x.shape[:-1], y.shape[1]))
+
+
 class _float8_linear_fn(torch.autograd.Function):
     """y = x W^T (+ bias) with every matmul of forward and backward in fp8.  A bias is added to the product rounded to its
     type, and its gradient is the column sum of dY in that type, as ``x @ w.t() + bias`` has them.
@@ -143,7 +150,7 @@ class _float8_linear_fn(torch.autograd.Function):
                 ctx.layouts = layouts
                 ctx.kb = None if layouts[0] else layouts[2:]
                 ctx.save_for_backward(xs if need_dw else None, ws if need_dx else None, sx, sw)
-                return y if x.dim() == 2 else y.reshape(*x.shape[:-1], n)
+                return _output(y, x)
         tn = not emulate and not emulate_bw and _native.tn_ok(m, k, n)
         if tn:
             x8, _, sx = _cast_for_gemm(x2, e4m3_dtype, dl("input"), is_amax_initialized, True, False, True, False)
@@ -167,7 +174,7 @@ class _float8_linear_fn(torch.autograd.Function):
             ctx.save_for_backward(x8t, w8t, sx, sw)
         if bias is not None:
             y = y + bias.to(y.dtype)
-        return y.reshape(*x.shape[:-1], n)
+        return _output(y, x)
 
     @staticmethod
     def backward(ctx, dy):

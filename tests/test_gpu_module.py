@@ -997,3 +997,28 @@ def test_bias_with_a_forward_mode_derivative_is_added_outside(f8):
         mod[0].bias = fwd.make_dual(bias, torch.ones_like(bias))
         y, tangent = fwd.unpack_dual(mod(torch.randn(64, 512, device=DEV, dtype=torch.bfloat16)))
         assert torch.equal(tangent, torch.ones_like(y))
+
+
+@pytest.mark.parametrize("shape", [(512, 1024), (2, 256, 1024), (300, 520), (3, 100, 520)])
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("native", [True, False])
+def test_outputs_may_be_changed_in_place(f8, monkeypatch, shape, bias, native):
+    """``relu_(layer(x))`` and ``y += residual`` behind a layer, as behind nn.Linear: the gradients of the forms that write elsewhere."""
+    from float8_experimental_amd import _native
+
+    if not native:
+        monkeypatch.setattr(_native, "linear_forward", lambda *a: None)
+    torch.manual_seed(0)
+    mod = f8.convert_to_float8_training(torch.nn.Sequential(torch.nn.Linear(shape[-1], 512, bias=bias, device=DEV, dtype=torch.bfloat16)))
+    x0 = torch.randn(shape, device=DEV, dtype=torch.bfloat16)
+    r = torch.randn(*shape[:-1], 512, device=DEV, dtype=torch.bfloat16)
+
+    def step(change):
+        x = x0.clone().requires_grad_()
+        mod.zero_grad()
+        y = change(mod(x))
+        y.backward(r)
+        return [y.detach(), x.grad] + [p.grad for p in mod.parameters()]
+
+    for inplace, other in ((torch.relu_, torch.relu), (lambda y: y.add_(r), lambda y: y + r)):
+        assert all(torch.equal(p, q) for p, q in zip(step(inplace), step(other)))

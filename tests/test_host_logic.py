@@ -403,3 +403,35 @@ def test_layers_with_one_fp8_copy_save_only_what_backward_reads(monkeypatch, nee
         x, w = (torch.empty(r, k, device="cuda", dtype=torch.bfloat16) for r in (m, n))
         _, xs, ws, *_ = torch.ops.f8mi.linear_fwd(x, w, need_dx, need_dw, None, None)
     assert xs.numel() == (m * k if need_dw else 0) and ws.numel() == (n * k if need_dx else 0)
+
+
+@pytest.mark.parametrize("shape", [(4, 6), (2, 2, 6), (6,)])
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("bias", [True, False])
+def test_outputs_may_be_changed_in_place(monkeypatch, shape, native, bias):
+    """``relu_(layer(x))`` and ``y += residual``, as behind nn.Linear, with the gradients of the forms that write elsewhere.  The
+    kernels are stood in for by plain products."""
+    k, n = 6, 8
+    scale = torch.ones(())
+    monkeypatch.setattr(_native, "linear_layouts", lambda *a: (True, 1, 1, 1))
+    monkeypatch.setattr(_native, "linear_forward", lambda x, w, *a: (x @ w.t(), x, w, scale, scale) if native else None)
+    monkeypatch.setattr(_native, "linear_backward", lambda *a: None)
+    monkeypatch.setattr(_native, "tn_ok", lambda *a: True)
+    monkeypatch.setattr(_native, "cast_dynamic", lambda t, *a, **kw: (t, t.t(), scale))
+    monkeypatch.setattr(_native, "gemm_kb_ex", lambda a, at, sa, b, bt, sb, dtype: (a.t() if at else a) @ b)
+    monkeypatch.setattr(_native, "gemm_nt_kb", lambda a, sa, b, sb, dtype: a @ b.t())
+    torch.manual_seed(0)
+    mod = Float8Linear.from_float(nn.Linear(k, n, bias=bias), config=cfg())
+    x0, r = torch.randn(shape), torch.randn(*shape[:-1], n)
+
+    def step(change):
+        x = x0.clone().requires_grad_()
+        mod.zero_grad()
+        y = mod(x)
+        assert not y._is_view()
+        y = change(y)
+        (y * r).sum().backward()
+        return [y.detach(), x.grad] + [p.grad for p in mod.parameters()]
+
+    for inplace, other in ((torch.relu_, torch.relu), (lambda y: y.add_(r), lambda y: y + r)):
+        assert all(torch.equal(p, q) for p, q in zip(step(inplace), step(other)))
