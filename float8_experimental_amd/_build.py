@@ -45,11 +45,11 @@ def build_extension() -> None:
 
     import torch
 
-    root = os.path.dirname(torch.__file__)
+    root, rocm = os.path.dirname(torch.__file__), os.path.dirname(os.path.dirname(HIPCC))
     subprocess.run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include",
-                    "-I" + sysconfig.get_paths()["include"], "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+                    f"-I{rocm}/include", "-I" + sysconfig.get_paths()["include"], "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
                     f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", EXT_SRC, "-o", EXT_LIB, f"-L{root}/lib",
-                    "-ltorch_python", "-ltorch_cpu", "-lc10"], check=True)
+                    "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"], check=True)
 
 
 def build(verbose: bool = True, out: str = LIB, defines=()) -> str:

@@ -522,10 +522,10 @@ def linear_forward(x: torch.Tensor, weight: torch.Tensor, layouts, need_dx: bool
 
 
 def linear_backward(dy: torch.Tensor, x_saved, w_saved, x_scale, w_scale, k: int, layouts, need_dx: bool, need_dw: bool, delayed_dy,
-                    bias_dtype: Optional[torch.dtype] = None, fp32_weight: bool = False):
+                    fp32_weight: bool = False):
     """Cast and products of the fused Float8Linear's backward as one native call: (grad_input, grad_weight), or None (see
-    ``linear_forward``).  With ``bias_dtype`` also the gradient of the bias, in that type.  The gradient of an fp32 weight may
-    come in fp32, with the values that dy's type holds: what a conversion behind the product makes of it."""
+    ``linear_forward``).  The gradient of an fp32 weight may come in fp32, with the values that dy's type holds: what a
+    conversion behind the product makes of it."""
     if not dy.is_cuda:
         return None
     idx = torch._C._cuda_getDevice()
@@ -533,12 +533,18 @@ def linear_backward(dy: torch.Tensor, x_saved, w_saved, x_scale, w_scale, k: int
     one_copy, _, kb_dx, kb_dw = layouts
     return ext().linear_backward(dy, x_saved, w_saved, x_scale, w_scale, k, one_copy, kb_dx, kb_dw, need_dx, need_dw, delayed_dy,
                                  None if ws is None else ws.data_ptr(), idx, torch._C._cuda_getCurrentRawStream(idx),
-                                 None if bias_dtype is None else _DT[bias_dtype], fp32_weight)
+                                 fp32_weight)
+
+
+def add_bias(y: torch.Tensor, bias: torch.Tensor, added: bool) -> torch.Tensor:
+    """``y + bias.to(y.dtype)``, or what y holds where the kernels have added the bias (``added``), with a history: a node of its
+    own, whose gradient of the bias is ``column_sum``."""
+    return ext().add_bias(y, bias, added)
 
 
 def column_sum(dy: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """The columns of ``dy`` [m, n] summed, rounded to its type, in ``dtype``: the gradient of a bias.  In the order of
-    f8mi_column_sum, as ``linear_backward`` has it, wherever its kernel reads ``dy`` as it is; else torch's sum."""
+    f8mi_column_sum, as ``add_bias`` has it, wherever its kernel reads ``dy`` as it is; else torch's sum."""
     m, n = dy.shape
     if not (dy.is_cuda and dy.dtype in _DT and dtype in _DT and m > 0 and n > 0 and dy.stride(1) == 1 and dy.stride(0) >= n):
         return dy.sum(0).to(dtype)

@@ -15,7 +15,11 @@
 #include <dlfcn.h>
 
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/f8mi.h"
@@ -31,7 +35,7 @@ struct Lib {
     decltype(&f8mi_gemm_nt_ws) gemm_nt_ws;
     decltype(&f8mi_gemm_nt_kb_ws) gemm_nt_kb_ws;
     decltype(&f8mi_gemm_kb_ex) gemm_kb_ex;
-    // null in a library without them: two products one by one, a bias and its gradient by torch
+    // null in a library without them: two products one by one, a bias by torch
     decltype(&f8mi_gemm_pair) gemm_pair;
     decltype(&f8mi_gemm_kb_bias) gemm_kb_bias;
     decltype(&f8mi_column_sum) column_sum;
@@ -210,18 +214,6 @@ struct Call {
         return gemm(a, sa, bt, sb, layout, m, n, kc, out).add_(bias.to(out));
     }
 
-    // the gradient of a bias: the columns of dy summed, in dy's type, then in that of the bias
-    at::Tensor column_sum(const at::Tensor& dy, at::ScalarType bias_type) const {
-        if (!L.column_sum || !L.column_sum_workspace_bytes) return dy.sum(0).to(bias_type);
-        const int64_t rows = dy.size(0), cols = dy.size(1);
-        const int dt = dtype_code(dy.scalar_type());
-        const int64_t bytes = L.column_sum_workspace_bytes(rows, cols, dt);
-        const at::Tensor out = make({cols}, bias_type), ws = bytes ? make({bytes / 4}, at::kFloat) : at::Tensor();
-        check(L.column_sum(dy.data_ptr(), rows, cols, dy.stride(0), dt, out.data_ptr(), dtype_code(bias_type), bytes ? ws.data_ptr() : nullptr, bytes, stream),
-              "f8mi_column_sum");
-        return out;
-    }
-
     at::Tensor gemm_tr(const at::Tensor& a, bool a_tr, const at::Tensor& sa, const at::Tensor& bt, const at::Tensor& sb, int64_t m, int64_t n,
                        int64_t k, at::ScalarType out) const {
         at::Tensor c = make({m, n}, out);
@@ -323,11 +315,10 @@ PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 }
 
 // linear_backward(dy [m, n], saved of x, saved of weight, scale of x, scale of weight, k, one_copy, kb_dx, kb_dw, need_dx, need_dw,
-//                 delayed_dy, delayed_workspace, device, stream, type of the bias = None, fp32 weight = False) -> (grad of x [m, k], grad of
-//                 weight [n, k] and, with such a type, grad of the bias [n]) or None.  The gradient of an fp32 weight comes in fp32 where a
-//                 kernel stores it so, with the values of dy's type; else in that type.
+//                 delayed_dy, delayed_workspace, device, stream, fp32 weight = False) -> (grad of x [m, k], grad of weight [n, k]) or None.
+//                 The gradient of an fp32 weight comes in fp32 where a kernel stores it so, with the values of dy's type; else in that type.
 PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
-    if (!expect(n_args, 15, "linear_backward", 2)) return nullptr;
+    if (!expect(n_args, 15, "linear_backward", 1)) return nullptr;
     return guarded([&]() -> PyObject* {
         const Call c{as_ptr(a[14]), as_int(a[13]), as_ptr(a[12])};
         const at::Tensor dy = matrix(a[0], c.device);
@@ -348,13 +339,9 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             const int layout = one_copy ? F8MI_LAYOUT_KBLOCK64 : t == &xs ? kb_dw : kb_dx;
             if (fp8_code(t->scalar_type()) < 0 || !t->is_contiguous() || t->sizes() != copy_sizes(rows, kc, layout)) Py_RETURN_NONE;
         }
-        const bool need_db = n_args > 15 && a[15] != Py_None;
-        const bool wide = n_args > 16 && as_int(a[16]) && dy.scalar_type() != at::kFloat;
-        const int bias_dt = need_db ? as_int(a[15]) : F8MI_FP32;
-        const at::ScalarType bias_type = bias_dt == F8MI_BF16 ? at::kBFloat16 : bias_dt == F8MI_FP16 ? at::kHalf : at::kFloat;
-        at::Tensor g8, g8t, sg, dx, dw, db;
+        const bool wide = n_args > 15 && as_int(a[15]) && dy.scalar_type() != at::kFloat;
+        at::Tensor g8, g8t, sg, dx, dw;
         const auto compute = [&] {
-            if (need_db) db = c.column_sum(dy, bias_type);
             if (one_copy) {
                 c.cast(dy, go, F8MI_E5M2, true, F8MI_LAYOUT_KBLOCK64, false, 0, g8, g8t, sg);
                 if (need_dx && need_dw && L.gemm_pair) {
@@ -377,8 +364,62 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             const WithoutGil no_gil;
             compute();
         }
-        if (need_db) return wrap_all(dx, dw, db);
         return wrap_all(dx, dw);
+    });
+}
+
+// Whether a kernel may take t's memory for its values, and nobody has to see the operators: no subclass, functional transform, dispatch mode
+// or lazy negation.
+bool memory_holds_values(const at::Tensor& t) {
+    using K = c10::DispatchKey;
+    constexpr c10::DispatchKeySet others({K::Python, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Batched, K::Functionalize, K::Negative, K::Conjugate, K::ZeroTensor});
+    return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(others) && !c10::impl::TorchDispatchModeTLS::any_modes_set();
+}
+
+// The gradient of a bias: the columns of dy summed in fp32, rounded to dy's type, in the type of the bias.
+at::Tensor bias_gradient(const at::Tensor& dy, at::ScalarType type) {
+    const at::Tensor d = dy.reshape({-1, dy.size(-1)});
+    if (!L.column_sum || !L.column_sum_workspace_bytes || at::GradMode::is_enabled() || !memory_holds_values(d) || dtype_code(d.scalar_type()) < 0 || d.numel() == 0 || d.stride(1) != 1 || d.stride(0) < d.size(1))
+        return d.sum(0).to(type);  // with create_graph a sum that has a gradient itself
+    const c10::DeviceGuard guard(d.device());
+    const int64_t rows = d.size(0), cols = d.size(1);
+    const int dt = dtype_code(d.scalar_type());
+    const int64_t bytes = L.column_sum_workspace_bytes(rows, cols, dt);
+    const at::Tensor out = at::empty({cols}, d.options().dtype(type)), ws = bytes ? at::empty({bytes / 4}, d.options().dtype(at::kFloat)) : at::Tensor();
+    const int rc = L.column_sum(d.data_ptr(), rows, cols, d.stride(0), dt, out.data_ptr(), dtype_code(type), bytes ? ws.data_ptr() : nullptr, bytes,
+                                c10::hip::getCurrentHIPStream(d.get_device()).stream());
+    TORCH_CHECK(rc == 0, "f8mi_column_sum failed with code ", rc, ": ", L.last_error());
+    return out;
+}
+
+// y + bias as a node of its own behind the product's, as an addition is one: asked for the gradient of the bias alone, autograd leaves the
+// product's node, its saved tensors and the maxima of a delayed dy alone.  added: y holds the sum already, and nobody else has it: its memory
+// is the result, neither a view (which a caller could not change in place) nor marked as changed (which compiled autograd does not take).
+struct AddBias : torch::autograd::Function<AddBias> {
+    static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& y, const at::Tensor& bias, bool added) {
+        ctx->saved_data["type"] = (int64_t)bias.scalar_type();
+        return added ? at::_unsafe_view(y, y.sizes()) : y + bias.to(y.scalar_type());
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, const torch::autograd::variable_list& grads) {
+        at::Tensor db;
+        if (ctx->needs_input_grad(1)) db = bias_gradient(grads[0], (at::ScalarType)ctx->saved_data["type"].toInt());
+        return {grads[0], db, at::Tensor()};
+    }
+};
+
+// add_bias(y, bias, added) -> y + bias with a history.  For a bias of one of the kernels' types.
+PyObject* add_bias(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    if (!expect(n_args, 3, "add_bias")) return nullptr;
+    return guarded([&]() -> PyObject* {
+        if (!THPVariable_Check(a[0]) || !THPVariable_Check(a[1])) return PyErr_Format(PyExc_TypeError, "add_bias takes two tensors");
+        const at::Tensor y = THPVariable_Unpack(a[0]), bias = THPVariable_Unpack(a[1]);
+        const bool added = PyObject_IsTrue(a[2]);
+        at::Tensor out;
+        {
+            const WithoutGil no_gil;
+            out = AddBias::apply(y, bias, added);
+        }
+        return wrap(out);
     });
 }
 
@@ -476,6 +517,7 @@ PyMethodDef methods[] = {
     {"load", load, METH_VARARGS, nullptr},
     {"linear_forward", (PyCFunction)(void (*)(void))linear_forward, METH_FASTCALL, nullptr},
     {"linear_backward", (PyCFunction)(void (*)(void))linear_backward, METH_FASTCALL, nullptr},
+    {"add_bias", (PyCFunction)(void (*)(void))add_bias, METH_FASTCALL, nullptr},
     {"inference_linear", (PyCFunction)(void (*)(void))inference_linear, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

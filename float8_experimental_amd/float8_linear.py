@@ -113,8 +113,8 @@ def _output(y: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
 
 
 class _float8_linear_fn(torch.autograd.Function):
-    """y = x W^T (+ bias) with every matmul of forward and backward in fp8.  A bias is added to the product rounded to its
-    type, and its gradient is the column sum of dY in that type, as ``x @ w.t() + bias`` has them.
+    """y = x W^T with every matmul of forward and backward in fp8.  ``bias`` (in a tuple: it has no gradient here, see
+    ``_native.add_bias``) is added to the product rounded to its type, as ``x @ w.t() + bias`` has it.
 
     Each of the three GEMMs contracts a different dimension (in_features, out_features, tokens).
     When all three are multiples of 128 (and at least 384) each tensor is cast ONCE, k-blocked over
@@ -140,7 +140,7 @@ class _float8_linear_fn(torch.autograd.Function):
         ctx.x_shape = x.shape
         ctx.layouts = None
         ctx.fp32_weight = weight.dtype is torch.float32
-        ctx.bias_dtype = None if bias is None else bias.dtype
+        bias = None if bias is None else bias[0]
         if not emulate and not emulate_bw and (is_amax_initialized or not mod.has_any_delayed_scaling):
             layouts = _native.linear_layouts(m, k, n)
             done = _native.linear_forward(x2, weight, layouts, need_dx, need_dw, mod._delayed_pair("input"), mod._delayed_pair("weight"),
@@ -181,25 +181,14 @@ class _float8_linear_fn(torch.autograd.Function):
         mod = ctx.mod
         need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         dy2 = dy.reshape(-1, dy.shape[-1])
-        dx = dw = db = None
-        need_db = ctx.bias_dtype is not None and ctx.needs_input_grad[4]
-        if need_db and torch.is_grad_enabled():  # with create_graph: a sum that has a gradient itself
-            db = dy2.sum(0).to(ctx.bias_dtype)
-            need_db = False
-        if not (need_dx or need_dw):
-            if need_db:
-                db = _native.column_sum(dy2, ctx.bias_dtype)
-            return None, None, None, None, db
+        dx = dw = None
         saved = ctx.saved_tensors  # once: non-reentrant checkpointing refuses to unpack a tensor a second time
-        if ctx.layouts is not None:
+        if ctx.layouts is not None and (need_dx or need_dw):
             done = _native.linear_backward(dy2, *saved, ctx.x_shape[-1], ctx.layouts, need_dx, need_dw,
-                                           mod._delayed_pair("grad_output"), ctx.bias_dtype if need_db else None, ctx.fp32_weight)
+                                           mod._delayed_pair("grad_output"), ctx.fp32_weight)
             if done is not None:
-                dx, dw, *native_db = done
-                return (dx if dx is None or len(ctx.x_shape) == 2 else dx.reshape(ctx.x_shape), dw, None, None,
-                        native_db[0] if need_db else db)
-        if need_db:
-            db = _native.column_sum(dy2, ctx.bias_dtype)
+                dx, dw = done
+                return dx if dx is None or len(ctx.x_shape) == 2 else dx.reshape(ctx.x_shape), dw, None, None, None
         dlg = mod._delayed_buffers("grad_output")
         if ctx.kb is None:  # one copy per tensor: x8 [K/64, M, 64], w8 [K/64, N, 64], g8 [N/64, M, 64]
             x8, w8, sx, sw = saved
@@ -208,7 +197,7 @@ class _float8_linear_fn(torch.autograd.Function):
                 dx = _native.gemm_kb_ex(g8, False, sg, w8, True, sw, dy.dtype).reshape(ctx.x_shape)
             if need_dw:  # grad_weight = dY^T @ x: both read transposed
                 dw = _native.gemm_kb_ex(g8, True, sg, x8, True, sx, dy.dtype)
-            return dx, dw, None, None, db
+            return dx, dw, None, None, None
         x8t, w8t, sx, sw = saved
         kb_dx, kb_dw = ctx.kb
         g8, g8t, sg = _cast_for_gemm(dy2, e5m2_dtype, dlg, ctx.is_amax_initialized, need_dx, need_dw, kb_dx, kb_dw)
@@ -224,7 +213,7 @@ class _float8_linear_fn(torch.autograd.Function):
                 dw = torch.ops.aten.mm_float8_emulated(g8t, sg, x8t.t(), sx, dy.dtype)
             else:
                 dw = _gemm(g8t, sg, x8t, sx, dy.dtype, kb_dw)
-        return dx, dw, None, None, db
+        return dx, dw, None, None, None
 
 
 class Float8Linear(torch.nn.Linear):
@@ -438,8 +427,11 @@ class Float8Linear(torch.nn.Linear):
         x = self._autocast_input(input)
         bias = self.bias
         inside = bias is not None and self._bias_inside(x, bias)
-        output = _float8_linear_fn.apply(x, self.weight, self, self.is_amax_initialized, bias if inside else None)
-        if bias is not None and not inside:
+        output = _float8_linear_fn.apply(x, self.weight, self, self.is_amax_initialized, (bias,) if inside else None)
+        if inside:
+            if bias.requires_grad and torch.is_grad_enabled():
+                output = _native.add_bias(output, bias, True)
+        elif bias is not None:
             output = output + bias.to(output.dtype)
         if self.has_any_delayed_scaling:
             self.float8_post_forward()
@@ -452,9 +444,11 @@ class Float8Linear(torch.nn.Linear):
                 and bias.dtype in _HP_DTYPES and not self.config.emulate and torch.autograd.forward_ad._current_level < 0)
 
     def _add_bias(self, output: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
-        """The addition outside the fused function; its gradient in the same order of sums where that function would take it."""
-        if not self._bias_inside(output, bias):
+        """The addition behind a product without a bias; its gradient in the same order of sums as behind one with it."""
+        if not (self._bias_inside(output, bias) and bias.requires_grad and torch.is_grad_enabled()):
             return output + bias.to(output.dtype)
+        if not torch.compiler.is_compiling():
+            return _native.add_bias(output, bias, False)
         from ._custom_ops import add_bias
 
         return add_bias(output, bias)

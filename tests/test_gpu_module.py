@@ -1022,3 +1022,57 @@ def test_outputs_may_be_changed_in_place(f8, monkeypatch, shape, bias, native):
 
     for inplace, other in ((torch.relu_, torch.relu), (lambda y: y.add_(r), lambda y: y + r)):
         assert all(torch.equal(p, q) for p, q in zip(step(inplace), step(other)))
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_gradient_of_the_bias_alone_leaves_the_product_alone(f8, monkeypatch, native):
+    """Asked for the gradient of the bias only, backward neither casts dY (which would fold its maximum into the delayed buffers) nor
+    frees what the product's gradients need; and it takes a batch of gradients, which the product's backward does not."""
+    from float8_experimental_amd import _native
+
+    if not native:
+        monkeypatch.setattr(_native, "linear_forward", lambda *a: None)
+    kind = f8.CastConfig(scaling_type=f8.ScalingType.DELAYED)
+    config = f8.Float8LinearConfig(cast_config_input=kind, cast_config_weight=kind, cast_config_grad_output=kind)
+    torch.manual_seed(0)
+    mod = f8.convert_to_float8_training(torch.nn.Sequential(torch.nn.Linear(1024, 512, device=DEV, dtype=torch.bfloat16)), config=config)
+    x = torch.randn(2, 256, 1024, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    dy = torch.randn(2, 256, 512, device=DEV, dtype=torch.bfloat16)
+    mod(x).backward(dy)
+    f8.sync_float8_amax_and_scale_history(mod)
+    w, b = mod[0].weight, mod[0].bias
+    y = mod(x)
+    before = [t.clone() for t in mod.buffers()]
+    (db,) = torch.autograd.grad(y, b, 4 * dy)
+    (dbs,) = torch.autograd.grad(y, b, torch.stack([dy, -dy]), is_grads_batched=True)
+    assert all(torch.equal(p, q) for p, q in zip(before, mod.buffers()))
+    dw, dx = torch.autograd.grad(y, (w, x), 2 * dy)
+    assert not all(torch.equal(p, q) for p, q in zip(before, mod.buffers()))
+    mod.zero_grad()
+    x.grad = None
+    f8.sync_float8_amax_and_scale_history(mod)
+    mod(x).backward(dy)
+    assert torch.equal(db, 4 * b.grad) and dw.shape == w.shape and dx.shape == x.shape
+    # torch's sum of a batch: 512 fp32 additions in another order, then the rounding to bf16
+    exact = dy.double().sum((0, 1))
+    bound = 512 * 2.0**-24 * dy.double().abs().sum((0, 1))
+    assert ((dbs.double() - torch.stack([exact, -exact])).abs() <= bound + (exact.abs() + bound) * 2.0**-8).all()
+
+
+@pytest.mark.parametrize("bias", [True, False])
+def test_backward_under_compiled_autograd(f8, bias):
+    torch.manual_seed(0)
+    mod = f8.convert_to_float8_training(torch.nn.Sequential(torch.nn.Linear(1024, 512, bias=bias, device=DEV, dtype=torch.bfloat16)))
+    x = torch.randn(2, 256, 1024, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    dy = torch.randn(2, 256, 512, device=DEV, dtype=torch.bfloat16)
+
+    def step():
+        mod.zero_grad()
+        x.grad = None
+        mod(x).backward(dy)
+        return [x.grad] + [p.grad for p in mod.parameters()]
+
+    want = step()
+    with torch._dynamo.compiled_autograd._enable(lambda gm: gm):
+        got = step()
+    assert all(torch.equal(p, q) for p, q in zip(got, want))
