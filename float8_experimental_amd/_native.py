@@ -340,7 +340,10 @@ def gemm_plan(m: int, n: int, k: int, aligned: bool = True, split_k: bool = True
 def _as_2d(x: torch.Tensor) -> Tuple[torch.Tensor, int, int, int]:
     """(tensor whose memory is read, rows, cols, row stride) -- copies only when the layout needs it.  A tensor
     expanded over all its leading dimensions (what autograd hands to backward after ``y.sum()``) is passed as ONE row
-    with row stride 0: the kernels read that row for every output row, nothing of rows x cols is materialised."""
+    with row stride 0: the kernels read that row for every output row, nothing of rows x cols is materialised.  A lazy
+    negation is carried out: its memory does not hold its values."""
+    if x.is_neg():
+        x = x.resolve_neg()
     if x.dim() == 2 and x.stride(1) == 1 and x.stride(0) >= x.shape[1] and x.shape[0] > 0 and x.shape[1] > 0:
         return x, x.shape[0], x.shape[1], x.stride(0)
     if x.dim() >= 2 and x.shape[-1] > 0 and x.numel() > x.shape[-1] and all(
@@ -352,6 +355,14 @@ def _as_2d(x: torch.Tensor) -> Tuple[torch.Tensor, int, int, int]:
     cols = x.shape[-1] if x.dim() > 0 else 1
     rows = x.numel() // cols if cols else 0
     return x, rows, cols, cols
+
+
+def _checked_bias(bias: Optional[torch.Tensor], n: int, dtype: torch.dtype, device: torch.device) -> Optional[torch.Tensor]:
+    """The bias of a product whose memory holds its values."""
+    if bias is None:
+        return None
+    assert bias.dtype == dtype and bias.numel() == n and bias.is_contiguous() and bias.device == device
+    return bias.resolve_neg()
 
 
 def amax_scale(x: torch.Tensor, float8_dtype: torch.dtype, math_dtype: Optional[torch.dtype] = None,
@@ -546,7 +557,8 @@ def column_sum(dy: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """The columns of ``dy`` [m, n] summed, rounded to its type, in ``dtype``: the gradient of a bias.  In the order of
     f8mi_column_sum, as ``add_bias`` has it, wherever its kernel reads ``dy`` as it is; else torch's sum."""
     m, n = dy.shape
-    if not (dy.is_cuda and dy.dtype in _DT and dtype in _DT and m > 0 and n > 0 and dy.stride(1) == 1 and dy.stride(0) >= n):
+    if not (dy.is_cuda and dy.dtype in _DT and dtype in _DT and m > 0 and n > 0 and dy.stride(1) == 1 and dy.stride(0) >= n
+            and not dy.is_neg()):
         return dy.sum(0).to(dtype)
     _check_device(dy.device)
     need = lib().f8mi_column_sum_workspace_bytes(m, n, _DT[dy.dtype])
@@ -682,8 +694,7 @@ def gemm_nt_kb(a_kb: torch.Tensor, a_scale: torch.Tensor, bt_kb: torch.Tensor, b
         out = torch.empty((m, n), dtype=out_dtype, device=a_kb.device)
     else:
         assert out.shape == (m, n) and out.dtype == out_dtype and out.is_contiguous()
-    if bias is not None:
-        assert bias.dtype == out_dtype and bias.numel() == n and bias.is_contiguous() and bias.device == a_kb.device
+    bias = _checked_bias(bias, n, out_dtype, a_kb.device)
     _check_device(a_kb.device)
     ws, ws_bytes = gemm_workspace(a_kb.device, m, k, n) if split_k else (None, 0)
     rc = lib().f8mi_gemm_nt_kb_ws(a_kb.data_ptr(), _F8[a_kb.dtype], bt_kb.data_ptr(), _F8[bt_kb.dtype], m, n, k,
@@ -709,8 +720,7 @@ def gemm_kb_ex(a_kb: torch.Tensor, a_transposed: bool, a_scale: torch.Tensor, bt
     for s in (a_scale, b_scale):
         assert s.dtype == torch.float32 and s.numel() == 1 and s.device == a_kb.device, "scales: 1 fp32 element on the operands' device"
     out = torch.empty((m, n), dtype=out_dtype, device=a_kb.device)
-    if bias is not None:
-        assert bias.dtype == out_dtype and bias.numel() == n and bias.is_contiguous() and bias.device == a_kb.device
+    bias = _checked_bias(bias, n, out_dtype, a_kb.device)
     _check_device(a_kb.device)
     rc = lib().f8mi_gemm_kb_ex(a_kb.data_ptr(), _F8[a_kb.dtype], int(a_transposed), bt_kb.data_ptr(), _F8[bt_kb.dtype],
                                int(b_transposed), m, n, k, a_scale.data_ptr(), b_scale.data_ptr(), out.data_ptr(),
@@ -750,8 +760,7 @@ def gemm_nt(a: torch.Tensor, a_scale: torch.Tensor, bt: torch.Tensor, b_scale: t
         out = torch.empty((m, n), dtype=out_dtype, device=a.device)
     else:
         assert out.shape == (m, n) and out.dtype == out_dtype and out.is_contiguous()
-    if bias is not None:
-        assert bias.dtype == out_dtype and bias.numel() == n and bias.is_contiguous() and bias.device == a.device
+    bias = _checked_bias(bias, n, out_dtype, a.device)
     _check_device(a.device)
     ws, ws_bytes = gemm_workspace(a.device, m, k, n) if split_k else (None, 0)
     rc = lib().f8mi_gemm_nt_ws(a.data_ptr(), _F8[a.dtype], lda, bt.data_ptr(), _F8[bt.dtype], ldb, m, n, k,
@@ -787,8 +796,7 @@ def scaled_mm(a: torch.Tensor, a_scale: torch.Tensor, b: torch.Tensor, b_scale: 
     if b_rowmajor and (a_rowmajor or a_colmajor) and m > 0 and n > 0 and k > 1 and n > 1 and (a_rowmajor or m > 1):
         for s in (a_scale, b_scale):
             assert s.dtype == torch.float32 and s.numel() == 1 and s.device == a.device, "scales: 1 fp32 element on the operands' device"
-        if bias is not None:
-            assert bias.dtype == out_dtype and bias.numel() == n and bias.is_contiguous() and bias.device == a.device
+        bias = _checked_bias(bias, n, out_dtype, a.device)
         _check_device(a.device)
         out = torch.empty((m, n), dtype=out_dtype, device=a.device)
         a_tr = not a_rowmajor

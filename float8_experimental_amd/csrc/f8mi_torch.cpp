@@ -68,11 +68,12 @@ std::vector<int64_t> copy_sizes(int64_t rows, int64_t kc, int layout) {
     return {padded(kc, layout) / 64, rows, 64};
 }
 
-// Undefined: not taken.  A plain tensor (or Parameter) on the current device: nothing of a subclass, no other layout ...
+// Undefined: not taken.  A plain tensor (or Parameter) on the current device: nothing of a subclass, no other layout, no lazy negation ...
 at::Tensor plain(PyObject* o, int device) {
     if (!THPVariable_CheckExact(o)) return {};
     const at::Tensor& t = THPVariable_Unpack(o);
-    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.get_device() == device ? t : at::Tensor();
+    constexpr c10::DispatchKeySet lazy({c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
+    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(lazy) && t.get_device() == device ? t : at::Tensor();
 }
 // ... that the cast kernels read as it is: 2-D, not empty, unit column stride
 at::Tensor matrix(PyObject* o, int device) {

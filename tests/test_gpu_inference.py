@@ -385,3 +385,20 @@ def test_few_row_linear_is_taken_where_its_workgroups_are_few(m, n, dtype, one_k
     launches = [nat.prof_read(kernel)[0] for kernel in (nat.K_CAST, nat.K_GEMM)]
     nat.prof_reset()
     assert launches == [0 if one_kernel else 1, 1]
+
+
+@pytest.mark.parametrize("m", [4, 64, 512])
+@pytest.mark.parametrize("which", ["x", "bias"])
+def test_lazy_negations_are_carried_out(m, which):
+    from float8_experimental_amd import inference
+
+    torch.manual_seed(0)
+    lin = torch.nn.Linear(1024, 512, device=DEV, dtype=torch.bfloat16).requires_grad_(False)
+    made = {"x": torch.randn(m, 1024, device=DEV, dtype=torch.bfloat16), "bias": lin.bias.detach().clone()}
+
+    def call(negate):
+        t = {name: negate(v) if name == which else v for name, v in made.items()}
+        lin.bias = torch.nn.Parameter(t["bias"], requires_grad=False)
+        return inference.Float8InferenceLinear.from_float(lin, inference.QuantConfig(inference.ActivationCasting.DYNAMIC), True)(t["x"])
+
+    assert torch.equal(call(torch._neg_view), call(torch.neg))

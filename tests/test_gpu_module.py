@@ -1076,3 +1076,26 @@ def test_backward_under_compiled_autograd(f8, bias):
     with torch._dynamo.compiled_autograd._enable(lambda gm: gm):
         got = step()
     assert all(torch.equal(p, q) for p, q in zip(got, want))
+
+
+@pytest.mark.parametrize("m,k,n", [(512, 1024, 512), (512, 520, 1000), (4, 512, 512)])
+@pytest.mark.parametrize("which", ["x", "weight", "bias", "dy"])
+def test_lazy_negations_are_carried_out(f8, m, k, n, which):
+    """A tensor whose negation is still to be done (``torch._neg_view``, the imaginary part of a conjugate) has other values than its
+    memory: the outputs and gradients of the tensor that holds them."""
+    torch.manual_seed(0)
+    made = {name: torch.randn(s, device=DEV, dtype=torch.bfloat16) for name, s in (("x", (m, k)), ("weight", (n, k)), ("bias", (n,)), ("dy", (m, n)))}
+
+    def step(negate, composed):
+        t = {name: negate(v) if name == which else v for name, v in made.items()}
+        lin = torch.nn.Linear(k, n, device=DEV, dtype=torch.bfloat16)
+        lin.weight, lin.bias = torch.nn.Parameter(t["weight"]), torch.nn.Parameter(t["bias"])
+        mod = f8.convert_to_float8_training(torch.nn.Sequential(lin))[0]
+        x = t["x"].detach().requires_grad_()
+        y = mod.forward_composed(x) if composed else mod(x)
+        y.backward(t["dy"])
+        return y.detach(), x.grad, mod.weight.grad, mod.bias.grad
+
+    assert torch.nn.Parameter(torch._neg_view(made[which])).is_neg()
+    for composed in (False, True):
+        assert all(torch.equal(p, q) for p, q in zip(step(torch._neg_view, composed), step(torch.neg, composed)))
