@@ -13,6 +13,8 @@ import threading
 from typing import Optional, Tuple
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # F8MI_LIB names another build of the library (same ABI) to load instead of the in-tree one: a switch for measurements
@@ -232,6 +234,18 @@ def _raw_stream(dev: torch.device) -> int:
 
 def _stream(t: torch.Tensor) -> int:
     return _raw_stream(t.device)
+
+
+def _function_mode_active() -> bool:
+    """True under a ``TorchFunctionMode`` that may want to see an operator; ``torch.set_default_device`` is one that does not."""
+    return any(not isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack())
+
+
+def operators_are_watched() -> bool:
+    """True where somebody has to see operators that a kernel would take along: a functional transform, a dispatch or function
+    mode, a trace."""
+    return (torch._C._len_torch_dispatch_stack() != 0 or torch._C._functorch.peek_interpreter_stack() is not None
+            or (torch._C._len_torch_function_stack() != 0 and _function_mode_active()) or torch.jit.is_tracing())
 
 
 _checked_devices = set()

@@ -15,8 +15,6 @@ from typing import Callable, Optional
 
 import torch
 import torch.nn as nn
-from torch.overrides import _get_current_function_mode_stack
-from torch.utils._device import DeviceContext
 
 from . import _custom_ops  # noqa: F401  (registers torch.ops.f8mi.*)
 from . import _native
@@ -142,11 +140,6 @@ def _inference_linear_traced(x2: torch.Tensor, weight: "Float8Tensor", static_sc
 WEIGHT_ONLY_MAX_ROWS = 128
 
 
-def _function_mode_active() -> bool:
-    """True under a ``TorchFunctionMode`` that may want to see ``F.linear``; ``torch.set_default_device`` is one that does not."""
-    return any(not isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack())
-
-
 def _weight_only_kernels_take(input: torch.Tensor, weight: "Float8Tensor") -> bool:
     """True if the weight-only kernels compute what ``F.linear(input, weight.to_original_precision())`` would: plain
     tensors of the weight's own type on the current device whose memory holds their values (not sparse, nested or a lazy
@@ -163,8 +156,7 @@ def _weight_only_kernels_take(input: torch.Tensor, weight: "Float8Tensor") -> bo
             and data.is_contiguous() and scale.dim() == 0 and scale.dtype == torch.float32
             and not (torch.is_grad_enabled() and (input.requires_grad or weight.requires_grad or data.requires_grad))
             and not torch.is_autocast_enabled() and torch.autograd.forward_ad._current_level < 0
-            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0
-            and not (torch._C._len_torch_function_stack() and _function_mode_active()) and not torch.jit.is_tracing())
+            and not _native.operators_are_watched())
 
 
 def _weight_only_linear(input: torch.Tensor, weight: "Float8Tensor") -> torch.Tensor:

@@ -1099,3 +1099,46 @@ def test_lazy_negations_are_carried_out(f8, m, k, n, which):
     assert torch.nn.Parameter(torch._neg_view(made[which])).is_neg()
     for composed in (False, True):
         assert all(torch.equal(p, q) for p, q in zip(step(torch._neg_view, composed), step(torch.neg, composed)))
+
+
+@pytest.mark.parametrize("composed", [False, True])
+def test_modes_and_traces_see_the_addition_of_the_bias(f8, composed):
+    """Under a dispatch or function mode or a trace the bias is added by an operator of its own, as are the columns of dY; with the
+    bits of the addition inside.  torch.set_default_device is a function mode that asks for nothing."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    seen = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    class Function(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    torch.manual_seed(0)
+    lin = f8.convert_to_float8_training(torch.nn.Sequential(torch.nn.Linear(1024, 512, device=DEV, dtype=torch.bfloat16)))[0]
+    forward = lin.forward_composed if composed else lin
+    x, dy = torch.randn(512, 1024, device=DEV, dtype=torch.bfloat16), torch.randn(512, 512, device=DEV, dtype=torch.bfloat16)
+    want = forward(x).detach()
+    with torch.device("cuda"):
+        assert lin._bias_inside(x, lin.bias)
+    with Dispatch():
+        assert torch.equal(forward(x).detach(), want)
+    assert torch.ops.aten.add.Tensor in seen
+    y = forward(x)
+    seen.clear()
+    with Dispatch():
+        torch.autograd.grad(y, lin.bias, dy)
+    assert torch.ops.aten.sum.dim_IntList in seen
+    seen.clear()
+    with Function():
+        assert torch.equal(forward(x).detach(), want)
+    assert torch.Tensor.add in seen or torch.Tensor.__add__ in seen
+    if not composed:  # Float8Tensor, a subclass, is not for the tracer
+        with torch.no_grad():
+            graph = torch.jit.trace(lin, x, check_trace=False).inlined_graph
+        assert "aten::add" in [node.kind() for node in graph.nodes()]
