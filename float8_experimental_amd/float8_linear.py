@@ -441,8 +441,8 @@ class Float8Linear(torch.nn.Linear):
         """True where the fused function takes the bias along: plain tensors on the GPU and nothing that would have to see the
         addition as an operation of its own (subclasses, modes, traces, forward-mode derivatives, which the function has none of)."""
         return (type(x) in _PLAIN and type(bias) in _PLAIN and x.is_cuda and bias.is_cuda and bias.shape == self.weight.shape[:1]
-                and bias.dtype in _HP_DTYPES and not bias.is_neg() and not self.config.emulate and torch.autograd.forward_ad._current_level < 0
-                and (torch.compiler.is_compiling() or not _native.operators_are_watched()))
+                and bias.dtype in _HP_DTYPES and not self.config.emulate and torch.autograd.forward_ad._current_level < 0
+                and (torch.compiler.is_compiling() or not (bias.is_neg() or _native.operators_are_watched())))
 
     def _add_bias(self, output: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
         """The addition behind a product without a bias; its gradient in the same order of sums as behind one with it."""
