@@ -795,8 +795,10 @@ constexpr int EXCHANGE_WORDS = 8192;
 static __device__ __align__(256) uint64_t exchange_words[EXCHANGE_STREAMS][EXCHANGE_WORDS];
 static std::atomic<uint64_t*> g_exchange_words[STATIC_MAX_DEVICES];
 static std::atomic<uintptr_t> g_exchange_streams[STATIC_MAX_DEVICES][EXCHANGE_STREAMS];
+static std::atomic<uint32_t> g_exchange_last[STATIC_MAX_DEVICES][EXCHANGE_STREAMS];  // tag of the set's last launch
 static std::atomic<uint32_t> g_exchange_given[STATIC_MAX_DEVICES];
 static std::atomic<uint32_t> g_exchange_tag{0};
+constexpr uint32_t EXCHANGE_LATELY = 64;  // launches
 
 static int exchange_set(int dev, hipStream_t stream) {
     static thread_local char own;  // one handle stands for every thread's own stream
@@ -809,7 +811,8 @@ static int exchange_set(int dev, hipStream_t stream) {
 }
 
 // Words and a tag for one launch on `stream`; words null: none to be had.  An error code if the runtime reports one.
-static int begin_exchange(hipStream_t stream, uint32_t wait_ticks, TaggedWords& e) {
+// streams: how many streams of the device, this one among them, had one of the last EXCHANGE_LATELY launches.
+static int begin_exchange(hipStream_t stream, uint32_t wait_ticks, TaggedWords& e, int* streams = nullptr) {
     e = TaggedWords{nullptr, 0, wait_ticks};
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {  // of the default stream, say, while a blocking one is captured: launches are taken
@@ -821,9 +824,18 @@ static int begin_exchange(hipStream_t stream, uint32_t wait_ticks, TaggedWords& 
     if (check_hip(hipGetDevice(&dev), "hipGetDevice")) return F8MI_ERR_HIP;
     uint64_t* base = device_array(HIP_SYMBOL(exchange_words), g_exchange_words, "exchange_words");
     if (!base) return F8MI_ERR_HIP;
-    e.words = base + (size_t)exchange_set(dev, stream) * EXCHANGE_WORDS;
+    const int set = exchange_set(dev, stream);
+    e.words = base + (size_t)set * EXCHANGE_WORDS;
     e.tag = g_exchange_tag.fetch_add(1, std::memory_order_relaxed) + 1;
     if (!e.tag) e.tag = g_exchange_tag.fetch_add(1, std::memory_order_relaxed) + 1;  // 0 is what the words start with
+    g_exchange_last[dev][set].store(e.tag, std::memory_order_relaxed);
+    if (streams) {
+        *streams = 0;
+        for (const auto& last : g_exchange_last[dev]) {
+            const uint32_t tag = last.load(std::memory_order_relaxed);
+            *streams += tag && e.tag - tag < EXCHANGE_LATELY;  // (another thread's may be newer: not counted)
+        }
+    }
     return F8MI_OK;
 }
 
@@ -1173,23 +1185,31 @@ static int launch_cast_pair(int dt_a, int dt_b, int tile_rows, hipStream_t strea
 }
 
 
-// Rows of the tiles that both get in one launch, 0: not in one.  Two 16-bit tensors may have half as many tiles again as one tensor: in two
+// Rows of the tiles that both get in one launch, 0: not in one.  Two 16-bit tensors may have half as many tiles again as one tensor (`large`): in two
 // launches each of them waits for its own words, together once.  us, two launches / one: 2048 x 4096 with 3072 x 4096 (1280 tiles) 25.9 /
 // 21.0, with 4096 x 4096 (1536) 29.1 / 24.1, both copies 33.1 / 26.7; 3000 x 3000 with 3100 x 3000, both copies 30.0 / 22.3; 1024 x 4096 with 5120 x 4096
-// (two launches, one of them for the maxima) 26.0 / 24.3.  Six workgroups of eight leave other kernels a quarter of the chip.  Two such pairs on streams of
-// their own at the same time: 23.7 / 23.0 a pair, but three: 24 / 47 (some wait for the others' places).  fp32 has room for five.
-static int pair_tile_rows(const f8mi_cast_job& a, const f8mi_cast_job& b) {
+// (two launches, one of them for the maxima) 26.0 / 24.3.  Six workgroups of eight leave other kernels a quarter of the chip.  Seven (1792 tiles) are
+// faster alone and slower beside each other: 3072 x 4096 with 4096 x 4096 32.1 / 29.2, on two streams at once 27.2 / 31.8; 1024 x 4096 with
+// 6144 x 4096 29.9 / 29.2 and 25.0 / 73.6.  fp32 has room for five.
+static int pair_tile_rows(const f8mi_cast_job& a, const f8mi_cast_job& b, bool* large) {
     const int64_t tiles = tiles_of(a) + tiles_of(b);
+    *large = false;
     if (const int rows = resident_tile_rows(tiles * CAST_TILE, CAST_TILE)) return rows;
-    return b.in_dtype != F8MI_FP32 && tiles <= std::min(RESIDENT_PAIR_TILES, 6 * cu_count()) ? CAST_TILE : 0;
+    *large = b.in_dtype != F8MI_FP32 && tiles <= std::min(RESIDENT_PAIR_TILES, 6 * cu_count());
+    return *large ? CAST_TILE : 0;
 }
+// Streams whose large pairs may be there at once.  us a pair of 2048 x 4096 with 4096 x 4096, two launches / one: on two streams 23.7 / 22.4, on
+// three 23.4 / 45.8, both copies 28.4 / 56.1 (some hold the places that others wait for).
+constexpr int LARGE_PAIR_STREAMS = 2;
 // Both casts in the launch that exchanges maxima.  F8MI_ERR_UNSUPPORTED, and nothing queued: not in one.
-static int cast_dynamic_pair_one_launch(const f8mi_cast_job& a, const f8mi_cast_job& b, uint32_t wait_ticks, hipStream_t stream) {
-    const int tile_rows = pair_tile_rows(a, b);
+static int cast_dynamic_pair_one_launch(const f8mi_cast_job& a, const f8mi_cast_job& b, uint32_t wait_ticks, hipStream_t stream, int large_pair_streams) {
+    bool large;
+    const int tile_rows = pair_tile_rows(a, b, &large);
     if (!tile_rows) return F8MI_ERR_UNSUPPORTED;
     TaggedWords tagged;
-    if (const int rc = begin_exchange(stream, wait_ticks, tagged)) return rc;
-    if (!tagged.words) return F8MI_ERR_UNSUPPORTED;
+    int streams = 0;
+    if (const int rc = begin_exchange(stream, wait_ticks, tagged, &streams)) return rc;
+    if (!tagged.words || (large && streams > large_pair_streams)) return F8MI_ERR_UNSUPPORTED;
     CastJob ja = kernel_job(a, tile_rows), jb = kernel_job(b, tile_rows);
     ja.scale_out = a.scale_dev;
     jb.scale_out = b.scale_dev;
@@ -1220,7 +1240,7 @@ extern "C" int f8mi_cast_one_launch(const f8mi_cast_job* a, const f8mi_cast_job*
     hipStream_t stream = (hipStream_t)stream_;
     if (!a || !pair_ok(*a, b ? *b : *a) || (delayed && (!a->amax_dev || (b && !b->amax_dev)))) { set_error("f8mi_cast_one_launch: bad job"); return F8MI_ERR_INVALID_ARG; }
     int rc;
-    if (b) rc = delayed ? cast_delayed_pair_one_launch(*a, *b, wait_ticks, stream) : cast_dynamic_pair_one_launch(*a, *b, wait_ticks, stream);
+    if (b) rc = delayed ? cast_delayed_pair_one_launch(*a, *b, wait_ticks, stream) : cast_dynamic_pair_one_launch(*a, *b, wait_ticks, stream, EXCHANGE_STREAMS);
     else if (delayed) rc = cast_delayed_one_launch(a->x, a->rows, a->cols, a->ld, a->in_dtype, a->scale_dev, F8MI_E4M3FN, a->out, a->out_layout, a->out_t, a->out_t_layout, a->amax_dev, wait_ticks, stream);
     else return f8mi_cast_dynamic_resident(a->x, a->rows, a->cols, a->ld, a->in_dtype, F8MI_E4M3FN, a->scale_dev, a->out, a->out_layout, a->out_t, a->out_t_layout, wait_ticks, stream_);
     if (rc == F8MI_ERR_UNSUPPORTED) set_error("f8mi_cast_one_launch: more tiles than one launch takes, or a stream that is being captured");
@@ -1231,7 +1251,7 @@ extern "C" int f8mi_cast_dynamic_pair(const f8mi_cast_job* a, const f8mi_cast_jo
     hipStream_t stream = (hipStream_t)stream_;
     if (!a || !b) { set_error("f8mi_cast_dynamic_pair: null job"); return F8MI_ERR_INVALID_ARG; }
     if (workspace && (uintptr_t)workspace % 16 == 0 && pair_ok(*a, *b)) {
-        const int one = cast_dynamic_pair_one_launch(*a, *b, EXCHANGE_WAIT_TICKS, stream);
+        const int one = cast_dynamic_pair_one_launch(*a, *b, EXCHANGE_WAIT_TICKS, stream, LARGE_PAIR_STREAMS);
         if (one != F8MI_ERR_UNSUPPORTED) return one;
         // one of them too large for a launch of its own: both through the two launches it takes
         if (two_launches_pay(*a, *b) && a->ld && b->ld &&

@@ -851,6 +851,48 @@ def test_cast_of_two_tensors_of_up_to_six_tiles_a_cu(nat, dts, shapes):
     test_cast_of_two_tensors_equals_two_casts(nat, dts, shapes)
 
 
+def test_large_pairs_are_one_launch_on_two_streams_and_two_on_three(nat):
+    """Three launches that fill three quarters of the chip each hold the places that the others' workgroups wait for.  A stream counts while
+    it had one of the last 64 such launches."""
+    xs = [heavy(s, torch.bfloat16, 90 + i).to(DEV) for i, s in enumerate([(2048, 4096), (4096, 4096), (64, 128), (64, 128)])]
+    outs, scales = [torch.zeros(x.shape, device=DEV, dtype=torch.uint8) for x in xs], torch.zeros(len(xs), device=DEV)
+    jobs = [CastJob(x.data_ptr(), *x.shape, x.stride(0), scales[i:].data_ptr(), outs[i].data_ptr(), None, None, nat._DT[x.dtype], 0, 0) for i, x in enumerate(xs)]
+    want = [nat.cast(x, nat.amax_scale(x, torch.float8_e4m3fn)[1], torch.float8_e4m3fn)[0] for x in xs]
+    streams, ws = [torch.cuda.Stream() for _ in range(3)], [torch.empty_like(nat.workspace(xs[0].device)) for _ in range(3)]
+    torch.cuda.synchronize()
+
+    def casts(first, i):
+        assert nat.lib().f8mi_cast_dynamic_pair(ctypes.byref(jobs[first]), ctypes.byref(jobs[first + 1]), ws[i].data_ptr(), streams[i].cuda_stream) == 0
+
+    def launches(i):
+        nat.prof_reset()
+        nat.prof_enable(True)
+        try:
+            casts(0, i)
+        finally:
+            nat.prof_enable(False)
+        torch.cuda.synchronize()
+        count = nat.prof_read(nat.K_CAST)[0]
+        nat.prof_reset()
+        for o, w in zip(outs[:2], want):
+            assert torch.equal(o, w.view(torch.uint8))
+            o.zero_()
+        torch.cuda.synchronize()
+        return count
+
+    for _ in range(64):
+        casts(2, 0)
+    torch.cuda.synchronize()
+    assert launches(0) == 1
+    casts(2, 1)
+    assert launches(0) == 1 and launches(1) == 1
+    casts(2, 2)
+    assert [launches(i) for i in range(3)] == [2, 2, 2]
+    for _ in range(64):
+        casts(2, 0)
+    assert launches(0) == 1
+
+
 def _rand_fp8(shape, tdt, seed, scale=1.0):
     g = torch.Generator().manual_seed(seed)
     v = torch.randn(shape, generator=g) * scale
