@@ -35,7 +35,6 @@ struct Lib {
     decltype(&f8mi_gemm_nt_ws) gemm_nt_ws;
     decltype(&f8mi_gemm_nt_kb_ws) gemm_nt_kb_ws;
     decltype(&f8mi_gemm_kb_ex) gemm_kb_ex;
-    // null in a library without them: two products one by one, a bias by torch
     decltype(&f8mi_gemm_pair) gemm_pair;
     decltype(&f8mi_gemm_kb_bias) gemm_kb_bias;
     decltype(&f8mi_column_sum) column_sum;
@@ -203,7 +202,7 @@ struct Call {
     at::Tensor gemm_biased(const at::Tensor& a, const at::Tensor& sa, const at::Tensor& bt, const at::Tensor& sb, int layout, int64_t m, int64_t n,
                            int64_t kc, at::ScalarType out, const at::Tensor& bias) const {
         const int64_t k = padded(kc, layout);
-        if (layout != F8MI_LAYOUT_ROWMAJOR && L.gemm_kb_bias && (bias.scalar_type() == out || bias.scalar_type() == at::kFloat)) {
+        if (layout != F8MI_LAYOUT_ROWMAJOR && (bias.scalar_type() == out || bias.scalar_type() == at::kFloat)) {
             const at::Tensor c = make({m, n}, out);
             const int rc = L.gemm_kb_bias(a.data_ptr(), bt.data_ptr(), m, n, k, (const float*)sa.data_ptr(), (const float*)sb.data_ptr(), c.data_ptr(),
                                           dtype_code(out), n, bias.data_ptr(), dtype_code(bias.scalar_type()), F8MI_GEMM_WORKSPACE_BYTES, stream);
@@ -345,7 +344,7 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         const auto compute = [&] {
             if (one_copy) {
                 c.cast(dy, go, F8MI_E5M2, true, F8MI_LAYOUT_KBLOCK64, false, 0, g8, g8t, sg);
-                if (need_dx && need_dw && L.gemm_pair) {
+                if (need_dx && need_dw) {
                     c.gemm_two({g8, sg, ws, sw, false, true, F8MI_LAYOUT_KBLOCK64, m, k, n, dx}, {g8, sg, xs, sx, true, true, F8MI_LAYOUT_KBLOCK64, n, k, m, dw}, dy.scalar_type(), wide);
                     return;
                 }
@@ -353,7 +352,7 @@ PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
                 if (need_dw) dw = c.gemm_tr(g8, true, sg, xs, sx, n, k, m, dy.scalar_type());
             } else {
                 c.cast(dy, go, F8MI_E5M2, need_dx, kb_dx, need_dw, kb_dw, g8, g8t, sg);
-                if (need_dx && need_dw && kb_dx != F8MI_LAYOUT_ROWMAJOR && kb_dw != F8MI_LAYOUT_ROWMAJOR && L.gemm_pair) {
+                if (need_dx && need_dw && kb_dx != F8MI_LAYOUT_ROWMAJOR && kb_dw != F8MI_LAYOUT_ROWMAJOR) {
                     c.gemm_two({g8, sg, ws, sw, false, false, kb_dx, m, k, n, dx}, {g8t, sg, xs, sx, false, false, kb_dw, n, k, m, dw}, dy.scalar_type(), wide);
                     return;
                 }
@@ -380,7 +379,7 @@ bool memory_holds_values(const at::Tensor& t) {
 // The gradient of a bias: the columns of dy summed in fp32, rounded to dy's type, in the type of the bias.
 at::Tensor bias_gradient(const at::Tensor& dy, at::ScalarType type) {
     const at::Tensor d = dy.reshape({-1, dy.size(-1)});
-    if (!L.column_sum || !L.column_sum_workspace_bytes || at::GradMode::is_enabled() || !memory_holds_values(d) || dtype_code(d.scalar_type()) < 0 || d.numel() == 0 || d.stride(1) != 1 || d.stride(0) < d.size(1))
+    if (at::GradMode::is_enabled() || !memory_holds_values(d) || dtype_code(d.scalar_type()) < 0 || d.numel() == 0 || d.stride(1) != 1 || d.stride(0) < d.size(1))
         return d.sum(0).to(type);  // with create_graph a sum that has a gradient itself
     const c10::DeviceGuard guard(d.device());
     const int64_t rows = d.size(0), cols = d.size(1);
@@ -499,11 +498,10 @@ PyObject* load(PyObject*, PyObject* args) {
     get(L.gemm_plan, "f8mi_gemm_plan");
     get(L.cast_dynamic_pair, "f8mi_cast_dynamic_pair");
     get(L.cast_delayed_pair, "f8mi_cast_delayed_pair");
-    const auto get_if_there = [&](auto& f, const char* name) { f = reinterpret_cast<std::decay_t<decltype(f)>>(dlsym(h, name)); };
-    get_if_there(L.gemm_pair, "f8mi_gemm_pair");
-    get_if_there(L.gemm_kb_bias, "f8mi_gemm_kb_bias");
-    get_if_there(L.column_sum, "f8mi_column_sum");
-    get_if_there(L.column_sum_workspace_bytes, "f8mi_column_sum_workspace_bytes");
+    get(L.gemm_pair, "f8mi_gemm_pair");
+    get(L.gemm_kb_bias, "f8mi_gemm_kb_bias");
+    get(L.column_sum, "f8mi_column_sum");
+    get(L.column_sum_workspace_bytes, "f8mi_column_sum_workspace_bytes");
     if (missing) {
         L.gemm_plan = nullptr;
         return PyErr_Format(PyExc_ImportError, "%s does not export %s", path, missing);

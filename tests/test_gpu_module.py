@@ -871,6 +871,10 @@ int f8mi_cast_delayed_pair(void) { return slow(); }
 int f8mi_gemm_nt_ws(void) { return slow(); }
 int f8mi_gemm_nt_kb_ws(void) { return slow(); }
 int f8mi_gemm_kb_ex(void) { return slow(); }
+int f8mi_gemm_pair(void) { return slow(); }
+int f8mi_gemm_kb_bias(void) { return slow(); }
+int64_t f8mi_column_sum_workspace_bytes(int64_t rows, int64_t cols, int dtype) { return 0; }
+int f8mi_column_sum(void) { return slow(); }
 int f8mi_linear_few_rows(void) { return slow(); }
 """
 
