@@ -611,7 +611,10 @@ static int gemm_job(const f8mi_gemm_job& j, void* stream) {
 // step's time per 128 of k (more where all CUs run them), a launch 2.25 us by itself, and 256 workgroups run at a time, those
 // of the longer tiles first.  Fitted to 425 pairs of products of 384 - 16384 tokens and 512 - 28672 features, both kinds of operands, timed as two
 // launches and in each of the nine pairs of tiles: with the choice they are 1.19 times as fast as two launches (always the best: 1.21; the
-// same tiles on both sides only: 1.15), and slower by more than 2 % in fourteen cases (8 % in the worst: 6656 tokens, 1920 -> 5504).
+// same tiles on both sides only: 1.15).  One launch has to be estimated at less than PAIR_MARGIN of two, as the estimates are not better than
+// that: of 1000 other pairs for which it is at less than 0.96, those that were slower by more than 2 % as chosen, the slowest, and how many times as
+// fast all of them were, with 0.96: 9, 8 %, 1.259; 0.94: 4, 6 % (384 tokens, 7040 -> 13696), 1.255; 0.90: 2, 6 %, 1.240.
+constexpr double PAIR_MARGIN = 0.94;
 struct PairTiles { int rows, cols; double us, step_us, crowded; };
 constexpr PairTiles PAIR_TILES[4] = {{}, {128, 128, 2.05, 0.447, 1.13}, {128, 256, 3.48, 0.636, 1.12}, {256, 256, 6.34, 1.06, 1.09}};
 constexpr double PAIR_LAUNCH_US = 2.25;
@@ -661,7 +664,7 @@ static int pair_tiles(const f8mi_gemm_job& a, const f8mi_gemm_job& b) {
     if (tiles_of(PAIR_TILES[F8MI_PAIR_TILES256], a.m, a.n) + tiles_of(PAIR_TILES[F8MI_PAIR_TILES256], b.m, b.n) > 16 * PAIR_WORKGROUPS) return F8MI_PAIR_BY_SIZE;
     const double us_a = single_us(a), us_b = single_us(b);
     if (us_a == 0.0 || us_b == 0.0) return F8MI_PAIR_BY_SIZE;
-    double best_us = 0.96 * (us_a + us_b);  // the estimates are not better than that
+    double best_us = PAIR_MARGIN * (us_a + us_b);
     int best = F8MI_PAIR_BY_SIZE;
     for (int ka = F8MI_PAIR_TILES128; ka <= F8MI_PAIR_TILES256; ka++) {
         if (ka != F8MI_PAIR_TILES256 && tiles_of(PAIR_TILES[ka], a.m, a.n) > 4 * PAIR_WORKGROUPS) continue;

@@ -1125,6 +1125,64 @@ def test_gemm_pair_equals_the_products_one_by_one(nat, tokens, k, n, out_dt):
         assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), 15, nat._stream(g)) == nat.ERR_UNSUPPORTED
 
 
+# Results in the columns of a wider matrix: rows at even and odd pitches and addresses, the same and different ones for the two products (which one
+# launch takes only from operands read transposed); the columns beside them are left alone.
+@pytest.mark.parametrize("tokens,k,n", [(385, 391, 413), (512, 1024, 1024), (1408, 512, 640)])
+@pytest.mark.parametrize("wider,at", [((3, 0), (0, 0)), ((1, 1), (1, 0)), ((2, 1), (0, 1)), ((2, 2), (1, 1)), ((2, 4), (0, 1))])
+@pytest.mark.parametrize("out_dt", [torch.bfloat16, torch.float32])
+def test_gemm_pair_writes_into_wider_matrices(nat, tokens, k, n, wider, at, out_dt):
+    g, w, x = (_rand_fp8(s, t, sum(s), 4.0).to(DEV) for s, t in (((tokens, n), torch.float8_e5m2), ((n, k), torch.float8_e4m3fn), ((tokens, k), torch.float8_e4m3fn)))
+    sg, sw, sx = (torch.tensor(s, device=DEV) for s in (2.0, 0.25, 0.5))
+    turned = lambda t: t.view(torch.uint8).t().contiguous().view(t.dtype)
+    pad = lambda v: -(-v // 128) * 128
+    forms = [(0, [_to_kb_padded(t)[0] for t in (g, turned(w), turned(g), turned(x))])]
+    if tokens % 128 == 0 and k % 128 == 0 and n % 128 == 0:
+        forms.append((1, [_to_kb(g), _to_kb(w), _to_kb(g), _to_kb(x)]))
+    for tr, (a0, b0, a1, b1) in forms:
+        if tr:
+            want = [nat.gemm_kb_ex(a0, False, sg, b0, True, sw, out_dt), nat.gemm_kb_ex(a1, True, sg, b1, True, sx, out_dt)]
+        else:
+            want = [nat.gemm_nt_kb(a0, sg, b0, sw, out_dt, split_k=False), nat.gemm_nt_kb(a1, sg, b1, sx, out_dt, split_k=False)]
+        jobs = (GemmJob * 2)()
+        memory = [torch.empty(c.shape[0] * (c.shape[1] + more) + at_, device=DEV, dtype=out_dt) for c, more, at_ in zip(want, wider, at)]
+        rows_of = lambda i: memory[i][at[i]:].view(want[i].shape[0], -1)
+        for i, (job, a, b, sb, (rows, cols, kc), a_tr) in enumerate(zip(jobs, (a0, a1), (b0, b1), (sw, sx), ((tokens, k, pad(n)), (n, k, pad(tokens))), (0, tr))):
+            job.a, job.bt, job.a_fmt, job.b_fmt, job.a_tr, job.b_tr = a.data_ptr(), b.data_ptr(), nat.E5M2, nat.E4M3FN, a_tr, tr
+            job.m, job.n, job.k, job.sa, job.sb, job.c, job.ldc, job.dtype = rows, cols, kc, sg.data_ptr(), sb.data_ptr(), rows_of(i).data_ptr(), cols + wider[i], nat._DT[out_dt]
+        odd = [out_dt is not torch.float32 and bool(job.ldc % 2 or job.c % 4) for job in jobs]
+        for tiles in (0, 1 | 1 << 2, 2 | 2 << 2, 3 | 3 << 2):
+            for t in memory:
+                t.fill_(7.0)
+            rc = nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), tiles, nat._stream(g))
+            if tiles and not tr and odd[0] != odd[1]:
+                assert rc == nat.ERR_UNSUPPORTED
+                continue
+            assert rc == 0, nat.lib().f8mi_last_error()
+            for i, c in enumerate(want):
+                assert torch.equal(rows_of(i)[:, :c.shape[1]], c) and (rows_of(i)[:, c.shape[1]:] == 7.0).all() and (memory[i][:at[i]] == 7.0).all(), (tr, tiles, i)
+
+
+# By the rule, one launch where the estimate for it is clearly the lower one, two where it is within the estimates' error (measured slower: by 8 and
+# 7 %) or higher.
+@pytest.mark.parametrize("tokens,k,n,launches", [(512, 1024, 1024, 1), (2048, 4096, 4096, 1), (640, 18048, 5248, 2), (6656, 2048, 3584, 2), (4096, 4096, 4096, 2)])
+def test_gemm_pair_is_one_launch_where_the_estimate_is_clear(nat, tokens, k, n, launches):
+    g, w, x = (torch.zeros(a * b, device=DEV, dtype=torch.uint8) for a, b in ((tokens, n), (n, k), (tokens, k)))
+    got, one = [torch.ones(a, k, device=DEV, dtype=torch.bfloat16) for a in (tokens, n)], torch.ones((), device=DEV)
+    jobs = (GemmJob * 2)()
+    for job, b, (rows, cols, kc), c, a_tr in zip(jobs, (w, x), ((tokens, k, n), (n, k, tokens)), got, (0, 1)):
+        job.a, job.bt, job.a_fmt, job.b_fmt, job.a_tr, job.b_tr = g.data_ptr(), b.data_ptr(), nat.E5M2, nat.E4M3FN, a_tr, 1
+        job.m, job.n, job.k, job.sa, job.sb, job.c, job.ldc, job.dtype = rows, cols, kc, one.data_ptr(), one.data_ptr(), c.data_ptr(), cols, nat._DT[torch.bfloat16]
+    nat.prof_reset()
+    nat.prof_enable(True)
+    try:
+        assert nat.lib().f8mi_gemm_pair(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), 0, nat._stream(g)) == 0, nat.lib().f8mi_last_error()
+    finally:
+        nat.prof_enable(False)
+    count = nat.prof_read(nat.K_GEMM)[0]
+    nat.prof_reset()
+    assert count == launches and not any(t.any() for t in got)
+
+
 # grad_weight's 16-bit result stored in fp32, beside grad_input in one launch on each of the tiles and by itself (a first product that one launch
 # does not take): 128 x 128, 128 x 256, 256 x 256 with and without a sparse last round, 256 x 224; odd and even step counts, odd rows of grad_input.
 @pytest.mark.parametrize("tokens,k,n", [(384, 1024, 512), (512, 4096, 2048), (384, 4096, 4096), (512, 4096, 4352), (384, 14336, 2048), (512, 513, 700),
@@ -1186,6 +1244,13 @@ def test_gemm_adds_a_bias_to_the_rounded_product(nat, m, n, k, plan, out_dt, bia
     assert call(nat._DT[bias_dt]) == 0, nat.lib().f8mi_last_error()
     want = nat.gemm_nt_kb(ka, sa, kbt, sb, out_dt) + bias.to(out_dt)
     assert torch.equal(c, want)
+    for more, at in ((1, 0), (2, 1), (3, 1)):  # into a wider matrix: rows at other pitches and addresses, which other tiles may take
+        memory = torch.full((m * (n + more) + at,), 7.0, device=DEV, dtype=out_dt)
+        rows = memory[at:].view(m, n + more)
+        rc = nat.lib().f8mi_gemm_kb_bias(ka.data_ptr(), kbt.data_ptr(), m, n, k, sa.data_ptr(), sb.data_ptr(), rows.data_ptr(), nat._DT[out_dt], n + more,
+                                         bias.data_ptr(), nat._DT[bias_dt], nat.GEMM_WORKSPACE_BYTES, nat._stream(a))
+        assert rc == 0, nat.lib().f8mi_last_error()
+        assert torch.equal(rows[:, :n], want) and (rows[:, n:] == 7.0).all() and (memory[:at] == 7.0).all()
 
 
 # One row and one workgroup's rows with one more or less; columns that leave a lane some of its eight or four; several chunks; rows at any
