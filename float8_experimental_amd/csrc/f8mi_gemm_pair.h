@@ -2,11 +2,12 @@
 //
 // One after the other, each product fills the chip and drains it again, and the workgroups of its last round leave the rest of the CUs idle.
 // In one launch the tiles of the second start where those of the first end, those of the longer contraction first.  Both products have the
-// same work, so a product of few tiles that each take long runs beside one of many that do not.  us, one after the other / together (tokens,
-// in -> out features; tiles): 512, 1024 -> 1024: 12.3 / 7.1 (128 x 128); 384, 2048 -> 5120: 27.3 / 18.0 (128 x 128); 1664, 3328 -> 2560: 40.3 /
-// 31.7 (128 x 256); 2048, 4096 -> 4096: 60.5 / 56.7 (256 x 256); 3584, 2816 -> 11648: 196.7 / 166.9; 2981, 2989 -> 8117: 158 / 125; 4096, 4096
-// -> 4096, one full round each: 101.3 / 99.4; 8192, 4096 -> 14336: 617 / 630, where the rule in f8mi_gemm.hip stays with two.  Tiles of the
-// first and of the second product, two of one kind / of their own: 7040, 2560 -> 512: 36.4 / 24.6; 512, 6400 -> 15232: 145.6 / 128.8; 1209, 1408 -> 6144: 29.5 / 23.6.
+// same work, so a product of few tiles that each take long runs beside one of many that do not.  us back to back, one after the other / together (tokens,
+// in -> out features; tiles): 512, 1024 -> 1024: 12.4 / 7.2 (128 x 128); 384, 2048 -> 5120: 28.4 / 18.7 (128 x 128 and 256 x 256); 1664, 3328 -> 2560:
+// 41.0 / 30.1 (256 x 256); 2048, 4096 -> 4096: 55.8 / 51.8 (256 x 256); 3584, 2816 -> 11648: 187 / 164; 2981, 2989 -> 8117: 141 / 117; where the rule in
+// f8mi_gemm.hip stays with two: 4096, 4096 -> 4096, one full round each: 93.7 / 94.1; 8192, 4096 -> 14336: 616 / 619.  Tiles of the
+// first and of the second product, the best two of one kind / of their own as chosen: 7040, 2560 -> 512: 32.4 / 28.8; 8192, 4096 -> 1024: 66.4 / 62.7; 1209, 1408 ->
+// 6144: 29.5 / 23.5.  Few tokens in wide layers gain little: 512, 6400 -> 15232: 150 / 149, though 135 with 128 x 128 beside 256 x 256, which the estimate does not see.
 // The tiles are the ones that a product by itself runs on (f8mi_gemm_dma16_impl.h, f8mi_gemm_mid_impl.h): the same bits.
 #pragma once
 #include "f8mi_gemm_util.h"

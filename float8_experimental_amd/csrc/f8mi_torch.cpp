@@ -316,7 +316,8 @@ PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 
 // linear_backward(dy [m, n], saved of x, saved of weight, scale of x, scale of weight, k, one_copy, kb_dx, kb_dw, need_dx, need_dw,
 //                 delayed_dy, delayed_workspace, device, stream, fp32 weight = False) -> (grad of x [m, k], grad of weight [n, k]) or None.
-//                 The gradient of an fp32 weight comes in fp32 where a kernel stores it so, with the values of dy's type; else in that type.
+//                 The gradient of an fp32 weight comes in fp32 where a kernel stores it so (both gradients wanted, products on tiles), with the
+//                 values of dy's type; else in that type.
 PyObject* linear_backward(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     if (!expect(n_args, 15, "linear_backward", 1)) return nullptr;
     return guarded([&]() -> PyObject* {
