@@ -844,11 +844,39 @@ def test_cast_of_two_tensors_equals_two_casts(nat, dts, shapes):
                     assert torch.equal(a, wa) or (torch.isnan(a).all() and torch.isnan(wa).all())
 
 
-# 16-bit pairs past what one tensor may have: ragged, the most tiles one launch takes together (1536) and a row more.
+# 16-bit pairs past what one tensor may have: ragged, one with more tiles than that by itself, the most tiles one launch takes together (1536) and a
+# row more.  After 64 launches on this stream no other one counts.
 @pytest.mark.parametrize("dts", ["bf16 bf16", "fp16 fp16", "bf16 fp32"])
-@pytest.mark.parametrize("shapes", [((3000, 3000), (3100, 3001)), ((2048, 4096), (4096, 4096)), ((2049, 4096), (4096, 4096))])
+@pytest.mark.parametrize("shapes", [((3000, 3000), (3100, 3001)), ((100, 100), (6000, 4090)), ((6000, 4090), (100, 100)), ((2048, 4096), (4096, 4096)),
+                                    ((2049, 4096), (4096, 4096))])
 def test_cast_of_two_tensors_of_up_to_six_tiles_a_cu(nat, dts, shapes):
+    x, out, scale = torch.ones(64, 128, device=DEV, dtype=torch.bfloat16), torch.zeros(64, 128, device=DEV, dtype=torch.uint8), torch.zeros((), device=DEV)
+    job = CastJob(x.data_ptr(), 64, 128, 128, scale.data_ptr(), out.data_ptr(), None, None, nat._DT[x.dtype], 0, 0)
+    for _ in range(64):
+        assert nat.lib().f8mi_cast_one_launch(ctypes.byref(job), ctypes.byref(job), 0, 6000, nat._stream(x)) == 0
     test_cast_of_two_tensors_equals_two_casts(nat, dts, shapes)
+
+
+# The same where nobody waits for anybody: more words than one tensor by itself may have, most of them missing.
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("shapes", [((3000, 3000), (3100, 3001)), ((100, 100), (6000, 4090)), ((6000, 4090), (100, 100)), ((2048, 4096), (4096, 4096))])
+def test_large_pairs_that_do_not_wait(nat, dt, shapes):
+    f8dt = torch.float8_e4m3fn
+    base = [heavy(s, TORCH_DT[dt], 70 + i).to(DEV) for i, s in enumerate(shapes)]
+    special = [x.clone() for x in base]
+    special[0].view(-1)[-1], special[1].view(-1)[0] = float("nan"), float("-inf")
+    for xs in (base, special):
+        jobs, got, want = (CastJob * 2)(), [], []
+        for x, job in zip(xs, jobs):
+            scale = nat.amax_scale(x, f8dt, want_amax=False)[1]
+            want.append((*nat.cast(x, scale, f8dt, want_out_t=True, out_kblock=nat.KBLOCK_PAD, out_t_kblock=nat.KBLOCK_PAD), scale))
+            got.append((*(torch.zeros_like(t.view(torch.uint8)) for t in want[-1][:2]), torch.zeros((), device=DEV)))
+            job.x, job.rows, job.cols, job.ld, job.dtype, job.layout, job.layout_t = x.data_ptr(), *x.shape, x.stride(0), nat._DT[x.dtype], nat.KBLOCK_PAD, nat.KBLOCK_PAD
+            job.out, job.out_t, job.scale = (t.data_ptr() for t in got[-1])
+        assert nat.lib().f8mi_cast_one_launch(ctypes.byref(jobs[0]), ctypes.byref(jobs[1]), 0, 0, nat._stream(xs[0])) == 0, nat.lib().f8mi_last_error()
+        for (q, qt, s), (wq, wqt, ws) in zip(got, want):
+            assert same_bytes_mod_nan_sign(fp8_bytes(q), fp8_bytes(wq)) and same_bytes_mod_nan_sign(fp8_bytes(qt), fp8_bytes(wqt))
+            assert torch.equal(s, ws) or (torch.isnan(s).all() and torch.isnan(ws).all())
 
 
 def test_large_pairs_are_one_launch_on_two_streams_and_two_on_three(nat):
