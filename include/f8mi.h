@@ -258,7 +258,7 @@ typedef struct f8mi_cast_job {
 } f8mi_cast_job;
 
 /* f8mi_cast_dynamic of `a`, then of `b`, both to e4m3: the same bits, in one launch where the chip holds both (at most 1024 tiles
- * together, 1536 of 16-bit types), in two instead of three or four where one is larger than that.  Everything else is the two calls. */
+ * together, 1536 of 16-bit types while at most two streams make such casts), in two instead of three or four where one is larger than that.  Everything else is the two calls. */
 int f8mi_cast_dynamic_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream);
 /* f8mi_cast_delayed of `a`, then of `b`, both to e4m3, in one launch up to 2048 tiles together. */
 int f8mi_cast_delayed_pair(const f8mi_cast_job* a, const f8mi_cast_job* b, void* workspace, void* stream);
